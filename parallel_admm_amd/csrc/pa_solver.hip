@@ -511,25 +511,19 @@ __global__ void k_vertex_p(int n, float hinv, int have_contacts, const double* _
     st3(p, i, pi);
 }
 
-// The friction-cone projection of contact c with barycentric weights b and
-// its vertices' p values p0..p3 (formula of ADMMImplCPU::_project_one_contact,
-// admm_impl_cpu.cpp:411-448), with the contact's friction coefficient from
-// K.w: r_c += du unless keep, and Gamma_k du into entry slot sl.k of each
-// dynamic vertex k.
-__device__ __forceinline__ void contact_du_core(int c, float4 b, float3 p0, float3 p1, float3 p2, float3 p3, bool keep,
-                                                const float4* __restrict__ nrm, const float4* __restrict__ K, float4* __restrict__ rc,
-                                                const float4* __restrict__ G, int4 sl, float4* __restrict__ gdu) {
+// The friction-cone projection of one contact with barycentric weights b, its
+// vertices' p values p0..p3, normal n4, K (the friction coefficient in K.w)
+// and dual r4 (formula of ADMMImplCPU::_project_one_contact,
+// admm_impl_cpu.cpp:411-448): returns du, the change of r_c.
+__device__ __forceinline__ float3 contact_du_core(float4 b, float3 p0, float3 p1, float3 p2, float3 p3, float4 n4, float4 kk, float4 r4) {
     float3 u = f3(0.f, 0.f, 0.f);
     u = u + b.x * p0;
     u = u + b.y * p1;
     u = u + b.z * p2;
     u = u + b.w * p3;
-    float4 kk = K[c];
     u = u + f3(kk.x, kk.y, kk.z);
     const float mu = kk.w;
-    float4 r4 = rc[c];
     float3 r = f3(r4.x, r4.y, r4.z);
-    float4 n4 = nrm[c];
     float3 nn = f3(n4.x, n4.y, n4.z);
     float3 us = u - r;
     float uN = dot3(nn, us);
@@ -542,23 +536,7 @@ __device__ __forceinline__ void contact_du_core(int c, float4 b, float3 p0, floa
         else uT = (1.f - alpha / tau) * uT;
     }
     float3 unew = uN * nn + uT;
-    float3 d = unew - u;
-    if (!keep) rc[c] = make_float4(r.x + d.x, r.y + d.y, r.z + d.z, 0.f);
-    // Gamma_k du goes straight into the entry slot of vertex k (dynamic
-    // vertices only), so the per-vertex gather reads contiguous entries
-    const float4 g = G[c];
-    const float gk[4] = {g.x, g.y, g.z, g.w};
-    const int sk[4] = {sl.x, sl.y, sl.z, sl.w};
-#pragma unroll
-    for (int k = 0; k < 4; k++)
-        if (sk[k] >= 0) gdu[sk[k]] = make_float4(gk[k] * d.x, gk[k] * d.y, gk[k] * d.z, 0.f);
-}
-
-// The projection of contact c (vertices v, weights b) on the current p.
-__device__ __forceinline__ void contact_du_one(int c, int4 v, float4 b, bool keep, const float4* __restrict__ nrm,
-                                               const float4* __restrict__ K, const float* __restrict__ p, float4* __restrict__ rc,
-                                               const float4* __restrict__ G, const int4* __restrict__ slot, float4* __restrict__ gdu) {
-    contact_du_core(c, b, ld3(p, v.x), ld3(p, v.y), ld3(p, v.z), ld3(p, v.w), keep, nrm, K, rc, G, slot[c], gdu);
+    return unew - u;
 }
 
 // One Jacobi sweep of the friction-cone projection, one lane per contact.
@@ -569,7 +547,19 @@ __global__ void k_contact_du(int nc, const int4* __restrict__ cv, const float4* 
     int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= nc) return;
     const bool keep = stop && stop[0]; // the iteration runs past the stop: r_c stays
-    contact_du_one(c, cv[c], bary[c], keep, nrm, K, p, rc, G, slot, gdu);
+    const int4 v = cv[c];
+    const float4 r = rc[c];
+    const float3 d = contact_du_core(bary[c], ld3(p, v.x), ld3(p, v.y), ld3(p, v.z), ld3(p, v.w), nrm[c], K[c], r);
+    if (!keep) rc[c] = make_float4(r.x + d.x, r.y + d.y, r.z + d.z, 0.f);
+    // Gamma_k du goes straight into the entry slot of vertex k (dynamic
+    // vertices only), so the per-vertex gather reads contiguous entries
+    const float4 g = G[c];
+    const int4 sl = slot[c];
+    const float gk[4] = {g.x, g.y, g.z, g.w};
+    const int sk[4] = {sl.x, sl.y, sl.z, sl.w};
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        if (sk[k] >= 0) gdu[sk[k]] = make_float4(gk[k] * d.x, gk[k] * d.y, gk[k] * d.z, 0.f);
 }
 
 // slot[c].k = position of (contact c, vertex k) in the sorted vertex entry
@@ -606,80 +596,207 @@ __global__ void k_vertex_gather(int ne_max, int n, float* __restrict__ p, const 
 }
 
 // Every Jacobi sweep of one contact projection in a single 1024-lane
-// workgroup, for contact sets of at most 1024 NPT contacts: per sweep the
-// update of k_contact_du and the gather of k_vertex_gather, with the same
-// arithmetic in the same order (bit-identical results), separated by
-// workgroup barriers instead of kernel boundaries.  A sweep is about two
-// dependent memory rounds:
-// - lane t owns contacts t + 1024 k (k < NPT), whose vertex ids and weights it
-//   keeps in registers, so their p loads issue at once; r_c is only ever read
-//   by the lane that wrote it;
-// - lane t owns entries [EPT t, EPT t + EPT) of the sorted vertex entry list
-//   (at most 4 per contact); it keeps their run-start vertices in registers, loads
-//   the entries' Gamma du and the p of every vertex whose run starts there at
-//   once, then sums each such run in entry order (a run that goes past the
-//   lane's entries continues from memory) and writes p.
+// workgroup, for contact sets of at most 1024 NPT contacts: the Gamma r_c term
+// of k_vertex_p, then per sweep the update of k_contact_du and the gather of
+// k_vertex_gather, with the same arithmetic in the same order (bit-identical
+// results), separated by workgroup barriers instead of kernel boundaries.
+// A projection is a chain of 2 sweeps dependent rounds on one CU, so what
+// bounds it is a round's latency and instruction count.  What a round
+// exchanges lives in LDS (through L2 a sweep took 4-7 us), what only its lane
+// reads in registers:
+// - lane t owns contacts t + 1024 k (k < NPT): weights, normal, K, Gamma, r_c
+//   and the p of its static vertices;
+// - a vertex's entries are one run of the sorted entry list; lane t owns runs
+//   t + 1024 j and adds each one's entries, in order, to its vertex's p.  A
+//   run is read eight entries at a time before they are added (the cap of a
+//   draped cloth has runs of 30 and more, and a read per add was 2 us a
+//   sweep);
+// - buf holds one float4 per entry (Gamma_k du), then the p of each run.  Runs
+//   that no longer fit behind the entries (only possible with over 1024
+//   contacts, most of whose vertices are distinct) keep p in global memory.
+// Ten sweeps (gs_max_iter 10), everything through L2 before: a side-16 cloth
+// draped over its sphere 36.6 -> 17.1 us, cloth256 landing (about 600
+// contacts) 38-48 -> 27.8 us, a side-95 cloth 47 -> 24 us (up to 1024
+// contacts) and 68 -> 36 us (above).
+constexpr int CONTACT_WG_SLOTS = 10000;
 template <int NPT>
 __global__ void __launch_bounds__(1024) k_contact_sweeps_wg(int nc, int n, int sweeps, const int4* __restrict__ cv,
                                                             const float4* __restrict__ bary, const float4* __restrict__ nrm,
-                                                            const float4* __restrict__ K, float* __restrict__ p, float4* __restrict__ rc,
+                                                            const float4* __restrict__ K, float* p, float4* __restrict__ rc,
                                                             const float4* __restrict__ G, const int4* __restrict__ slot,
-                                                            float4* __restrict__ gdu, const uint32_t* __restrict__ vptr,
-                                                            const int2* __restrict__ erun, const int32_t* __restrict__ stop) {
-    constexpr int EPT = 4 * NPT;
-    const int t = threadIdx.x;
-    const bool keep = stop && stop[0];
+                                                            const uint32_t* __restrict__ vptr, const int2* __restrict__ erun,
+                                                            const int32_t* __restrict__ stop) {
+    constexpr int EPT = 4 * NPT, NE = 1024 * EPT, SLOTS = NPT == 1 ? 2 * NE : CONTACT_WG_SLOTS;
+    constexpr unsigned NONE = 0xffffu;
+    __shared__ float4 buf[SLOTS];
+    __shared__ int wsum[16];
+    uint16_t* const map = reinterpret_cast<uint16_t*>(buf); // set-up: run number of a run-start entry,
+    uint16_t* const first = map + NE;                       // and a run's first entry
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const bool keep = stop && stop[0]; // the iteration runs past the stop: r_c stays
     const int ne = (int)vptr[n];
-    int4 cvr[NPT];
-    float4 br[NPT];
+    const int e0 = EPT * t;
+
+    // contacts of this lane: what every sweep reads, once
+    int4 v[NPT], sl[NPT];
+    float4 b[NPT], n4[NPT], kk[NPT], g4[NPT], r4[NPT];
 #pragma unroll
     for (int k = 0; k < NPT; k++) {
         const int c = t + 1024 * k;
-        cvr[k] = c < nc ? cv[c] : make_int4(0, 0, 0, 0);
-        br[k] = c < nc ? bary[c] : make_float4(0.f, 0.f, 0.f, 0.f);
+        const bool on = c < nc;
+        v[k] = on ? cv[c] : make_int4(0, 0, 0, 0);
+        sl[k] = on ? slot[c] : make_int4(-1, -1, -1, -1);
+        b[k] = on ? bary[c] : make_float4(0.f, 0.f, 0.f, 0.f);
+        n4[k] = on ? nrm[c] : make_float4(0.f, 0.f, 0.f, 0.f);
+        kk[k] = on ? K[c] : make_float4(0.f, 0.f, 0.f, 0.f);
+        g4[k] = on ? G[c] : make_float4(0.f, 0.f, 0.f, 0.f);
+        r4[k] = on ? rc[c] : make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    const int e0 = EPT * t;
-    int rv[EPT]; // vertex whose run starts at the entry, else -1
+    // number the runs: an exclusive scan of the run starts among each lane's EPT entries
+    unsigned starts = 0;
 #pragma unroll
-    for (int j = 0; j < EPT; j++) rv[j] = e0 + j < ne ? erun[e0 + j].x : -1;
+    for (int j = 0; j < EPT; j++)
+        if (e0 + j < ne && erun[e0 + j].x >= 0) starts |= 1u << j;
+    int inc = __popc(starts);
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += y;
+    }
+    if (lane == 63) wsum[wave] = inc;
+    __syncthreads();
+    int rbase = inc - __popc(starts), nrun = 0;
+    for (int w = 0; w < 16; w++) {
+        if (w < wave) rbase += wsum[w];
+        nrun += wsum[w];
+    }
+#pragma unroll
+    for (int j = 0; j < EPT; j++)
+        if (starts >> j & 1) {
+            const int r = rbase + __popc(starts & ((1u << j) - 1));
+            map[e0 + j] = (uint16_t)r;
+            first[r] = (uint16_t)(e0 + j);
+        }
+    __syncthreads();
+    const int pcap = SLOTS - ne; // runs whose p fits behind the entries
+    // per contact vertex: its run and its entry (dynamic, two packed per
+    // register) or its p (static)
+    unsigned run[NPT][2], ent[NPT][2];
+    float3 ps[NPT][4];
+#pragma unroll
+    for (int k = 0; k < NPT; k++) {
+        const int vk[4] = {v[k].x, v[k].y, v[k].z, v[k].w}, sk[4] = {sl[k].x, sl[k].y, sl[k].z, sl[k].w};
+        unsigned rk[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            rk[q] = sk[q] >= 0 ? (unsigned)map[vptr[vk[q]]] : NONE;
+            ps[k][q] = t + 1024 * k < nc && sk[q] < 0 ? ld3(p, vk[q]) : f3(0.f, 0.f, 0.f);
+        }
+        run[k][0] = rk[0] | rk[1] << 16;
+        run[k][1] = rk[2] | rk[3] << 16;
+        ent[k][0] = ((unsigned)sk[0] & NONE) | (unsigned)sk[1] << 16;
+        ent[k][1] = ((unsigned)sk[2] & NONE) | (unsigned)sk[3] << 16;
+    }
+    auto half = [](const unsigned(&w)[2], int q) { return q & 1 ? w[q >> 1] >> 16 : w[q >> 1] & 0xffffu; };
+    // this lane's runs: entries [se & 0xffff, se >> 16), empty where it has none
+    unsigned se[EPT];
+#pragma unroll
+    for (int j = 0; j < EPT; j++) {
+        const int r = t + 1024 * j;
+        se[j] = r < nrun ? (unsigned)first[r] | (unsigned)(r + 1 < nrun ? first[r + 1] : ne) << 16 : 0u;
+    }
+    __syncthreads();
+    // entries hold (r_c, Gamma_k): p += Gamma r_c (k_vertex_p has written the rest of p)
+#pragma unroll
+    for (int k = 0; k < NPT; k++) {
+        const float gk[4] = {g4[k].x, g4[k].y, g4[k].z, g4[k].w};
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const unsigned e = half(ent[k], q);
+            if (e != NONE) buf[e] = make_float4(r4[k].x, r4[k].y, r4[k].z, gk[q]);
+        }
+    }
+    __syncthreads();
+    // s = the run's entries folded in order by add, eight read at a time
+    auto sum_run = [&](unsigned w, auto add) {
+        float3 s = f3(0.f, 0.f, 0.f);
+        const int end = (int)(w >> 16);
+        for (int e = (int)(w & 0xffffu); e < end; e += 8) {
+            float4 g[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) g[u] = buf[e + u]; // past the run's end: other entries or p, dropped below
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const float3 a = add(s, g[u]);
+                if (e + u < end) s = a;
+            }
+        }
+        return s;
+    };
+#pragma unroll
+    for (int j = 0; j < EPT; j++) {
+        const int r = t + 1024 * j;
+        if (r >= nrun) break;
+        const int vtx = erun[se[j] & 0xffffu].x;
+        const float3 s = sum_run(se[j], [](float3 s, float4 g) { return s + g.w * f3(g.x, g.y, g.z); });
+        const float3 pv = ld3(p, vtx) + s;
+        if (r < pcap) buf[ne + r] = make_float4(pv.x, pv.y, pv.z, 0.f);
+        else st3(p, vtx, pv);
+    }
+    __syncthreads();
     for (int sw = 0; sw < sweeps; sw++) {
 #pragma unroll
-        for (int k = 0; k < NPT; k++) {
-            const int c = t + 1024 * k;
-            if (c < nc) contact_du_one(c, cvr[k], br[k], keep, nrm, K, p, rc, G, slot, gdu);
-        }
+        for (int k = 0; k < NPT; k++)
+            if (t + 1024 * k < nc) {
+                float3 pv[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int r = (int)half(run[k], q);
+                    const float4 w = buf[ne + (r < pcap ? r : 0)];
+                    pv[q] = f3(w.x, w.y, w.z);
+                    if (r == (int)NONE) {
+                        pv[q] = ps[k][q];
+                    } else if (NPT > 1 && r >= pcap) {
+                        const int4 vv = cv[t + 1024 * k];
+                        pv[q] = ld3(p, q == 0 ? vv.x : q == 1 ? vv.y : q == 2 ? vv.z : vv.w);
+                    }
+                }
+                const float3 d = contact_du_core(b[k], pv[0], pv[1], pv[2], pv[3], n4[k], kk[k], r4[k]);
+                r4[k] = make_float4(r4[k].x + d.x, r4[k].y + d.y, r4[k].z + d.z, 0.f);
+                const float gk[4] = {g4[k].x, g4[k].y, g4[k].z, g4[k].w};
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const unsigned e = half(ent[k], q);
+                    if (e != NONE) buf[e] = make_float4(gk[q] * d.x, gk[q] * d.y, gk[q] * d.z, 0.f);
+                }
+            }
         __syncthreads();
-        float3 g[EPT], pv[EPT];
 #pragma unroll
         for (int j = 0; j < EPT; j++) {
-            const float4 gj = e0 + j < ne ? gdu[e0 + j] : make_float4(0.f, 0.f, 0.f, 0.f);
-            g[j] = f3(gj.x, gj.y, gj.z);
-            pv[j] = rv[j] >= 0 ? ld3(p, rv[j]) : f3(0.f, 0.f, 0.f);
-        }
-        // runs are contiguous and cover every entry below ne: an entry that
-        // starts no run belongs to the open one
-        int cur = -1;
-        float3 sum = f3(0.f, 0.f, 0.f), pc = f3(0.f, 0.f, 0.f);
-#pragma unroll
-        for (int j = 0; j < EPT; j++) {
-            if (rv[j] >= 0) {
-                if (cur >= 0) st3(p, cur, pc + sum);
-                cur = rv[j];
-                sum = f3(0.f, 0.f, 0.f);
-                pc = pv[j];
+            const int r = t + 1024 * j;
+            if (r >= nrun) break;
+            const float3 s = sum_run(se[j], [](float3 s, float4 g) { return s + f3(g.x, g.y, g.z); });
+            if (NPT == 1 || r < pcap) {
+                const float4 w = buf[ne + r];
+                buf[ne + r] = make_float4(w.x + s.x, w.y + s.y, w.z + s.z, 0.f);
+            } else {
+                const int vtx = erun[se[j] & 0xffffu].x;
+                st3(p, vtx, ld3(p, vtx) + s);
             }
-            if (cur >= 0 && e0 + j < ne) sum = sum + g[j];
-        }
-        if (cur >= 0) {
-            const int end = (int)vptr[cur + 1];
-            for (int q = e0 + EPT; q < end; q++) {
-                const float4 gq = gdu[q];
-                sum = sum + f3(gq.x, gq.y, gq.z);
-            }
-            st3(p, cur, pc + sum);
         }
         __syncthreads();
     }
+#pragma unroll
+    for (int j = 0; j < EPT; j++) {
+        const int r = t + 1024 * j;
+        if (r < nrun && r < pcap) {
+            const float4 w = buf[ne + r];
+            st3(p, erun[se[j] & 0xffffu].x, f3(w.x, w.y, w.z));
+        }
+    }
+    if (!keep)
+#pragma unroll
+        for (int k = 0; k < NPT; k++)
+            if (t + 1024 * k < nc) rc[t + 1024 * k] = r4[k];
 }
 
 // ---------------------------------------------------------------------------
@@ -2832,18 +2949,18 @@ void Backend::contact_setup(float eps, float gamma_, float hinv) {
 
 void Backend::contact_project(bool) {
     const float hinv = (float)(1.0 / cfg.dt);
-    hipLaunchKernelGGL(k_vertex_p, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, n, hinv, nc > 0 ? 1 : 0, x.p, x0.p, Uc.p, p.p, vptr.p,
-                       vent.p, gam.p, rc.p);
+    const bool wg = nc > 0 && nc <= contact_wg_max; // the whole projection in one workgroup: no launch per sweep
+    hipLaunchKernelGGL(k_vertex_p, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, n, hinv, nc > 0 && !wg ? 1 : 0, x.p, x0.p, Uc.p, p.p,
+                       vptr.p, vent.p, gam.p, rc.p);
     PA_LAUNCH_CHECK();
-    if (nc == 0) return;
-    if (nc <= contact_wg_max) { // every sweep in one workgroup: no launch per sweep
-        if (cfg.gs_max_iter > 0)
-            hipLaunchKernelGGL((nc <= 1024 ? k_contact_sweeps_wg<1> : k_contact_sweeps_wg<2>), dim3(1), dim3(1024), 0, stream, nc, n,
-                               cfg.gs_max_iter, det->c.v.p, det->c.bary.p, det->c.nrm.p, kc.p, p.p, rc.p, (const float4*)gam.p,
-                               (const int4*)cslot.p, gdu.p, (const uint32_t*)vptr.p, (const int2*)erun.p, (const int32_t*)stop_guard);
+    if (wg) {
+        hipLaunchKernelGGL((nc <= 1024 ? k_contact_sweeps_wg<1> : k_contact_sweeps_wg<2>), dim3(1), dim3(1024), 0, stream, nc, n,
+                           cfg.gs_max_iter, det->c.v.p, det->c.bary.p, det->c.nrm.p, kc.p, p.p, rc.p, (const float4*)gam.p,
+                           (const int4*)cslot.p, (const uint32_t*)vptr.p, (const int2*)erun.p, (const int32_t*)stop_guard);
         PA_LAUNCH_CHECK();
         return;
     }
+    if (nc == 0) return;
     for (int g = 0; g < cfg.gs_max_iter; g++) contact_sweep_once();
 }
 

@@ -450,6 +450,38 @@ def test_contact_sweeps_in_one_workgroup_match_per_sweep_launches(pa, tol):
             np.testing.assert_array_equal(a, c)
 
 
+@pytest.mark.parametrize("pairs", [1, 1024, 1025, 1500, 2048])
+def test_contact_sweeps_in_one_workgroup_with_distinct_vertices(pa, pairs):
+    """Isolated triangle pairs, one vertex of the upper triangle over the lower
+    one: one contact of four distinct vertices per pair, so the entry and run
+    counts are the largest the contact count allows, on both sides of the
+    one-contact-per-lane limit and past the runs whose p fits in LDS.  The
+    one-workgroup sweeps give the same bits as the per-sweep launches."""
+    from parallel_admm_amd.configs import config_for
+
+    cfg = config_for("cloth32")
+    d = cfg.thickness
+    lower = np.array([[0, 0, 0], [0.01, 0, 0], [0, 0, 0.01]])
+    upper = np.array([[0.0033, 0.5 * d, 0.0033], [0.0063, 0.01, 0.0033], [0.0033, 0.01, 0.0063]])
+    cell = np.concatenate([lower, upper])
+    k = np.arange(pairs)
+    shift = 0.05 * np.stack([k % 40, np.zeros(pairs), k // 40], axis=1)
+    x = (cell[None] + shift[:, None]).reshape(-1, 3)
+    tris = np.arange(6 * pairs).reshape(-1, 3)
+    sc = pa.Scene.from_mesh(x, len(x), np.full(len(x), 1.0), tris=tris, tri_k=np.full(len(tris), 1e3))
+    v = np.random.default_rng(5).normal(size=x.shape) * 1e-3  # moves a vertex by 0.02 mm a step: every pair stays within d
+    out = []
+    for wg in (2048, 0):
+        b = pa.ADMMBackendHIP.from_scene(sc, cfg)
+        b.set_contact_sweep_wg(wg)
+        b.set_state(v=v)
+        st = b.step()
+        assert st["n_contacts_max"] == pairs
+        out.append((*b.get_state(), *b.get_duals()))
+    for a, c in zip(*out):
+        np.testing.assert_array_equal(a, c)
+
+
 def test_step_overflow_rolls_back(pa):
     from parallel_admm_amd.configs import config_for
 
