@@ -155,7 +155,9 @@ struct Backend {
     DBuf<float4> gam, kc, rc;
     DBuf<int32_t> cslot;  // per contact: entry slot of each of its 4 vertices (-1: static)
     DBuf<float4> gdu;     // per vertex entry: Gamma_k du of the last sweep
-    DBuf<uint32_t> vcnt, vptr, vfill, vent;
+    DBuf<uint32_t> vcnt, vptr, vent; // contacts per vertex; entries per dynamic vertex (offsets, sorted entries 4 c + k)
+    DBuf<int4> vloc;                 // per contact: its place among each vertex's contacts, any order
+    DBuf<uint32_t> vraw;             // entries in their runs, unsorted
     DBuf<int2> erun;      // per vertex entry: (vertex, end of its entries) on its first entry, else (-1, 0)
     int contact_wg_max = CONTACT_WG_MAX; // contact sets up to this size sweep in one workgroup
     PrimScratch scratch;
@@ -255,7 +257,7 @@ struct Backend {
 
     // sub-phases (also used by step)
     void local_step(bool first_iter, hipStream_t s = nullptr);
-    void contact_setup(float eps, float gamma, float hinv);
+    void contact_setup(float eps, float gamma, float hinv, bool counted = false);
     void contact_project(bool first_iter);
     void contact_sweep_once();
     void rhs(bool want_residual, bool first_iter);

@@ -39,6 +39,15 @@ struct ContactBuffers {
     DBuf<double> dist;
 };
 
+// Per-vertex contact counts wanted by the caller of Detector::detect: cnt[v]
+// (n entries, cleared by the detection) counts the contacts of vertex v, and
+// loc[c] holds, for each vertex of contact c, its place among them (any order).
+struct VertexCount {
+    uint32_t* cnt = nullptr;
+    int4* loc = nullptr;
+    int64_t n = 0;
+};
+
 struct Detector {
     hipStream_t stream = nullptr;     // stream work is issued on (the backend's once attached)
     hipStream_t own_stream = nullptr; // created here when none was given; destroyed here
@@ -50,10 +59,18 @@ struct Detector {
     Tree ft, et;
     ContactBuffers c;   // canonical list
     ContactBuffers stg; // staging list in discovery order (single traversal)
-    DBuf<int32_t> st_seg; // segment of each staged contact
-    DBuf<uint32_t> qcount, qoffset; // nv + ne segment counts / offsets (PT per query vertex, EE per smaller edge id)
-    DBuf<uint32_t> qfill;           // nv + ne: slots taken per segment by the scatter
-    DBuf<uint32_t> total;           // [0] contacts found (segment counts), [1] stack overflow flag, [2] staged contacts
+    DBuf<int2> st_seg;      // per staged contact: its segment and its place in the segment's unsorted order
+    DBuf<int32_t> seg_key;  // partner ids in segment order, unsorted inside a segment
+    // one buffer, cleared by one launch per detection: total[0] contacts found
+    // (segment counts), [1] stack overflow flags, [2] staged contacts;
+    // ovf_count[0..1]; qcount: nv + ne segment counts (PT per query vertex, EE
+    // per smaller edge id)
+    DBuf<uint32_t> counts;
+    uint32_t* total = nullptr;
+    uint32_t* ovf_count = nullptr;
+    uint32_t* qcount = nullptr;
+    DBuf<uint32_t> qoffset;       // nv + ne segment offsets
+    uint32_t* total_host = nullptr; // pinned: total[0..2] after the scan
     // Leaf hits of the collect pass: per query a slab of up to 32 sorted leaf
     // indices (strided by the query count) and the number of hits; hits past
     // the slab as (query, leaf) pairs in an overflow list of one entry per
@@ -61,7 +78,6 @@ struct Detector {
     DBuf<int32_t> cand_pt, cand_ee;
     DBuf<uint32_t> ccount_pt, ccount_ee;
     DBuf<int2> ovf_pt, ovf_ee;
-    DBuf<uint32_t> ovf_count;
     int64_t single_pass_fallbacks = 0; // detections that reran as a single pass (short stack or overflow list too small)
     bool force_single_pass = false;    // every detection runs the single pass
     PrimScratch scratch;
@@ -91,7 +107,8 @@ struct Detector {
     // work queued on this->stream has run (the last kernels are queued after
     // the host reads the count).  Sets found_total and throws PA_ERR_OVERFLOW
     // (list unspecified) if more than `cap` contacts were found.
-    int detect(const double* x, bool refit = false);
+    // With vc, also counts the contacts of every vertex.
+    int detect(const double* x, bool refit = false, VertexCount vc = VertexCount());
     // Enables segmented mode: vseg (n_all host ints) in [0, nseg), nseg <= 2048.
     void set_segments(const int32_t* vseg_host, int nseg);
     void set_stream(hipStream_t s) { stream = s; }

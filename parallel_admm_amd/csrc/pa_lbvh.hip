@@ -13,9 +13,9 @@
 // Point-triangle: one lane per surface vertex; its pairs form the vertex's
 // segment.  Edge-edge: one lane per sorted leaf k, visiting only leaves after
 // k, so each unordered pair is tested once; the pair belongs to the segment of
-// its smaller edge id.  Segment counts -> exclusive scan -> scatter of the
-// staged pairs into their segments -> per-segment sort by partner id: the list
-// comes out in canonical order, bit-identical on every run, with no global sort.
+// its smaller edge id.  Segment counts -> exclusive scan -> partner ids into
+// their segments -> every pair to its rank in its segment: the list comes out
+// in canonical order, bit-identical on every run, with no global sort.
 //
 // Segmented mode (merged scenes): keys carry the scene id above a 21-bit
 // Morton code, so every scene is one subtree and queries start at their own
@@ -426,35 +426,6 @@ __device__ inline void write_contact(const QueryOut& o, int idx, int type, int p
     o.dist[idx] = dist;
 }
 
-// Insertion sort of one query's segment by partner id (prim1).
-__device__ inline void sort_segment(const QueryOut& o, int begin, int end) {
-    for (int a = begin + 1; a < end; a++) {
-        int32_t key = o.prim1[a];
-        int32_t t0 = o.type[a], p0 = o.prim0[a];
-        int4 vv = o.v[a];
-        float4 bb = o.bary[a], nn = o.nrm[a];
-        double dd = o.dist[a];
-        int b = a - 1;
-        while (b >= begin && o.prim1[b] > key) {
-            o.type[b + 1] = o.type[b];
-            o.prim0[b + 1] = o.prim0[b];
-            o.prim1[b + 1] = o.prim1[b];
-            o.v[b + 1] = o.v[b];
-            o.bary[b + 1] = o.bary[b];
-            o.nrm[b + 1] = o.nrm[b];
-            o.dist[b + 1] = o.dist[b];
-            b--;
-        }
-        o.type[b + 1] = t0;
-        o.prim0[b + 1] = p0;
-        o.prim1[b + 1] = key;
-        o.v[b + 1] = vv;
-        o.bary[b + 1] = bb;
-        o.nrm[b + 1] = nn;
-        o.dist[b + 1] = dd;
-    }
-}
-
 // Slot in the staging list for every lane of the wave that reaches this call
 // together (one atomic per wave and call site; lanes that diverged away are
 // not counted).
@@ -554,7 +525,7 @@ inline int test_rows(int nq) { return std::max(1, std::min(CAND, (1 << 22) / std
 // against the triangle at sorted leaf lf; an accepted pair goes to the
 // staging list and qcount[q] counts it.
 __device__ inline void pt_candidate(int q, int v, dv3 p, int lf, const double2* __restrict__ leafd, int n_dyn, double dhat,
-                                    uint32_t* __restrict__ qcount, const QueryOut& st, int32_t* __restrict__ st_seg,
+                                    uint32_t* __restrict__ qcount, const QueryOut& st, int2* __restrict__ st_seg,
                                     uint32_t* __restrict__ counter) {
     const double2* L = leafd + (size_t)leaf_stride<3>() * lf;
     const double2 u0 = L[0], u1 = L[1], u2 = L[2], u3 = L[3], u4 = L[4];
@@ -564,11 +535,11 @@ __device__ inline void pt_candidate(int q, int v, dv3 p, int lf, const double2* 
     const dv3 t0 = dmk(u0.x, u0.y, u1.x), t1 = dmk(u1.y, u2.x, u2.y), t2 = dmk(u3.x, u3.y, u4.x);
     const PTOut r = point_triangle(p, t0, t1, t2);
     if (!pt_accept(r, dhat)) return;
-    atomicAdd(&qcount[q], 1u);
+    const uint32_t place = atomicAdd(&qcount[q], 1u);
     const int idx = stage_slot(counter);
     if (idx < st.cap) {
         write_contact(st, idx, 0, v, f, make_int4(v, a, b, c), pt_fields(p, t0, t1, t2, r, dhat), r.dist);
-        st_seg[idx] = q;
+        st_seg[idx] = make_int2(q, (int)place);
     }
 }
 
@@ -613,7 +584,7 @@ template <int MODE, int SK>
 __global__ void __launch_bounds__(QBLK) k_query_pt(const double* __restrict__ x, const int32_t* __restrict__ surf_verts, int nv,
                                                    int n_dyn, int nf, const float4* __restrict__ rec,
                                                    const double2* __restrict__ leafd, double dhat, float gap, uint32_t* __restrict__ qcount,
-                                                   QueryOut st, int32_t* __restrict__ st_seg, uint32_t* __restrict__ counter,
+                                                   QueryOut st, int2* __restrict__ st_seg, uint32_t* __restrict__ counter,
                                                    uint32_t* __restrict__ flags, const int32_t* __restrict__ vseg,
                                                    const int32_t* __restrict__ roots, int32_t* __restrict__ cand,
                                                    uint32_t* __restrict__ ccount, int2* __restrict__ ovf, uint32_t* __restrict__ ovf_count) {
@@ -672,7 +643,7 @@ __global__ void __launch_bounds__(QBLK) k_query_pt(const double* __restrict__ x,
 // i: it goes to the staging list with segment seg0 + i and qcount[i] counts it.
 __device__ inline void ee_candidate(int e, int a0, int a1, dv3 A0, dv3 A1, int lf, const double2* __restrict__ leafd, int n_dyn,
                                     double dhat, uint32_t* __restrict__ qcount, int seg0, const QueryOut& st,
-                                    int32_t* __restrict__ st_seg, uint32_t* __restrict__ counter) {
+                                    int2* __restrict__ st_seg, uint32_t* __restrict__ counter) {
     const double2* L = leafd + (size_t)leaf_stride<2>() * lf;
     const double2 u0 = L[0], u1 = L[1], u2 = L[2];
     const int4 m = *reinterpret_cast<const int4*>(L + 3);
@@ -685,11 +656,11 @@ __device__ inline void ee_candidate(int e, int a0, int a1, dv3 A0, dv3 A1, int l
     const dv3 P0 = first ? A0 : B0, P1 = first ? A1 : B1, Q0 = first ? B0 : A0, Q1 = first ? B1 : A1;
     const EEOut r = segment_segment(P0, P1, Q0, Q1);
     if (!ee_accept(r, dhat)) return;
-    atomicAdd(&qcount[i], 1u);
+    const uint32_t place = atomicAdd(&qcount[i], 1u);
     const int idx = stage_slot(counter);
     if (idx < st.cap) {
         write_contact(st, idx, 1, i, j, make_int4(i0, i1, j0, j1), ee_fields(P0, P1, Q0, Q1, r, dhat), r.dist);
-        st_seg[idx] = seg0 + i;
+        st_seg[idx] = make_int2(seg0 + i, (int)place);
     }
 }
 
@@ -712,7 +683,7 @@ template <int MODE, int SK>
 __global__ void __launch_bounds__(QBLK) k_query_ee(int ne, int n_dyn, const float4* __restrict__ rec,
                                                    const double2* __restrict__ leafd, double dhat,
                                                    float gap, uint32_t* __restrict__ qcount, int seg0, QueryOut st,
-                                                   int32_t* __restrict__ st_seg, uint32_t* __restrict__ counter,
+                                                   int2* __restrict__ st_seg, uint32_t* __restrict__ counter,
                                                    uint32_t* __restrict__ flags, const int32_t* __restrict__ vseg,
                                                    const int32_t* __restrict__ roots, int32_t* __restrict__ cand,
                                                    uint32_t* __restrict__ ccount, int2* __restrict__ ovf, uint32_t* __restrict__ ovf_count) {
@@ -762,33 +733,54 @@ __global__ void __launch_bounds__(QBLK) k_query_ee(int ne, int n_dyn, const floa
     }
 }
 
-// Staged contact c goes to its segment: position qoffset[seg] + qfill[seg]++
-// (qfill zeroed beforehand); k_sort_segments then fixes the order inside each
-// segment.
-__global__ void k_scatter_contacts(int n, const int32_t* __restrict__ st_seg, QueryOut st, const uint32_t* __restrict__ qoffset,
-                                   uint32_t* __restrict__ qfill, QueryOut o) {
+// Canonical order of the staged contacts: segment by segment, sorted by
+// partner id inside a segment.  The partner ids go to their segments first
+// (in the order the test pass met them), then every staged contact counts the
+// smaller ids of its segment (a pair occurs once, so ids are distinct) and
+// moves straight to its final place.  The counts are independent loads over
+// one lane per contact; an insertion sort by one lane per segment moved each
+// 68-byte record several times in a dependent chain (13-30 us per detection
+// for segments of 10 to 30).
+__global__ void k_segment_keys(int n, const int2* __restrict__ st_seg, const int32_t* __restrict__ prim1,
+                               const uint32_t* __restrict__ qoffset, int32_t* __restrict__ seg_key) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= n) return;
-    const int sg = st_seg[c];
-    const int idx = (int)(qoffset[sg] + atomicAdd(&qfill[sg], 1u));
-    if (idx >= o.cap) return;
+    const int2 sg = st_seg[c];
+    seg_key[qoffset[sg.x] + sg.y] = prim1[c];
+}
+
+__global__ void k_place_contacts(int n, const int2* __restrict__ st_seg, QueryOut st, const uint32_t* __restrict__ qoffset,
+                                 const uint32_t* __restrict__ qcount, const int32_t* __restrict__ seg_key, QueryOut o, VertexCount vc) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= n) return;
+    const int sg = st_seg[c].x;
+    const int begin = (int)qoffset[sg], cnt = (int)qcount[sg];
+    const int key = st.prim1[c];
+    const int4 v = st.v[c];
+    int rank = 0;
+    for (int q = 0; q < cnt; q += 8) {
+        int k[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) k[u] = seg_key[begin + min(q + u, cnt - 1)];
+#pragma unroll
+        for (int u = 0; u < 8; u++) rank += q + u < cnt && k[u] < key ? 1 : 0;
+    }
+    const int idx = begin + rank;
     o.type[idx] = st.type[c];
     o.prim0[idx] = st.prim0[c];
-    o.prim1[idx] = st.prim1[c];
-    o.v[idx] = st.v[c];
+    o.prim1[idx] = key;
+    o.v[idx] = v;
     o.bary[idx] = st.bary[c];
     o.nrm[idx] = st.nrm[c];
     o.dist[idx] = st.dist[c];
-}
-
-// Sorts each of `n` segments [qoffset[s], qoffset[s] + qcount[s]) (clamped to
-// the capacity) by partner id.
-__global__ void k_sort_segments(int n, const uint32_t* __restrict__ qcount, const uint32_t* __restrict__ qoffset, QueryOut o) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const int begin = (int)qoffset[s];
-    const int end = min(begin + (int)qcount[s], o.cap);
-    if (end - begin > 1) sort_segment(o, begin, end);
+    if (vc.cnt) {
+        int4 l;
+        l.x = (int)atomicAdd(&vc.cnt[v.x], 1u);
+        l.y = (int)atomicAdd(&vc.cnt[v.y], 1u);
+        l.z = (int)atomicAdd(&vc.cnt[v.z], 1u);
+        l.w = (int)atomicAdd(&vc.cnt[v.w], 1u);
+        vc.loc[idx] = l;
+    }
 }
 
 } // namespace
@@ -845,9 +837,12 @@ Detector::Detector(int n_all_, int n_dyn_, int nv_, const int32_t* sv, int nf_, 
     c.bary.alloc(cap);
     c.nrm.alloc(cap);
     c.dist.alloc(cap);
-    qcount.alloc((size_t)nv + ne + 1);
+    counts.alloc((size_t)nv + ne + 8);
+    total = counts.p;
+    ovf_count = counts.p + 3;
+    qcount = counts.p + 8; // 16-byte aligned for the scan
     qoffset.alloc((size_t)nv + ne + 1);
-    qfill.alloc((size_t)nv + ne + 1);
+    PA_HIP(hipHostMalloc((void**)&total_host, 3 * sizeof(uint32_t), hipHostMallocDefault));
     stg.cap = cap;
     stg.type.alloc(cap);
     stg.prim0.alloc(cap);
@@ -857,14 +852,13 @@ Detector::Detector(int n_all_, int n_dyn_, int nv_, const int32_t* sv, int nf_, 
     stg.nrm.alloc(cap);
     stg.dist.alloc(cap);
     st_seg.alloc(cap);
+    seg_key.alloc(cap);
     cand_pt.alloc((size_t)CAND * std::max(nv, 1));
     cand_ee.alloc((size_t)CAND * std::max(ne, 1));
     ccount_pt.alloc(std::max(nv, 1));
     ccount_ee.alloc(std::max(ne, 1));
     ovf_pt.alloc(std::max(nv, 1));
     ovf_ee.alloc(std::max(ne, 1));
-    ovf_count.alloc(2);
-    total.alloc(3);
     PA_HIP(hipStreamSynchronize(stream));
 }
 
@@ -875,6 +869,7 @@ Detector::~Detector() {
     }
     if (ev_fork) (void)hipEventDestroy(ev_fork);
     if (ev_join) (void)hipEventDestroy(ev_join);
+    if (total_host) (void)hipHostFree(total_host); // every scan that writes it is waited for in detect()
     if (own_stream) {
         (void)hipStreamSynchronize(own_stream);
         (void)hipStreamDestroy(own_stream);
@@ -987,12 +982,10 @@ void Detector::set_segments(const int32_t* vs, int count) {
     }
 }
 
-int Detector::detect(const double* x, bool refit) {
+int Detector::detect(const double* x, bool refit, VertexCount vc) {
     refit = refit && built;
     // the edge tree (build, query) runs on the side stream beside the triangle tree
-    fill<uint32_t>(total.p, 0u, 3, stream);
-    fill<uint32_t>(qcount.p, 0u, (int64_t)nv + ne, stream);
-    fill<uint32_t>(ovf_count.p, 0u, 2, stream);
+    fill2<uint32_t>(counts.p, 8 + (int64_t)nv + ne, vc.cnt, vc.cnt ? vc.n : 0, 0u, stream);
     PA_HIP(hipEventRecord(ev_fork, stream));
     PA_HIP(hipStreamWaitEvent(side, ev_fork, 0));
     const float gap = (float)(dhat * 1.001);
@@ -1008,14 +1001,14 @@ int Detector::detect(const double* x, bool refit) {
     // the triangle tree.
     auto ee_pass = [&](auto mode, auto sk, hipStream_t s, dim3 grid) {
         hipLaunchKernelGGL((k_query_ee<decltype(mode)::value, decltype(sk)::value>), grid, dim3(QBLK), 0, s, ne, n_dyn,
-                           (const float4*)et.rec.p, (const double2*)et.leafd.p, dhat, gap, qcount.p + nv, nv, st, st_seg.p, total.p + 2,
-                           total.p, (const int32_t*)vseg.p, ee_roots, cand_ee.p, ccount_ee.p, ovf_ee.p, ovf_count.p + 1);
+                           (const float4*)et.rec.p, (const double2*)et.leafd.p, dhat, gap, qcount + nv, nv, st, st_seg.p, total + 2,
+                           total, (const int32_t*)vseg.p, ee_roots, cand_ee.p, ccount_ee.p, ovf_ee.p, ovf_count + 1);
         PA_LAUNCH_CHECK();
     };
     auto pt_pass = [&](auto mode, auto sk, hipStream_t s, dim3 grid) {
         hipLaunchKernelGGL((k_query_pt<decltype(mode)::value, decltype(sk)::value>), grid, dim3(QBLK), 0, s, x, surf_verts.p, nv,
-                           n_dyn, nf, (const float4*)ft.rec.p, (const double2*)ft.leafd.p, dhat, gap, qcount.p, st, st_seg.p,
-                           total.p + 2, total.p, (const int32_t*)vseg.p, pt_roots, cand_pt.p, ccount_pt.p, ovf_pt.p, ovf_count.p);
+                           n_dyn, nf, (const float4*)ft.rec.p, (const double2*)ft.leafd.p, dhat, gap, qcount, st, st_seg.p,
+                           total + 2, total, (const int32_t*)vseg.p, pt_roots, cand_pt.p, ccount_pt.p, ovf_pt.p, ovf_count);
         PA_LAUNCH_CHECK();
     };
     using M0 = std::integral_constant<int, 0>;
@@ -1038,21 +1031,21 @@ int Detector::detect(const double* x, bool refit) {
     PA_HIP(hipEventRecord(ev_join, side));
     PA_HIP(hipStreamWaitEvent(stream, ev_join, 0));
     uint32_t h[3] = {0u, 0u, 0u};
-    if (two) {
-        scan_exclusive(qcount.p, qoffset.p, (int64_t)nv + ne, total.p, scratch, stream);
-        PA_HIP(hipMemcpyAsync(h, total.p, sizeof(h), hipMemcpyDeviceToHost, stream));
+    auto count_found = [&](uint32_t* o) { // segment offsets; the totals reach the host with the scan's last launch
+        scan_exclusive(qcount, qoffset.p, (int64_t)nv + ne, total, scratch, stream, total_host);
         PA_HIP(hipStreamSynchronize(stream));
+        for (int k = 0; k < 3; k++) o[k] = total_host[k];
+    };
+    if (two) {
+        count_found(h);
     }
     if (!two || h[1] != 0) {
         // the short stack or an overflow list was too small: the single pass
         // (traversal and test together, full stack) for both queries
-        fill<uint32_t>(total.p, 0u, 3, stream);
-        fill<uint32_t>(qcount.p, 0u, (int64_t)nv + ne, stream);
+        fill<uint32_t>(counts.p, 0u, 8 + (int64_t)nv + ne, stream);
         if (ne > 0) ee_pass(M2{}, LS{}, stream, dim3(query_grid(ne)));
         if (nv > 0) pt_pass(M2{}, LS{}, stream, dim3(query_grid(nv)));
-        scan_exclusive(qcount.p, qoffset.p, (int64_t)nv + ne, total.p, scratch, stream);
-        PA_HIP(hipMemcpyAsync(h, total.p, sizeof(h), hipMemcpyDeviceToHost, stream));
-        PA_HIP(hipStreamSynchronize(stream));
+        count_found(h);
         if (two) single_pass_fallbacks++;
     }
     found_total = h[0];
@@ -1068,12 +1061,11 @@ int Detector::detect(const double* x, bool refit) {
     if (n_contacts > 0) {
         // canonical order: segments in query order (PT by vertex, EE by the
         // smaller edge id), each sorted by partner id
-        fill<uint32_t>(qfill.p, 0u, (int64_t)nv + ne, stream);
-        hipLaunchKernelGGL(k_scatter_contacts, dim3(grid_for(n_contacts, BLK)), dim3(BLK), 0, stream, n_contacts, (const int32_t*)st_seg.p,
-                           st, (const uint32_t*)qoffset.p, qfill.p, o);
+        hipLaunchKernelGGL(k_segment_keys, dim3(grid_for(n_contacts, BLK)), dim3(BLK), 0, stream, n_contacts, (const int2*)st_seg.p,
+                           (const int32_t*)stg.prim1.p, (const uint32_t*)qoffset.p, seg_key.p);
         PA_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_sort_segments, dim3(grid_for(nv + ne, BLK)), dim3(BLK), 0, stream, nv + ne, (const uint32_t*)qcount.p,
-                           (const uint32_t*)qoffset.p, o);
+        hipLaunchKernelGGL(k_place_contacts, dim3(grid_for(n_contacts, BLK)), dim3(BLK), 0, stream, n_contacts, (const int2*)st_seg.p, st,
+                           (const uint32_t*)qoffset.p, (const uint32_t*)qcount, (const int32_t*)seg_key.p, o, vc);
         PA_LAUNCH_CHECK();
     }
     return n_contacts;

@@ -4,61 +4,101 @@
 namespace pa {
 namespace {
 
-constexpr int SCAN_BLOCK = 256;
-constexpr int SCAN_ITEMS = 4;
-constexpr int SCAN_TILE = SCAN_BLOCK * SCAN_ITEMS;
+// Exclusive scan.  Up to SCAN_ONE values: one workgroup, one launch.  Above:
+// two launches, k_scan_sums (each tile's sum) and k_scan_apply, where every
+// tile adds up the sums before it (a few thousand values at most here, read by
+// 1024 lanes) and scans itself.  Launches bound these scans, not bytes: the
+// scans here are over 1e3 to 1e6 counts, and a launch costs 2-3 us and its
+// dependent dispatch as much again; the recursive tile scan took up to five.
+constexpr int SCAN_BLOCK = 1024;
+constexpr int SCAN_TILE = 4 * SCAN_BLOCK;
+constexpr int SCAN_ONE = 16 * SCAN_BLOCK;
 
-// Block-wide exclusive scan of one value per thread (256 threads = 4 waves).
+// Four consecutive values from i on, 0 past n (in is 16-byte aligned).
+__device__ inline uint4 scan_load(const uint32_t* in, int64_t i, int64_t n) {
+    if (i + 4 <= n) return *reinterpret_cast<const uint4*>(in + i);
+    return make_uint4(i < n ? in[i] : 0u, i + 1 < n ? in[i + 1] : 0u, i + 2 < n ? in[i + 2] : 0u, 0u);
+}
+__device__ inline void scan_store(uint32_t* out, int64_t i, int64_t n, uint4 v) {
+    if (i + 4 <= n) {
+        *reinterpret_cast<uint4*>(out + i) = v;
+        return;
+    }
+    if (i < n) out[i] = v.x;
+    if (i + 1 < n) out[i + 1] = v.y;
+    if (i + 2 < n) out[i + 2] = v.z;
+}
+
+// Block-wide exclusive scan of one value per thread (16 waves).
 __device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t* sh_wave, uint32_t* block_total) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    // inclusive scan inside the wave
-    uint32_t x = v;
+    uint32_t x = v; // inclusive scan inside the wave
     for (int o = 1; o < 64; o <<= 1) {
-        uint32_t y = __shfl_up(x, o, 64);
+        const uint32_t y = __shfl_up(x, o, 64);
         if (lane >= o) x += y;
     }
     if (lane == 63) sh_wave[wave] = x;
     __syncthreads();
-    uint32_t base = 0;
-    for (int w = 0; w < wave; w++) base += sh_wave[w];
-    if (block_total) *block_total = sh_wave[0] + sh_wave[1] + sh_wave[2] + sh_wave[3];
+    uint32_t base = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < SCAN_BLOCK / 64; w++) {
+        if (w < wave) base += sh_wave[w];
+        all += sh_wave[w];
+    }
+    *block_total = all;
     return base + x - v;
 }
 
-__global__ void __launch_bounds__(SCAN_BLOCK) k_scan_tiles(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
-                                                          int64_t n, uint32_t* __restrict__ tile_sums) {
-    __shared__ uint32_t sh_wave[4];
-    const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
-    uint32_t v[SCAN_ITEMS];
+__device__ inline void scan_publish(uint32_t t, uint32_t* total, uint32_t* host3) {
+    if (total) *total = t;
+    if (host3) {
+        host3[0] = t;
+        host3[1] = total[1];
+        host3[2] = total[2];
+    }
+}
+
+__global__ void __launch_bounds__(SCAN_BLOCK) k_scan_one(const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total, uint32_t* host3) {
+    __shared__ uint32_t sh_wave[SCAN_BLOCK / 64];
+    const int64_t i0 = 16 * (int64_t)threadIdx.x;
+    uint4 v[4];
     uint32_t sum = 0;
 #pragma unroll
-    for (int k = 0; k < SCAN_ITEMS; k++) {
-        v[k] = (base + k < n) ? in[base + k] : 0u;
-        sum += v[k];
+    for (int k = 0; k < 4; k++) {
+        v[k] = scan_load(in, i0 + 4 * k, n);
+        sum += v[k].x + v[k].y + v[k].z + v[k].w;
     }
-    uint32_t tot;
-    uint32_t ex = block_exclusive_scan(sum, sh_wave, &tot);
+    uint32_t all;
+    uint32_t ex = block_exclusive_scan(sum, sh_wave, &all); // its barrier: every load is done before a store
 #pragma unroll
-    for (int k = 0; k < SCAN_ITEMS; k++) {
-        if (base + k < n) out[base + k] = ex;
-        ex += v[k];
+    for (int k = 0; k < 4; k++) {
+        const uint4 o = make_uint4(ex, ex + v[k].x, ex + v[k].x + v[k].y, ex + v[k].x + v[k].y + v[k].z);
+        scan_store(out, i0 + 4 * k, n, o);
+        ex = o.w + v[k].w;
     }
-    if (threadIdx.x == 0) tile_sums[blockIdx.x] = tot;
+    if (threadIdx.x == 0) scan_publish(all, total, host3);
 }
 
-__global__ void k_scan_add(uint32_t* __restrict__ out, int64_t n, const uint32_t* __restrict__ tile_offsets) {
-    const int64_t i = (int64_t)blockIdx.x * SCAN_TILE + threadIdx.x;
-    const uint32_t add = tile_offsets[blockIdx.x];
-#pragma unroll
-    for (int k = 0; k < SCAN_ITEMS; k++) {
-        int64_t e = i + (int64_t)k * SCAN_BLOCK;
-        if (e < n) out[e] += add;
-    }
+__global__ void __launch_bounds__(SCAN_BLOCK) k_scan_sums(const uint32_t* __restrict__ in, int64_t n, uint32_t* __restrict__ sums) {
+    __shared__ uint32_t sh_wave[SCAN_BLOCK / 64];
+    const uint4 v = scan_load(in, (int64_t)blockIdx.x * SCAN_TILE + 4 * (int64_t)threadIdx.x, n);
+    uint32_t all;
+    block_exclusive_scan(v.x + v.y + v.z + v.w, sh_wave, &all);
+    if (threadIdx.x == 0) sums[blockIdx.x] = all;
 }
 
-__global__ void k_scan_total(const uint32_t* __restrict__ in, const uint32_t* __restrict__ out, int64_t n,
-                             uint32_t* __restrict__ total) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) *total = n > 0 ? out[n - 1] + in[n - 1] : 0u;
+__global__ void __launch_bounds__(SCAN_BLOCK) k_scan_apply(const uint32_t* in, uint32_t* out, int64_t n, const uint32_t* __restrict__ sums,
+                                                          uint32_t* total, uint32_t* host3) {
+    __shared__ uint32_t sh_base[SCAN_BLOCK / 64], sh_wave[SCAN_BLOCK / 64];
+    const int64_t i = (int64_t)blockIdx.x * SCAN_TILE + 4 * (int64_t)threadIdx.x;
+    const uint4 v = scan_load(in, i, n);
+    uint32_t before = 0;
+    for (unsigned b = threadIdx.x; b < blockIdx.x; b += SCAN_BLOCK) before += sums[b];
+    uint32_t base, all;
+    block_exclusive_scan(before, sh_base, &base);
+    uint32_t ex = base + block_exclusive_scan(v.x + v.y + v.z + v.w, sh_wave, &all);
+    scan_store(out, i, n, make_uint4(ex, ex + v.x, ex + v.x + v.y, ex + v.x + v.y + v.z));
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) scan_publish(base + all, total, host3);
 }
 
 // Histogram of one 8-bit digit per tile; hist is digit-major [256][ntiles].
@@ -124,41 +164,22 @@ __global__ void __launch_bounds__(RS_BLOCK) k_rs_scatter(const uint32_t* __restr
     }
 }
 
-void scan_rec(const uint32_t* in, uint32_t* out, int64_t n, PrimScratch& s, int depth, hipStream_t st) {
-    if (n <= 0) return;
-    const int64_t tiles = (n + SCAN_TILE - 1) / SCAN_TILE;
-    DBuf<uint32_t>& sums = depth == 0 ? s.scan_a : (depth == 1 ? s.scan_b : s.scan_c);
-    PA_CHECK(depth < 3, PA_ERR_INVALID, "scan too large");
-    sums.reserve((size_t)tiles + 1);
-    hipLaunchKernelGGL(k_scan_tiles, dim3((unsigned)tiles), dim3(SCAN_BLOCK), 0, st, in, out, n, sums.p);
-    PA_LAUNCH_CHECK();
-    if (tiles > 1) {
-        scan_rec(sums.p, sums.p, tiles, s, depth + 1, st);
-        hipLaunchKernelGGL(k_scan_add, dim3((unsigned)tiles), dim3(SCAN_BLOCK), 0, st, out, n, sums.p);
-        PA_LAUNCH_CHECK();
-    } else {
-        // single tile: its offset is zero already
-    }
-}
-
 } // namespace
 
-void scan_exclusive(const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total, PrimScratch& s, hipStream_t st) {
-    if (n <= 0) {
-        if (total) fill<uint32_t>(total, 0u, 1, st);
+void scan_exclusive(const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total, PrimScratch& s, hipStream_t st, uint32_t* host3) {
+    PA_CHECK(!host3 || total, PA_ERR_INVALID, "scan: host3 needs total");
+    PA_CHECK(((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0, PA_ERR_INVALID, "scan: unaligned array");
+    if (n <= SCAN_ONE) { // also n <= 0: the total is 0
+        hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(SCAN_BLOCK), 0, st, in, out, n, total, host3);
+        PA_LAUNCH_CHECK();
         return;
     }
-    if (total) {
-        // The total needs the last input value, which `out` may overwrite when it aliases `in`.
-        DBuf<uint32_t>& last = s.last;
-        last.reserve(1);
-        PA_HIP(hipMemcpyAsync(last.p, in + n - 1, sizeof(uint32_t), hipMemcpyDeviceToDevice, st));
-        scan_rec(in, out, n, s, 0, st);
-        hipLaunchKernelGGL(k_scan_total, dim3(1), dim3(64), 0, st, last.p, out + n - 1, (int64_t)1, total);
-        PA_LAUNCH_CHECK();
-    } else {
-        scan_rec(in, out, n, s, 0, st);
-    }
+    const int64_t tiles = (n + SCAN_TILE - 1) / SCAN_TILE;
+    s.sums.reserve((size_t)tiles);
+    hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)tiles), dim3(SCAN_BLOCK), 0, st, in, n, s.sums.p);
+    PA_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)tiles), dim3(SCAN_BLOCK), 0, st, in, out, n, (const uint32_t*)s.sums.p, total, host3);
+    PA_LAUNCH_CHECK();
 }
 
 void radix_sort_pairs(uint32_t* keys, uint32_t* vals, int64_t n, int bits, PrimScratch& s, hipStream_t st) {
@@ -174,7 +195,7 @@ void radix_sort_pairs(uint32_t* keys, uint32_t* vals, int64_t n, int bits, PrimS
         const int shift = 8 * pss;
         hipLaunchKernelGGL(k_rs_hist, dim3(ntiles), dim3(RS_BLOCK), 0, st, ka, n, shift, hist.p, ntiles);
         PA_LAUNCH_CHECK();
-        scan_rec(hist.p, hist.p, (int64_t)ntiles * 256, s, 0, st);
+        scan_exclusive(hist.p, hist.p, (int64_t)ntiles * 256, nullptr, s, st);
         hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles), dim3(RS_BLOCK), 0, st, ka, va, kb, vb, n, shift, hist.p, ntiles);
         PA_LAUNCH_CHECK();
         std::swap(ka, kb);

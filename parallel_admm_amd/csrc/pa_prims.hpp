@@ -19,15 +19,30 @@ template <class T> inline void fill(T* p, T v, int64_t n, hipStream_t s) {
     PA_LAUNCH_CHECK();
 }
 
+// Two fills in one launch: p[0..n) and q[0..m) = v.
+template <class T> __global__ void k_fill2(T* __restrict__ p, int64_t n, T* __restrict__ q, int64_t m, T v) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = v;
+    else if (i - n < m) q[i - n] = v;
+}
+template <class T> inline void fill2(T* p, int64_t n, T* q, int64_t m, T v, hipStream_t s) {
+    if (n + m <= 0) return;
+    hipLaunchKernelGGL(k_fill2<T>, dim3(grid_for(n + m, 256)), dim3(256), 0, s, p, n, q, m, v);
+    PA_LAUNCH_CHECK();
+}
+
 // Scratch for scan/sort; grown on demand.
 struct PrimScratch {
-    DBuf<uint32_t> scan_a, scan_b, scan_c;
-    DBuf<uint32_t> hist, keys_alt, vals_alt, last;
+    DBuf<uint32_t> sums, hist, keys_alt, vals_alt;
 };
 
 // out[i] = sum_{j<i} in[j]; if total != nullptr, *total (device) = sum of all.
-// in and out may alias.
-void scan_exclusive(const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total, PrimScratch& s, hipStream_t st);
+// in and out are 16-byte aligned and may alias; total is outside both.  host3
+// (pinned host memory, with total): the same launch also writes total[0..2]
+// there, so the caller reads them after a stream synchronisation without a
+// copy.
+void scan_exclusive(const uint32_t* in, uint32_t* out, int64_t n, uint32_t* total, PrimScratch& s, hipStream_t st,
+                    uint32_t* host3 = nullptr);
 
 // Sorts (keys, vals) by the low `bits` bits of keys, stably.  Result in keys/vals.
 void radix_sort_pairs(uint32_t* keys, uint32_t* vals, int64_t n, int bits, PrimScratch& s, hipStream_t st);

@@ -418,55 +418,35 @@ __global__ void __launch_bounds__(BLK) k_dual_elem(ElemArgs a, int want_res, con
 // ---------------------------------------------------------------------------
 // Contacts (reference src/solver/contact_solver.cu:90-431).
 // ---------------------------------------------------------------------------
-__global__ void k_contact_count(int nc, const int4* __restrict__ cv, uint32_t* __restrict__ cnt) {
+// Contact counts per vertex (all vertices), and each contact's place among its
+// vertices' contacts (any order): what the detection's last kernel does itself
+// within a step.
+__global__ void k_contact_count(int nc, const int4* __restrict__ cv, uint32_t* __restrict__ cnt, int4* __restrict__ loc) {
     int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= nc) return;
-    int4 v = cv[c];
-    atomicAdd(&cnt[v.x], 1u);
-    atomicAdd(&cnt[v.y], 1u);
-    atomicAdd(&cnt[v.z], 1u);
-    atomicAdd(&cnt[v.w], 1u);
+    int4 v = cv[c], l;
+    l.x = (int)atomicAdd(&cnt[v.x], 1u);
+    l.y = (int)atomicAdd(&cnt[v.y], 1u);
+    l.z = (int)atomicAdd(&cnt[v.z], 1u);
+    l.w = (int)atomicAdd(&cnt[v.w], 1u);
+    loc[c] = l;
 }
 
-__global__ void k_contact_fill(int nc, int n, const int4* __restrict__ cv, const uint32_t* __restrict__ vptr,
-                               uint32_t* __restrict__ vfill, uint32_t* __restrict__ vent) {
+// The entries of dynamic vertices into their runs, unsorted (vraw), and per
+// contact S_c = eps + sum_i b_i^2 w_i^-1 cnt_i; Gamma_ci = b_i / (S_c w_i); K_c = h^-1 h_cN gamma n
+// with the contact's friction coefficient (that of its first vertex) in K.w; r_c = 0.
+__global__ void k_contact_fill(int nc, int n, float eps, float gam, float hinv, const int4* __restrict__ cv, const int4* __restrict__ loc,
+                               const uint32_t* __restrict__ vptr, uint32_t* __restrict__ vraw, const float4* __restrict__ bary,
+                               const float4* __restrict__ nrm, const uint32_t* __restrict__ cnt, const float* __restrict__ wc,
+                               const float* __restrict__ wc_inv, const float* __restrict__ mu_v, float4* __restrict__ G,
+                               float4* __restrict__ K, float4* __restrict__ rc) {
     int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= nc) return;
-    int4 v = cv[c];
-    int vs[4] = {v.x, v.y, v.z, v.w};
+    const int4 v = cv[c], l = loc[c];
+    const int vs[4] = {v.x, v.y, v.z, v.w}, ls[4] = {l.x, l.y, l.z, l.w};
 #pragma unroll
     for (int k = 0; k < 4; k++)
-        if (vs[k] < n) {
-            uint32_t pos = vptr[vs[k]] + atomicAdd(&vfill[vs[k]], 1u);
-            vent[pos] = (uint32_t)(4 * c + k);
-        }
-}
-
-// Per-vertex entries sorted ascending (contact order) so gathers sum in a fixed order.
-__global__ void k_contact_sort(int n, const uint32_t* __restrict__ vptr, uint32_t* __restrict__ vent) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint32_t b = vptr[i], e = vptr[i + 1];
-    for (uint32_t a = b + 1; a < e; a++) {
-        uint32_t key = vent[a];
-        uint32_t q = a;
-        while (q > b && vent[q - 1] > key) {
-            vent[q] = vent[q - 1];
-            q--;
-        }
-        vent[q] = key;
-    }
-}
-
-// S_c = eps + sum_i b_i^2 w_i^-1 cnt_i; Gamma_ci = b_i / (S_c w_i); K_c = h^-1 h_cN gamma n
-// with the contact's friction coefficient (that of its first vertex) in K.w; r_c = 0.
-__global__ void k_contact_scc(int nc, int n, float eps, float gam, float hinv, const int4* __restrict__ cv,
-                              const float4* __restrict__ bary, const float4* __restrict__ nrm, const uint32_t* __restrict__ cnt,
-                              const float* __restrict__ wc, const float* __restrict__ wc_inv, const float* __restrict__ mu_v,
-                              float4* __restrict__ G, float4* __restrict__ K, float4* __restrict__ rc) {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nc) return;
-    int4 v = cv[c];
+        if (vs[k] < n) vraw[vptr[vs[k]] + ls[k]] = (uint32_t)(4 * c + k);
     float4 b = bary[c];
     float Sc = eps;
     Sc += b.x * b.x * wc_inv[v.x] * (float)cnt[v.x];
@@ -483,6 +463,40 @@ __global__ void k_contact_scc(int nc, int n, float eps, float gam, float hinv, c
     float s = hinv * nn.w * gam;
     K[c] = make_float4(s * nn.x, s * nn.y, s * nn.z, mu_v[v.x]);
     rc[c] = make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
+// Sorts every vertex's entries ascending (contact order, so that gathers sum in
+// a fixed order), one lane per (contact, vertex): the entry's place is the
+// number of smaller entries in its run.  vent gets the sorted entries, slot[c].k
+// the place of (contact c, vertex k), -1 for static vertices, and erun[e]
+// (vertex, end of its entries) on a vertex's first entry, (-1, 0) on the
+// others.  Counting reads a run eight entries at a time; the insertion sort by
+// one lane per vertex that stood here was a chain of dependent loads and
+// stores over runs of 10 to 40 entries, 32-85 us per detection on single
+// scenes.
+__global__ void k_contact_rank(int nc, int n, const int4* __restrict__ cv, const uint32_t* __restrict__ vptr,
+                               const uint32_t* __restrict__ vraw, uint32_t* __restrict__ vent, int32_t* __restrict__ slot,
+                               int2* __restrict__ erun) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= 4 * nc) return;
+    const int v = reinterpret_cast<const int32_t*>(cv)[i];
+    if (v >= n) {
+        slot[i] = -1;
+        return;
+    }
+    const int begin = (int)vptr[v], end = (int)vptr[v + 1];
+    int rank = 0;
+    for (int q = begin; q < end; q += 8) {
+        uint32_t k[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) k[u] = vraw[min(q + u, end - 1)];
+#pragma unroll
+        for (int u = 0; u < 8; u++) rank += q + u < end && k[u] < (uint32_t)i ? 1 : 0;
+    }
+    const int e = begin + rank;
+    vent[e] = (uint32_t)i;
+    slot[i] = e;
+    erun[e] = rank == 0 ? make_int2(v, end) : make_int2(-1, 0);
 }
 
 __device__ inline float3 gather_contacts(int i, const uint32_t* __restrict__ vptr, const uint32_t* __restrict__ vent,
@@ -560,20 +574,6 @@ __global__ void k_contact_du(int nc, const int4* __restrict__ cv, const float4* 
 #pragma unroll
     for (int k = 0; k < 4; k++)
         if (sk[k] >= 0) gdu[sk[k]] = make_float4(gk[k] * d.x, gk[k] * d.y, gk[k] * d.z, 0.f);
-}
-
-// slot[c].k = position of (contact c, vertex k) in the sorted vertex entry
-// list, -1 for static vertices; erun[e] = (vertex, end of its entries) on a
-// vertex's first entry, (-1, 0) on the others.
-__global__ void k_contact_slots(int n, const uint32_t* __restrict__ vptr, const uint32_t* __restrict__ vent, int32_t* __restrict__ slot,
-                                int2* __restrict__ erun) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t e0 = vptr[i], e1 = vptr[i + 1];
-    for (uint32_t e = e0; e < e1; e++) {
-        slot[vent[e]] = (int32_t)e;
-        erun[e] = e == e0 ? make_int2(i, (int)e1) : make_int2(-1, 0);
-    }
 }
 
 // p_v += sum of the Gamma du entries of v (contact order), one lane per
@@ -2811,7 +2811,8 @@ void Backend::assemble_and_upload(const double* x0h) {
     gdu.alloc(4 * (size_t)cap);
     vcnt.alloc(n_all);
     vptr.alloc((size_t)n + 1);
-    vfill.alloc(n);
+    vloc.alloc(cap);
+    vraw.alloc(4 * (size_t)cap);
     vent.alloc(4 * (size_t)cap);
     erun.alloc(4 * (size_t)cap);
     x_host.assign(x0h, x0h + 3 * (size_t)n_all);
@@ -2919,32 +2920,25 @@ void Backend::dual_update(bool want_res) {
     }
 }
 
-void Backend::contact_setup(float eps, float gamma_, float hinv) {
+// counted: the detection has filled vcnt and vloc.
+void Backend::contact_setup(float eps, float gamma_, float hinv, bool counted) {
     nc = det ? det->n_contacts : 0;
-    fill<uint32_t>(vcnt.p, 0u, n_all, stream);
-    fill<uint32_t>(vfill.p, 0u, n, stream);
-    if (nc > 0)
-        hipLaunchKernelGGL(k_contact_count, dim3(grid_for(nc, BLK)), dim3(BLK), 0, stream, nc, det->c.v.p, vcnt.p);
-    PA_LAUNCH_CHECK();
-    // per-vertex contact slots over dynamic vertices; static vertices keep
-    // their counts (they enter S_c) but get no slots
-    DBuf<uint32_t>& tmp = scratch.keys_alt;
-    tmp.reserve((size_t)n + 1);
-    PA_HIP(hipMemcpyAsync(tmp.p, vcnt.p, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, stream));
-    scan_exclusive(tmp.p, vptr.p, n, vptr.p + n, scratch, stream);
-    if (nc > 0) {
-        hipLaunchKernelGGL(k_contact_fill, dim3(grid_for(nc, BLK)), dim3(BLK), 0, stream, nc, n, det->c.v.p, vptr.p, vfill.p, vent.p);
-        PA_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_contact_sort, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, n, vptr.p, vent.p);
-        PA_LAUNCH_CHECK();
-        fill<int32_t>(cslot.p, -1, 4 * (int64_t)nc, stream);
-        hipLaunchKernelGGL(k_contact_slots, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, n, (const uint32_t*)vptr.p, (const uint32_t*)vent.p,
-                           cslot.p, erun.p);
-        PA_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_contact_scc, dim3(grid_for(nc, BLK)), dim3(BLK), 0, stream, nc, n, eps, gamma_, hinv, det->c.v.p,
-                           det->c.bary.p, det->c.nrm.p, vcnt.p, wc.p, wc_inv.p, (const float*)mu_v.p, gam.p, kc.p, rc.p);
+    if (nc == 0) return;
+    if (!counted) {
+        fill<uint32_t>(vcnt.p, 0u, n_all, stream);
+        hipLaunchKernelGGL(k_contact_count, dim3(grid_for(nc, BLK)), dim3(BLK), 0, stream, nc, (const int4*)det->c.v.p, vcnt.p, vloc.p);
         PA_LAUNCH_CHECK();
     }
+    // per-vertex contact entries over dynamic vertices; static vertices keep
+    // their counts (they enter S_c) but get no entries
+    scan_exclusive(vcnt.p, vptr.p, n, vptr.p + n, scratch, stream);
+    hipLaunchKernelGGL(k_contact_fill, dim3(grid_for(nc, BLK)), dim3(BLK), 0, stream, nc, n, eps, gamma_, hinv, (const int4*)det->c.v.p,
+                       (const int4*)vloc.p, (const uint32_t*)vptr.p, vraw.p, (const float4*)det->c.bary.p, (const float4*)det->c.nrm.p,
+                       (const uint32_t*)vcnt.p, (const float*)wc.p, (const float*)wc_inv.p, (const float*)mu_v.p, gam.p, kc.p, rc.p);
+    PA_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_contact_rank, dim3(grid_for(4 * (int64_t)nc, BLK)), dim3(BLK), 0, stream, nc, n, (const int4*)det->c.v.p,
+                       (const uint32_t*)vptr.p, (const uint32_t*)vraw.p, vent.p, cslot.p, erun.p);
+    PA_LAUNCH_CHECK();
 }
 
 void Backend::contact_project(bool) {
@@ -4028,12 +4022,13 @@ int Backend::admm_loop(pa_step_stats& S, float eps, float gam_, float hinv) {
                 break;
             }
             try {
-                det->detect(x.p, it > 0); // rebuild at the step's first detection, refit later ones
+                // rebuild at the step's first detection, refit later ones
+                det->detect(x.p, it > 0, VertexCount{vcnt.p, vloc.p, n_all});
             } catch (...) {
                 if (overlap) join(); // the rollback writes x, which the side stream reads
                 throw;
             }
-            contact_setup(eps, gam_, hinv);
+            contact_setup(eps, gam_, hinv, true);
             ws_window_begin();
             S.detections++;
             S.n_contacts_max = std::max(S.n_contacts_max, nc);

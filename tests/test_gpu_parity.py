@@ -69,6 +69,32 @@ def test_detector_matches_oracle_folded_cloth(pa, jitter):
     _check_contacts_equal(gi, gr, oi, orr)
 
 
+@pytest.mark.parametrize("faces", [3, 8, 9, 40, 200])
+def test_detector_orders_long_segments(pa, faces):
+    """One vertex over the hub of a fan of static triangles: it is in contact
+    with every face, so its segment of the list has `faces` entries (below, at
+    and past the eight that are ranked at a time), numbered in an order that is
+    not the order in which the traversal meets them."""
+    from parallel_admm_amd.configs import config_for
+
+    cfg = config_for("cloth32")
+    a = 2 * np.pi * np.arange(faces) / faces
+    fan = np.concatenate([[[0.0, 0.0, 0.0]], np.stack([0.1 * np.cos(a), 0 * a, 0.1 * np.sin(a)], axis=1)])
+    x = np.concatenate([[[0, 0.5 * cfg.thickness, 0], [0.05, 0.05, 0], [0, 0.05, 0.05]], fan])
+    k = np.random.default_rng(2).permutation(faces)
+    tris = np.concatenate([[[0, 1, 2]], np.stack([np.full(faces, 3), 4 + (k + 1) % faces, 4 + k], axis=1)])
+    density = np.concatenate([np.full(3, 1.0), np.full(faces + 1, 1e12)])
+    sc = pa.Scene.from_mesh(x, 3, density, tris=tris, tri_k=np.full(len(tris), 1e3))
+    det = _detector(pa, sc, cfg)
+    det.detect(x)
+    gi, gr = det.contacts()
+    o = _oracle(sc.mesh(), cfg)
+    o.detect(x, brute_force=True)
+    oi, orr = o.contacts()
+    assert np.sum((gi[:, 0] == 0) & (gi[:, 1] == 0)) >= faces
+    _check_contacts_equal(gi, gr, oi, orr)
+
+
 def test_single_pass_and_two_pass_queries_agree(pa):
     """The two query passes (collect leaf hits, then test them) and the single
     pass (traversal and FP64 test together) give the same list, bit for bit:
