@@ -256,7 +256,7 @@ struct Backend {
     void set_vertex_mu(const double* mu);
 
     // sub-phases (also used by step)
-    void local_step(bool first_iter, hipStream_t s = nullptr);
+    void local_step(hipStream_t s = nullptr);
     void contact_setup(float eps, float gamma, float hinv, bool counted = false);
     void contact_project(bool first_iter);
     void contact_sweep_once();
@@ -270,8 +270,9 @@ struct Backend {
     void get_track_frames(int32_t* frames) const;
     void set_track_frames(const int32_t* frames, int count);
     // defer_last (direct solve): the last pass leaves x += d to the next
-    // dual update (dx_pending), which applies it before reading x
-    int global_solve(int max_iter, double tol, bool defer_last = false);
+    // dual update (dx_pending), which applies it before reading x.
+    // resid_ready (direct solve): cg_r holds b - A x already (left by rhs)
+    int global_solve(int max_iter, double tol, bool defer_last = false, bool resid_ready = false);
     bool dx_pending = false;
     void pcg_iteration(int it, bool fused, int& pc, int& rc);
     hipGraphExec_t pcg_pair_graph(bool first_pair);
@@ -281,7 +282,8 @@ struct Backend {
     // cg_z = M^-1 r, partial r.z into cg_part[*, 6..8]; with skip_pre0 the
     // level-0 pre-smoothing was already done by k_cg_update_pre.
     void precondition(const float* r, bool skip_pre0 = false);
-    void dual_update(bool want_residual);
+    void dual_vertices(bool want_residual);
+    void elem_update(bool want_residual, bool last, bool next_check, hipStream_t s);
     void residual_read(double* rp, double* rd);
     void residual_enqueue(int it);
     int3 resid_blocks();

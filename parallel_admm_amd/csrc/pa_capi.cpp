@@ -570,7 +570,7 @@ pa_status pa_backend_project_elastic(pa_backend* b, const double* x, const doubl
         std::vector<float> uf(ue, ue + 3 * (size_t)B.m), zf(3 * (size_t)B.m);
         B.x.upload(x, 3 * (size_t)B.n_all, B.stream);
         B.Ue.upload(uf.data(), uf.size(), B.stream);
-        B.local_step(true);
+        B.local_step();
         B.z.download(zf.data(), zf.size(), B.stream);
         PA_HIP(hipStreamSynchronize(B.stream));
         for (size_t i = 0; i < zf.size(); i++) zo[i] = zf[i];

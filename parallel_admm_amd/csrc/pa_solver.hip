@@ -5,14 +5,16 @@
 // does, src/solver/backend_cpu/admm_impl_cpu.cpp:264-359):
 //   prologue        k_begin_step (+ k_spmv_add for Damp x0)
 //   per iteration   [detection every dcd_interval]
-//                   k_local        z = prox(D x + Ue) per constraint (tri/tet/bend/pin in one launch)
-//                   k_vertex_p     p = (x - x0 + Uc)/h + Gamma r_c      (contact on)
+//                   [k_elem        z = prox(D x + Ue) per constraint (tri/tet/bend/pin in one launch), first iteration]
+//                   k_vertex_p     p += Gamma r_c                       (contact on; p = (x - x0 + Uc)/h before)
 //                   G x (k_contact_du, k_vertex_gather)                  (friction-cone sweeps;
-//                                  up to 2048 contacts all G of them in k_contact_sweeps_wg)
+//                                  up to 2048 contacts all of this in k_contact_sweeps_wg)
 //                   k_rhs          b = M x~ + Damp x0 + h^2 D^T We^2 (z - Ue) + h^2 Wc (h p + x0 - Uc)
+//                                  (and b - A x with the direct solve)
 //                   global solve   A x = b: FP64 residual + FP32 correction (the direct factor, or PCG
 //                                  with a smoothed-aggregation AMG V-cycle or Jacobi preconditioner)
-//                   k_dual_elem / k_dual_vert   Ue += D x - z, Uc += x - x0 - h p (+ residual sums)
+//                   k_dual_vert    x += correction, Uc += x - x0 - h p, p = (x - x0 + Uc)/h (+ residual sums)
+//                   k_elem         Ue += D x - z (+ residual sums), then z of the next iteration
 //                   k_resid_final  residual check (the stop test on the device with the direct solve)
 //   epilogue        k_end_step     v = (x - x0)/h
 // D is applied matrix-free from the constraint rest data; D^T We^2 is a
@@ -129,10 +131,11 @@ __device__ inline void block_reduce_parts(const double* __restrict__ part, int n
 // Positions and velocities are FP64: x~ = x0 + h v and v = (x - x0)/h are
 // formed without the cancellation an FP32 position would carry.  bconst =
 // M x~ + bpin, bpin holding the pins' targets (the pin rows of z are kept
-// relative to the pin position).
-__global__ void k_begin_step(int n_all, int n, double h, double g, const uint8_t* __restrict__ pinned, double* __restrict__ x,
+// relative to the pin position).  p starts as the velocity on static vertices
+// and as (x~ - x0 + Uc) / h, the first iteration's value, on dynamic ones.
+__global__ void k_begin_step(int n_all, int n, double h, float hinv, double g, const uint8_t* __restrict__ pinned, double* __restrict__ x,
                              const double* __restrict__ v, double* __restrict__ x0, float* __restrict__ p, double* __restrict__ bconst,
-                             const double* __restrict__ mass, const double* __restrict__ bpin) {
+                             const double* __restrict__ mass, const double* __restrict__ bpin, const float* __restrict__ Uc) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n_all) return;
     const double3 xi = ld3(x, i);
@@ -147,8 +150,10 @@ __global__ void k_begin_step(int n_all, int n, double h, double g, const uint8_t
         bconst[3 * i] = mi * xt.x + bpin[3 * i];
         bconst[3 * i + 1] = mi * xt.y + bpin[3 * i + 1];
         bconst[3 * i + 2] = mi * xt.z + bpin[3 * i + 2];
+        st3(p, i, hinv * (to_f3(xt - xi) + ld3(Uc, i)));
+    } else {
+        st3(p, i, to_f3(vi));
     }
-    st3(p, i, to_f3(vi));
 }
 
 // flag[0] |= 1 if any of x (3 n_all) or v (3 n_all) is not finite.
@@ -228,51 +233,64 @@ __device__ inline int elem_of(const ElemArgs& a, int* c) {
     return *c < a.n_pin ? 3 : -1;
 }
 
-// D x for constraint c of `type`: rows into dx[], returns number of rows and
+// D x for constraint c of type TYPE: ELEM_ROWS<TYPE> rows into dx[]; returns the
 // first row.  Edge vectors and the bending sum are formed from the FP64
 // positions and rounded once.  A pin row is kept relative to its target:
 // dx = x_v - pin position (its z is 0, and the target enters the right-hand
 // side through bpin), so no FP32 value holds an absolute position.
-__device__ inline int elem_dx(const ElemArgs& a, int type, int c, const double* __restrict__ x, float3 dx[3], int* row0, float* w) {
-    if (type == 0) {
+template <int TYPE> constexpr int ELEM_ROWS = TYPE == 0 ? 2 : TYPE == 1 ? 3 : 1;
+template <int TYPE>
+__device__ inline int elem_dx(const ElemArgs& a, int c, const double* __restrict__ x, float3 (&dx)[ELEM_ROWS<TYPE>], float* w) {
+    if constexpr (TYPE == 0) {
         int4 t = a.tri_v[c];
         float4 B = a.tri_binv[c]; // row-major 2x2
+        *w = a.tri_w[c];
         const double3 xa = ld3(x, t.x);
         const float3 e1 = to_f3(ld3(x, t.y) - xa), e2 = to_f3(ld3(x, t.z) - xa);
         dx[0] = B.x * e1 + B.z * e2;
         dx[1] = B.y * e1 + B.w * e2;
-        *row0 = a.tri_row0 + 2 * c;
-        *w = a.tri_w[c];
-        return 2;
-    }
-    if (type == 1) {
+        return a.tri_row0 + 2 * c;
+    } else if constexpr (TYPE == 1) {
         int4 t = a.tet_v[c];
         const float* B = a.tet_binv + 9 * c; // row-major 3x3
+        *w = a.tet_w[c];
         const double3 xa = ld3(x, t.x);
         const float3 e1 = to_f3(ld3(x, t.y) - xa), e2 = to_f3(ld3(x, t.z) - xa), e3 = to_f3(ld3(x, t.w) - xa);
 #pragma unroll
         for (int r = 0; r < 3; r++) dx[r] = (B[r] * e1 + B[3 + r] * e2) + B[6 + r] * e3;
-        *row0 = a.tet_row0 + 3 * c;
-        *w = a.tet_w[c];
-        return 3;
-    }
-    if (type == 2) {
+        return a.tet_row0 + 3 * c;
+    } else if constexpr (TYPE == 2) {
         // sum_e coef_e x_e = sum_e coef_e (x_e - x_ref) + (sum_e coef_e) x_ref with
         // the row sum in FP64: the FP32 coefficients then multiply only
-        // differences of nearby positions
+        // differences of nearby positions.  The ring is read four entries at a
+        // time (a padded entry has coefficient 0 and the reference vertex).
         const int e0 = a.bend_ptr[c], e1 = a.bend_ptr[c + 1];
-        const double3 xr = e1 > e0 ? ld3(x, a.bend_idx[e0]) : d3(0.0, 0.0, 0.0);
-        double3 s = a.bend_sum[c] * xr;
-        for (int e = e0 + 1; e < e1; e++) s = s + (double)a.bend_coef[e] * (ld3(x, a.bend_idx[e]) - xr);
-        dx[0] = to_f3(s);
-        *row0 = a.bend_row0 + c;
         *w = a.bend_w[c];
-        return 1;
+        const int ref = e1 > e0 ? a.bend_idx[e0] : 0;
+        const double3 xr = e1 > e0 ? ld3(x, ref) : d3(0.0, 0.0, 0.0);
+        double3 s = a.bend_sum[c] * xr;
+        for (int e = e0 + 1; e < e1; e += 4) {
+            int id[4];
+            float cf[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                id[u] = e + u < e1 ? a.bend_idx[e + u] : ref;
+                cf[u] = e + u < e1 ? a.bend_coef[e + u] : 0.f;
+            }
+            double3 q[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) q[u] = ld3(x, id[u]);
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (e + u < e1) s = s + (double)cf[u] * (q[u] - xr);
+        }
+        dx[0] = to_f3(s);
+        return a.bend_row0 + c;
+    } else {
+        *w = a.pin_w[c];
+        dx[0] = to_f3(ld3(x, a.pin_v[c]) - ld3(a.pin_pos, c));
+        return a.pin_row0 + c;
     }
-    dx[0] = to_f3(ld3(x, a.pin_v[c]) - ld3(a.pin_pos, c));
-    *row0 = a.pin_row0 + c;
-    *w = a.pin_w[c];
-    return 1;
 }
 
 // Stiefel polar factor of F = [y0 y1] (3x2): P = F (F^T F)^{-1/2}, using the
@@ -367,52 +385,68 @@ __device__ inline void prox_tet(float3& y0, float3& y1, float3& y2) {
     y2 = 0.5f * (r2 + y2);
 }
 
-// z = prox(D x + Ue); zprev <- previous z (zero on the first iteration).  A
-// pin row's prox is its target, which is 0 in the relative form of elem_dx.
-__global__ void __launch_bounds__(BLK) k_local(ElemArgs a, int first_iter, const double* __restrict__ x, const float* __restrict__ Ue,
-                                               float* __restrict__ z, float* __restrict__ zprev) {
-    int c;
-    int type = elem_of(a, &c);
-    if (type < 0) return;
-    float3 y[3];
-    int row0;
+// The elastic part of the iterations, one pass over the constraints at a
+// given x.  DUAL (the end of iteration k): Ue += D x - z, and with want_res the
+// residual sums w^2 |Dx - z|^2 and w^2 |Dx|^2 into part[blk*6 + 0..1] (for a
+// pin row |Dx|^2 is the absolute |x_v|^2, as D x = x_v in the residual's
+// definition).  LOCAL (the start of iteration k + 1, at the same x):
+// z = prox(D x + Ue), zprev <- the old z where it is wanted; a pin row's prox is
+// its target, which is 0 in the relative form of elem_dx.  Both together read
+// the constraint, its vertices, z and Ue once: 25 us per iteration at 256x256
+// vertices against 22 us for each of the two as a pass of its own.
+enum { ELEM_DUAL = 1, ELEM_LOCAL = 2 };
+template <int MODE, int TYPE>
+__device__ inline void elem_pass(const ElemArgs& a, int c, bool keep, const double* __restrict__ x, float* __restrict__ Ue,
+                                 float* __restrict__ z, float* __restrict__ zprev, double (&acc)[2]) {
+    constexpr int NR = ELEM_ROWS<TYPE>;
+    float3 dx[NR], u[NR], zz[NR];
     float w;
-    int nr = elem_dx(a, type, c, x, y, &row0, &w);
-    for (int r = 0; r < nr; r++) {
-        y[r] = y[r] + ld3(Ue, row0 + r);
-        st3(zprev, row0 + r, first_iter ? f3(0.f, 0.f, 0.f) : ld3(z, row0 + r));
+    const int row0 = elem_dx<TYPE>(a, c, x, dx, &w);
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        u[r] = ld3(Ue, row0 + r);
+        if constexpr ((MODE & ELEM_DUAL) != 0) zz[r] = ld3(z, row0 + r);
     }
-    if (type == 0) prox_tri(y[0], y[1]);
-    else if (type == 1) prox_tet(y[0], y[1], y[2]);
-    else if (type == 2) y[0] = 0.5f * y[0];
-    else y[0] = f3(0.f, 0.f, 0.f);
-    for (int r = 0; r < nr; r++) st3(z, row0 + r, y[r]);
-}
-
-// Ue += D x - z; residual sums w^2 |Dx - z|^2 and w^2 |Dx|^2 into part[blk*6 + 0..1]
-// (for a pin row |Dx|^2 is the absolute |x_v|^2, as D x = x_v in the residual's definition).
-__global__ void __launch_bounds__(BLK) k_dual_elem(ElemArgs a, int want_res, const double* __restrict__ x, const float* __restrict__ z,
-                                                   float* __restrict__ Ue, double* __restrict__ part, const int32_t* __restrict__ stop) {
-    const bool keep = stop && stop[0]; // the iteration runs past the stop: Ue stays
-    int c;
-    int type = elem_of(a, &c);
-    double acc[2] = {0, 0};
-    if (type >= 0) {
-        float3 dx[3];
-        int row0;
-        float w;
-        int nr = elem_dx(a, type, c, x, dx, &row0, &w);
-        for (int r = 0; r < nr; r++) {
-            float3 zz = ld3(z, row0 + r);
-            float3 d = dx[r] - zz;
-            if (!keep) st3(Ue, row0 + r, ld3(Ue, row0 + r) + d);
-            double w2 = (double)w * (double)w;
+    if constexpr ((MODE & ELEM_DUAL) != 0) {
+#pragma unroll
+        for (int r = 0; r < NR; r++) {
+            const float3 d = dx[r] - zz[r];
+            u[r] = u[r] + d;
+            if (!keep) st3(Ue, row0 + r, u[r]);
+            if ((MODE & ELEM_LOCAL) && zprev) st3(zprev, row0 + r, zz[r]);
+            const double w2 = (double)w * (double)w;
             acc[0] += w2 * (((double)d.x * d.x + (double)d.y * d.y) + (double)d.z * d.z);
-            const double3 da = type == 3 ? ld3(x, a.pin_v[c]) : to_d3(dx[r]);
+            const double3 da = TYPE == 3 ? ld3(x, a.pin_v[c]) : to_d3(dx[r]);
             acc[1] += w2 * ((da.x * da.x + da.y * da.y) + da.z * da.z);
         }
     }
-    if (want_res) block_sum_write<2>(acc, part, 6, 0, xcd_block_chunked<32>());
+    if constexpr ((MODE & ELEM_LOCAL) != 0) {
+        float3 y[NR];
+#pragma unroll
+        for (int r = 0; r < NR; r++) y[r] = dx[r] + u[r];
+        if constexpr (TYPE == 0) prox_tri(y[0], y[1]);
+        else if constexpr (TYPE == 1) prox_tet(y[0], y[1], y[2]);
+        else if constexpr (TYPE == 2) y[0] = 0.5f * y[0];
+        else y[0] = f3(0.f, 0.f, 0.f);
+#pragma unroll
+        for (int r = 0; r < NR; r++) st3(z, row0 + r, y[r]);
+    }
+}
+
+template <int MODE>
+__global__ void __launch_bounds__(BLK) k_elem(ElemArgs a, int want_res, const double* __restrict__ x, float* __restrict__ Ue,
+                                              float* __restrict__ z, float* __restrict__ zprev, double* __restrict__ part,
+                                              const int32_t* __restrict__ stop) {
+    const bool keep = stop && stop[0]; // the iteration runs past the stop: Ue stays
+    int c;
+    const int type = elem_of(a, &c);
+    double acc[2] = {0, 0};
+    if (type == 0) elem_pass<MODE, 0>(a, c, keep, x, Ue, z, zprev, acc);
+    else if (type == 1) elem_pass<MODE, 1>(a, c, keep, x, Ue, z, zprev, acc);
+    else if (type == 2) elem_pass<MODE, 2>(a, c, keep, x, Ue, z, zprev, acc);
+    else if (type == 3) elem_pass<MODE, 3>(a, c, keep, x, Ue, z, zprev, acc);
+    if constexpr ((MODE & ELEM_DUAL) != 0)
+        if (want_res) block_sum_write<2>(acc, part, 6, 0, xcd_block_chunked<32>());
 }
 
 // ---------------------------------------------------------------------------
@@ -499,30 +533,33 @@ __global__ void k_contact_rank(int nc, int n, const int4* __restrict__ cv, const
     erun[e] = rank == 0 ? make_int2(v, end) : make_int2(-1, 0);
 }
 
-__device__ inline float3 gather_contacts(int i, const uint32_t* __restrict__ vptr, const uint32_t* __restrict__ vent,
-                                         const float4* __restrict__ G, const float4* __restrict__ src) {
-    float3 s = f3(0.f, 0.f, 0.f);
-    for (uint32_t e = vptr[i]; e < vptr[i + 1]; e++) {
-        uint32_t ent = vent[e];
-        uint32_t c = ent >> 2, k = ent & 3u;
-        float4 g = G[c];
-        float gk = k == 0 ? g.x : (k == 1 ? g.y : (k == 2 ? g.z : g.w));
-        float4 d = src[c];
-        s = s + gk * f3(d.x, d.y, d.z);
-    }
-    return s;
-}
-
-// p = (x - x0 + Uc) / h, then p += Gamma r_c (dynamic vertices).
-__global__ void k_vertex_p(int n, float hinv, int have_contacts, const double* __restrict__ x, const double* __restrict__ x0,
-                           const float* __restrict__ Uc, float* __restrict__ p, const uint32_t* __restrict__ vptr,
+// p += Gamma r_c on the vertices with contacts (p holds (x - x0 + Uc) / h from
+// k_begin_step or k_dual_vert), one lane per entry of the sorted list: the lane
+// of a vertex's first entry sums its run in contact order, four entries read
+// at a time.
+__global__ void k_vertex_p(int ne_max, int n, float* __restrict__ p, const uint32_t* __restrict__ vptr, const int2* __restrict__ erun,
                            const uint32_t* __restrict__ vent, const float4* __restrict__ G, const float4* __restrict__ rc) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    float3 pi = to_f3(ld3(x, i) - ld3(x0, i)) + ld3(Uc, i);
-    pi = hinv * pi;
-    if (have_contacts) pi = pi + gather_contacts(i, vptr, vent, G, rc);
-    st3(p, i, pi);
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= ne_max) return;
+    const int ne = (int)vptr[n];
+    const int2 run = erun[e];
+    if (e >= ne || run.x < 0) return;
+    const float3 pv = ld3(p, run.x);
+    float3 s = f3(0.f, 0.f, 0.f);
+    for (int q = e; q < run.y; q += 4) {
+        float gk[4];
+        float4 d[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const uint32_t ent = vent[min(q + u, run.y - 1)];
+            gk[u] = reinterpret_cast<const float*>(G)[ent]; // Gamma of (contact ent / 4, vertex ent % 4)
+            d[u] = rc[ent >> 2];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+            if (q + u < run.y) s = s + gk[u] * f3(d[u].x, d[u].y, d[u].z);
+    }
+    st3(p, run.x, pv + s);
 }
 
 // The friction-cone projection of one contact with barycentric weights b, its
@@ -929,37 +966,107 @@ __global__ void k_ws_log(int nc, float s, const float* __restrict__ feat, const 
     o[11] = s * ((r.x * t4.x + r.y * t4.y) + r.z * t4.z);
 }
 
+// System matrix rows for the residual of the global solve (off-diagonal CSR
+// and diagonal, A = hi + lo), and where r goes.
+struct ResidArgs {
+    const int32_t* ptr;
+    const int32_t* col;
+    const float *val, *val_lo, *diag, *diag_lo;
+    const double* x;
+    float* r;
+};
+
 // b = bconst + sum_e coef_e (z - Ue)[row_e] + h^2 wc (h p + x0 - Uc), accumulated in FP64.
 // With want_res, also |sum coef (z - zprev)|^2 and |sum coef z|^2 into part[blk*6 + 4..5],
 // with the pins' targets (bpin) added back to z (and to z - zprev on the
 // first iteration, where zprev is 0), as the pin rows of z are relative.
 // LPR lanes share a vertex (each takes every LPR-th entry of its D^T row
-// list) and combine with shuffles, so a vertex's dependent gathers of z and
-// Ue are spread over LPR lanes.
-template <int LPR>
-__global__ void __launch_bounds__(BLK) k_rhs(int n, float h, int contact, int want_res, int first_iter, const int32_t* __restrict__ dt_ptr,
+// list, RU at a time) and combine with shuffles, so a vertex's dependent
+// gathers of z and Ue are spread over LPR lanes.
+// RESID (the direct solve): the row's residual r = b - A x in FP64 as well, so
+// that b need not go through memory (store_b: later refinement passes read it).
+// Both sums of a row are chains of dependent loads of like length; the matrix
+// row's are issued first and its vertices arrive during the gather of z and Ue.
+// At 256x256 vertices 25 us against 22 + 13 us in two launches, at 16x16 6
+// against 5 + 9 (k_cg_resid64 also forms the norms that only PCG uses).
+constexpr int RU = 3;
+template <int LPR, bool RESID>
+__global__ void __launch_bounds__(BLK) k_rhs(int n, float h, int contact, int want_res, int first_iter, int store_b,
+                                             const int32_t* __restrict__ dt_ptr,
                                              const int32_t* __restrict__ dt_row, const float* __restrict__ dt_coef,
                                              const float* __restrict__ z, const float* __restrict__ zprev, const float* __restrict__ Ue,
                                              const double* __restrict__ bconst, const double* __restrict__ wch2, const float* __restrict__ p,
                                              const double* __restrict__ x0, const float* __restrict__ Uc, const double* __restrict__ bpin,
-                                             double* __restrict__ b, double* __restrict__ part) {
+                                             double* __restrict__ b, double* __restrict__ part, ResidArgs A) {
     // XCD-contiguous numbering: neighbouring vertices gather shared rows from one L2
     const int t = xcd_block() * blockDim.x + threadIdx.x;
     const int i = t / LPR, sub = t % LPR;
     double acc[2] = {0, 0};
-    double s[3] = {0, 0, 0}, s1[3] = {0, 0, 0}, s2[3] = {0, 0, 0};
+    double s[3] = {0, 0, 0}, s1[3] = {0, 0, 0}, s2[3] = {0, 0, 0}, ax[3] = {0, 0, 0};
     if (i < n) {
-        for (int e = dt_ptr[i] + sub; e < dt_ptr[i + 1]; e += LPR) {
-            const int r = dt_row[e];
-            const double cf = dt_coef[e];
+        int ae0 = 0, ae1 = 0;
+        double av[RU], xv[RU][3];
+        if (RESID) {
+            ae0 = A.ptr[i] + sub;
+            ae1 = A.ptr[i + 1];
 #pragma unroll
-            for (int a = 0; a < 3; a++) {
-                const double zr = z[3 * r + a];
-                s[a] += cf * (zr - (double)Ue[3 * r + a]);
-                if (want_res) {
-                    s1[a] += cf * (zr - (double)zprev[3 * r + a]);
-                    s2[a] += cf * zr;
+            for (int u = 0; u < RU; u++) {
+                const int e = ae0 + u * LPR;
+                const int c = e < ae1 ? A.col[e] : i;
+                av[u] = e < ae1 ? (double)A.val[e] + (double)A.val_lo[e] : 0.0;
+#pragma unroll
+                for (int a = 0; a < 3; a++) xv[u][a] = A.x[3 * c + a];
+            }
+        }
+        const int e1 = dt_ptr[i + 1];
+        for (int e0 = dt_ptr[i] + sub; e0 < e1; e0 += RU * LPR) {
+            int r[RU];
+            double cf[RU];
+#pragma unroll
+            for (int u = 0; u < RU; u++) {
+                const int e = e0 + u * LPR;
+                r[u] = dt_row[min(e, e1 - 1)];
+                cf[u] = e < e1 ? (double)dt_coef[e] : 0.0;
+            }
+            float zr[RU][3], ur[RU][3], pr[RU][3];
+#pragma unroll
+            for (int u = 0; u < RU; u++)
+#pragma unroll
+                for (int a = 0; a < 3; a++) {
+                    zr[u][a] = z[3 * r[u] + a];
+                    ur[u][a] = Ue[3 * r[u] + a];
+                    pr[u][a] = want_res && !first_iter ? zprev[3 * r[u] + a] : 0.f;
                 }
+#pragma unroll
+            for (int u = 0; u < RU; u++)
+                if (e0 + u * LPR < e1)
+#pragma unroll
+                    for (int a = 0; a < 3; a++) {
+                        s[a] += cf[u] * ((double)zr[u][a] - (double)ur[u][a]);
+                        if (want_res) {
+                            s1[a] += cf[u] * ((double)zr[u][a] - (double)pr[u][a]);
+                            s2[a] += cf[u] * (double)zr[u][a];
+                        }
+                    }
+        }
+        if (RESID) {
+#pragma unroll
+            for (int u = 0; u < RU; u++)
+#pragma unroll
+                for (int a = 0; a < 3; a++) ax[a] += av[u] * xv[u][a];
+            for (int e0 = ae0 + RU * LPR; e0 < ae1; e0 += RU * LPR) {
+#pragma unroll
+                for (int u = 0; u < RU; u++) {
+                    const int e = e0 + u * LPR;
+                    const int c = e < ae1 ? A.col[e] : i;
+                    av[u] = e < ae1 ? (double)A.val[e] + (double)A.val_lo[e] : 0.0;
+#pragma unroll
+                    for (int a = 0; a < 3; a++) xv[u][a] = A.x[3 * c + a];
+                }
+#pragma unroll
+                for (int u = 0; u < RU; u++)
+#pragma unroll
+                    for (int a = 0; a < 3; a++) ax[a] += av[u] * xv[u][a];
             }
         }
     }
@@ -968,6 +1075,7 @@ __global__ void __launch_bounds__(BLK) k_rhs(int n, float h, int contact, int wa
 #pragma unroll
         for (int a = 0; a < 3; a++) {
             s[a] += __shfl_xor(s[a], o, LPR);
+            if (RESID) ax[a] += __shfl_xor(ax[a], o, LPR);
             if (want_res) {
                 s1[a] += __shfl_xor(s1[a], o, LPR);
                 s2[a] += __shfl_xor(s2[a], o, LPR);
@@ -975,11 +1083,13 @@ __global__ void __launch_bounds__(BLK) k_rhs(int n, float h, int contact, int wa
         }
     if (i < n && sub == 0) {
         const double wv = contact ? wch2[i] : 0.0;
+        const double di = RESID ? (double)A.diag[i] + (double)A.diag_lo[i] : 0.0;
 #pragma unroll
         for (int a = 0; a < 3; a++) {
             double bi = bconst[3 * i + a] + s[a];
             if (wv != 0.0) bi += wv * (((double)h * p[3 * i + a] + x0[3 * i + a]) - (double)Uc[3 * i + a]);
-            b[3 * i + a] = bi;
+            if (!RESID || store_b) b[3 * i + a] = bi;
+            if (RESID) A.r[3 * i + a] = (float)(bi - (ax[a] + di * A.x[3 * i + a]));
         }
         if (want_res) {
 #pragma unroll
@@ -998,9 +1108,9 @@ __global__ void __launch_bounds__(BLK) k_rhs(int n, float h, int contact, int wa
 // Uc += x - x0 - h p; residual sums wc |x - x0 - h p|^2, wc |x - x0|^2 into part[blk*6 + 2..3].
 // With dxg non-null the global solve's last correction is applied here
 // first: x += dxg (what k_axpy_d would have done), then the dual update on the
-// new x.
-__global__ void __launch_bounds__(BLK) k_dual_vert(int n, float h, int contact, int want_res, double* __restrict__ x,
-                                                   const double* __restrict__ x0, const float* __restrict__ p, const double* __restrict__ wch2,
+// new x.  p becomes the next iteration's (x - x0 + Uc) / h.
+__global__ void __launch_bounds__(BLK) k_dual_vert(int n, float h, float hinv, int contact, int want_res, double* __restrict__ x,
+                                                   const double* __restrict__ x0, float* __restrict__ p, const double* __restrict__ wch2,
                                                    float* __restrict__ Uc, double* __restrict__ part, double h2inv,
                                                    const int32_t* __restrict__ stop, const float* __restrict__ dxg) {
     const bool keep = stop && stop[0]; // the iteration runs past the stop: x and Uc stay
@@ -1013,7 +1123,9 @@ __global__ void __launch_bounds__(BLK) k_dual_vert(int n, float h, int contact, 
     if (i < n && contact) {
         const float3 dx = to_f3(ld3(x, i) - ld3(x0, i));
         float3 d = dx - h * ld3(p, i);
-        if (!keep) st3(Uc, i, ld3(Uc, i) + d);
+        const float3 uc = ld3(Uc, i) + d;
+        if (!keep) st3(Uc, i, uc);
+        st3(p, i, hinv * (dx + uc));
         const double w = wch2[i] * h2inv;
         if (want_res && w != 0.0) {
             acc[0] = w * (((double)d.x * d.x + (double)d.y * d.y) + (double)d.z * d.z);
@@ -1028,7 +1140,7 @@ __global__ void __launch_bounds__(BLK) k_dual_vert(int n, float h, int contact, 
 // residual sqrt(s4) / max(1, sqrt(s5)).  With stop non-null, a residual
 // max(r_p, r_d) <= tol sets stop[0] (the iterations enqueued after this one
 // then leave the state alone), and a check after that leaves out untouched.
-// Component pair q of the partials (0-1 k_dual_elem, 2-3 k_dual_vert, 4-5
+// Component pair q of the partials (0-1 k_elem, 2-3 k_dual_vert, 4-5
 // k_rhs) is read from its kernel's first nq[q] blocks only, so the slots need
 // no clearing between checks (the skipped slots would add zeros).
 __global__ void __launch_bounds__(BLK) k_resid_final(const double* __restrict__ part, int3 nq, double* __restrict__ out, double tol,
@@ -1076,7 +1188,6 @@ template <int LPR> __device__ inline float3 group_sum(float3 s) {
 // (ptr -> col/val -> gathered vector) instead of one per entry.  Unused slots
 // pass value 0 and column 0, an index every matrix here has (the row index
 // would not do: the prolongators have more rows than columns).
-constexpr int RU = 3;
 template <int LPR, class F>
 __device__ inline void row_foreach(int i, int rows, int sub, const int32_t* __restrict__ ptr, const int32_t* __restrict__ col,
                                    const float* __restrict__ val, F&& f) {
@@ -2895,29 +3006,35 @@ static ElemArgs make_elem_args(const Backend& B) {
 
 static int elem_grid(const ElemArgs& a, int n_pin) { return a.blk_bend + grid_for(n_pin, BLK); }
 
-void Backend::local_step(bool first_iter, hipStream_t s) {
+// z = prox(D x + Ue) at the step's first x.
+void Backend::local_step(hipStream_t s) {
     ElemArgs a = make_elem_args(*this);
     int g = elem_grid(a, hc.n_pin);
     if (g == 0) return;
-    hipLaunchKernelGGL(k_local, dim3(g), dim3(BLK), 0, s ? s : stream, a, first_iter ? 1 : 0, x.p, Ue.p, z.p, zprev.p);
+    hipLaunchKernelGGL(k_elem<ELEM_LOCAL>, dim3(g), dim3(BLK), 0, s ? s : stream, a, 0, x.p, Ue.p, z.p, (float*)nullptr, (double*)nullptr,
+                       (const int32_t*)nullptr);
     PA_LAUNCH_CHECK();
 }
 
-// k_dual_vert first: it also applies a deferred global-solve correction to x,
-// which k_dual_elem then reads.
-void Backend::dual_update(bool want_res) {
-    ElemArgs a = make_elem_args(*this);
-    int g = elem_grid(a, hc.n_pin);
-    hipLaunchKernelGGL(k_dual_vert, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, n, (float)cfg.dt, cfg.enable_contact, want_res ? 1 : 0,
-                       x.p, x0.p, p.p, wch2.p, Uc.p, res_part.p, 1.0 / (cfg.dt * cfg.dt), (const int32_t*)stop_guard,
-                       dx_pending ? (const float*)cg_d.p : nullptr);
+// Applies a deferred global-solve correction to x as well, which elem_update
+// then reads.
+void Backend::dual_vertices(bool want_res) {
+    hipLaunchKernelGGL(k_dual_vert, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, n, (float)cfg.dt, (float)(1.0 / cfg.dt),
+                       cfg.enable_contact, want_res ? 1 : 0, x.p, x0.p, p.p, wch2.p, Uc.p, res_part.p, 1.0 / (cfg.dt * cfg.dt),
+                       (const int32_t*)stop_guard, dx_pending ? (const float*)cg_d.p : nullptr);
     PA_LAUNCH_CHECK();
     dx_pending = false;
-    if (g > 0) {
-        hipLaunchKernelGGL(k_dual_elem, dim3(g), dim3(BLK), 0, stream, a, want_res ? 1 : 0, x.p, z.p, Ue.p, res_part.p,
-                           (const int32_t*)stop_guard);
-        PA_LAUNCH_CHECK();
-    }
+}
+
+// The elastic dual update of this iteration and, unless it is the last, the
+// local step of the next one (next_check: that one's residual needs zprev).
+void Backend::elem_update(bool want_res, bool last, bool next_check, hipStream_t s) {
+    ElemArgs a = make_elem_args(*this);
+    const int g = elem_grid(a, hc.n_pin);
+    if (g == 0) return;
+    hipLaunchKernelGGL((last ? k_elem<ELEM_DUAL> : k_elem<ELEM_DUAL | ELEM_LOCAL>), dim3(g), dim3(BLK), 0, s, a, want_res ? 1 : 0, x.p, Ue.p,
+                       z.p, next_check ? zprev.p : (float*)nullptr, res_part.p, (const int32_t*)stop_guard);
+    PA_LAUNCH_CHECK();
 }
 
 // counted: the detection has filled vcnt and vloc.
@@ -2942,19 +3059,17 @@ void Backend::contact_setup(float eps, float gamma_, float hinv, bool counted) {
 }
 
 void Backend::contact_project(bool) {
-    const float hinv = (float)(1.0 / cfg.dt);
-    const bool wg = nc > 0 && nc <= contact_wg_max; // the whole projection in one workgroup: no launch per sweep
-    hipLaunchKernelGGL(k_vertex_p, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, n, hinv, nc > 0 && !wg ? 1 : 0, x.p, x0.p, Uc.p, p.p,
-                       vptr.p, vent.p, gam.p, rc.p);
-    PA_LAUNCH_CHECK();
-    if (wg) {
+    if (nc == 0) return;
+    if (nc <= contact_wg_max) { // the whole projection in one workgroup: no launch per sweep
         hipLaunchKernelGGL((nc <= 1024 ? k_contact_sweeps_wg<1> : k_contact_sweeps_wg<2>), dim3(1), dim3(1024), 0, stream, nc, n,
                            cfg.gs_max_iter, det->c.v.p, det->c.bary.p, det->c.nrm.p, kc.p, p.p, rc.p, (const float4*)gam.p,
                            (const int4*)cslot.p, (const uint32_t*)vptr.p, (const int2*)erun.p, (const int32_t*)stop_guard);
         PA_LAUNCH_CHECK();
         return;
     }
-    if (nc == 0) return;
+    hipLaunchKernelGGL(k_vertex_p, dim3(grid_for(4 * (int64_t)nc, BLK)), dim3(BLK), 0, stream, 4 * nc, n, p.p, (const uint32_t*)vptr.p,
+                       (const int2*)erun.p, (const uint32_t*)vent.p, (const float4*)gam.p, (const float4*)rc.p);
+    PA_LAUNCH_CHECK();
     for (int g = 0; g < cfg.gs_max_iter; g++) contact_sweep_once();
 }
 
@@ -2967,12 +3082,16 @@ void Backend::contact_sweep_once() {
     PA_LAUNCH_CHECK();
 }
 
+// The right-hand side, and with the direct solve also the residual of its
+// first pass (cg_r): global_solve then starts from it.
 void Backend::rhs(bool want_res, bool first_iter) {
+    const ResidArgs A{a_ptr.p, a_col.p, a_val.p, a_val_lo.p, a_diag.p, a_diag_lo.p, x.p, cg_r.p};
+    const int store_b = cfg.global_refine > 1 ? 1 : 0;
     with_lpr(rhs_lpr, [&](auto c) {
         constexpr int P = decltype(c)::value;
-        hipLaunchKernelGGL(k_rhs<P>, dim3(grid_for((int64_t)n * P, BLK)), dim3(BLK), 0, stream, n, (float)cfg.dt, cfg.enable_contact,
-                           want_res ? 1 : 0, first_iter ? 1 : 0, dt_ptr.p, dt_row.p, dt_coef.p, z.p, zprev.p, Ue.p, bconst.p, wch2.p,
-                           p.p, x0.p, Uc.p, bpin.p, b.p, res_part.p);
+        hipLaunchKernelGGL((use_chol ? k_rhs<P, true> : k_rhs<P, false>), dim3(grid_for((int64_t)n * P, BLK)), dim3(BLK), 0, stream, n,
+                           (float)cfg.dt, cfg.enable_contact, want_res ? 1 : 0, first_iter ? 1 : 0, store_b, dt_ptr.p, dt_row.p, dt_coef.p,
+                           z.p, zprev.p, Ue.p, bconst.p, wch2.p, p.p, x0.p, Uc.p, bpin.p, b.p, res_part.p, A);
     });
     PA_LAUNCH_CHECK();
 }
@@ -3479,7 +3598,7 @@ void Backend::chol_solve(const float* r, float* d) {
     }
 }
 
-int Backend::global_solve(int max_iter, double tol, bool defer_last) {
+int Backend::global_solve(int max_iter, double tol, bool defer_last, bool resid_ready) {
     const int nb = cg_blocks;
     const int passes = std::max(1, cfg.global_refine);
     // the fused iteration needs a real level 0 (nl >= 2); a one-level
@@ -3501,12 +3620,14 @@ int Backend::global_solve(int max_iter, double tol, bool defer_last) {
     };
     if (use_chol) { // direct solve: each pass applies the factor to the FP64 residual, no read-back
         for (int pass = 0; pass < passes; pass++) {
-            with_lpr(a_lpr, [&](auto c) {
-                constexpr int P = decltype(c)::value;
-                hipLaunchKernelGGL(k_cg_resid64<P>, dim3(nb), dim3(PBLK), 0, stream, n, a_ptr.p, a_col.p, a_val.p, a_val_lo.p,
-                                   a_diag.p, a_diag_lo.p, b.p, x.p, cg_r.p, cg_d.p, cg_part.p);
-            });
-            PA_LAUNCH_CHECK();
+            if (pass > 0 || !resid_ready) {
+                with_lpr(a_lpr, [&](auto c) {
+                    constexpr int P = decltype(c)::value;
+                    hipLaunchKernelGGL(k_cg_resid64<P>, dim3(nb), dim3(PBLK), 0, stream, n, a_ptr.p, a_col.p, a_val.p, a_val_lo.p,
+                                       a_diag.p, a_diag_lo.p, b.p, x.p, cg_r.p, cg_d.p, cg_part.p);
+                });
+                PA_LAUNCH_CHECK();
+            }
             chol_solve(cg_r.p, cg_d.p);
             if (defer_last && pass == passes - 1) { // x += d is applied by the next dual update
                 dx_pending = true;
@@ -3582,8 +3703,8 @@ int Backend::global_solve(int max_iter, double tol, bool defer_last) {
     return total_iters;
 }
 
-// Blocks of the three kernels that write the residual partials (k_dual_elem,
-// k_dual_vert, k_rhs), as launched by dual_update and rhs.
+// Blocks of the three kernels that write the residual partials (k_elem,
+// k_dual_vert, k_rhs), as launched by elem_update, dual_vertices and rhs.
 int3 Backend::resid_blocks() {
     ElemArgs a = make_elem_args(*this);
     return make_int3(elem_grid(a, hc.n_pin), grid_for(n, BLK), grid_for((int64_t)n * rhs_lpr, BLK));
@@ -3899,15 +4020,15 @@ void Backend::step_impl(pa_step_stats* st) {
         ws_active = can_warm && attempt == 0;
         hipEvent_t e;
         mark_begin(5, &e);
-        hipLaunchKernelGGL(k_begin_step, dim3(grid_for(n_all, BLK)), dim3(BLK), 0, stream, n_all, n, hd, cfg.g, pinned.p, x.p, v.p, x0.p,
-                           p.p, bconst.p, mass.p, (const double*)bpin.p);
+        if (!cfg.warmstart_ue) fill<float>(Ue.p, 0.f, 3 * (int64_t)m, stream);
+        if (!cfg.warmstart_uc) fill<float>(Uc.p, 0.f, 3 * (int64_t)n, stream);
+        hipLaunchKernelGGL(k_begin_step, dim3(grid_for(n_all, BLK)), dim3(BLK), 0, stream, n_all, n, hd, hinv, cfg.g, pinned.p, x.p, v.p, x0.p,
+                           p.p, bconst.p, mass.p, (const double*)bpin.p, (const float*)Uc.p);
         PA_LAUNCH_CHECK();
         if (nnz_dm > 0) {
             hipLaunchKernelGGL(k_spmv_add, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, n, dm_ptr.p, dm_col.p, dm_val.p, x0.p, bconst.p);
             PA_LAUNCH_CHECK();
         }
-        if (!cfg.warmstart_ue) fill<float>(Ue.p, 0.f, 3 * (int64_t)m, stream);
-        if (!cfg.warmstart_uc) fill<float>(Uc.p, 0.f, 3 * (int64_t)n, stream);
         mark_end(5, e);
         it = admm_loop(S, eps, gam_, hinv);
         if (!ws_restart) break;
@@ -3966,15 +4087,26 @@ int Backend::admm_loop(pa_step_stats& S, float eps, float gam_, float hinv) {
     res_log.clear(); // this attempt's checks
     double best = std::numeric_limits<double>::infinity();
     int it = 0;
-    // The elastic local step (z from x, Ue) and the contact phase (detection,
+    // The elastic part (Ue and z from x) and the contact phase (detection,
     // projection: p from x, x0, Uc) are independent until the right-hand
-    // side: the local step runs on the side stream beside them.  Phase
-    // timing (profiling bit 1) keeps them in sequence.
+    // side: the elastic pass runs on the side stream beside them.  Where an
+    // iteration is checked its elastic pass stays on the main stream, before
+    // the check (which must precede every later write).  Phase timing
+    // (profiling bit 1) keeps them in sequence.
     const bool overlap = !(profiling & 2);
+    bool side_busy = false;
+    auto fork = [&]() {
+        PA_HIP(hipEventRecord(ev_fork, stream));
+        PA_HIP(hipStreamWaitEvent(side, ev_fork, 0));
+        side_busy = true;
+    };
     auto join = [&]() {
+        if (!side_busy) return;
+        side_busy = false;
         PA_HIP(hipEventRecord(ev_join, side));
         PA_HIP(hipStreamWaitEvent(stream, ev_join, 0));
     };
+    auto checked = [&](int q) { return cfg.residual_tol > 0 && (q + 1) % cfg.residual_interval == 0; };
     // Stop test on the device (direct solve, no learned warm start): the
     // check of iteration q is read back once iteration q + 1 is enqueued, or
     // before a detection, so the queue does not drain at every check.  An
@@ -4008,24 +4140,22 @@ int Backend::admm_loop(pa_step_stats& S, float eps, float gam_, float hinv) {
                 break; // it == q + 1
             }
         }
-        if (overlap) {
-            PA_HIP(hipEventRecord(ev_fork, stream));
-            PA_HIP(hipStreamWaitEvent(side, ev_fork, 0));
-            local_step(it == 0, side);
+        if (it == 0 && overlap) {
+            fork();
+            local_step(side);
         }
         if (contact && it % cfg.dcd_interval == 0) {
             mark_begin(0, &e);
             ws_window_end();
             if (ws_restart) {
                 mark_end(0, e);
-                if (overlap) join();
                 break;
             }
             try {
                 // rebuild at the step's first detection, refit later ones
                 det->detect(x.p, it > 0, VertexCount{vcnt.p, vloc.p, n_all});
             } catch (...) {
-                if (overlap) join(); // the rollback writes x, which the side stream reads
+                join(); // the rollback writes x, which the side stream reads
                 throw;
             }
             contact_setup(eps, gam_, hinv, true);
@@ -4034,9 +4164,9 @@ int Backend::admm_loop(pa_step_stats& S, float eps, float gam_, float hinv) {
             S.n_contacts_max = std::max(S.n_contacts_max, nc);
             mark_end(0, e);
         }
-        if (!overlap) {
+        if (it == 0 && !overlap) {
             mark_begin(1, &e);
-            local_step(it == 0);
+            local_step();
             mark_end(1, e);
         }
         if (contact) {
@@ -4044,18 +4174,25 @@ int Backend::admm_loop(pa_step_stats& S, float eps, float gam_, float hinv) {
             contact_project(it == 0);
             mark_end(2, e);
         }
-        if (overlap) join();
-        const bool check = cfg.residual_tol > 0 && ((it + 1) % cfg.residual_interval == 0);
+        join();
+        const bool check = checked(it);
         mark_begin(3, &e);
         rhs(check, it == 0);
         mark_end(3, e);
         mark_begin(4, &e);
         const int gi = (nscene && !use_amg && !use_chol) ? batch_solve(cfg.global_max_iter, cfg.global_tol)
-                                                         : global_solve(cfg.global_max_iter, cfg.global_tol, true);
+                                                         : global_solve(cfg.global_max_iter, cfg.global_tol, true, use_chol);
         S.global_iters += gi;
         mark_end(4, e);
         mark_begin(1, &e);
-        dual_update(check);
+        dual_vertices(check);
+        const bool last = it + 1 >= cfg.admm_max_iter;
+        if (overlap && !check && !last) {
+            fork();
+            elem_update(false, last, checked(it + 1), side);
+        } else {
+            elem_update(check, last, checked(it + 1), stream);
+        }
         mark_end(1, e);
         if (lagged) {
             if (check) residual_enqueue(it);
@@ -4092,6 +4229,7 @@ int Backend::admm_loop(pa_step_stats& S, float eps, float gam_, float hinv) {
             }
         }
     }
+    join();
     if (lagged && pending >= 0 && take_check(pending)) S.converged = 1; // the last iteration's check
     if (ws_active && !ws_restart) ws_judge(); // the last window of the attempt
     return it;
