@@ -392,8 +392,8 @@ __device__ inline void prox_tet(float3& y0, float3& y1, float3& y2) {
 // definition).  LOCAL (the start of iteration k + 1, at the same x):
 // z = prox(D x + Ue), zprev <- the old z where it is wanted; a pin row's prox is
 // its target, which is 0 in the relative form of elem_dx.  Both together read
-// the constraint, its vertices, z and Ue once: 25 us per iteration at 256x256
-// vertices against 22 us for each of the two as a pass of its own.
+// the constraint, its vertices, z and Ue once: 10.4 us per iteration at 256x256
+// vertices against 22.7 + 21.2 us as two passes with a runtime row count.
 enum { ELEM_DUAL = 1, ELEM_LOCAL = 2 };
 template <int MODE, int TYPE>
 __device__ inline void elem_pass(const ElemArgs& a, int c, bool keep, const double* __restrict__ x, float* __restrict__ Ue,
@@ -987,11 +987,14 @@ struct ResidArgs {
 // that b need not go through memory (store_b: later refinement passes read it).
 // Both sums of a row are chains of dependent loads of like length; the matrix
 // row's are issued first and its vertices arrive during the gather of z and Ue.
-// At 256x256 vertices 25 us against 22 + 13 us in two launches, at 16x16 6
-// against 5 + 9 (k_cg_resid64 also forms the norms that only PCG uses).
+// At 256x256 vertices 31 us (checked, RES) against 21.7 + 12.7 us in two
+// launches, at 16x16 5.8 against 4.9 + 9.4 (k_cg_resid64 also forms the norms
+// that only PCG uses), on a 160-scene batch 134 against 110 + 77.  The matrix
+// row is read ahead only without the residual sums: with them it would take
+// 106 registers and half the waves.
 constexpr int RU = 3;
-template <int LPR, bool RESID>
-__global__ void __launch_bounds__(BLK) k_rhs(int n, float h, int contact, int want_res, int first_iter, int store_b,
+template <int LPR, bool RESID, bool RES>
+__global__ void __launch_bounds__(BLK) k_rhs(int n, float h, int contact, int first_iter, int store_b,
                                              const int32_t* __restrict__ dt_ptr,
                                              const int32_t* __restrict__ dt_row, const float* __restrict__ dt_coef,
                                              const float* __restrict__ z, const float* __restrict__ zprev, const float* __restrict__ Ue,
@@ -1001,22 +1004,27 @@ __global__ void __launch_bounds__(BLK) k_rhs(int n, float h, int contact, int wa
     // XCD-contiguous numbering: neighbouring vertices gather shared rows from one L2
     const int t = xcd_block() * blockDim.x + threadIdx.x;
     const int i = t / LPR, sub = t % LPR;
+    constexpr bool AHEAD = RESID && !RES;
     double acc[2] = {0, 0};
     double s[3] = {0, 0, 0}, s1[3] = {0, 0, 0}, s2[3] = {0, 0, 0}, ax[3] = {0, 0, 0};
     if (i < n) {
-        int ae0 = 0, ae1 = 0;
+        // entries ae .. of the matrix row, RU at a time: (value, x of its column)
+        int ae = 0, ae1 = 0;
         double av[RU], xv[RU][3];
-        if (RESID) {
-            ae0 = A.ptr[i] + sub;
-            ae1 = A.ptr[i + 1];
+        auto a_load = [&]() {
 #pragma unroll
             for (int u = 0; u < RU; u++) {
-                const int e = ae0 + u * LPR;
+                const int e = ae + u * LPR;
                 const int c = e < ae1 ? A.col[e] : i;
                 av[u] = e < ae1 ? (double)A.val[e] + (double)A.val_lo[e] : 0.0;
 #pragma unroll
                 for (int a = 0; a < 3; a++) xv[u][a] = A.x[3 * c + a];
             }
+        };
+        if (RESID) {
+            ae = A.ptr[i] + sub;
+            ae1 = A.ptr[i + 1];
+            if (AHEAD) a_load();
         }
         const int e1 = dt_ptr[i + 1];
         for (int e0 = dt_ptr[i] + sub; e0 < e1; e0 += RU * LPR) {
@@ -1035,7 +1043,7 @@ __global__ void __launch_bounds__(BLK) k_rhs(int n, float h, int contact, int wa
                 for (int a = 0; a < 3; a++) {
                     zr[u][a] = z[3 * r[u] + a];
                     ur[u][a] = Ue[3 * r[u] + a];
-                    pr[u][a] = want_res && !first_iter ? zprev[3 * r[u] + a] : 0.f;
+                    pr[u][a] = RES && !first_iter ? zprev[3 * r[u] + a] : 0.f;
                 }
 #pragma unroll
             for (int u = 0; u < RU; u++)
@@ -1043,32 +1051,20 @@ __global__ void __launch_bounds__(BLK) k_rhs(int n, float h, int contact, int wa
 #pragma unroll
                     for (int a = 0; a < 3; a++) {
                         s[a] += cf[u] * ((double)zr[u][a] - (double)ur[u][a]);
-                        if (want_res) {
+                        if (RES) {
                             s1[a] += cf[u] * ((double)zr[u][a] - (double)pr[u][a]);
                             s2[a] += cf[u] * (double)zr[u][a];
                         }
                     }
         }
-        if (RESID) {
-#pragma unroll
-            for (int u = 0; u < RU; u++)
-#pragma unroll
-                for (int a = 0; a < 3; a++) ax[a] += av[u] * xv[u][a];
-            for (int e0 = ae0 + RU * LPR; e0 < ae1; e0 += RU * LPR) {
-#pragma unroll
-                for (int u = 0; u < RU; u++) {
-                    const int e = e0 + u * LPR;
-                    const int c = e < ae1 ? A.col[e] : i;
-                    av[u] = e < ae1 ? (double)A.val[e] + (double)A.val_lo[e] : 0.0;
-#pragma unroll
-                    for (int a = 0; a < 3; a++) xv[u][a] = A.x[3 * c + a];
-                }
+        if (RESID)
+            for (bool loaded = AHEAD; ae < ae1; ae += RU * LPR, loaded = false) {
+                if (!loaded) a_load();
 #pragma unroll
                 for (int u = 0; u < RU; u++)
 #pragma unroll
                     for (int a = 0; a < 3; a++) ax[a] += av[u] * xv[u][a];
             }
-        }
     }
 #pragma unroll
     for (int o = LPR / 2; o > 0; o >>= 1)
@@ -1076,7 +1072,7 @@ __global__ void __launch_bounds__(BLK) k_rhs(int n, float h, int contact, int wa
         for (int a = 0; a < 3; a++) {
             s[a] += __shfl_xor(s[a], o, LPR);
             if (RESID) ax[a] += __shfl_xor(ax[a], o, LPR);
-            if (want_res) {
+            if (RES) {
                 s1[a] += __shfl_xor(s1[a], o, LPR);
                 s2[a] += __shfl_xor(s2[a], o, LPR);
             }
@@ -1091,7 +1087,7 @@ __global__ void __launch_bounds__(BLK) k_rhs(int n, float h, int contact, int wa
             if (!RESID || store_b) b[3 * i + a] = bi;
             if (RESID) A.r[3 * i + a] = (float)(bi - (ax[a] + di * A.x[3 * i + a]));
         }
-        if (want_res) {
+        if (RES) {
 #pragma unroll
             for (int a = 0; a < 3; a++) {
                 const double bp = bpin[3 * i + a];
@@ -1102,7 +1098,7 @@ __global__ void __launch_bounds__(BLK) k_rhs(int n, float h, int contact, int wa
             acc[1] = (s2[0] * s2[0] + s2[1] * s2[1]) + s2[2] * s2[2];
         }
     }
-    if (want_res) block_sum_write<2>(acc, part, 6, 4, xcd_block());
+    if (RES) block_sum_write<2>(acc, part, 6, 4, xcd_block());
 }
 
 // Uc += x - x0 - h p; residual sums wc |x - x0 - h p|^2, wc |x - x0|^2 into part[blk*6 + 2..3].
@@ -3089,8 +3085,10 @@ void Backend::rhs(bool want_res, bool first_iter) {
     const int store_b = cfg.global_refine > 1 ? 1 : 0;
     with_lpr(rhs_lpr, [&](auto c) {
         constexpr int P = decltype(c)::value;
-        hipLaunchKernelGGL((use_chol ? k_rhs<P, true> : k_rhs<P, false>), dim3(grid_for((int64_t)n * P, BLK)), dim3(BLK), 0, stream, n,
-                           (float)cfg.dt, cfg.enable_contact, want_res ? 1 : 0, first_iter ? 1 : 0, store_b, dt_ptr.p, dt_row.p, dt_coef.p,
+        hipLaunchKernelGGL((use_chol ? (want_res ? k_rhs<P, true, true> : k_rhs<P, true, false>)
+                                     : (want_res ? k_rhs<P, false, true> : k_rhs<P, false, false>)),
+                           dim3(grid_for((int64_t)n * P, BLK)), dim3(BLK), 0, stream, n, (float)cfg.dt, cfg.enable_contact,
+                           first_iter ? 1 : 0, store_b, dt_ptr.p, dt_row.p, dt_coef.p,
                            z.p, zprev.p, Ue.p, bconst.p, wch2.p, p.p, x0.p, Uc.p, bpin.p, b.p, res_part.p, A);
     });
     PA_LAUNCH_CHECK();
