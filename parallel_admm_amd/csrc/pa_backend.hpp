@@ -114,29 +114,29 @@ struct Backend {
     // init (pa_chol.hpp), FP32 copies in the layouts the level kernels read
     bool use_chol = false;
     int chol_levels = 0;                  // levels below the dense tops
-    std::vector<int> chol_lvl_lds;        // wide levels: LDS bytes of the fused forward and backward launches
-    std::vector<uint8_t> chol_lvl_wide;   // 1: many supernodes (a workgroup each), 0: few (split over tiles)
-    // narrow levels: tile lists (supernode, first row or column) of the three split launches
-    std::vector<int32_t> chol_sf_ptr, chol_sg_ptr, chol_sx_ptr; // per level: ranges in the tile arrays
-    std::vector<int> chol_sf_lds, chol_sg_lds, chol_sx_lds;
-    DBuf<int2> chol_sf_tiles, chol_sg_tiles, chol_sx_tiles;
-    DBuf<float> chol_g;                   // backward: g of the split levels (elimination order)
-    int chol_top_tiles = 0, chol_top_lds = 0;
-    std::vector<int32_t> chol_lvl_ptr;    // non-top supernodes of height h: chol_lvl_sup[ptr[h] .. ptr[h + 1])
-    DBuf<int32_t> chol_lvl_sup, chol_perm, chol_col0, chol_below, chol_rel, chol_child_ptr, chol_child, chol_top_pos, chol_top_ridx;
-    DBuf<int64_t> chol_below_ptr, chol_l21_off, chol_inv_off, chol_top_ptr, chol_gat, chol_sinv_off;
+    // per level: ranges in the tile arrays, lanes along rows (up) or per column
+    // (down), LDS bytes
+    std::vector<int32_t> chol_up_ptr, chol_down_ptr;
+    std::vector<int> chol_rg, chol_lp, chol_up_lds, chol_down_lds;
+    DBuf<uint8_t> chol_up_tiles, chol_down_tiles; // CholTile descriptors (pa_solver.hip)
+    DBuf<float> chol_panels;              // [D; -W] per supernode, column-major
+    DBuf<int32_t> chol_gat_rows;          // per front row: the children's update-vector entries added there
+    DBuf<int32_t> chol_ipos, chol_below;  // place of each unknown in elimination order; rows below of each supernode
+    int chol_top_tiles = 0, chol_top_lds = 0, chol_top_nv = 1;
+    DBuf<int32_t> chol_top_pos;
+    DBuf<int64_t> chol_top_ptr, chol_gat, chol_sinv_off;
     int chol_gmax = 1;                    // width of the dense tops' gather table chol_gat (entries -1: none)
     DBuf<int2> chol_tiles;                // (top block, first row) of each workgroup of the dense-top launch
-    DBuf<float> chol_l21, chol_linv;      // L21 (nbelow x width) and L11^-1 (width x width), column-major
-    DBuf<float> chol_sinv;                // dense tops: S^-1, row-major
-    DBuf<float> chol_y, chol_x, chol_u;   // forward result and solution (elimination order), update vectors
+    DBuf<float> chol_sinv;                // dense tops: S^-1, row-major, rows padded to whole float4s
+    DBuf<float> chol_f, chol_x, chol_u;   // fronts' column right-hand sides and solution (elimination order), update vectors
     DBuf<float> chol_ftop;                // right-hand side of every dense-top entry (3 per entry)
-    int64_t chol_entries = 0;             // stored factor entries (L21, L11^-1, S^-1)
+    int64_t chol_entries = 0;             // stored factor entries (panels, S^-1)
     int64_t chol_top_cols = 0, chol_top_sq = 0; // dense tops: sum of m and of m^2
     double chol_setup_ms = 0;
     void chol_setup(const std::vector<int32_t>& aptr, const std::vector<int32_t>& acol, const std::vector<double>& aval,
                     const double* x0h);
-    void chol_solve(const float* r, float* d); // d = A^-1 r (3 interleaved columns, FP32)
+    void chol_solve(const float* r); // chol_x = A^-1 r
+    void chol_top_launch(const float* r);
     // scripted animation of static vertex ranges (ScriptAnimator rigid and
     // point-sequence scripts)
     struct RigidTrack {

@@ -27,10 +27,13 @@
 #include <roctracer/roctx.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstring>
 #include <limits>
+#include <new>
+#include <thread>
 #include <type_traits>
 
 namespace pa {
@@ -967,13 +970,14 @@ __global__ void k_ws_log(int nc, float s, const float* __restrict__ feat, const 
 }
 
 // System matrix rows for the residual of the global solve (off-diagonal CSR
-// and diagonal, A = hi + lo), and where r goes.
+// and diagonal, A = hi + lo), and where r goes: row i to place ipos[i].
 struct ResidArgs {
     const int32_t* ptr;
     const int32_t* col;
     const float *val, *val_lo, *diag, *diag_lo;
     const double* x;
     float* r;
+    const int32_t* ipos;
 };
 
 // b = bconst + sum_e coef_e (z - Ue)[row_e] + h^2 wc (h p + x0 - Uc), accumulated in FP64.
@@ -1080,12 +1084,13 @@ __global__ void __launch_bounds__(BLK) k_rhs(int n, float h, int contact, int fi
     if (i < n && sub == 0) {
         const double wv = contact ? wch2[i] : 0.0;
         const double di = RESID ? (double)A.diag[i] + (double)A.diag_lo[i] : 0.0;
+        const int64_t o = RESID ? A.ipos[i] : 0;
 #pragma unroll
         for (int a = 0; a < 3; a++) {
             double bi = bconst[3 * i + a] + s[a];
             if (wv != 0.0) bi += wv * (((double)h * p[3 * i + a] + x0[3 * i + a]) - (double)Uc[3 * i + a]);
             if (!RESID || store_b) b[3 * i + a] = bi;
-            if (RESID) A.r[3 * i + a] = (float)(bi - (ax[a] + di * A.x[3 * i + a]));
+            if (RESID) A.r[3 * o + a] = (float)(bi - (ax[a] + di * A.x[3 * i + a]));
         }
         if (RES) {
 #pragma unroll
@@ -1102,19 +1107,21 @@ __global__ void __launch_bounds__(BLK) k_rhs(int n, float h, int contact, int fi
 }
 
 // Uc += x - x0 - h p; residual sums wc |x - x0 - h p|^2, wc |x - x0|^2 into part[blk*6 + 2..3].
-// With dxg non-null the global solve's last correction is applied here
-// first: x += dxg (what k_axpy_d would have done), then the dual update on the
-// new x.  p becomes the next iteration's (x - x0 + Uc) / h.
+// With dxg non-null the direct solve's last correction (in elimination order,
+// vertex i at ipos[i]) is applied here first: x += dxg (what k_axpy_d would have
+// done), then the dual update on the new x.  p becomes the next iteration's (x - x0 + Uc) / h.
 __global__ void __launch_bounds__(BLK) k_dual_vert(int n, float h, float hinv, int contact, int want_res, double* __restrict__ x,
                                                    const double* __restrict__ x0, float* __restrict__ p, const double* __restrict__ wch2,
                                                    float* __restrict__ Uc, double* __restrict__ part, double h2inv,
-                                                   const int32_t* __restrict__ stop, const float* __restrict__ dxg) {
+                                                   const int32_t* __restrict__ stop, const float* __restrict__ dxg,
+                                                   const int32_t* __restrict__ ipos) {
     const bool keep = stop && stop[0]; // the iteration runs past the stop: x and Uc stay
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     double acc[2] = {0, 0};
     if (i < n && dxg && !keep) {
+        const int64_t o = ipos[i];
 #pragma unroll
-        for (int a = 0; a < 3; a++) x[3 * i + a] += (double)dxg[3 * i + a];
+        for (int a = 0; a < 3; a++) x[3 * i + a] += (double)dxg[3 * o + a];
     }
     if (i < n && contact) {
         const float3 dx = to_f3(ld3(x, i) - ld3(x0, i));
@@ -1216,13 +1223,14 @@ template <int LPR> __device__ inline float3 row_dot(int r, int rows, int sub, co
 // Start of one refinement pass: r = b - A x with A = hi + lo and FP64
 // accumulation (the exact residual of the FP64 iterate); the FP32 PCG for the
 // correction d starts from d = 0 with r32 = r.  Partials: |b|^2 at 0..2,
-// |r|^2 at 3..5.
+// |r|^2 at 3..5.  With ipos (the direct solve) row i of r goes to place
+// ipos[i], and d is left alone.
 template <int LPR>
 __global__ void __launch_bounds__(PBLK) k_cg_resid64(int n, const int32_t* __restrict__ ptr, const int32_t* __restrict__ col,
                                                     const float* __restrict__ val, const float* __restrict__ val_lo,
                                                     const float* __restrict__ diag, const float* __restrict__ diag_lo,
                                                     const double* __restrict__ bvec, const double* __restrict__ x, float* __restrict__ r,
-                                                    float* __restrict__ d, double* __restrict__ part) {
+                                                    float* __restrict__ d, double* __restrict__ part, const int32_t* __restrict__ ipos) {
     const int sub = threadIdx.x % LPR;
     double acc[6] = {0, 0, 0, 0, 0, 0};
     for (int r0 = xcd_block() * (PBLK / LPR); r0 < n; r0 += gridDim.x * (PBLK / LPR)) {
@@ -1258,8 +1266,8 @@ __global__ void __launch_bounds__(PBLK) k_cg_resid64(int n, const int32_t* __res
             for (int k = 0; k < 3; k++) {
                 const double bk = bvec[3 * i + k];
                 const double rk = bk - (ax[k] + di * x[3 * i + k]);
-                r[3 * i + k] = (float)rk;
-                d[3 * i + k] = 0.f;
+                r[3 * (int64_t)(ipos ? ipos[i] : i) + k] = (float)rk;
+                if (!ipos) d[3 * i + k] = 0.f;
                 acc[k] += bk * bk;
                 acc[3 + k] += rk * rk;
             }
@@ -1308,10 +1316,11 @@ __global__ void k_copy(int64_t m, const float* __restrict__ a, float* __restrict
 }
 
 // x += d, skipped once stop[0] is set (stop may be null).
-__global__ void k_axpy_d(int n, const float* __restrict__ d, double* __restrict__ x, const int32_t* __restrict__ stop) {
+__global__ void k_axpy_d(int n, const float* __restrict__ d, const int32_t* __restrict__ ipos, double* __restrict__ x,
+                         const int32_t* __restrict__ stop) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= 3 * n || (stop && stop[0])) return;
-    x[i] += (double)d[i];
+    x[i] += (double)(ipos ? d[3 * (int64_t)ipos[i / 3] + i % 3] : d[i]);
 }
 
 // q = A pd (off-diagonal CSR + diagonal); partial p.q at 0..2
@@ -1838,418 +1847,256 @@ __global__ void __launch_bounds__(BLK) k_amg_coarse(int nc, int ncp, const float
 
 // ---------------------------------------------------------------------------
 // Direct global solve with the prefactored supernodal Cholesky (pa_chol.hpp).
-// Below the dense tops, one launch per tree level and one workgroup per
-// supernode (FP32, factor blocks column-major):
-//   forward (leaves first):  F = [r(cols); 0] + extend-add of the children's
-//     update vectors; y = L11^-1 F(cols); u = F(below) - L21 y (to the parent)
-//   backward (down from the tops):  g = y - L21^T x(below); x(cols) = L11^-T g
-// and between them one launch for every tree's dense top: f = r(top) + the
-// update vectors its boundary children send up, x(top) = S^-1 f.  Factor
-// blocks reach LDS in column chunks (4096 or 8192 floats), loaded with
-// 16 independent loads in flight per lane; every product then reads LDS.
-// r and d are in the unknowns' own order, y and x in elimination order.
+// Every vector is in elimination order and a supernode's columns are
+// consecutive there.  With F the right-hand side of a supernode's front (r on
+// its columns plus the children's update vectors), D = (L11 L11^T)^-1 and
+// W = L21 L11^-1 of its factor blocks, one launch per tree level below the
+// dense tops:
+//   up (leaves first):        u = F(below) - W F(cols), to the parent
+//   down (from the tops on):  x(cols) = D F(cols) - W^T x(below)
+// and between them every tree's dense top: f = r(top) + the update vectors its
+// boundary children send up, x(top) = S^-1 f.
+//
+// What bounds a level is its chain of dependent loads, not its bytes (below
+// 3 MB but for the leaves), so a level is one product in each direction: with
+// the triangular blocks L11^-1 and L21 themselves a level needed y = L11^-1 F
+// before u and L21^T x before x, in two phases with a barrier (or, spread over
+// tiles, two launches).  D and W take no more storage than L11^-1 and L21,
+// and up reads only W.  A supernode's panel [D; -W] is column-major with its
+// rows padded to whole float4s.  Everything a tile needs to find its data is
+// in one descriptor, and where a row of F comes from is a table, so the chain
+// is descriptor -> (panel, table, r) -> children's u -> product.
+//
+// At 256x256 vertices (7 levels and the top): up 4 x 13.3 + 3 x 11.0 ->
+// 7 x 7.5 us, down 4 x (7.4 + 4.3) + 3 x 9.5 -> 6 x 5.0 + 7.4 us.
 // ---------------------------------------------------------------------------
-constexpr int CHOL_TOP_ROWS = 4;  // rows of S^-1 per workgroup (one per wave)
-constexpr int CHOL_KC_MAX = 256;  // columns per chunk in the transposed products
-// Levels with at least CHOL_WIDE_MIN supernodes run one 256-lane workgroup per
-// supernode (several share a CU); levels with fewer, larger supernodes split
-// each over tiles of the split kernels below, so a level still spans the chip.
-constexpr int CHOL_WIDE_MIN = 256;
-constexpr int CHOL_BIG_TILE_MAX = 2048; // wide levels up to this many supernodes stage 8192-float factor tiles, larger ones 4096
-
-struct CholArgs {
-    const int32_t* sup;       // supernodes of this level
-    const int32_t* perm;
-    const int32_t* col0;
-    const int64_t* below_ptr;
-    const int32_t* below;
-    const int32_t* rel;
-    const int32_t* child_ptr;
-    const int32_t* child;
-    const int64_t* l21_off;
-    const int64_t* inv_off;
+struct CholTile {
+    int64_t panel;     // the supernode's [D; -W] in the panel array
+    int32_t c0, w, nb; // its columns' first position, their number, rows below
+    int32_t first;     // up: first row of u of this tile; down: first column
+    int32_t below;     // its rows below in chol_below and chol_u
+    int32_t gat, kids; // its table in chol_gat_rows: kids entries per row of the front (-1: none)
+    int32_t pad;
 };
+constexpr int CHOL_BLK = 256;
+// Dissection leaves hold up to 160 unknowns in systems of up to this many, 64
+// above.  Larger leaves save a level, two launches of about 6 us, and cost
+// host set-up (about 25,000 more flops per unknown): 256x256 cloth step
+// 12.5 -> 12.1 ms, tet box 4.31 -> 3.84, side-95 cloth 4.03 -> 3.67, but a
+// 160-scene batch of 500,000 unknowns, whose levels are wide, 36.9 -> 36.3.
+constexpr int CHOL_BIG_LEAF_N = 1 << 17;
+constexpr int CHOL_INFLIGHT = 8; // float4 panel loads in flight per lane
 
-// Copies len floats from global memory into LDS, 16 loads in flight per lane.
-template <int BLK>
-__device__ inline void chol_stage(float* __restrict__ dst, const float* __restrict__ src, int len) {
-    for (int t0 = threadIdx.x; t0 < len; t0 += 16 * BLK) {
-        float v[16];
+__device__ inline int chol_pad4(int v) { return (v + 3) & ~3; }
+
+// Adds the children's update-vector entries of front row `row` to v, in child order.
+__device__ inline float3 chol_gather(const CholTile& T, int row, const int32_t* __restrict__ gat, const float* u, float3 v) {
+    const int32_t* g = gat + T.gat + (int64_t)row * T.kids;
+    int k = 0;
+    for (; k + 2 <= T.kids; k += 2) {
+        const int a = g[k], b = g[k + 1];
+        const float3 ua = a >= 0 ? ld3(u, a) : f3(0.f, 0.f, 0.f), ub = b >= 0 ? ld3(u, b) : f3(0.f, 0.f, 0.f);
+        v = v + ua;
+        v = v + ub;
+    }
+    if (k < T.kids && g[k] >= 0) v = v + ld3(u, g[k]);
+    return v;
+}
+
+// Rows first .. first + 4 RG of u.  RG lanes take four rows each (one float4 of
+// a panel column), 256 / RG groups of lanes share the columns.  A small RG
+// gives a level more tiles, a large one gathers F fewer times.
+template <int RG>
+__global__ void __launch_bounds__(CHOL_BLK) k_chol_up(const CholTile* __restrict__ tiles, const float* __restrict__ panels,
+                                                      const int32_t* __restrict__ gat, const float* __restrict__ r, float* __restrict__ F,
+                                                      float* u) {
+    constexpr int PARTS = CHOL_BLK / RG, RT = 4 * RG, U = CHOL_INFLIGHT;
+    extern __shared__ float4 chol_sh4[];
+    __shared__ float red[CHOL_BLK / 64][3 * RT];
+    float4* const Fs = chol_sh4; // w: F of the columns
+    const CholTile T = tiles[blockIdx.x];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int wp = chol_pad4(T.w), ld = wp + chol_pad4(T.nb);
+    const int j = T.first + 4 * (t % RG), part = t / RG;
+    const float* P = panels + T.panel + wp + j;
+    float4 pv[U];
+    auto load = [&](int k0) {
 #pragma unroll
-        for (int q = 0; q < 16; q++) {
-            const int t = t0 + q * BLK;
-            v[q] = t < len ? src[t] : 0.f;
+        for (int q = 0; q < U; q++) {
+            const int k = k0 + part + q * PARTS;
+            pv[q] = j < T.nb && k < T.w ? *reinterpret_cast<const float4*>(P + (int64_t)k * ld) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
+    };
+    load(0);
+    for (int i = t; i < T.w; i += CHOL_BLK) {
+        const float3 f = chol_gather(T, i, gat, u, ld3(r, T.c0 + i));
+        Fs[i] = make_float4(f.x, f.y, f.z, 0.f);
+        if (T.first == 0) st3(F, T.c0 + i, f);
+    }
+    float3 fb = f3(0.f, 0.f, 0.f);
+    if (t < RT && T.first + t < T.nb) fb = chol_gather(T, T.w + T.first + t, gat, u, fb);
+    __syncthreads();
+    if (T.nb == 0) return;
+    float3 acc[4];
 #pragma unroll
-        for (int q = 0; q < 16; q++) {
-            const int t = t0 + q * BLK;
-            if (t < len) dst[t] = v[q];
-        }
-    }
-}
-
-// out[c] = sum over rows r >= lo(c) of T[r + c rows] v[r], for the kc <= BLK
-// columns of an LDS chunk T (column-major, `rows` rows); lo(c) = tri ? c +
-// tri_base : 0.  BLK / kc consecutive threads share a column, each taking a
-// strided share of its rows (consecutive rows on consecutive lanes); the
-// shares go through LDS (red, BLK float3) and are summed in a fixed order.
-template <int BLK>
-__device__ inline void chol_col_dots(const float* __restrict__ T, int rows, int kc, const float* __restrict__ v, bool tri,
-                                     int tri_base, float* __restrict__ red, float* __restrict__ out) {
-    const int parts = BLK / kc;
-    const int c = threadIdx.x / parts, part = threadIdx.x % parts;
-    float3 acc = f3(0.f, 0.f, 0.f);
-    if (c < kc) {
-        const int lo = tri ? c + tri_base : 0;
-        for (int r = lo + part; r < rows; r += parts) acc = acc + T[r + c * rows] * ld3(v, r);
-    }
-    st3(red, threadIdx.x, acc);
-    __syncthreads();
-    if (threadIdx.x < kc) {
-        float3 s3 = f3(0.f, 0.f, 0.f);
-        for (int q = 0; q < parts; q++) s3 = s3 + ld3(red, threadIdx.x * parts + q);
-        st3(out, threadIdx.x, s3);
-    }
-    __syncthreads();
-}
-
-// LDS floats of a level launch for a supernode (w, nb): the larger of the
-// forward's F, ys and chunk and the backward's xb, g, partials, sums and chunk.
-template <int BLK, int TILE> constexpr int chol_lds_floats(int w, int nb) {
-    return (3 * (w + nb) + 3 * w > 3 * (nb + w) + 3 * BLK + 3 * CHOL_KC_MAX ? 3 * (w + nb) + 3 * w
-                                                                          : 3 * (nb + w) + 3 * BLK + 3 * CHOL_KC_MAX) +
-           TILE;
-}
-
-template <int BLK, int TILE>
-__global__ void __launch_bounds__(BLK) k_chol_fwd(CholArgs a, const float* __restrict__ l21, const float* __restrict__ linv,
-                                                  const float* __restrict__ r, float* __restrict__ y, float* __restrict__ u) {
-    extern __shared__ float chol_sh[];
-    const int s = a.sup[blockIdx.x];
-    const int c0 = a.col0[s], w = a.col0[s + 1] - c0;
-    const int64_t b0 = a.below_ptr[s];
-    const int nb = (int)(a.below_ptr[s + 1] - b0), nr = w + nb;
-    float* F = chol_sh;            // 3 nr
-    float* ys = F + 3 * nr;        // 3 w
-    float* T = ys + 3 * w;         // TILE
-    for (int i = threadIdx.x; i < nr; i += BLK) st3(F, i, i < w ? ld3(r, a.perm[c0 + i]) : f3(0.f, 0.f, 0.f));
-    for (int i = threadIdx.x; i < w; i += BLK) st3(ys, i, f3(0.f, 0.f, 0.f));
-    __syncthreads();
-    for (int ci = a.child_ptr[s]; ci < a.child_ptr[s + 1]; ci++) { // children in order: no two writers of one row at once
-        const int c = a.child[ci];
-        const int64_t cb = a.below_ptr[c];
-        const int nbc = (int)(a.below_ptr[c + 1] - cb);
-        for (int k = threadIdx.x; k < nbc; k += BLK) {
-            const int l = a.rel[cb + k];
-            st3(F, l, ld3(F, l) + ld3(u, cb + k));
-        }
-        __syncthreads();
-    }
-    // ys = L11^-1 F(cols), column chunks of L11^-1 (lower triangular: k <= i)
-    const float* Li = linv + a.inv_off[s];
-    const int kc1 = max(1, TILE / w);
-    for (int k0 = 0; k0 < w; k0 += kc1) {
-        const int kc = min(kc1, w - k0);
-        chol_stage<BLK>(T, Li + (int64_t)k0 * w, kc * w);
-        __syncthreads();
-        for (int i = threadIdx.x; i < w; i += BLK) {
-            float3 acc = ld3(ys, i);
-            const int kend = min(kc, i - k0 + 1);
-            for (int kk = 0; kk < kend; kk++) acc = acc + T[i + kk * w] * ld3(F, k0 + kk);
-            st3(ys, i, acc);
-        }
-        __syncthreads();
-    }
-    for (int i = threadIdx.x; i < w; i += BLK) st3(y, c0 + i, ld3(ys, i));
-    // u = F(below) - L21 ys, column chunks of L21, accumulated in F(below)
-    if (nb == 0) return;
-    const float* L = l21 + a.l21_off[s];
-    const int kc2 = max(1, TILE / nb);
-    for (int k0 = 0; k0 < w; k0 += kc2) {
-        const int kc = min(kc2, w - k0);
-        chol_stage<BLK>(T, L + (int64_t)k0 * nb, kc * nb);
-        __syncthreads();
-        for (int j = threadIdx.x; j < nb; j += BLK) {
-            float3 acc = ld3(F, w + j);
-            for (int kk = 0; kk < kc; kk++) acc = acc - T[j + kk * nb] * ld3(ys, k0 + kk);
-            st3(F, w + j, acc);
-        }
-        __syncthreads();
-    }
-    for (int j = threadIdx.x; j < nb; j += BLK) st3(u, b0 + j, ld3(F, w + j));
-}
-
-template <int BLK, int TILE>
-__global__ void __launch_bounds__(BLK) k_chol_bwd(CholArgs a, const float* __restrict__ l21, const float* __restrict__ linv,
-                                                  const float* __restrict__ y, float* __restrict__ x, float* __restrict__ d) {
-    extern __shared__ float chol_sh[];
-    const int s = a.sup[blockIdx.x];
-    const int c0 = a.col0[s], w = a.col0[s + 1] - c0;
-    const int64_t b0 = a.below_ptr[s];
-    const int nb = (int)(a.below_ptr[s + 1] - b0);
-    float* xb = chol_sh;              // 3 nb: the solution at the rows below (solved by the ancestors)
-    float* g = xb + 3 * nb;           // 3 w
-    float* red = g + 3 * w;           // 3 BLK
-    float* dots = red + 3 * BLK;      // 3 CHOL_KC_MAX
-    float* T = dots + 3 * CHOL_KC_MAX; // TILE
-    for (int j = threadIdx.x; j < nb; j += BLK) st3(xb, j, ld3(x, a.below[b0 + j]));
-    for (int k = threadIdx.x; k < w; k += BLK) st3(g, k, ld3(y, c0 + k));
-    __syncthreads();
-    // g -= L21^T xb, column chunks of L21
-    if (nb > 0) {
-        const float* L = l21 + a.l21_off[s];
-        const int kc1 = max(1, min(CHOL_KC_MAX, TILE / nb));
-        for (int k0 = 0; k0 < w; k0 += kc1) {
-            const int kc = min(kc1, w - k0);
-            chol_stage<BLK>(T, L + (int64_t)k0 * nb, kc * nb);
-            __syncthreads();
-            chol_col_dots<BLK>(T, nb, kc, xb, false, 0, red, dots);
-            if (threadIdx.x < kc) st3(g, k0 + threadIdx.x, ld3(g, k0 + threadIdx.x) - ld3(dots, threadIdx.x));
-            __syncthreads();
-        }
-    }
-    // x(cols) = L11^-T g: column i of L11^-1 against g over k >= i
-    const float* Li = linv + a.inv_off[s];
-    const int kc2 = max(1, min(CHOL_KC_MAX, TILE / w));
-    for (int i0 = 0; i0 < w; i0 += kc2) {
-        const int kc = min(kc2, w - i0);
-        chol_stage<BLK>(T, Li + (int64_t)i0 * w, kc * w);
-        __syncthreads();
-        chol_col_dots<BLK>(T, w, kc, g, true, i0, red, dots);
-        if (threadIdx.x < kc) {
-            const float3 v = ld3(dots, threadIdx.x);
-            st3(x, c0 + i0 + threadIdx.x, v);
-            st3(d, a.perm[c0 + i0 + threadIdx.x], v);
-        }
-        __syncthreads();
-    }
-}
-
-// Narrow levels (few, large supernodes) split every supernode over several
-// workgroups, each named by a tile (supernode, first row or column):
-//   k_chol_fwd_split  tile (s, j0): F(cols) and y = L11^-1 F(cols) (the j0 = 0
-//                     tile stores y), then rows j0 .. j0 + R of u = F(below) - L21 y
-//   k_chol_bwd_g      tile (s, k0): g(k) = y(k) - L21(:, k)^T x(below), CHOL_SPLIT_KC columns
-//   k_chol_bwd_x      tile (s, i0): x(i) = sum over k >= i of L11^-1(k, i) g(k)
-// The transposed products take one wave per column (lanes along the
-// column, a shuffle reduction).
-constexpr int CHOL_SPLIT_BLK = 256;
-constexpr int CHOL_SPLIT_KC = 8;     // columns per backward tile
-constexpr int CHOL_SPLIT_ROWS = 32;  // rows of u per forward tile
-constexpr int CHOL_SPLIT_TILE = 8192; // floats of factor per LDS chunk
-
-__global__ void __launch_bounds__(CHOL_SPLIT_BLK) k_chol_fwd_split(CholArgs a, const int2* __restrict__ tiles, int rows_per_tile,
-                                                                   const float* __restrict__ l21, const float* __restrict__ linv,
-                                                                   const float* __restrict__ r, float* __restrict__ y,
-                                                                   float* __restrict__ u) {
-    extern __shared__ float chol_sh[];
-    constexpr int BLK = CHOL_SPLIT_BLK, TILE = CHOL_SPLIT_TILE, RP = CHOL_SPLIT_ROWS;
-    const int2 tl = tiles[blockIdx.x];
-    const int s = tl.x, j0 = tl.y;
-    const int c0 = a.col0[s], w = a.col0[s + 1] - c0;
-    const int64_t b0 = a.below_ptr[s];
-    const int nb = (int)(a.below_ptr[s + 1] - b0);
-    const int R = min(rows_per_tile, nb - j0); // rows of u in this tile (<= 0: none)
-    float* F = chol_sh;          // 3 w
-    float* ys = F + 3 * w;       // 3 w
-    float* Fb = ys + 3 * w;      // 3 RP
-    float* red = Fb + 3 * RP;    // 3 BLK
-    float* T = red + 3 * BLK;    // TILE
-    for (int i = threadIdx.x; i < w; i += BLK) {
-        st3(F, i, ld3(r, a.perm[c0 + i]));
-        st3(ys, i, f3(0.f, 0.f, 0.f));
-    }
-    for (int j = threadIdx.x; j < R; j += BLK) st3(Fb, j, f3(0.f, 0.f, 0.f));
-    __syncthreads();
-    for (int ci = a.child_ptr[s]; ci < a.child_ptr[s + 1]; ci++) { // children in order; rows of one child are distinct
-        const int c = a.child[ci];
-        const int64_t cb = a.below_ptr[c];
-        const int nbc = (int)(a.below_ptr[c + 1] - cb);
-        for (int k = threadIdx.x; k < nbc; k += BLK) {
-            const int l = a.rel[cb + k];
-            if (l < w) st3(F, l, ld3(F, l) + ld3(u, cb + k));
-            else if (l - w >= j0 && l - w < j0 + R) st3(Fb, l - w - j0, ld3(Fb, l - w - j0) + ld3(u, cb + k));
-        }
-        __syncthreads();
-    }
-    const float* Li = linv + a.inv_off[s];
-    const int kc1 = max(1, TILE / w);
-    for (int k0 = 0; k0 < w; k0 += kc1) {
-        const int kc = min(kc1, w - k0);
-        chol_stage<BLK>(T, Li + (int64_t)k0 * w, kc * w);
-        __syncthreads();
-        for (int i = threadIdx.x; i < w; i += BLK) {
-            float3 acc = ld3(ys, i);
-            const int kend = min(kc, i - k0 + 1);
-            for (int kk = 0; kk < kend; kk++) acc = acc + T[i + kk * w] * ld3(F, k0 + kk);
-            st3(ys, i, acc);
-        }
-        __syncthreads();
-    }
-    if (j0 == 0)
-        for (int i = threadIdx.x; i < w; i += BLK) st3(y, c0 + i, ld3(ys, i));
-    if (R <= 0) return;
-    // rows j0 .. j0 + R of L21, column chunks staged as RP-row strips
-    // (T[kk RP + row]); four lanes per row, each a quarter of the columns
-    const float* L = l21 + a.l21_off[s] + j0;
-    const int row = threadIdx.x % RP, grp = threadIdx.x / RP; // BLK / RP = 4 groups
-    float3 acc = f3(0.f, 0.f, 0.f);
-    const int kc3 = TILE / RP;
-    for (int k0 = 0; k0 < w; k0 += kc3) {
-        const int kc = min(kc3, w - k0), len = kc * RP;
-        for (int t0 = threadIdx.x; t0 < len; t0 += 16 * BLK) {
-            float v[16];
+    for (int q = 0; q < 4; q++) acc[q] = f3(0.f, 0.f, 0.f);
+    for (int k0 = 0; k0 < T.w; k0 += U * PARTS) {
+        if (k0 > 0) load(k0);
 #pragma unroll
-            for (int q = 0; q < 16; q++) {
-                const int t = t0 + q * BLK, kk = t / RP, rr = t % RP;
-                v[q] = (t < len && rr < R) ? L[(int64_t)(k0 + kk) * nb + rr] : 0.f;
-            }
-#pragma unroll
-            for (int q = 0; q < 16; q++) {
-                const int t = t0 + q * BLK;
-                if (t < len) T[t] = v[q];
-            }
+        for (int q = 0; q < U; q++) {
+            const float4 g = Fs[min(k0 + part + q * PARTS, T.w - 1)];
+            const float3 fk = f3(g.x, g.y, g.z);
+            acc[0] = acc[0] + pv[q].x * fk;
+            acc[1] = acc[1] + pv[q].y * fk;
+            acc[2] = acc[2] + pv[q].z * fk;
+            acc[3] = acc[3] + pv[q].w * fk;
         }
-        __syncthreads();
-        for (int kk = grp; kk < kc; kk += BLK / RP) acc = acc + T[kk * RP + row] * ld3(ys, k0 + kk);
-        __syncthreads();
     }
-    st3(red, threadIdx.x, acc);
+#pragma unroll
+    for (int o = RG; o < 64; o <<= 1)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            acc[q].x += __shfl_xor(acc[q].x, o, 64);
+            acc[q].y += __shfl_xor(acc[q].y, o, 64);
+            acc[q].z += __shfl_xor(acc[q].z, o, 64);
+        }
+    if (lane < RG)
+#pragma unroll
+        for (int q = 0; q < 4; q++) st3(red[wave], 4 * lane + q, acc[q]);
     __syncthreads();
-    if (grp == 0 && row < R) {
-        float3 t = ld3(Fb, row);
-        for (int q = 0; q < BLK / RP; q++) t = t - ld3(red, q * RP + row);
-        st3(u, b0 + j0 + row, t);
+    if (t < RT && T.first + t < T.nb) {
+#pragma unroll
+        for (int q = 0; q < CHOL_BLK / 64; q++) fb = fb + ld3(red[q], t);
+        st3(u, T.below + T.first + t, fb);
     }
 }
 
-__global__ void __launch_bounds__(CHOL_SPLIT_BLK) k_chol_bwd_g(CholArgs a, const int2* __restrict__ tiles, const float* __restrict__ l21,
-                                                               const float* __restrict__ y, const float* __restrict__ x,
-                                                               float* __restrict__ g) {
-    extern __shared__ float chol_sh[];
-    constexpr int PARTS = CHOL_SPLIT_BLK / CHOL_SPLIT_KC;
-    const int2 tl = tiles[blockIdx.x];
-    const int s = tl.x, k0 = tl.y;
-    const int c0 = a.col0[s], w = a.col0[s + 1] - c0;
-    const int64_t b0 = a.below_ptr[s];
-    const int nb = (int)(a.below_ptr[s + 1] - b0);
-    float* red = chol_sh;                    // 3 CHOL_SPLIT_BLK
-    float* xb = red + 3 * CHOL_SPLIT_BLK;    // 3 nb
-    for (int j = threadIdx.x; j < nb; j += CHOL_SPLIT_BLK) st3(xb, j, ld3(x, a.below[b0 + j]));
+// Columns first .. first + 256 / LP of x: LP lanes share a column of the panel,
+// four rows each, and combine with shuffles.
+template <int LP>
+__global__ void __launch_bounds__(CHOL_BLK) k_chol_down(const CholTile* __restrict__ tiles, const float* __restrict__ panels,
+                                                        const int32_t* __restrict__ below, const float* __restrict__ F, float* x) {
+    constexpr int U = CHOL_INFLIGHT;
+    extern __shared__ float4 chol_sh4[];
+    const CholTile T = tiles[blockIdx.x];
+    const int t = threadIdx.x, s = t % LP, col = T.first + t / LP;
+    const int wp = chol_pad4(T.w), ld = wp + chol_pad4(T.nb);
+    float* const v = reinterpret_cast<float*>(chol_sh4); // 3 x ld: [F(cols); x(below)], zeros in the padding
+    const float* P = panels + T.panel + (int64_t)col * ld + 4 * s;
+    float4 pv[U];
+    auto load = [&](int l0) {
+#pragma unroll
+        for (int q = 0; q < U; q++) {
+            const int l = l0 + q * 4 * LP;
+            pv[q] = col < T.w && l + 4 * s < ld ? *reinterpret_cast<const float4*>(P + l) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    };
+    load(0);
+    for (int l = t; l < ld; l += CHOL_BLK) {
+        float3 e = f3(0.f, 0.f, 0.f);
+        if (l < T.w) e = ld3(F, T.c0 + l);
+        else if (l >= wp && l - wp < T.nb) e = ld3(x, below[T.below + l - wp]);
+        v[l] = e.x;
+        v[ld + l] = e.y;
+        v[2 * ld + l] = e.z;
+    }
     __syncthreads();
-    // PARTS consecutive lanes share a column and take consecutive rows
-    const int c = threadIdx.x / PARTS, part = threadIdx.x % PARTS, k = k0 + c;
     float3 acc = f3(0.f, 0.f, 0.f);
-    if (k < w) {
-        const float* Lk = a.l21_off[s] + l21 + (int64_t)k * nb;
-        for (int j = part; j < nb; j += PARTS) acc = acc + Lk[j] * ld3(xb, j);
+    for (int l0 = 0; l0 < ld; l0 += U * 4 * LP) {
+        if (l0 > 0) load(l0);
+#pragma unroll
+        for (int q = 0; q < U; q++) {
+            const int l = min(l0 + q * 4 * LP + 4 * s, ld - 4);
+            const float4 p = pv[q], vx = *reinterpret_cast<const float4*>(v + l), vy = *reinterpret_cast<const float4*>(v + ld + l),
+                         vz = *reinterpret_cast<const float4*>(v + 2 * ld + l);
+            acc.x += (p.x * vx.x + p.y * vx.y) + (p.z * vx.z + p.w * vx.w);
+            acc.y += (p.x * vy.x + p.y * vy.y) + (p.z * vy.z + p.w * vy.w);
+            acc.z += (p.x * vz.x + p.y * vz.y) + (p.z * vz.z + p.w * vz.w);
+        }
     }
-    st3(red, threadIdx.x, acc);
-    __syncthreads();
-    if (threadIdx.x < CHOL_SPLIT_KC && k0 + threadIdx.x < w) {
-        float3 t = f3(0.f, 0.f, 0.f);
-        for (int q = 0; q < PARTS; q++) t = t + ld3(red, threadIdx.x * PARTS + q);
-        st3(g, c0 + k0 + threadIdx.x, ld3(y, c0 + k0 + threadIdx.x) - t);
+#pragma unroll
+    for (int o = LP / 2; o > 0; o >>= 1) {
+        acc.x += __shfl_xor(acc.x, o, LP);
+        acc.y += __shfl_xor(acc.y, o, LP);
+        acc.z += __shfl_xor(acc.z, o, LP);
     }
+    if (s == 0 && col < T.w) st3(x, T.c0 + col, acc);
 }
 
-__global__ void __launch_bounds__(CHOL_SPLIT_BLK) k_chol_bwd_x(CholArgs a, const int2* __restrict__ tiles, const float* __restrict__ linv,
-                                                               const float* __restrict__ g, float* __restrict__ x, float* __restrict__ d) {
-    extern __shared__ float chol_sh[];
-    constexpr int PARTS = CHOL_SPLIT_BLK / CHOL_SPLIT_KC;
-    const int2 tl = tiles[blockIdx.x];
-    const int s = tl.x, i0 = tl.y;
-    const int c0 = a.col0[s], w = a.col0[s + 1] - c0;
-    float* red = chol_sh;                  // 3 CHOL_SPLIT_BLK
-    float* gs = red + 3 * CHOL_SPLIT_BLK;  // 3 w
-    for (int k = threadIdx.x; k < w; k += CHOL_SPLIT_BLK) st3(gs, k, ld3(g, c0 + k));
-    __syncthreads();
-    const int c = threadIdx.x / PARTS, part = threadIdx.x % PARTS, i = i0 + c;
-    float3 acc = f3(0.f, 0.f, 0.f);
-    if (i < w) {
-        const float* Lc = linv + a.inv_off[s] + (int64_t)i * w; // column i: (k, i) at i w + k
-        for (int k = i + part; k < w; k += PARTS) acc = acc + Lc[k] * ld3(gs, k);
-    }
-    st3(red, threadIdx.x, acc);
-    __syncthreads();
-    if (threadIdx.x < CHOL_SPLIT_KC && i0 + threadIdx.x < w) {
-        float3 t = f3(0.f, 0.f, 0.f);
-        for (int q = 0; q < PARTS; q++) t = t + ld3(red, threadIdx.x * PARTS + q);
-        st3(x, c0 + i0 + threadIdx.x, t);
-        st3(d, a.perm[c0 + i0 + threadIdx.x], t);
-    }
-}
-
-// Dense tops, in two launches.  k_chol_top_f assembles every top entry's
-// right-hand side once: f = r at its unknown plus the update-vector entries
-// the boundary children send up (at most gmax each, in a fixed order).
+// Dense tops.  k_chol_top_f assembles every top entry's right-hand side once:
+// f = r at its position plus the update-vector entries the boundary children
+// send up (at most gmax each, in a fixed order).  Where there is no level
+// below the tops f is r itself (pos non-null) and the launch falls away.
 // k_chol_top: workgroup (block, row0) forms CHOL_TOP_ROWS rows of S^-1 f for
-// its tree's top, one wave per row; the row of S^-1 is loaded into registers
-// first, f (contiguous) meanwhile into LDS.  Every entry is one unknown
-// (ridx), updated in place.
+// its tree's top, one wave per row.  A row is up to NV float4s per lane (rows
+// padded to whole float4s), all in flight before f arrives in LDS; the lanes'
+// sums combine with shuffles.  NV follows the largest top, so a small one does
+// not step over the loads of a large one.  256x256 vertices (3036 columns,
+// 37 MB): 13.2 us against 15.5 with scalar loads and lane 0 adding 64 sums from
+// LDS; a 256-column top 3.5 against 8.0.
+constexpr int CHOL_TOP_ROWS = 4;   // rows of S^-1 per workgroup (one per wave)
 constexpr int CHOL_TOP_BLK = 256;
-constexpr int CHOL_TOP_MAX = 4096; // largest dense top (64 values per lane)
+constexpr int CHOL_TOP_MAX = 4096; // largest dense top (16 float4s per lane)
 constexpr int CHOL_TOP_GMAX = 8;   // most update-vector entries gathered into one top entry
 
-__global__ void k_chol_top_f(int ntop, const int32_t* __restrict__ ridx, const int64_t* __restrict__ gat_fix, int gmax,
+__global__ void k_chol_top_f(int ntop, const int32_t* __restrict__ pos, const int64_t* __restrict__ gat_fix, int gmax,
                              const float* __restrict__ r, const float* __restrict__ u, float* __restrict__ ftop) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= ntop) return;
     int64_t ge[CHOL_TOP_GMAX];
 #pragma unroll
     for (int k = 0; k < CHOL_TOP_GMAX; k++) ge[k] = k < gmax ? gat_fix[(int64_t)q * gmax + k] : -1;
-    float3 fv = ld3(r, ridx[q]);
+    float3 fv = ld3(r, pos[q]);
 #pragma unroll
     for (int k = 0; k < CHOL_TOP_GMAX; k++)
         if (ge[k] >= 0) fv = fv + ld3(u, ge[k]);
     st3(ftop, q, fv);
 }
 
+template <int NV>
 __global__ void __launch_bounds__(CHOL_TOP_BLK) k_chol_top(const int2* __restrict__ tiles, const int64_t* __restrict__ top_ptr,
-                                                           const int32_t* __restrict__ top_pos, const int32_t* __restrict__ ridx,
-                                                           const int64_t* __restrict__ sinv_off, const float* __restrict__ sinv,
-                                                           const float* __restrict__ ftop, float* __restrict__ x, float* __restrict__ d) {
-    extern __shared__ float chol_sh[];
-    constexpr int NV = CHOL_TOP_MAX / 64;
-    constexpr int PER = CHOL_TOP_MAX / CHOL_TOP_BLK; // f entries per lane
+                                                           const int32_t* __restrict__ top_pos, const int64_t* __restrict__ sinv_off,
+                                                           const float* __restrict__ sinv, const float* __restrict__ f,
+                                                           const int32_t* __restrict__ pos, float* __restrict__ x) {
+    extern __shared__ float4 chol_sh4[];
     const int2 tl = tiles[blockIdx.x];
     const int64_t p0 = top_ptr[tl.x];
-    const int m = (int)(top_ptr[tl.x + 1] - p0);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int i0 = tl.y + wave;
-    // the row of S^-1 in flight first ...
-    const float* S = sinv + sinv_off[tl.x];
-    float s0[NV];
+    const int m = (int)(top_ptr[tl.x + 1] - p0), mp = chol_pad4(m);
+    const int lane = threadIdx.x & 63, i0 = tl.y + (threadIdx.x >> 6);
+    const float* S = sinv + sinv_off[tl.x] + (int64_t)i0 * mp + 4 * lane;
+    float4 s0[NV];
+#pragma unroll
+    for (int t = 0; t < NV; t++)
+        s0[t] = i0 < m && 4 * lane + 256 * t < mp ? *reinterpret_cast<const float4*>(S + 256 * t) : make_float4(0.f, 0.f, 0.f, 0.f);
+    float* const v = reinterpret_cast<float*>(chol_sh4); // 3 x mp
 #pragma unroll
     for (int t = 0; t < NV; t++) {
-        const int j = lane + 64 * t;
-        s0[t] = (i0 < m && j < m) ? S[(int64_t)i0 * m + j] : 0.f;
-    }
-    // ... then f of this top into LDS
-    float* f = chol_sh; // 3 m
-#pragma unroll
-    for (int t = 0; t < PER; t++) {
-        const int q = threadIdx.x + t * CHOL_TOP_BLK;
-        if (q < m) st3(f, q, ld3(ftop, p0 + q));
+        const int q = threadIdx.x + CHOL_TOP_BLK * t;
+        if (q < mp) {
+            const float3 e = q < m ? ld3(f, pos ? (int64_t)pos[p0 + q] : p0 + q) : f3(0.f, 0.f, 0.f);
+            v[q] = e.x;
+            v[mp + q] = e.y;
+            v[2 * mp + q] = e.z;
+        }
     }
     __syncthreads();
-    float3 a0 = f3(0.f, 0.f, 0.f);
+    float3 a = f3(0.f, 0.f, 0.f);
 #pragma unroll
     for (int t = 0; t < NV; t++) {
-        const int j = lane + 64 * t;
-        if (j < m) a0 = a0 + s0[t] * ld3(f, j);
+        const int j = min(4 * lane + 256 * t, mp - 4);
+        const float4 p = s0[t], vx = *reinterpret_cast<const float4*>(v + j), vy = *reinterpret_cast<const float4*>(v + mp + j),
+                     vz = *reinterpret_cast<const float4*>(v + 2 * mp + j);
+        a.x += (p.x * vx.x + p.y * vx.y) + (p.z * vx.z + p.w * vx.w);
+        a.y += (p.x * vy.x + p.y * vy.y) + (p.z * vy.z + p.w * vy.w);
+        a.z += (p.x * vz.x + p.y * vz.y) + (p.z * vz.z + p.w * vz.w);
     }
-    // per-lane sums through LDS (after f's last use), added in lane order
-    __syncthreads();
-    float* red = chol_sh; // 3 CHOL_TOP_BLK
-    st3(red, threadIdx.x, a0);
-    __syncthreads();
-    if (lane == 0 && i0 < m) {
-        float3 t = f3(0.f, 0.f, 0.f);
-        for (int q = 0; q < 64; q++) t = t + ld3(red, wave * 64 + q);
-        st3(x, top_pos[p0 + i0], t);
-        st3(d, ridx[p0 + i0], t);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        a.x += __shfl_xor(a.x, o, 64);
+        a.y += __shfl_xor(a.y, o, 64);
+        a.z += __shfl_xor(a.z, o, 64);
     }
+    if (lane == 0 && i0 < m) st3(x, top_pos[p0 + i0], a);
 }
 
 // Rigid animation of static vertices (reference ScriptAnimator::animate_rigid,
@@ -3017,7 +2864,7 @@ void Backend::local_step(hipStream_t s) {
 void Backend::dual_vertices(bool want_res) {
     hipLaunchKernelGGL(k_dual_vert, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, n, (float)cfg.dt, (float)(1.0 / cfg.dt),
                        cfg.enable_contact, want_res ? 1 : 0, x.p, x0.p, p.p, wch2.p, Uc.p, res_part.p, 1.0 / (cfg.dt * cfg.dt),
-                       (const int32_t*)stop_guard, dx_pending ? (const float*)cg_d.p : nullptr);
+                       (const int32_t*)stop_guard, dx_pending ? (const float*)chol_x.p : nullptr, (const int32_t*)chol_ipos.p);
     PA_LAUNCH_CHECK();
     dx_pending = false;
 }
@@ -3081,7 +2928,7 @@ void Backend::contact_sweep_once() {
 // The right-hand side, and with the direct solve also the residual of its
 // first pass (cg_r): global_solve then starts from it.
 void Backend::rhs(bool want_res, bool first_iter) {
-    const ResidArgs A{a_ptr.p, a_col.p, a_val.p, a_val_lo.p, a_diag.p, a_diag_lo.p, x.p, cg_r.p};
+    const ResidArgs A{a_ptr.p, a_col.p, a_val.p, a_val_lo.p, a_diag.p, a_diag_lo.p, x.p, cg_r.p, chol_ipos.p};
     const int store_b = cfg.global_refine > 1 ? 1 : 0;
     with_lpr(rhs_lpr, [&](auto c) {
         constexpr int P = decltype(c)::value;
@@ -3114,11 +2961,7 @@ double Backend::spmv_time_ms(int reps) {
         PA_HIP(hipEventRecord(e0, stream));
         for (int r = 0; r < reps; r++) {
             if (use_chol) { // the dense-top product on the last solve's vectors
-                hipLaunchKernelGGL(k_chol_top, dim3(chol_top_tiles), dim3(CHOL_TOP_BLK), chol_top_lds, stream,
-                                   (const int2*)chol_tiles.p, (const int64_t*)chol_top_ptr.p, (const int32_t*)chol_top_pos.p,
-                                   (const int32_t*)chol_top_ridx.p, (const int64_t*)chol_sinv_off.p, (const float*)chol_sinv.p,
-                                   (const float*)chol_ftop.p, chol_x.p, cg_d.p);
-                PA_LAUNCH_CHECK();
+                chol_top_launch(cg_r.p);
                 continue;
             }
             with_lpr(a_lpr, [&](auto c) {
@@ -3393,170 +3236,219 @@ void Backend::chol_setup(const std::vector<int32_t>& aptr, const std::vector<int
     Ah.val = aval;
     SupernodalFactor F;
     try {
-        F = chol_factor(Ah, x0h, 64, CHOL_TOP_MAX);
+        F = chol_factor(Ah, x0h, n <= CHOL_BIG_LEAF_N ? 160 : 64, CHOL_TOP_MAX);
     } catch (const std::exception& e) {
         throw Error(PA_ERR_NOT_SPD, std::string("direct solve set-up: ") + e.what());
     }
     const int ns = F.nsuper;
-    // level lists of the supernodes below the dense tops, and their LDS needs
+    PA_CHECK(F.below.size() < ((size_t)1 << 31), PA_ERR_INVALID, "direct solve: too many rows below the diagonal blocks");
+    // supernodes below the dense tops by height
     chol_levels = F.lower_levels;
-    chol_lvl_ptr.assign(chol_levels + 1, 0);
+    std::vector<int32_t> lvl_ptr(chol_levels + 1, 0);
     for (int k = 0; k < ns; k++)
-        if (!F.is_top[k]) chol_lvl_ptr[F.height[k] + 1]++;
-    chol_lvl_wide.assign(chol_levels, 0);
-    chol_lvl_lds.assign(chol_levels, 0);
-    chol_sf_lds.assign(chol_levels, 0);
-    chol_sg_lds.assign(chol_levels, 0);
-    chol_sx_lds.assign(chol_levels, 0);
-    // wide levels: 2 = the larger factor tile (up to CHOL_BIG_TILE_MAX supernodes, where the
-    // level's workgroups fit the chip at once), 1 = the smaller one (more workgroups per CU)
-    for (int h = 0; h < chol_levels; h++)
-        chol_lvl_wide[h] = chol_lvl_ptr[h + 1] < CHOL_WIDE_MIN ? 0 : chol_lvl_ptr[h + 1] <= CHOL_BIG_TILE_MAX ? 2 : 1;
-    for (int k = 0; k < ns; k++) {
-        if (F.is_top[k]) continue;
-        const int h = F.height[k], w = F.width(k), nb = F.nbelow(k);
-        PA_CHECK(w <= 4096 && nb <= 4096, PA_ERR_INVALID, "direct solve: a supernode is too large (use precond 1)");
-        if (chol_lvl_wide[h]) {
-            const int fl = chol_lvl_wide[h] == 2 ? chol_lds_floats<256, 8192>(w, nb) : chol_lds_floats<256, 4096>(w, nb);
-            chol_lvl_lds[h] = std::max(chol_lvl_lds[h], (int)sizeof(float) * fl);
-        } else {
-            chol_sf_lds[h] = std::max(chol_sf_lds[h], (int)sizeof(float) * (6 * w + 3 * CHOL_SPLIT_ROWS + 3 * CHOL_SPLIT_BLK +
-                                                                           CHOL_SPLIT_TILE));
-            chol_sg_lds[h] = std::max(chol_sg_lds[h], (int)sizeof(float) * 3 * (CHOL_SPLIT_BLK + std::max(1, nb)));
-            chol_sx_lds[h] = std::max(chol_sx_lds[h], (int)sizeof(float) * 3 * (CHOL_SPLIT_BLK + std::max(1, w)));
-        }
-        PA_CHECK(std::max({chol_lvl_lds[h], chol_sf_lds[h], chol_sg_lds[h], chol_sx_lds[h]}) <= 65536, PA_ERR_INVALID,
-                 "direct solve: a front is too large for one workgroup's LDS (use precond 1)");
-    }
-    for (int h = 0; h < chol_levels; h++) chol_lvl_ptr[h + 1] += chol_lvl_ptr[h];
-    std::vector<int32_t> lvl_sup(std::max(1, chol_lvl_ptr[chol_levels]));
+        if (!F.is_top[k]) lvl_ptr[F.height[k] + 1]++;
+    for (int h = 0; h < chol_levels; h++) lvl_ptr[h + 1] += lvl_ptr[h];
+    std::vector<int32_t> lvl_sup(lvl_ptr[chol_levels]);
     {
-        std::vector<int32_t> fill(chol_lvl_ptr.begin(), chol_lvl_ptr.end() - 1);
+        std::vector<int32_t> fill(lvl_ptr.begin(), lvl_ptr.end() - 1);
         for (int k = 0; k < ns; k++)
             if (!F.is_top[k]) lvl_sup[fill[F.height[k]]++] = k;
     }
-    // split launches of the narrow levels: tiles per level
+    // panels [D; -W], column-major, both blocks' rows padded to whole float4s
+    auto pad4 = [](int64_t v) { return (v + 3) & ~(int64_t)3; };
+    std::vector<int64_t> panel_off(ns + 1, 0);
+    for (int k = 0; k < ns; k++) panel_off[k + 1] = panel_off[k] + (F.is_top[k] ? 0 : (pad4(F.width(k)) + pad4(F.nbelow(k))) * F.width(k));
+    std::vector<float> panels(std::max<int64_t>(4, panel_off[ns]), 0.f);
     {
-        std::vector<int2> sf, sg, sx;
-        chol_sf_ptr.assign(chol_levels + 1, 0);
-        chol_sg_ptr.assign(chol_levels + 1, 0);
-        chol_sx_ptr.assign(chol_levels + 1, 0);
-        for (int h = 0; h < chol_levels; h++) {
-            if (!chol_lvl_wide[h])
-                for (int q = chol_lvl_ptr[h]; q < chol_lvl_ptr[h + 1]; q++) {
-                    const int k = lvl_sup[q], w = F.width(k), nb = F.nbelow(k);
-                    for (int j0 = 0; j0 < std::max(1, nb); j0 += CHOL_SPLIT_ROWS) sf.push_back(make_int2(k, j0));
-                    for (int k0 = 0; k0 < w; k0 += CHOL_SPLIT_KC) sg.push_back(make_int2(k, k0));
-                    for (int i0 = 0; i0 < w; i0 += CHOL_SPLIT_KC) sx.push_back(make_int2(k, i0));
+        std::atomic<int> next{0};
+        auto work = [&, max_nb = (size_t)F.max_rows]() noexcept {
+            std::unique_ptr<double[]> col(new (std::nothrow) double[max_nb + 1]);
+            if (!col) return; // the other workers, or the check below, take the rest
+            for (int k; (k = next.fetch_add(1)) < ns;) {
+                if (F.is_top[k]) continue;
+                const int64_t w = F.width(k), nb = F.nbelow(k), nr = w + nb, wp = pad4(w), ld = wp + pad4(nb);
+                const double* L21 = F.panel.data() + F.panel_off[k] + w;
+                const double* Li = F.linv.data() + F.inv_off[k];
+                for (int64_t i = 0; i < w; i++) {
+                    float* o = panels.data() + panel_off[k] + i * ld;
+                    for (int64_t j = 0; j < w; j++) { // D = L11^-T L11^-1
+                        double acc = 0;
+                        for (int64_t q = std::max(i, j); q < w; q++) acc += Li[i * w + q] * Li[j * w + q];
+                        o[j] = (float)acc;
+                    }
+                    std::fill_n(col.get(), nb, 0.0); // column i of W = L21 L11^-1
+                    for (int64_t q = i; q < w; q++) {
+                        const double l = Li[i * w + q];
+                        const double* c = L21 + q * nr;
+                        for (int64_t j = 0; j < nb; j++) col[j] += c[j] * l;
+                    }
+                    for (int64_t j = 0; j < nb; j++) o[wp + j] = (float)-col[j];
                 }
-            chol_sf_ptr[h + 1] = (int32_t)sf.size();
-            chol_sg_ptr[h + 1] = (int32_t)sg.size();
-            chol_sx_ptr[h + 1] = (int32_t)sx.size();
+            }
+        };
+        std::vector<std::thread> pool;
+        const unsigned nt = std::max(1u, std::min({16u, std::thread::hardware_concurrency(), (unsigned)std::max(1, ns / 8)}));
+        try {
+            pool.reserve(nt);
+            for (unsigned q = 1; q < nt; q++) pool.emplace_back(work);
+        } catch (const std::exception&) { // fewer workers
         }
-        for (auto* v : {&sf, &sg, &sx})
-            if (v->empty()) v->push_back(make_int2(0, 0));
-        chol_sf_tiles.upload(sf, stream);
-        chol_sg_tiles.upload(sg, stream);
-        chol_sx_tiles.upload(sx, stream);
+        work();
+        for (std::thread& q : pool) q.join();
+        PA_CHECK(next.load() >= ns, PA_ERR_INVALID, "direct solve set-up: out of memory");
     }
-    // dense tops: workgroup tiles and LDS
+    // where the rows of every front come from: the children's update-vector entries
+    std::vector<int32_t> gat_off(ns, 0), gat_rows;
+    for (int k = 0; k < ns; k++) {
+        const int kids = F.child_ptr[k + 1] - F.child_ptr[k];
+        if (F.is_top[k] || kids == 0) continue;
+        PA_CHECK(gat_rows.size() < ((size_t)1 << 30), PA_ERR_INVALID, "direct solve: front tables too large");
+        gat_off[k] = (int32_t)gat_rows.size();
+        gat_rows.resize(gat_rows.size() + (size_t)kids * (F.width(k) + F.nbelow(k)), -1);
+        for (int q = 0; q < kids; q++) {
+            const int c = F.child[F.child_ptr[k] + q];
+            for (int64_t e = F.below_ptr[c]; e < F.below_ptr[c + 1]; e++) gat_rows[gat_off[k] + (size_t)F.rel[e] * kids + q] = (int32_t)e;
+        }
+    }
+    if (gat_rows.empty()) gat_rows.push_back(-1);
+    // tiles of every level.  The tile size is the largest that still gives the
+    // level CHOL_TILES_MIN workgroups (one per CU): narrow levels of large
+    // fronts spread over the chip, wide ones gather each front fewer times
+    // (256x256 cloth step: 13.7 ms at 2048, 13.0 at 1024, 12.5 at 256, 12.4 at 128).
+    constexpr int CHOL_TILES_MIN = 256;
+    std::vector<CholTile> up, down;
+    chol_up_ptr.assign(chol_levels + 1, 0);
+    chol_down_ptr.assign(chol_levels + 1, 0);
+    chol_rg.assign(chol_levels, 16);
+    chol_lp.assign(chol_levels, 8);
+    chol_up_lds.assign(chol_levels, 0);
+    chol_down_lds.assign(chol_levels, 0);
+    for (int h = 0; h < chol_levels; h++) {
+        auto count = [&](bool rows, int size) {
+            int64_t c = 0;
+            for (int q = lvl_ptr[h]; q < lvl_ptr[h + 1]; q++) {
+                const int v = rows ? F.nbelow(lvl_sup[q]) : F.width(lvl_sup[q]);
+                c += std::max(1, (v + size - 1) / size);
+            }
+            return c;
+        };
+        while (chol_rg[h] > 4 && count(true, 4 * chol_rg[h]) < CHOL_TILES_MIN) chol_rg[h] /= 2;
+        while (chol_lp[h] < 32 && count(false, CHOL_BLK / chol_lp[h]) < CHOL_TILES_MIN) chol_lp[h] *= 2;
+        for (int q = lvl_ptr[h]; q < lvl_ptr[h + 1]; q++) {
+            const int k = lvl_sup[q], w = F.width(k), nb = F.nbelow(k);
+            PA_CHECK(w <= 4096 && nb <= 4096, PA_ERR_INVALID, "direct solve: a supernode is too large (use precond 1)");
+            CholTile T{panel_off[k], F.col0[k], w, nb, 0, (int32_t)F.below_ptr[k], gat_off[k], F.child_ptr[k + 1] - F.child_ptr[k], 0};
+            for (T.first = 0; T.first < std::max(1, nb); T.first += 4 * chol_rg[h]) up.push_back(T);
+            for (T.first = 0; T.first < w; T.first += CHOL_BLK / chol_lp[h]) down.push_back(T);
+            chol_up_lds[h] = std::max(chol_up_lds[h], (int)sizeof(float4) * std::max(1, w));
+            chol_down_lds[h] = std::max<int>(chol_down_lds[h], (int)sizeof(float) * 3 * (pad4(w) + pad4(nb)));
+        }
+        PA_CHECK(chol_up_lds[h] <= 65536 - 4096 && chol_down_lds[h] <= 65536, PA_ERR_INVALID,
+                 "direct solve: a front is too large for one workgroup's LDS (use precond 1)");
+        chol_up_ptr[h + 1] = (int32_t)up.size();
+        chol_down_ptr[h + 1] = (int32_t)down.size();
+    }
+    // dense tops: workgroup tiles, LDS, and S^-1 with padded rows
     std::vector<int2> tiles;
     int max_m = 0;
+    std::vector<int64_t> sinv_off(F.sinv_off.size(), 0);
     for (size_t blk = 0; blk + 1 < F.top_ptr.size(); blk++) {
         const int m = (int)(F.top_ptr[blk + 1] - F.top_ptr[blk]);
         max_m = std::max(max_m, m);
         for (int r0 = 0; r0 < m; r0 += CHOL_TOP_ROWS) tiles.push_back(make_int2((int)blk, r0));
+        if (blk + 1 < sinv_off.size()) sinv_off[blk + 1] = sinv_off[blk] + (int64_t)m * pad4(m);
     }
     PA_CHECK(max_m <= CHOL_TOP_MAX, PA_ERR_INVALID, "direct solve: a dense top is too large");
+    std::vector<float> sinv;
+    for (size_t blk = 0; blk + 1 < F.top_ptr.size(); blk++) {
+        const int64_t m = F.top_ptr[blk + 1] - F.top_ptr[blk], mp = pad4(m);
+        sinv.resize(sinv_off[blk] + m * mp, 0.f);
+        const double* S = F.sinv.data() + F.sinv_off[blk];
+        for (int64_t i = 0; i < m; i++)
+            for (int64_t j = 0; j < m; j++) sinv[sinv_off[blk] + i * mp + j] = (float)S[i * m + j];
+    }
+    if (sinv.empty()) sinv.push_back(0.f);
     chol_top_tiles = (int)tiles.size();
-    chol_top_lds = (int)sizeof(float) * std::max(3 * max_m, 3 * CHOL_TOP_BLK);
-    // per top entry: its unknown, and a fixed-width list of the update-vector entries it gathers (-1: none)
+    chol_top_nv = 1;
+    while (256 * chol_top_nv < max_m) chol_top_nv *= 2;
+    chol_top_lds = (int)sizeof(float) * 3 * (int)pad4(std::max(max_m, 4));
+    // per top entry a fixed-width list of the update-vector entries it gathers (-1: none)
     const size_t ntop = F.top_pos.size();
-    std::vector<int32_t> ridx(std::max<size_t>(1, ntop), 0);
-    for (size_t q = 0; q < ntop; q++) ridx[q] = F.perm[F.top_pos[q]];
     chol_gmax = 1;
     for (size_t q = 0; q < ntop; q++) chol_gmax = std::max<int>(chol_gmax, (int)(F.gat_ptr[q + 1] - F.gat_ptr[q]));
     PA_CHECK(chol_gmax <= CHOL_TOP_GMAX, PA_ERR_INVALID, "direct solve: a dense-top entry gathers too many update vectors");
     std::vector<int64_t> gat_fix(std::max<size_t>(1, ntop) * chol_gmax, -1);
     for (size_t q = 0; q < ntop; q++)
         for (int64_t e = F.gat_ptr[q]; e < F.gat_ptr[q + 1]; e++) gat_fix[q * chol_gmax + (e - F.gat_ptr[q])] = F.gat[e];
-    // factor blocks in FP32, column-major
-    std::vector<int64_t> l21_off(ns + 1, 0);
-    for (int k = 0; k < ns; k++) l21_off[k + 1] = l21_off[k] + (F.is_top[k] ? 0 : (int64_t)F.nbelow(k) * F.width(k));
-    std::vector<int64_t> inv_off(ns + 1, 0);
-    for (int k = 0; k < ns; k++) inv_off[k + 1] = inv_off[k] + (F.is_top[k] ? 0 : (int64_t)F.width(k) * F.width(k));
-    std::vector<float> l21(std::max<int64_t>(1, l21_off[ns])), linv(std::max<int64_t>(1, inv_off[ns]));
-    for (int k = 0; k < ns; k++) {
-        if (F.is_top[k]) continue;
-        const int64_t w = F.width(k), nb = F.nbelow(k), nr = w + nb;
-        const double* P = F.panel.data() + F.panel_off[k];
-        float* L = l21.data() + l21_off[k];
-        for (int64_t c = 0; c < w; c++)
-            for (int64_t j = 0; j < nb; j++) L[c * nb + j] = (float)P[c * nr + w + j];
-        const double* Li = F.linv.data() + F.inv_off[k];
-        float* I = linv.data() + inv_off[k];
-        for (int64_t q = 0; q < w * w; q++) I[q] = (float)Li[q];
-    }
-    std::vector<float> sinv(std::max<size_t>(1, F.sinv.size()));
-    for (size_t q = 0; q < F.sinv.size(); q++) sinv[q] = (float)F.sinv[q];
     auto nonempty = [](std::vector<int32_t> v) {
         if (v.empty()) v.push_back(0);
         return v;
     };
-    chol_lvl_sup.upload(lvl_sup, stream);
-    chol_perm.upload(F.perm, stream);
-    chol_col0.upload(F.col0, stream);
-    chol_below_ptr.upload(F.below_ptr, stream);
+    if (up.empty()) up.push_back(CholTile{});
+    if (down.empty()) down.push_back(CholTile{});
+    if (tiles.empty()) tiles.push_back(make_int2(0, 0));
+    chol_up_tiles.reserve(up.size() * sizeof(CholTile));
+    chol_up_tiles.upload(reinterpret_cast<const uint8_t*>(up.data()), up.size() * sizeof(CholTile), stream);
+    chol_down_tiles.reserve(down.size() * sizeof(CholTile));
+    chol_down_tiles.upload(reinterpret_cast<const uint8_t*>(down.data()), down.size() * sizeof(CholTile), stream);
+    chol_panels.upload(panels, stream);
+    chol_gat_rows.upload(gat_rows, stream);
+    chol_ipos.upload(F.iperm, stream);
     chol_below.upload(nonempty(F.below), stream);
-    chol_rel.upload(nonempty(F.rel), stream);
-    chol_child_ptr.upload(F.child_ptr, stream);
-    chol_child.upload(nonempty(F.child), stream);
-    chol_l21_off.upload(l21_off, stream);
-    chol_inv_off.upload(inv_off, stream);
-    chol_l21.upload(l21, stream);
-    chol_linv.upload(linv, stream);
     chol_top_ptr.upload(F.top_ptr, stream);
     chol_top_pos.upload(nonempty(F.top_pos), stream);
-    chol_top_ridx.upload(ridx, stream);
     chol_gat.upload(gat_fix, stream);
-    chol_sinv_off.upload(F.sinv_off, stream);
+    chol_sinv_off.upload(sinv_off, stream);
     chol_sinv.upload(sinv, stream);
-    if (tiles.empty()) tiles.push_back(make_int2(0, 0));
     chol_tiles.upload(tiles, stream);
-    chol_y.alloc(3 * (size_t)n);
+    chol_f.alloc(3 * (size_t)n);
     chol_x.alloc(3 * (size_t)n);
-    chol_g.alloc(3 * (size_t)n);
     chol_u.alloc(3 * std::max<size_t>(1, F.below.size()));
     chol_ftop.alloc(3 * std::max<size_t>(1, ntop));
-    chol_entries = l21_off[ns] + inv_off[ns] + (int64_t)F.sinv.size();
+    chol_entries = panel_off[ns] + (int64_t)sinv.size();
     chol_top_cols = (int64_t)F.top_pos.size();
     chol_top_sq = (int64_t)F.sinv.size();
     use_chol = true;
     chol_setup_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
 }
 
-void Backend::chol_solve(const float* r, float* d) {
-    CholArgs a{nullptr, chol_perm.p, chol_col0.p, chol_below_ptr.p, chol_below.p, chol_rel.p,
-               chol_child_ptr.p, chol_child.p, chol_l21_off.p, chol_inv_off.p};
+// The dense-top product; r: the residual in elimination order, which is the
+// right-hand side itself where there is no level below the tops.
+void Backend::chol_top_launch(const float* r) {
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(chol_top_tiles), dim3(CHOL_TOP_BLK), chol_top_lds, stream, (const int2*)chol_tiles.p,
+                           (const int64_t*)chol_top_ptr.p, (const int32_t*)chol_top_pos.p, (const int64_t*)chol_sinv_off.p,
+                           (const float*)chol_sinv.p, chol_levels > 0 ? (const float*)chol_ftop.p : r,
+                           chol_levels > 0 ? (const int32_t*)nullptr : (const int32_t*)chol_top_pos.p, chol_x.p);
+    };
+    switch (chol_top_nv) {
+    case 1: go(k_chol_top<1>); break;
+    case 2: go(k_chol_top<2>); break;
+    case 4: go(k_chol_top<4>); break;
+    case 8: go(k_chol_top<8>); break;
+    default: go(k_chol_top<16>); break;
+    }
+    PA_LAUNCH_CHECK();
+}
+
+// chol_x = A^-1 r, both in elimination order (3 interleaved columns, FP32).
+void Backend::chol_solve(const float* r) {
+    const CholTile* up = reinterpret_cast<const CholTile*>(chol_up_tiles.p);
+    const CholTile* down = reinterpret_cast<const CholTile*>(chol_down_tiles.p);
     for (int h = 0; h < chol_levels; h++) {
-        const int cnt = chol_lvl_ptr[h + 1] - chol_lvl_ptr[h];
-        if (cnt == 0) continue;
-        a.sup = chol_lvl_sup.p + chol_lvl_ptr[h];
-        if (chol_lvl_wide[h]) {
-            hipLaunchKernelGGL((chol_lvl_wide[h] == 2 ? k_chol_fwd<256, 8192> : k_chol_fwd<256, 4096>), dim3(cnt), dim3(256), chol_lvl_lds[h],
-                               stream, a, (const float*)chol_l21.p, (const float*)chol_linv.p, r, chol_y.p, chol_u.p);
-        } else {
-            const int nt = chol_sf_ptr[h + 1] - chol_sf_ptr[h];
-            hipLaunchKernelGGL(k_chol_fwd_split, dim3(nt), dim3(CHOL_SPLIT_BLK), chol_sf_lds[h], stream, a,
-                               (const int2*)chol_sf_tiles.p + chol_sf_ptr[h], CHOL_SPLIT_ROWS, (const float*)chol_l21.p,
-                               (const float*)chol_linv.p, r, chol_y.p, chol_u.p);
-        }
+        const int nt = chol_up_ptr[h + 1] - chol_up_ptr[h];
+        if (nt == 0) continue;
+        hipLaunchKernelGGL((chol_rg[h] == 16 ? k_chol_up<16> : chol_rg[h] == 8 ? k_chol_up<8> : k_chol_up<4>), dim3(nt), dim3(CHOL_BLK),
+                           chol_up_lds[h], stream, up + chol_up_ptr[h], (const float*)chol_panels.p, (const int32_t*)chol_gat_rows.p, r,
+                           chol_f.p, chol_u.p);
         PA_LAUNCH_CHECK();
     }
     if (chol_top_tiles > 0) {
-        hipLaunchKernelGGL(k_chol_top_f, dim3(grid_for(chol_top_cols, BLK)), dim3(BLK), 0, stream, (int)chol_top_cols,
-                           (const int32_t*)chol_top_ridx.p, (const int64_t*)chol_gat.p, chol_gmax, r, (const float*)chol_u.p, chol_ftop.p);
-        PA_LAUNCH_CHECK();
+        if (chol_levels > 0) {
+            hipLaunchKernelGGL(k_chol_top_f, dim3(grid_for(chol_top_cols, BLK)), dim3(BLK), 0, stream, (int)chol_top_cols,
+                               (const int32_t*)chol_top_pos.p, (const int64_t*)chol_gat.p, chol_gmax, r, (const float*)chol_u.p, chol_ftop.p);
+            PA_LAUNCH_CHECK();
+        }
         hipEvent_t e0 = nullptr, e1 = nullptr;
         const bool mark = (profiling & 1) && !capturing;
         if (mark) {
@@ -3564,34 +3456,18 @@ void Backend::chol_solve(const float* r, float* d) {
             e1 = next_event();
             PA_HIP(hipEventRecord(e0, stream));
         }
-        hipLaunchKernelGGL(k_chol_top, dim3(chol_top_tiles), dim3(CHOL_TOP_BLK), chol_top_lds, stream, (const int2*)chol_tiles.p,
-                           (const int64_t*)chol_top_ptr.p, (const int32_t*)chol_top_pos.p, (const int32_t*)chol_top_ridx.p,
-                           (const int64_t*)chol_sinv_off.p, (const float*)chol_sinv.p, (const float*)chol_ftop.p, chol_x.p, d);
-        PA_LAUNCH_CHECK();
+        chol_top_launch(r);
         if (mark) {
             PA_HIP(hipEventRecord(e1, stream));
             spmv_marks.push_back({e0, e1});
         }
     }
     for (int h = chol_levels - 1; h >= 0; h--) {
-        const int cnt = chol_lvl_ptr[h + 1] - chol_lvl_ptr[h];
-        if (cnt == 0) continue;
-        a.sup = chol_lvl_sup.p + chol_lvl_ptr[h];
-        if (chol_lvl_wide[h]) {
-            hipLaunchKernelGGL((chol_lvl_wide[h] == 2 ? k_chol_bwd<256, 8192> : k_chol_bwd<256, 4096>), dim3(cnt), dim3(256), chol_lvl_lds[h],
-                               stream, a, (const float*)chol_l21.p, (const float*)chol_linv.p, (const float*)chol_y.p, chol_x.p, d);
-            PA_LAUNCH_CHECK();
-            continue;
-        }
-        const int ng = chol_sg_ptr[h + 1] - chol_sg_ptr[h];
-        hipLaunchKernelGGL(k_chol_bwd_g, dim3(ng), dim3(CHOL_SPLIT_BLK), chol_sg_lds[h], stream, a,
-                           (const int2*)chol_sg_tiles.p + chol_sg_ptr[h], (const float*)chol_l21.p, (const float*)chol_y.p,
-                           (const float*)chol_x.p, chol_g.p);
-        PA_LAUNCH_CHECK();
-        const int nx = chol_sx_ptr[h + 1] - chol_sx_ptr[h];
-        hipLaunchKernelGGL(k_chol_bwd_x, dim3(nx), dim3(CHOL_SPLIT_BLK), chol_sx_lds[h], stream, a,
-                           (const int2*)chol_sx_tiles.p + chol_sx_ptr[h], (const float*)chol_linv.p, (const float*)chol_g.p,
-                           chol_x.p, d);
+        const int nt = chol_down_ptr[h + 1] - chol_down_ptr[h];
+        if (nt == 0) continue;
+        hipLaunchKernelGGL((chol_lp[h] == 8 ? k_chol_down<8> : chol_lp[h] == 16 ? k_chol_down<16> : k_chol_down<32>), dim3(nt),
+                           dim3(CHOL_BLK), chol_down_lds[h], stream, down + chol_down_ptr[h], (const float*)chol_panels.p,
+                           (const int32_t*)chol_below.p, (const float*)chol_f.p, chol_x.p);
         PA_LAUNCH_CHECK();
     }
 }
@@ -3622,16 +3498,17 @@ int Backend::global_solve(int max_iter, double tol, bool defer_last, bool resid_
                 with_lpr(a_lpr, [&](auto c) {
                     constexpr int P = decltype(c)::value;
                     hipLaunchKernelGGL(k_cg_resid64<P>, dim3(nb), dim3(PBLK), 0, stream, n, a_ptr.p, a_col.p, a_val.p, a_val_lo.p,
-                                       a_diag.p, a_diag_lo.p, b.p, x.p, cg_r.p, cg_d.p, cg_part.p);
+                                       a_diag.p, a_diag_lo.p, b.p, x.p, cg_r.p, cg_d.p, cg_part.p, (const int32_t*)chol_ipos.p);
                 });
                 PA_LAUNCH_CHECK();
             }
-            chol_solve(cg_r.p, cg_d.p);
+            chol_solve(cg_r.p);
             if (defer_last && pass == passes - 1) { // x += d is applied by the next dual update
                 dx_pending = true;
                 break;
             }
-            hipLaunchKernelGGL(k_axpy_d, dim3(grid_for(3 * (int64_t)n, BLK)), dim3(BLK), 0, stream, n, cg_d.p, x.p, (const int32_t*)stop_guard);
+            hipLaunchKernelGGL(k_axpy_d, dim3(grid_for(3 * (int64_t)n, BLK)), dim3(BLK), 0, stream, n, (const float*)chol_x.p,
+                               (const int32_t*)chol_ipos.p, x.p, (const int32_t*)stop_guard);
             PA_LAUNCH_CHECK();
         }
         return passes;
@@ -3640,7 +3517,7 @@ int Backend::global_solve(int max_iter, double tol, bool defer_last, bool resid_
         with_lpr(a_lpr, [&](auto c) {
             constexpr int P = decltype(c)::value;
             hipLaunchKernelGGL(k_cg_resid64<P>, dim3(nb), dim3(PBLK), 0, stream, n, a_ptr.p, a_col.p, a_val.p, a_val_lo.p, a_diag.p,
-                               a_diag_lo.p, b.p, x.p, cg_r.p, cg_d.p, cg_part.p);
+                               a_diag_lo.p, b.p, x.p, cg_r.p, cg_d.p, cg_part.p, (const int32_t*)nullptr);
         });
         PA_LAUNCH_CHECK();
         if (per_scene) {
@@ -3695,7 +3572,8 @@ int Backend::global_solve(int max_iter, double tol, bool defer_last, bool resid_
                                (int)hs[19], scene_iters.p);
             PA_LAUNCH_CHECK();
         }
-        hipLaunchKernelGGL(k_axpy_d, dim3(grid_for(3 * (int64_t)n, BLK)), dim3(BLK), 0, stream, n, cg_d.p, x.p, (const int32_t*)stop_guard);
+        hipLaunchKernelGGL(k_axpy_d, dim3(grid_for(3 * (int64_t)n, BLK)), dim3(BLK), 0, stream, n, (const float*)cg_d.p,
+                           (const int32_t*)nullptr, x.p, (const int32_t*)stop_guard);
         PA_LAUNCH_CHECK();
     }
     return total_iters;

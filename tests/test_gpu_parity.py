@@ -262,6 +262,32 @@ def test_direct_solve_matches_llt(pa, passes):
         assert err < (2e-4 if passes == 1 else 1e-6)
 
 
+@pytest.mark.parametrize("sides", [(2,), (3,), (13,), (16, 2, 41), (64,), (65,), (80, 5, 64), (120,)], ids=str)
+def test_direct_solve_at_factor_edges(pa, sides):
+    """Cloths below, at and above a leaf's and a dense top's size (a 64 x 64
+    cloth is all top, a 65 x 65 one has a level below it), alone and in
+    forests, with row and column counts that are no multiples of the solve's
+    tiles.  One pass against the oracle's LLT: the FP32 panels and products
+    round at 6e-8 times a modest growth over the levels, so 1e-5 of the
+    correction."""
+    from parallel_admm_amd.configs import config_for
+
+    rng = np.random.default_rng(8)
+    cfg = config_for("batch")
+    parts = [pa.Scene.generate(4, side=s, radius=0.1, drop=0.3) for s in sides]
+    sc = parts[0] if len(parts) == 1 else pa.Scene.merge(parts)
+    m = sc.mesh()
+    n = sc.info["n_dyn"]
+    o = _oracle(m, cfg)
+    rhs = o.matrix(1) @ (m["x"][:n] + 0.01 * rng.standard_normal((n, 3)))
+    xo = o.solve(rhs)
+    x0 = m["x"][:n]
+    xg, _ = pa.ADMMBackendHIP.from_scene(sc, cfg).global_solve(rhs, x0)
+    err = np.linalg.norm(xg - xo) / np.linalg.norm(xo - x0)
+    print(f"sides {sides}: error / correction {err:.2e}")
+    assert err < 1e-5
+
+
 def test_global_solve_multi_pass_matches_llt(pa):
     """A 300 x 300 cloth (90,000 rows) is more rows than one pass of the fused
     PCG grid covers, so the kernels run their multi-pass variant (each pass
