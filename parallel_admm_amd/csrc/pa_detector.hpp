@@ -13,15 +13,13 @@ struct Tree {
     int n = 0;
     DBuf<float4> prim_box;   // 2 per primitive (lo, hi)
     DBuf<float4> leaf_box;   // 2 per sorted leaf (lo, hi)
-    int leaf_stride = 0;     // double2 per leaf in leafd (4 for edges, 6 for triangles)
-    DBuf<double2> leafd;     // per sorted leaf: FP64 vertex positions, then (primitive id, vertex ids)
+    DBuf<int4> leafid;       // per sorted leaf: primitive id and vertex ids
     DBuf<uint32_t> keys, ids; // sorted Morton codes and primitive ids
     DBuf<int32_t> child;     // 2 per internal node
     DBuf<int2> range;        // per internal node: first and last sorted leaf it covers
     DBuf<float4> rec;        // 8 per internal node: boxes, ids and last leaf of its up to four grandchildren
-    DBuf<float4> chunk64;    // 2 per 64-leaf chunk: union of its leaf boxes
-    DBuf<float4> chunk4k;    // 2 per 4096-leaf chunk
-    DBuf<float4> chunk256k;  // 2 per 262144-leaf chunk
+    DBuf<float4> blk_box;    // 2 per block of sorted leaves that the refit takes together
+    DBuf<int32_t> cross;     // [0] count, then the internal nodes whose range crosses such a block's boundary
     DBuf<int32_t> ipos;      // per internal node: float4 index of its record slot (-1: none)
     DBuf<int32_t> lpos;      // 2 per leaf: its slot in the parent's record, in the grandparent's (-1: none)
     DBuf<float4> scene;      // 2: scene box
@@ -58,20 +56,20 @@ struct Detector {
     DBuf<double> x_own; // positions uploaded through detect(host x)
     Tree ft, et;
     ContactBuffers c;   // canonical list
-    ContactBuffers stg; // staging list in discovery order (single traversal)
-    DBuf<int2> st_seg;      // per staged contact: its segment and its place in the segment's unsorted order
+    DBuf<int2> single_pairs; // single pass: accepted (query, leaf) pairs
     DBuf<int32_t> seg_key;  // partner ids in segment order, unsorted inside a segment
     // one buffer, cleared by one launch per detection: total[0] contacts found
-    // (segment counts), [1] stack overflow flags, [2] staged contacts;
+    // (segment counts), [1] limit flags, [2] pairs of the single pass;
     // ovf_count[0..1]; qcount: nv + ne segment counts (PT per query vertex, EE
-    // per smaller edge id)
+    // per smaller edge id); qfill: partner ids written per segment
     DBuf<uint32_t> counts;
     uint32_t* total = nullptr;
     uint32_t* ovf_count = nullptr;
     uint32_t* qcount = nullptr;
+    uint32_t* qfill = nullptr;
     DBuf<uint32_t> qoffset;       // nv + ne segment offsets
     uint32_t* total_host = nullptr; // pinned: total[0..2] after the scan
-    // Leaf hits of the collect pass: per query a slab of up to 32 sorted leaf
+    // Leaf hits of the collect pass: per query a slab of up to 16 sorted leaf
     // indices (strided by the query count) and the number of hits; hits past
     // the slab as (query, leaf) pairs in an overflow list of one entry per
     // query ([0] PT, [1] EE counts).
@@ -116,7 +114,6 @@ struct Detector {
   private:
     void build_tree(Tree& T, const double* x, bool faces, hipStream_t s, PrimScratch& scr, bool refit);
     bool built = false; // trees built at least once (a refit needs their order and topology)
-    void node_boxes(Tree& T, hipStream_t s);
 };
 
 } // namespace pa

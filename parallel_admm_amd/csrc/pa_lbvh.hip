@@ -6,15 +6,15 @@
 // -> node boxes from leaf ranges -> 128-byte wide node records (the boxes,
 // ids and last sorted leaf of a node's up to four grandchildren, a leaf child
 // standing in for its own pair, so a traversal step descends two levels with
-// one dependent load; the stack top's record is loaded ahead, so a pop needs
-// none) -> one traversal per query with the FP64 predicate,
-// accepted pairs appended to a staging list with their segment.
+// one dependent load) -> per query a traversal by 16 lanes that collects close
+// leaves, then the FP64 predicate on them, accepted pairs marked and counted
+// per segment.
 //
-// Point-triangle: one lane per surface vertex; its pairs form the vertex's
-// segment.  Edge-edge: one lane per sorted leaf k, visiting only leaves after
+// Point-triangle: one query per surface vertex; its pairs form the vertex's
+// segment.  Edge-edge: one query per sorted leaf k, visiting only leaves after
 // k, so each unordered pair is tested once; the pair belongs to the segment of
 // its smaller edge id.  Segment counts -> exclusive scan -> partner ids into
-// their segments -> every pair to its rank in its segment: the list comes out
+// their segments -> every pair's fields to its rank in its segment: the list comes out
 // in canonical order, bit-identical on every run, with no global sort.
 //
 // Segmented mode (merged scenes): keys carry the scene id above a 21-bit
@@ -39,7 +39,13 @@ namespace {
 
 constexpr int BLK = 256;
 constexpr int QBLK = 128;
-constexpr int STACK = 64;
+constexpr int STACK = 64;          // single pass: stack entries per lane
+constexpr int CAND = 16;           // collected hits per query before the overflow list
+constexpr int CBLK = 256;          // collect block (four waves)
+constexpr int CSTACK = 1024, CSTACK_HIGH = 768; // collect: stack entries per wave, and the depth-first threshold
+constexpr int COLLECT_BITS = 26;   // collect: node and leaf indices in a packed entry
+constexpr uint32_t COLLECT_MASK = (1u << COLLECT_BITS) - 1u;
+constexpr int TBLK = 256, TQ = 64; // test block and its queries
 
 __device__ inline float4 fmin4(float4 a, float4 b) { return make_float4(fminf(a.x, b.x), fminf(a.y, b.y), fminf(a.z, b.z), 0.f); }
 __device__ inline float4 fmax4(float4 a, float4 b) { return make_float4(fmaxf(a.x, b.x), fmaxf(a.y, b.y), fmaxf(a.z, b.z), 0.f); }
@@ -125,8 +131,9 @@ __device__ inline uint32_t quant10(float u) {
 }
 
 __global__ void k_morton(const float4* __restrict__ box, int n, const float4* __restrict__ scene, uint32_t* __restrict__ keys,
-                         uint32_t* __restrict__ ids) {
+                         uint32_t* __restrict__ ids, int32_t* __restrict__ cross) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) cross[0] = 0; // for k_record_slots
     if (i >= n) return;
     float4 slo = scene[0], shi = scene[1];
     float4 lo = box[2 * i], hi = box[2 * i + 1];
@@ -143,8 +150,9 @@ __global__ void k_morton(const float4* __restrict__ box, int n, const float4* __
 // (7 bits per axis) of the box centre in the box of all segments.
 __global__ void k_morton_seg(const float4* __restrict__ box, const int32_t* __restrict__ prims, int k, int n,
                              const int32_t* __restrict__ vseg, const float4* __restrict__ scene, uint32_t* __restrict__ keys,
-                             uint32_t* __restrict__ ids) {
+                             uint32_t* __restrict__ ids, int32_t* __restrict__ cross) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) cross[0] = 0; // for k_record_slots
     if (i >= n) return;
     float4 slo = scene[0], shi = scene[1];
     float4 lo = box[2 * i], hi = box[2 * i + 1];
@@ -220,17 +228,12 @@ __global__ void k_karras(const uint32_t* __restrict__ keys, const uint32_t* __re
 
 // Node boxes without cross-block synchronisation: an internal node covers
 // the contiguous sorted-leaf range [lo, hi] (Karras), so its box is the union
-// of that range, taken from the leaf boxes at the ends and from precomputed
-// unions of aligned 64- and 4096-leaf chunks in the middle.  (A bottom-up
-// climb with atomic visit flags needs device-scope fences, which write back
-// and invalidate the per-XCD L2 on this part.)
-// Leaf data of a tree over K-vertex primitives (K = 2 edges, 3 triangles):
-// per double2 slots of leaf_stride<K>, first the primitive's FP64 vertex
-// positions (3K doubles, a zero pads triangles to 10), then an int4 of its
-// primitive id and vertex ids (-1 for none).  A traversal tests a leaf with
-// this one load instead of the chain sorted id -> vertex ids -> positions.
-template <int K> constexpr int leaf_stride() { return (3 * K + 1) / 2 + 1; }
-
+// of that range (k_refit, k_cross_boxes).  (A bottom-up climb with atomic visit
+// flags needs device-scope fences, which write back and invalidate the per-XCD
+// L2 on this part.)
+// Leaf ids of a tree: per sorted leaf its primitive id and vertex ids (-1 for
+// none), written once per build, so a query tests a leaf's vertices with one
+// load instead of the chain sorted id -> vertex ids.
 // Wide node record i (8 float4): four slots, slot j = (lo, node id) at
 // 2j and (hi, last sorted leaf under the node) at 2j + 1, ids and leaf
 // positions as int bits in w.  Slots 0-1 come from the left child, 2-3 from
@@ -248,133 +251,175 @@ __device__ inline void put_slot(float4* __restrict__ rec, int p, float4 lo, floa
     rec[p + 1] = make_float4(hi.x, hi.y, hi.z, __int_as_float(last));
 }
 
-// Leaf k (sorted order): its box (into leaf_box and its record slots) and
-// its leaf data.  The box is the primitive box of k_prim_boxes
-// (outward-rounded FP32 of the FP64 positions), so a refit needs no
-// primitive boxes.
+// Refit of RB consecutive sorted leaves: their boxes from x (a box is the
+// primitive box of k_prim_boxes, the outward-rounded FP32 of the FP64
+// positions) into their record slots, the box of every internal node whose
+// leaf range lies inside the block, and the block's own box (blk_box).
+// Node i's range begins or ends at leaf i (Karras), so node i of this block
+// is the only kind that can.  Its box is the union of two overlapping windows
+// of a power of two leaves (a union may count a leaf twice), read from a table
+// of all such windows that the block builds in LDS in log2(RB) steps: a node
+// costs two reads whatever its range.  Unions straight from the leaf boxes and
+// from 64- and 4096-leaf chunks in memory were a chain of up to 30 dependent
+// loads per node and three more launches: 33 + 4 + 4 us of the 256x256 cloth's
+// refit (28 us of FP64 leaf copies besides; the queries now take their vertices
+// from x), now 29 + 9; 350 + 60 + 222 us of a 160-scene batch's edges, now
+// 233 + 93.  Blocks of 128 and 64 leaves list two and four times the crossing
+// nodes and were slower in sum (19 + 12 and 17 + 21 us on the cloth's edges).
+constexpr int RB = 256, RB_LEVELS = 9;
 template <int K>
-__global__ void k_leaf_data(const double* __restrict__ x, const int32_t* __restrict__ prims, const uint32_t* __restrict__ ids, int n,
-                            float4* __restrict__ leaf_box, double2* __restrict__ leafd, const int2* __restrict__ lpos,
-                            float4* __restrict__ rec) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const int pid = (int)ids[k];
-    int v[K];
-    double p[3 * K + 1];
+__global__ void __launch_bounds__(RB) k_refit(const double* __restrict__ x, const int4* __restrict__ leafid, int n,
+                                              float4* __restrict__ leaf_box, const int2* __restrict__ lpos, const int2* __restrict__ range, const int32_t* __restrict__ ipos, float4* __restrict__ blk_box,
+                                              float4* __restrict__ rec) {
+    __shared__ float win[RB_LEVELS][6][RB]; // win[l][.][a]: box of leaves [a, a + 2^l) of the block
+    const int t = threadIdx.x, b0 = blockIdx.x * RB, k = b0 + t;
+    const bool node = k < n - 1;
+    const int p = node ? ipos[k] : -1; // the root and its children sit in no slot
+    const int2 rg = node ? range[k] : make_int2(0, 0);
     float4 lo = make_float4(INFINITY, INFINITY, INFINITY, 0.f), hi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
+    if (k < n) {
+        const int2 lp = n > 1 ? lpos[k] : make_int2(-1, -1);
+        const int4 id = leafid[k];
+        const int v[3] = {id.y, id.z, id.w};
 #pragma unroll
-    for (int q = 0; q < K; q++) {
-        v[q] = prims[K * pid + q];
-        p[3 * q] = x[3 * v[q]];
-        p[3 * q + 1] = x[3 * v[q] + 1];
-        p[3 * q + 2] = x[3 * v[q] + 2];
-        lo = fmin4(lo, pos_lo(x, v[q]));
-        hi = fmax4(hi, pos_hi(x, v[q]));
-    }
-    p[3 * K] = 0.0;
-    leaf_box[2 * k] = lo;
-    leaf_box[2 * k + 1] = hi;
-    if (n > 1) {
-        const int2 lp = lpos[k];
+        for (int j = 0; j < K; j++) {
+            lo = fmin4(lo, pos_lo(x, v[j]));
+            hi = fmax4(hi, pos_hi(x, v[j]));
+        }
+        leaf_box[2 * k] = lo;
+        leaf_box[2 * k + 1] = hi;
         if (lp.x >= 0) put_slot(rec, lp.x, lo, hi, (n - 1) + k, k);
         if (lp.y >= 0) put_slot(rec, lp.y, lo, hi, (n - 1) + k, k);
     }
-    constexpr int NP = leaf_stride<K>() - 1;
-    double2* o = leafd + (size_t)leaf_stride<K>() * k;
+    auto put = [&](int l) {
+        win[l][0][t] = lo.x;
+        win[l][1][t] = lo.y;
+        win[l][2][t] = lo.z;
+        win[l][3][t] = hi.x;
+        win[l][4][t] = hi.y;
+        win[l][5][t] = hi.z;
+    };
+    auto get_lo = [&](int l, int a) { return make_float4(win[l][0][a], win[l][1][a], win[l][2][a], 0.f); };
+    auto get_hi = [&](int l, int a) { return make_float4(win[l][3][a], win[l][4][a], win[l][5][a], 0.f); };
+    put(0);
 #pragma unroll
-    for (int j = 0; j < NP; j++) o[j] = make_double2(p[2 * j], p[2 * j + 1]);
-    *reinterpret_cast<int4*>(o + NP) = make_int4(pid, v[0], v[1], K == 3 ? v[K - 1] : -1);
+    for (int l = 1; l < RB_LEVELS; l++) {
+        __syncthreads();
+        const int a = t + (1 << (l - 1)); // a window past the block's end is cut there
+        if (a < RB) {
+            lo = fmin4(lo, get_lo(l - 1, a));
+            hi = fmax4(hi, get_hi(l - 1, a));
+        }
+        put(l);
+    }
+    if (t == 0) {
+        blk_box[2 * blockIdx.x] = lo;
+        blk_box[2 * blockIdx.x + 1] = hi;
+    }
+    __syncthreads();
+    if (p < 0 || rg.x < b0 || rg.y >= b0 + RB) return; // the others: k_cross_boxes
+    const int len = rg.y - rg.x + 1, l = 31 - __clz(len), a = rg.x - b0, b = a + len - (1 << l);
+    put_slot(rec, p, fmin4(get_lo(l, a), get_lo(l, b)), fmax4(get_hi(l, a), get_hi(l, b)), k, rg.y);
+}
+
+// Boxes of the internal nodes whose range crosses a block boundary of k_refit
+// (cross[1 .. cross[0]], listed by the build), one wave each: the leaves of the
+// first and the last block that it covers in part, and the boxes of the blocks
+// between them, all loads independent.
+__global__ void __launch_bounds__(BLK) k_cross_boxes(const int32_t* __restrict__ cross, const int2* __restrict__ range,
+                                                     const int32_t* __restrict__ ipos, const float4* __restrict__ leaf_box,
+                                                     const float4* __restrict__ blk_box, float4* __restrict__ rec) {
+    const int lane = threadIdx.x & 63, count = cross[0];
+    for (int w = blockIdx.x * (BLK / 64) + (threadIdx.x >> 6); w < count; w += gridDim.x * (BLK / 64)) {
+        const int i = cross[1 + w], p = ipos[i];
+        if (p < 0) continue; // the root or a child of it
+        const int2 rg = range[i];
+        const int A = rg.x / RB, B = rg.y / RB;
+        float4 lo = make_float4(INFINITY, INFINITY, INFINITY, 0.f), hi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
+        auto take = [&](const float4* arr, int u, int v) { // boxes [u, v): lane u + lane, .. + 64, ..., four in flight
+            for (int e = u + lane; e < v; e += 256) {
+                float4 l[4], h[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int c = e + 64 * q < v ? e + 64 * q : e; // a repeated box leaves the union unchanged
+                    l[q] = arr[2 * c];
+                    h[q] = arr[2 * c + 1];
+                }
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    lo = fmin4(lo, l[q]);
+                    hi = fmax4(hi, h[q]);
+                }
+            }
+        };
+        take(leaf_box, rg.x, (A + 1) * RB);
+        take(leaf_box, B * RB, rg.y + 1);
+        take(blk_box, A + 1, B);
+        lo = wave_min4(lo);
+        hi = wave_max4(hi);
+        if (lane == 0) put_slot(rec, p, lo, hi, i, rg.y);
+    }
 }
 
 // Block b's place in the query order.  Workgroups go round-robin to the 8
 // XCDs (block b to XCD b mod 8); the query order is dealt to them in chunks
-// of XCD_CHUNK consecutive blocks, chunk c to XCD c mod 8, so spatially close
-// queries (consecutive in Morton order) share one L2 for the records and
-// leaf data they visit, while the chunks of a dense region still spread over
-// all XCDs.  The grid is padded to a multiple of 8 XCD_CHUNK blocks
-// (query_grid), which makes the map a permutation of the blocks.
-constexpr int XCD_CHUNK = 16;
-__device__ inline int xcd_block(int b) {
+// of `chunk` consecutive blocks, chunk c to XCD c mod 8, so spatially close
+// queries (consecutive in Morton order) share one L2 for the records they
+// visit, while the chunks of a dense region still spread over all XCDs.  The
+// grid is padded to a multiple of 8 chunks (query_grid), which makes the map a
+// permutation of the blocks.
+__device__ inline int xcd_block(int b, int chunk) {
     const int j = b >> 3; // the j-th block this XCD receives
-    return ((j / XCD_CHUNK) * 8 + (b & 7)) * XCD_CHUNK + j % XCD_CHUNK;
+    return ((j / chunk) * 8 + (b & 7)) * chunk + j % chunk;
 }
-inline int query_grid(int n) {
-    constexpr int m = 8 * XCD_CHUNK;
-    return (grid_for(n, QBLK) + m - 1) / m * m;
+// Chunks of up to 2048 queries; fewer where the launch is small, so that every
+// XCD gets at least four.
+inline int query_chunk(int n, int per_block) { return std::max(1, std::min(2048 / per_block, grid_for(n, per_block) / 32)); }
+inline int query_grid(int n, int per_block) {
+    const int m = 8 * query_chunk(n, per_block);
+    return (grid_for(n, per_block) + m - 1) / m * m;
 }
-
-// out[c] = union of in[c*64 .. c*64+63] (clamped to n), one wave per chunk.
-__global__ void __launch_bounds__(BLK) k_chunk_union(const float4* __restrict__ in, int n, float4* __restrict__ out, int nchunks) {
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63;
-    if (wave >= nchunks) return;
-    const int e = wave * 64 + lane;
-    float4 lo = make_float4(INFINITY, INFINITY, INFINITY, 0.f), hi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
-    if (e < n) {
-        lo = in[2 * e];
-        hi = in[2 * e + 1];
-    }
-    lo = wave_min4(lo);
-    hi = wave_max4(hi);
-    if (lane == 0) {
-        out[2 * wave] = lo;
-        out[2 * wave + 1] = hi;
-    }
+// Queries per wave: a power of two from 4 to 64 that leaves COLLECT_WAVES waves
+// where there are enough queries.
+constexpr int COLLECT_WAVES = 4096;
+inline int collect_qw(int n) {
+    int qw = 4;
+    while (qw < 64 && n / (2 * qw) >= COLLECT_WAVES) qw *= 2;
+    return qw;
 }
 
-// Box of internal node i (the union of the leaf boxes of its range [a, b))
-// into its record slot.  Levels: leaves, then unions of 64 leaves, of 4096,
-// and (c256k non-null) of 262144; at each level the range's ends up to the
-// next level's boundaries, the whole chunks between them at the next level.
-__global__ void k_node_boxes(int n, const int2* __restrict__ range, const int32_t* __restrict__ ipos, const float4* __restrict__ leaf_box,
-                             const float4* __restrict__ c64, const float4* __restrict__ c4k, const float4* __restrict__ c256k,
-                             float4* __restrict__ rec) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n - 1) return;
-    const int p = ipos[i];
-    if (p < 0) return; // the root and its children sit in no slot
-    const int2 rg = range[i];
-    float4 lo = make_float4(INFINITY, INFINITY, INFINITY, 0.f), hi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
-    // union of arr's boxes [u, v), eight loads in flight (a clamped index
-    // repeats a box of the range, which leaves the union unchanged)
-    auto take = [&](const float4* arr, int u, int v) {
-        for (; u < v; u += 8) {
-            float4 l[8], h[8];
-#pragma unroll
-            for (int t = 0; t < 8; t++) {
-                const int k = min(u + t, v - 1);
-                l[t] = arr[2 * k];
-                h[t] = arr[2 * k + 1];
-            }
-#pragma unroll
-            for (int t = 0; t < 8; t++) {
-                lo = fmin4(lo, l[t]);
-                hi = fmax4(hi, h[t]);
-            }
-        }
-    };
-    const float4* lv[4] = {leaf_box, c64, c4k, c256k};
-    int a = rg.x, b = rg.y + 1;
-#pragma unroll
-    for (int L = 0; L < 3; L++) {
-        if (L == 2 && !c256k) break;
-        const int a2 = min((a + 63) & ~63, b), b2 = max(b & ~63, a2);
-        take(lv[L], a, a2);
-        take(lv[L], b2, b);
-        a = a2 >> 6;
-        b = b2 >> 6;
-    }
-    take(c256k ? c256k : c4k, a, b);
-    put_slot(rec, p, lo, hi, i, rg.y);
+// Slot in the staging list for every lane of the wave that reaches this call
+// together (one atomic per wave and call site; lanes that diverged away are
+// not counted).
+__device__ inline int stage_slot(uint32_t* __restrict__ counter) {
+    const unsigned long long m = __ballot(1);
+    const int lane = __lane_id();
+    const int leader = __ffsll(m) - 1;
+    uint32_t base = 0;
+    if (lane == leader) base = atomicAdd(counter, (uint32_t)__popcll(m));
+    base = __shfl(base, leader);
+    return (int)(base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull)));
+}
+
+template <int K>
+__global__ void k_leaf_ids(const int32_t* __restrict__ prims, const uint32_t* __restrict__ ids, int n, int4* __restrict__ leafid) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    const int pid = (int)ids[k];
+    leafid[k] = make_int4(pid, prims[K * pid], prims[K * pid + 1], K == 3 ? prims[K * pid + K - 1] : -1);
 }
 
 // Record slots (build only): empty slots get their constant, and every node
 // that sits in a slot gets the slot's position (ipos for internal nodes;
 // lpos.x for a leaf kept by its parent, lpos.y in its grandparent's record),
-// each written by exactly one thread.
-__global__ void k_record_slots(int n, const int32_t* __restrict__ child, float4* __restrict__ rec, int32_t* __restrict__ ipos,
-                               int32_t* __restrict__ lpos) {
+// each written by exactly one thread.  Nodes whose range crosses a block
+// boundary of k_refit are listed in cross (any order; cross[0] counts them).
+__global__ void k_record_slots(int n, const int32_t* __restrict__ child, const int2* __restrict__ range, float4* __restrict__ rec,
+                               int32_t* __restrict__ ipos, int32_t* __restrict__ lpos, int32_t* __restrict__ cross) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n - 1) return;
+    const int2 rg = range[i];
+    if (rg.x / RB != rg.y / RB) cross[1 + stage_slot(reinterpret_cast<uint32_t*>(cross))] = i;
     const int l = child[2 * i], r = child[2 * i + 1];
     const bool li = l < n - 1, ri = r < n - 1;
     const int sl[4] = {li ? child[2 * l] : l, li ? child[2 * l + 1] : -1, ri ? child[2 * r] : r, ri ? child[2 * r + 1] : -1};
@@ -424,19 +469,6 @@ __device__ inline void write_contact(const QueryOut& o, int idx, int type, int p
     o.bary[idx] = make_float4((float)f.bary[0], (float)f.bary[1], (float)f.bary[2], (float)f.bary[3]);
     o.nrm[idx] = make_float4((float)f.n.x, (float)f.n.y, (float)f.n.z, (float)f.h_cN);
     o.dist[idx] = dist;
-}
-
-// Slot in the staging list for every lane of the wave that reaches this call
-// together (one atomic per wave and call site; lanes that diverged away are
-// not counted).
-__device__ inline int stage_slot(uint32_t* __restrict__ counter) {
-    const unsigned long long m = __ballot(1);
-    const int lane = __lane_id();
-    const int leader = __ffsll(m) - 1;
-    uint32_t base = 0;
-    if (lane == leader) base = atomicAdd(counter, (uint32_t)__popcll(m));
-    base = __shfl(base, leader);
-    return (int)(base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull)));
 }
 
 // Wide-record traversal for one query box from internal node `start`: calls
@@ -501,286 +533,430 @@ __device__ inline void traverse(const float4* __restrict__ rec, int start, int l
     }
 }
 
-// Queries run in two passes.  Collect (MODE 0): the traversal alone, on a
-// short stack (SHORT_STACK entries); the sorted index of each leaf it reaches
-// goes to the query's slab (the first CAND hits, strided by the query count:
+// Queries run in two passes.
+//
+// Collect: a wave takes QW queries and one stack of (query, node) pairs in LDS.
+// A step pops up to 16 pairs, four lanes each: every lane tests one child slot
+// of its node against its query's box; children that pass go back on the stack
+// and leaves to the wave's hit buffer, both packed by ballots.  With one lane
+// per query and a stack each, a launch took as long as its longest chain of
+// dependent loads (40 visits of 0.9 us on a 16 x 16 cloth, 130 at the fold of a
+// 256 x 256 one), the lanes that were done idled, and a visit read its 128-byte
+// record in eight 16-byte pieces per lane.  Here a wave's lanes are busy until
+// its last query is done, four of them read a record together, and a query's
+// nodes are visited many at a time.  Few queries give few waves, so QW falls
+// with their number (collect_qw) until a wave has four.
+// Hits are filtered 64 at a time by their vertex ids (pairs that share a vertex
+// or are both static, most of the hits in a cloth at rest) before they go to
+// the query's slab (the first CAND, strided by the query count:
 // cand[h * nq + q]) or, past CAND, to a shared overflow list of (query, leaf)
-// pairs (capacity nq, filled in per-lane chunks); ccount[q] = hits.  Test
-// (MODE 1): lane (q, y) runs the exact FP64 predicate on slab rows y, y + R,
-// ... of query q (R = gridDim.y, test_rows: up to CAND rows for few queries,
-// one for millions), and lane (i, 0) also tests overflow entry i: no
-// traversal and few tests per lane, so a query with many close leaves no
-// longer holds its wave through a long serial chain.  Every reached
-// leaf is tested once, so the accepted set is that of the single pass
-// (MODE 2: traversal and test together, on a STACK-entry stack), which runs
-// instead when the short stack or the overflow list was too small (bits 0
-// and 1 of flags[1]).
-constexpr int CAND = 16;
-constexpr int SHORT_STACK = 32;
-// Slab rows spread over the test pass's grid: CAND (one test per lane) for up
-// to 2^18 queries, fewer as the query count grows, 1 from 2^22 queries on.
-inline int test_rows(int nq) { return std::max(1, std::min(CAND, (1 << 22) / std::max(nq, 1))); }
-
-// Point-triangle candidate: query vertex v (FP64 position p, segment q)
-// against the triangle at sorted leaf lf; an accepted pair goes to the
-// staging list and qcount[q] counts it.
-__device__ inline void pt_candidate(int q, int v, dv3 p, int lf, const double2* __restrict__ leafd, int n_dyn, double dhat,
-                                    uint32_t* __restrict__ qcount, const QueryOut& st, int2* __restrict__ st_seg,
-                                    uint32_t* __restrict__ counter) {
-    const double2* L = leafd + (size_t)leaf_stride<3>() * lf;
-    const double2 u0 = L[0], u1 = L[1], u2 = L[2], u3 = L[3], u4 = L[4];
-    const int4 m = *reinterpret_cast<const int4*>(L + 5);
-    const int f = m.x, a = m.y, b = m.z, c = m.w;
-    if (v == a || v == b || v == c || (v >= n_dyn && a >= n_dyn)) return;
-    const dv3 t0 = dmk(u0.x, u0.y, u1.x), t1 = dmk(u1.y, u2.x, u2.y), t2 = dmk(u3.x, u3.y, u4.x);
-    const PTOut r = point_triangle(p, t0, t1, t2);
-    if (!pt_accept(r, dhat)) return;
-    const uint32_t place = atomicAdd(&qcount[q], 1u);
-    const int idx = stage_slot(counter);
-    if (idx < st.cap) {
-        write_contact(st, idx, 0, v, f, make_int4(v, a, b, c), pt_fields(p, t0, t1, t2, r, dhat), r.dist);
-        st_seg[idx] = make_int2(q, (int)place);
-    }
-}
-
-// Hits of the collect pass: the first CAND in the query's slab, the rest in
-// the overflow list, where a lane reserves OVF_CHUNK entries at a time (one
-// atomic per chunk) and pads the unused end of its last chunk with query -1.
-// A reservation beyond the list's capacity sets bit 1 of flags[1].
-constexpr int OVF_CHUNK = 16;
-struct HitSink {
-    int hits = 0;
-    int chunk = -1; // start of the lane's current overflow chunk (-2: list full)
-    int fill = 0;   // entries used in it
-    __device__ inline void add(int q, int nq, int lf, int32_t* __restrict__ cand, int2* __restrict__ ovf, uint32_t* __restrict__ ovf_count,
-                               uint32_t* __restrict__ flags) {
-        if (hits < CAND) {
-            cand[(size_t)hits * nq + q] = lf;
-        } else if (chunk != -2) {
-            if (chunk < 0 || fill == OVF_CHUNK) {
-                const uint32_t b = atomicAdd(ovf_count, (uint32_t)OVF_CHUNK);
-                if (b + OVF_CHUNK > (uint32_t)nq) {
-                    atomicOr(&flags[1], 2u);
-                    chunk = -2;
-                } else {
-                    chunk = (int)b;
-                    fill = 0;
-                }
-            }
-            if (chunk >= 0) ovf[chunk + fill++] = make_int2(q, lf);
-        }
-        hits++;
-    }
-    __device__ inline void finish(int2* __restrict__ ovf) {
-        if (chunk >= 0)
-            for (int i = fill; i < OVF_CHUNK; i++) ovf[chunk + i] = make_int2(-1, -1);
-    }
+// pairs (capacity nq); ccount[q] counts them.
+//
+// Test: a block takes TQ queries and spreads their slab entries over its lanes;
+// each runs the exact FP64 predicate on its pair, and a lane of the launch also
+// tests one overflow entry.  Every kept hit is tested once, so the accepted set
+// is that of the single pass (k_single: one lane per query, traversal and test
+// together, on a STACK-entry stack), which runs instead when the shared stack
+// or the overflow list was too small (bits 0 and 1 of flags[1]).
+//
+// 256 x 256 cloth: EE collect 82 -> 44 us, test 42 -> 12, PT collect 46 -> 24,
+// test 13 -> 5; 16 x 16 cloth: collects 38 -> 9.4 and 28 -> 9.0 us; 160-scene
+// batch (1.5 million edges): EE collect 505 -> 530, test 340 -> 68, PT collect
+// 230 -> 267, test 390 -> 73.
+struct ListOut {
+    int32_t* cand;
+    uint32_t* ccount;
+    int2* ovf;
+    uint32_t* ovf_count;
+    uint32_t* flags;
 };
 
-// Point-triangle queries: one lane per surface vertex q.  Accepted pairs go
-// to the staging list (any order) with segment q, counted in qcount[q]
-// (zeroed beforehand).
-template <int MODE, int SK>
-__global__ void __launch_bounds__(QBLK) k_query_pt(const double* __restrict__ x, const int32_t* __restrict__ surf_verts, int nv,
-                                                   int n_dyn, int nf, const float4* __restrict__ rec,
-                                                   const double2* __restrict__ leafd, double dhat, float gap, uint32_t* __restrict__ qcount,
-                                                   QueryOut st, int2* __restrict__ st_seg, uint32_t* __restrict__ counter,
-                                                   uint32_t* __restrict__ flags, const int32_t* __restrict__ vseg,
-                                                   const int32_t* __restrict__ roots, int32_t* __restrict__ cand,
-                                                   uint32_t* __restrict__ ccount, int2* __restrict__ ovf, uint32_t* __restrict__ ovf_count) {
-    __shared__ int32_t stack[MODE == 1 ? 1 : SK][QBLK];
-    const int leaf0 = nf - 1;
-    if (MODE == 1) { // lane (q, blockIdx.y): slab rows blockIdx.y + i gridDim.y of query q; row 0 also overflow entry q
-        const int q = blockIdx.x * blockDim.x + threadIdx.x;
-        if (q >= nv || nf == 0) return;
-        const int nh = (int)min(ccount[q], (uint32_t)CAND);
-        if ((int)blockIdx.y < nh) {
-            const int v = surf_verts[q];
-            const dv3 p = ldd(x, v);
-            for (int h = blockIdx.y; h < nh; h += gridDim.y)
-                pt_candidate(q, v, p, cand[(size_t)h * nv + q], leafd, n_dyn, dhat, qcount, st, st_seg, counter);
-        }
-        if (blockIdx.y == 0 && !(flags[1] & 2u) && (uint32_t)q < min(*ovf_count, (uint32_t)nv)) { // a full list reruns as a single pass
-            const int2 o = ovf[q];
-            if (o.x >= 0) {
-                const int v = surf_verts[o.x];
-                pt_candidate(o.x, v, ldd(x, v), o.y, leafd, n_dyn, dhat, qcount, st, st_seg, counter);
-            }
-        }
-        return;
-    }
-    const int q = xcd_block(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (q >= nv) return;
-    if (nf == 0) {
-        if (MODE == 0) ccount[q] = 0;
-        return;
-    }
-    const int v = surf_verts[q];
-    const dv3 p = ldd(x, v);
-    HitSink sink;
-    auto leaf = [&](int node) {
-        if (MODE == 0) sink.add(q, nv, node - leaf0, cand, ovf, ovf_count, flags);
-        else pt_candidate(q, v, p, node - leaf0, leafd, n_dyn, dhat, qcount, st, st_seg, counter);
+// The two kinds of query.  Point-triangle: query q is surface vertex q.
+// Edge-edge: query k is the edge at sorted leaf k, which reaches only leaves
+// after k, so each unordered pair is tested once; a pair (i, j), i < j, is
+// evaluated with edge i first, as the canonical definition does.
+struct PTQuery {
+    const double* x;
+    const int32_t* surf_verts;
+    const int4* leafid; // of the triangle tree
+    const int32_t* vseg;
+    const int32_t* roots;
+    int nq, nleaf, n_dyn;
+    struct Q {
+        int v;
+        dv3 p;
     };
+    __device__ inline Q query(int q) const {
+        const int v = surf_verts[q];
+        return Q{v, ldd(x, v)};
+    }
     // start node: the root, or in segmented mode the vertex's segment subtree
-    const int start = roots ? roots[vseg[v]] : 0;
-    if (start < 0) {
-        // no triangle in this segment
-    } else if (start >= leaf0) {
-        leaf(start);
-    } else {
-        traverse<SK>(rec, start, leaf0, pos_lo(x, v), pos_hi(x, v), gap, -1, stack, flags, leaf);
+    __device__ inline int start(const Q& Q) const { return nleaf == 0 ? -1 : roots ? roots[vseg[Q.v]] : 0; }
+    __device__ inline void box(const Q& Q, float4* lo, float4* hi) const {
+        *lo = pos_lo(x, Q.v);
+        *hi = pos_hi(x, Q.v);
     }
-    if (MODE == 0) {
-        sink.finish(ovf);
-        ccount[q] = (uint32_t)sink.hits;
+    __device__ inline int after(int) const { return -1; }
+    __device__ inline int2 verts(const Q& Q) const { return make_int2(Q.v, -1); }
+    __device__ inline bool keep(int2 v, int lf) const {
+        const int4 m = leafid[lf];
+        return !(v.x == m.y || v.x == m.z || v.x == m.w || (v.x >= n_dyn && m.y >= n_dyn));
     }
-}
-
-// Edge-edge candidate: query edge e (vertices a0, a1, FP64 endpoints A0, A1)
-// against the edge at sorted leaf lf.  A pair (i, j), i < j, is evaluated
-// with edge i first, as the canonical definition does, and belongs to segment
-// i: it goes to the staging list with segment seg0 + i and qcount[i] counts it.
-__device__ inline void ee_candidate(int e, int a0, int a1, dv3 A0, dv3 A1, int lf, const double2* __restrict__ leafd, int n_dyn,
-                                    double dhat, uint32_t* __restrict__ qcount, int seg0, const QueryOut& st,
-                                    int2* __restrict__ st_seg, uint32_t* __restrict__ counter) {
-    const double2* L = leafd + (size_t)leaf_stride<2>() * lf;
-    const double2 u0 = L[0], u1 = L[1], u2 = L[2];
-    const int4 m = *reinterpret_cast<const int4*>(L + 3);
-    const int f = m.x, b0 = m.y, b1 = m.z;
-    if (a0 == b0 || a0 == b1 || a1 == b0 || a1 == b1 || (a0 >= n_dyn && b0 >= n_dyn)) return;
-    const dv3 B0 = dmk(u0.x, u0.y, u1.x), B1 = dmk(u1.y, u2.x, u2.y);
-    const bool first = e < f;
-    const int i = first ? e : f, j = first ? f : e;
-    const int i0 = first ? a0 : b0, i1 = first ? a1 : b1, j0 = first ? b0 : a0, j1 = first ? b1 : a1;
-    const dv3 P0 = first ? A0 : B0, P1 = first ? A1 : B1, Q0 = first ? B0 : A0, Q1 = first ? B1 : A1;
-    const EEOut r = segment_segment(P0, P1, Q0, Q1);
-    if (!ee_accept(r, dhat)) return;
-    const uint32_t place = atomicAdd(&qcount[i], 1u);
-    const int idx = stage_slot(counter);
-    if (idx < st.cap) {
-        write_contact(st, idx, 1, i, j, make_int4(i0, i1, j0, j1), ee_fields(P0, P1, Q0, Q1, r, dhat), r.dist);
-        st_seg[idx] = make_int2(seg0 + i, (int)place);
+    __device__ inline bool accept(const Q& Q, int lf, double dhat) const {
+        const int4 m = leafid[lf];
+        return pt_accept(point_triangle(Q.p, ldd(x, m.y), ldd(x, m.z), ldd(x, m.w)), dhat);
     }
-}
-
-// The query edge at sorted leaf k: id, vertices and FP64 endpoints.
-struct EEQuery {
-    int e, a0, a1;
-    dv3 A0, A1;
+    __device__ inline int2 segment(int q, const Q&, int lf) const { return make_int2(q, leafid[lf].x); } // (segment, partner)
+    __device__ inline int4 write(const Q& Q, int lf, double dhat, const QueryOut& o, int idx) const {
+        const int4 m = leafid[lf], vv = make_int4(Q.v, m.y, m.z, m.w);
+        const dv3 t0 = ldd(x, m.y), t1 = ldd(x, m.z), t2 = ldd(x, m.w);
+        const PTOut r = point_triangle(Q.p, t0, t1, t2);
+        write_contact(o, idx, 0, Q.v, m.x, vv, pt_fields(Q.p, t0, t1, t2, r, dhat), r.dist);
+        return vv;
+    }
 };
-__device__ inline EEQuery ee_query(const double2* __restrict__ leafd, int k) {
-    const double2* Lk = leafd + (size_t)leaf_stride<2>() * k;
-    const double2 w0 = Lk[0], w1 = Lk[1], w2 = Lk[2];
-    const int4 mk = *reinterpret_cast<const int4*>(Lk + 3);
-    return EEQuery{mk.x, mk.y, mk.z, dmk(w0.x, w0.y, w1.x), dmk(w1.y, w2.x, w2.y)};
-}
 
-// Edge-edge queries: lane k takes the edge at sorted leaf k and reaches only
-// leaves after k, so each unordered pair is tested once (qcount zeroed
-// beforehand).
-template <int MODE, int SK>
-__global__ void __launch_bounds__(QBLK) k_query_ee(int ne, int n_dyn, const float4* __restrict__ rec,
-                                                   const double2* __restrict__ leafd, double dhat,
-                                                   float gap, uint32_t* __restrict__ qcount, int seg0, QueryOut st,
-                                                   int2* __restrict__ st_seg, uint32_t* __restrict__ counter,
-                                                   uint32_t* __restrict__ flags, const int32_t* __restrict__ vseg,
-                                                   const int32_t* __restrict__ roots, int32_t* __restrict__ cand,
-                                                   uint32_t* __restrict__ ccount, int2* __restrict__ ovf, uint32_t* __restrict__ ovf_count) {
-    __shared__ int32_t stack[MODE == 1 ? 1 : SK][QBLK];
-    if (ne < 2) return;
-    const int leaf0 = ne - 1;
-    if (MODE == 1) { // lane (k, blockIdx.y): slab rows blockIdx.y + i gridDim.y of query k; row 0 also overflow entry k
-        const int k = blockIdx.x * blockDim.x + threadIdx.x;
-        if (k >= ne) return;
-        const int nh = (int)min(ccount[k], (uint32_t)CAND);
-        if ((int)blockIdx.y < nh) {
-            const EEQuery Q = ee_query(leafd, k);
-            for (int h = blockIdx.y; h < nh; h += gridDim.y)
-                ee_candidate(Q.e, Q.a0, Q.a1, Q.A0, Q.A1, cand[(size_t)h * ne + k], leafd, n_dyn, dhat, qcount, seg0, st, st_seg, counter);
-        }
-        if (blockIdx.y == 0 && !(flags[1] & 2u) && (uint32_t)k < min(*ovf_count, (uint32_t)ne)) { // a full list reruns as a single pass
-            const int2 o = ovf[k];
-            if (o.x >= 0) {
-                const EEQuery Q = ee_query(leafd, o.x);
-                ee_candidate(Q.e, Q.a0, Q.a1, Q.A0, Q.A1, o.y, leafd, n_dyn, dhat, qcount, seg0, st, st_seg, counter);
+struct EEQuery {
+    const double* x;
+    const int4* leafid; // of the edge tree
+    const int32_t* vseg;
+    const int32_t* roots;
+    int nq, nleaf, n_dyn, seg0; // segments seg0 + edge id
+    struct Q {
+        int e, a0, a1;
+        dv3 A0, A1;
+    };
+    __device__ inline Q query(int k) const {
+        const int4 m = leafid[k];
+        return Q{m.x, m.y, m.z, ldd(x, m.y), ldd(x, m.z)};
+    }
+    // a lone edge, of the tree or of its segment, has no partner (start is a leaf then)
+    __device__ inline int start(const Q& Q) const {
+        const int s = nleaf < 2 ? -1 : roots ? roots[vseg[Q.a0]] : 0;
+        return s >= nleaf - 1 ? -1 : s;
+    }
+    __device__ inline void box(const Q& Q, float4* lo, float4* hi) const {
+        *lo = make_float4(__double2float_rd(fmin(Q.A0.x, Q.A1.x)), __double2float_rd(fmin(Q.A0.y, Q.A1.y)),
+                          __double2float_rd(fmin(Q.A0.z, Q.A1.z)), 0.f);
+        *hi = make_float4(__double2float_ru(fmax(Q.A0.x, Q.A1.x)), __double2float_ru(fmax(Q.A0.y, Q.A1.y)),
+                          __double2float_ru(fmax(Q.A0.z, Q.A1.z)), 0.f);
+    }
+    __device__ inline int after(int k) const { return k; }
+    __device__ inline int2 verts(const Q& Q) const { return make_int2(Q.a0, Q.a1); }
+    __device__ inline bool keep(int2 v, int lf) const {
+        const int4 m = leafid[lf];
+        return !(v.x == m.y || v.x == m.z || v.y == m.y || v.y == m.z || (v.x >= n_dyn && m.y >= n_dyn));
+    }
+    // the pair's edges in canonical order: i < j
+    struct Pair {
+        int i, j;
+        int4 v;
+        dv3 P0, P1, Q0, Q1;
+    };
+    __device__ inline Pair pair(const Q& Q, int lf) const {
+        const int4 m = leafid[lf];
+        const dv3 B0 = ldd(x, m.y), B1 = ldd(x, m.z);
+        return Q.e < m.x ? Pair{Q.e, m.x, make_int4(Q.a0, Q.a1, m.y, m.z), Q.A0, Q.A1, B0, B1}
+                         : Pair{m.x, Q.e, make_int4(m.y, m.z, Q.a0, Q.a1), B0, B1, Q.A0, Q.A1};
+    }
+    __device__ inline bool accept(const Q& Q, int lf, double dhat) const {
+        const Pair p = pair(Q, lf);
+        return ee_accept(segment_segment(p.P0, p.P1, p.Q0, p.Q1), dhat);
+    }
+    __device__ inline int2 segment(int, const Q& Q, int lf) const { // (segment, partner)
+        const int f = leafid[lf].x;
+        return make_int2(seg0 + min(Q.e, f), max(Q.e, f));
+    }
+    __device__ inline int4 write(const Q& Q, int lf, double dhat, const QueryOut& o, int idx) const {
+        const Pair p = pair(Q, lf);
+        const EEOut r = segment_segment(p.P0, p.P1, p.Q0, p.Q1);
+        write_contact(o, idx, 1, p.i, p.j, p.v, ee_fields(p.P0, p.P1, p.Q0, p.Q1, r, dhat), r.dist);
+        return p.v;
+    }
+};
+
+// Compiler barrier between LDS accesses of lanes of one wave (the hardware
+// keeps a wave's LDS accesses in order).
+__device__ inline void wave_lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
+template <class QK, int QW>
+__global__ void __launch_bounds__(CBLK) k_collect(QK K, const float4* __restrict__ rec, float gap, int chunk, ListOut out) {
+    constexpr int W = CBLK / 64;
+    __shared__ uint32_t stack_[W][CSTACK]; // (query of the wave << COLLECT_BITS) | node
+    __shared__ uint32_t hit_[W][128];      // (query << COLLECT_BITS) | sorted leaf
+    __shared__ float4 blo_[W][QW], bhi_[W][QW]; // query boxes grown by gap; w: the query's vertex ids
+    __shared__ int cnt_[W][QW];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint32_t* const stack = stack_[wave];
+    uint32_t* const hit = hit_[wave];
+    float4 *const blo = blo_[wave], *const bhi = bhi_[wave];
+    int* const cnt = cnt_[wave];
+    const int q0 = (xcd_block(blockIdx.x, chunk) * W + wave) * QW;
+    const int leaf0 = K.nleaf - 1;
+    auto rank = [&](unsigned long long m) { return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u)); };
+    int sp = 0, nh = 0; // entries of stack and hit, the same in all lanes
+    {
+        int start = -1;
+        if (lane < QW) {
+            cnt[lane] = 0;
+            if (q0 + lane < K.nq) {
+                const auto Q = K.query(q0 + lane);
+                start = K.start(Q);
+                float4 lo, hi;
+                K.box(Q, &lo, &hi);
+                const int2 v = K.verts(Q);
+                blo[lane] = make_float4(__double2float_rd((double)lo.x - gap), __double2float_rd((double)lo.y - gap), __double2float_rd((double)lo.z - gap),
+                                         __int_as_float(v.x));
+                bhi[lane] = make_float4(__double2float_ru((double)hi.x + gap), __double2float_ru((double)hi.y + gap), __double2float_ru((double)hi.z + gap),
+                                         __int_as_float(v.y));
             }
         }
+        const bool node = start >= 0 && start < leaf0, leaf = start >= 0 && start >= leaf0; // a leaf: a one-leaf tree or segment
+        const unsigned long long mn = __ballot(node), ml = __ballot(leaf);
+        if (node) stack[rank(mn)] = (uint32_t)lane << COLLECT_BITS | (uint32_t)start;
+        if (leaf) hit[rank(ml)] = (uint32_t)lane << COLLECT_BITS | (uint32_t)(start - leaf0);
+        sp = __popcll(mn);
+        nh = __popcll(ml);
+    }
+    wave_lds_order();
+    // filters the last (up to) 64 buffered hits
+    auto flush = [&]() {
+        const int k = min(nh, 64);
+        bool over = false;
+        int q = 0, lf = 0;
+        if (lane < k) {
+            const uint32_t e = hit[nh - k + lane];
+            const int ql = (int)(e >> COLLECT_BITS);
+            q = q0 + ql;
+            lf = (int)(e & COLLECT_MASK);
+            if (K.keep(make_int2(__float_as_int(blo[ql].w), __float_as_int(bhi[ql].w)), lf)) {
+                const int pos = atomicAdd(&cnt[ql], 1);
+                if (pos < CAND) out.cand[(size_t)pos * K.nq + q] = lf;
+                else over = true;
+            }
+        }
+        const unsigned long long mo = __ballot(over);
+        if (mo) {
+            const int leader = __ffsll(mo) - 1, need = __popcll(mo);
+            uint32_t b = 0;
+            if (lane == leader) b = atomicAdd(out.ovf_count, (uint32_t)need);
+            b = __shfl(b, leader, 64);
+            if (b + need > (uint32_t)K.nq) {
+                if (lane == leader) atomicOr(&out.flags[1], 2u);
+            } else if (over) {
+                out.ovf[b + rank(mo)] = make_int2(q, lf);
+            }
+        }
+        nh -= k;
+        wave_lds_order();
+    };
+    while (sp > 0) {
+        // a nearly full stack is worked off one node at a time, depth first,
+        // which adds at most three entries per tree level
+        const int take = sp > CSTACK_HIGH ? 1 : min(16, sp), slot = lane >> 2;
+        const bool on = slot < take;
+        const uint32_t e = on ? stack[sp - 1 - slot] : 0u;
+        const int ql = (int)(e >> COLLECT_BITS);
+        float4 lo = make_float4(0.f, 0.f, 0.f, 0.f), hi = lo;
+        if (on) {
+            const float4* r = rec + 8 * (size_t)(e & COLLECT_MASK) + 2 * (lane & 3);
+            lo = r[0];
+            hi = r[1];
+        }
+        const float4 ql4 = blo[ql], qh4 = bhi[ql];
+        sp -= take;
+        const int id = __float_as_int(lo.w);
+        // an unused slot has id -1 and last leaf -1
+        const bool in = on && __float_as_int(hi.w) > K.after(q0 + ql) && !(lo.x > qh4.x || lo.y > qh4.y || lo.z > qh4.z || ql4.x > hi.x ||
+                                                                         ql4.y > hi.y || ql4.z > hi.z);
+        const bool leaf = id >= leaf0;
+        const unsigned long long mn = __ballot(in && !leaf), ml = __ballot(in && leaf);
+        wave_lds_order();
+        const uint32_t tag = (uint32_t)ql << COLLECT_BITS;
+        if (in && !leaf) {
+            const int at = sp + rank(mn);
+            if (at < CSTACK) stack[at] = tag | (uint32_t)id;
+        }
+        if (in && leaf) hit[nh + rank(ml)] = tag | (uint32_t)(id - leaf0);
+        sp += __popcll(mn);
+        nh += __popcll(ml);
+        if (sp > CSTACK) {
+            if (lane == 0) atomicOr(&out.flags[1], 1u);
+            sp = CSTACK;
+        }
+        wave_lds_order();
+        if (nh >= 64) flush(); // at most 63 stay, and a step adds at most 64
+    }
+    while (nh > 0) flush();
+    if (lane < QW && q0 + lane < K.nq) out.ccount[q0 + lane] = (uint32_t)cnt[lane];
+}
+
+// Exclusive prefix sums of the slab entries of queries q0 .. q0 + TQ into pre
+// (TQ + 1 values); returns their number.
+__device__ inline int slab_prefix(const uint32_t* __restrict__ ccount, int q0, int nq, int* pre) {
+    const int t = threadIdx.x;
+    if (t < TQ) { // one wave
+        int s = q0 + t < nq ? (int)min(ccount[q0 + t], (uint32_t)CAND) : 0;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int y = __shfl_up(s, d, 64);
+            if (t >= d) s += y;
+        }
+        pre[t + 1] = s;
+        if (t == 0) pre[0] = 0;
+    }
+    __syncthreads();
+    return pre[TQ];
+}
+// The query (0 .. TQ - 1) whose entries hold entry i.
+__device__ inline int slab_query(const int* pre, int i) {
+    int lo = 0;
+#pragma unroll
+    for (int s = TQ / 2; s > 0; s >>= 1)
+        if (pre[lo + s] <= i) lo += s;
+    return lo;
+}
+__device__ inline int ovf_entries(const ListOut& l, int nq) { // none if the list was too small (the detection reruns)
+    return l.flags[1] & 2u ? 0 : (int)min(*l.ovf_count, (uint32_t)nq);
+}
+
+// Accepted entries keep a mark in the leaf index's sign bit, and their segment
+// counts them; nothing is appended to a common list: one counter that every
+// wave with a contact adds to took 10 to 20 ns a wave, 330 us of a 160-scene
+// batch's two test launches.
+constexpr int ACCEPTED = (int)0x80000000;
+
+template <class QK>
+__global__ void __launch_bounds__(TBLK) k_test(QK K, ListOut l, double dhat, uint32_t* __restrict__ qcount) {
+    __shared__ int pre[TQ + 1];
+    const int q0 = blockIdx.x * TQ, total = slab_prefix(l.ccount, q0, K.nq, pre);
+    auto test = [&](int q, int32_t* entry) {
+        const auto Q = K.query(q);
+        const int lf = *entry;
+        if (!K.accept(Q, lf, dhat)) return;
+        *entry = lf | ACCEPTED;
+        atomicAdd(&qcount[K.segment(q, Q, lf).x], 1u);
+    };
+    for (int i = threadIdx.x; i < total; i += TBLK) {
+        const int s = slab_query(pre, i);
+        test(q0 + s, &l.cand[(size_t)(i - pre[s]) * K.nq + q0 + s]);
+    }
+    const int i = blockIdx.x * TBLK + threadIdx.x; // the launch has at least nq lanes
+    if (i < ovf_entries(l, K.nq)) test(l.ovf[i].x, &l.ovf[i].y);
+}
+
+// Canonical order of the accepted pairs: segment by segment (PT by vertex, EE
+// by the smaller edge id), sorted by partner id inside a segment.  PASS 0 puts
+// the partner ids into their segments (any order inside one).  PASS 1: every
+// pair counts the smaller ids of its segment (a pair occurs once, so they are
+// distinct), evaluates its contact and writes it to its final place.  The
+// counts are independent loads over one lane per contact; an insertion sort by
+// one lane per segment moved each 68-byte record several times in a dependent
+// chain (13-30 us per detection for segments of 10 to 30).
+struct PlaceArgs {
+    const uint32_t* qoffset;
+    const uint32_t* qcount;
+    uint32_t* qfill;
+    int32_t* seg_key;
+    double dhat;
+    QueryOut o;
+    VertexCount vc;
+};
+
+template <int PASS, class QK>
+__device__ inline void place_pair(const QK& K, int q, int lf, const PlaceArgs& a) {
+    const auto Q = K.query(q);
+    const int2 sp = K.segment(q, Q, lf);
+    const int begin = (int)a.qoffset[sp.x];
+    if (PASS == 0) {
+        a.seg_key[begin + (int)atomicAdd(&a.qfill[sp.x], 1u)] = sp.y;
         return;
     }
-    const int k = xcd_block(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (k >= ne) return;
-    // the query edge is leaf k itself
-    const EEQuery Q = ee_query(leafd, k);
-    HitSink sink;
-    auto leaf = [&](int node) {
-        if (MODE == 0) sink.add(k, ne, node - leaf0, cand, ovf, ovf_count, flags);
-        else ee_candidate(Q.e, Q.a0, Q.a1, Q.A0, Q.A1, node - leaf0, leafd, n_dyn, dhat, qcount, seg0, st, st_seg, counter);
-    };
-    // start node: the root, or in segmented mode the edge's segment subtree
-    // (a segment with one edge has no pair)
-    const int start = roots ? roots[vseg[Q.a0]] : 0;
-    if (start >= 0 && start < leaf0) {
-        const float4 qlo = make_float4(__double2float_rd(fmin(Q.A0.x, Q.A1.x)), __double2float_rd(fmin(Q.A0.y, Q.A1.y)),
-                                       __double2float_rd(fmin(Q.A0.z, Q.A1.z)), 0.f);
-        const float4 qhi = make_float4(__double2float_ru(fmax(Q.A0.x, Q.A1.x)), __double2float_ru(fmax(Q.A0.y, Q.A1.y)),
-                                       __double2float_ru(fmax(Q.A0.z, Q.A1.z)), 0.f);
-        traverse<SK>(rec, start, leaf0, qlo, qhi, gap, k, stack, flags, leaf);
-    }
-    if (MODE == 0) {
-        sink.finish(ovf);
-        ccount[k] = (uint32_t)sink.hits;
-    }
-}
-
-// Canonical order of the staged contacts: segment by segment, sorted by
-// partner id inside a segment.  The partner ids go to their segments first
-// (in the order the test pass met them), then every staged contact counts the
-// smaller ids of its segment (a pair occurs once, so ids are distinct) and
-// moves straight to its final place.  The counts are independent loads over
-// one lane per contact; an insertion sort by one lane per segment moved each
-// 68-byte record several times in a dependent chain (13-30 us per detection
-// for segments of 10 to 30).
-__global__ void k_segment_keys(int n, const int2* __restrict__ st_seg, const int32_t* __restrict__ prim1,
-                               const uint32_t* __restrict__ qoffset, int32_t* __restrict__ seg_key) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= n) return;
-    const int2 sg = st_seg[c];
-    seg_key[qoffset[sg.x] + sg.y] = prim1[c];
-}
-
-__global__ void k_place_contacts(int n, const int2* __restrict__ st_seg, QueryOut st, const uint32_t* __restrict__ qoffset,
-                                 const uint32_t* __restrict__ qcount, const int32_t* __restrict__ seg_key, QueryOut o, VertexCount vc) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= n) return;
-    const int sg = st_seg[c].x;
-    const int begin = (int)qoffset[sg], cnt = (int)qcount[sg];
-    const int key = st.prim1[c];
-    const int4 v = st.v[c];
+    const int cnt = (int)a.qcount[sp.x];
     int rank = 0;
-    for (int q = 0; q < cnt; q += 8) {
+    for (int e = 0; e < cnt; e += 8) {
         int k[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) k[u] = seg_key[begin + min(q + u, cnt - 1)];
+        for (int u = 0; u < 8; u++) k[u] = a.seg_key[begin + min(e + u, cnt - 1)];
 #pragma unroll
-        for (int u = 0; u < 8; u++) rank += q + u < cnt && k[u] < key ? 1 : 0;
+        for (int u = 0; u < 8; u++) rank += e + u < cnt && k[u] < sp.y ? 1 : 0;
     }
     const int idx = begin + rank;
-    o.type[idx] = st.type[c];
-    o.prim0[idx] = st.prim0[c];
-    o.prim1[idx] = key;
-    o.v[idx] = v;
-    o.bary[idx] = st.bary[c];
-    o.nrm[idx] = st.nrm[c];
-    o.dist[idx] = st.dist[c];
-    if (vc.cnt) {
-        int4 l;
-        l.x = (int)atomicAdd(&vc.cnt[v.x], 1u);
-        l.y = (int)atomicAdd(&vc.cnt[v.y], 1u);
-        l.z = (int)atomicAdd(&vc.cnt[v.z], 1u);
-        l.w = (int)atomicAdd(&vc.cnt[v.w], 1u);
-        vc.loc[idx] = l;
+    const int4 v = K.write(Q, lf, a.dhat, a.o, idx);
+    if (a.vc.cnt) {
+        int4 c;
+        c.x = (int)atomicAdd(&a.vc.cnt[v.x], 1u);
+        c.y = (int)atomicAdd(&a.vc.cnt[v.y], 1u);
+        c.z = (int)atomicAdd(&a.vc.cnt[v.z], 1u);
+        c.w = (int)atomicAdd(&a.vc.cnt[v.w], 1u);
+        a.vc.loc[idx] = c;
     }
+}
+
+// The accepted slab entries of TQ queries, gathered in LDS so that full waves
+// work on them, and the overflow entries.
+template <int PASS, class QK>
+__device__ inline void place_block(const QK& K, const ListOut& l, int block, const PlaceArgs& a, int* pre, uint16_t* list, int* count) {
+    const int t = threadIdx.x, q0 = block * TQ;
+    if (t == 0) *count = 0;
+    const int total = slab_prefix(l.ccount, q0, K.nq, pre); // its barrier also covers count
+    for (int i = t; i < total; i += TBLK) {
+        const int s = slab_query(pre, i), h = i - pre[s];
+        if (l.cand[(size_t)h * K.nq + q0 + s] & ACCEPTED) list[atomicAdd(count, 1)] = (uint16_t)(s * CAND + h);
+    }
+    __syncthreads();
+    for (int j = t; j < *count; j += TBLK) {
+        const int q = q0 + list[j] / CAND;
+        place_pair<PASS>(K, q, l.cand[(size_t)(list[j] % CAND) * K.nq + q] & ~ACCEPTED, a);
+    }
+    const int i = block * TBLK + t;
+    if (i < ovf_entries(l, K.nq) && (l.ovf[i].y & ACCEPTED)) place_pair<PASS>(K, l.ovf[i].x, l.ovf[i].y & ~ACCEPTED, a);
+}
+
+template <int PASS>
+__global__ void __launch_bounds__(TBLK) k_place(PTQuery PT, ListOut pl, int pt_blocks, EEQuery EE, ListOut el, PlaceArgs a) {
+    __shared__ int pre[TQ + 1];
+    __shared__ uint16_t list[TQ * CAND];
+    __shared__ int count;
+    if ((int)blockIdx.x < pt_blocks) place_block<PASS>(PT, pl, blockIdx.x, a, pre, list, &count);
+    else place_block<PASS>(EE, el, (int)blockIdx.x - pt_blocks, a, pre, list, &count);
+}
+
+// The single pass: accepted pairs to a list of (query, leaf) of capacity cap, EE
+// queries with the sign bit set; k_place_single then places them.
+template <class QK>
+__global__ void __launch_bounds__(QBLK) k_single(QK K, int mark, const float4* __restrict__ rec, float gap, double dhat,
+                                                 uint32_t* __restrict__ qcount, int2* __restrict__ pairs, int cap,
+                                                 uint32_t* __restrict__ counter, uint32_t* __restrict__ flags) {
+    __shared__ int32_t stack[STACK][QBLK];
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= K.nq) return;
+    const int leaf0 = K.nleaf - 1;
+    const typename QK::Q Q = K.query(q);
+    const int start = K.start(Q);
+    if (start < 0) return;
+    auto leaf = [&](int node) {
+        const int lf = node - leaf0;
+        if (!K.keep(K.verts(Q), lf) || !K.accept(Q, lf, dhat)) return;
+        atomicAdd(&qcount[K.segment(q, Q, lf).x], 1u);
+        const int idx = stage_slot(counter);
+        if (idx < cap) pairs[idx] = make_int2(q | mark, lf);
+    };
+    if (start >= leaf0) {
+        leaf(start);
+    } else {
+        float4 lo, hi;
+        K.box(Q, &lo, &hi);
+        traverse<STACK>(rec, start, leaf0, lo, hi, gap, K.after(q), stack, flags, leaf);
+    }
+}
+
+template <int PASS>
+__global__ void __launch_bounds__(TBLK) k_place_single(PTQuery PT, EEQuery EE, const int2* __restrict__ pairs, int n, PlaceArgs a) {
+    const int i = blockIdx.x * TBLK + threadIdx.x;
+    if (i >= n) return;
+    const int2 e = pairs[i];
+    if (e.x & ACCEPTED) place_pair<PASS>(EE, e.x & ~ACCEPTED, e.y, a);
+    else place_pair<PASS>(PT, e.x, e.y, a);
 }
 
 } // namespace
@@ -807,13 +983,12 @@ Detector::Detector(int n_all_, int n_dyn_, int nv_, const int32_t* sv, int nf_, 
     edges.alloc(2 * (size_t)ne);
     edges.upload(e, 2 * (size_t)ne, stream);
     edges_h.assign(e, e + 2 * (size_t)ne);
-    auto init_tree = [&](Tree& T, int n, int stride) {
+    auto init_tree = [&](Tree& T, int n) {
         T.n = n;
-        T.leaf_stride = stride;
         if (n == 0) return;
         T.prim_box.alloc(2 * (size_t)n);
         T.leaf_box.alloc(2 * (size_t)n);
-        T.leafd.alloc((size_t)T.leaf_stride * n);
+        T.leafid.alloc(n);
         T.ipos.alloc(std::max(n - 1, 1));
         T.lpos.alloc(2 * (size_t)n);
         T.keys.alloc(n);
@@ -821,14 +996,13 @@ Detector::Detector(int n_all_, int n_dyn_, int nv_, const int32_t* sv, int nf_, 
         T.child.alloc(2 * (size_t)std::max(n - 1, 1));
         T.range.alloc(std::max(n - 1, 1));
         T.rec.alloc(8 * (size_t)std::max(n - 1, 1));
-        T.chunk64.alloc(2 * (size_t)((n + 63) / 64));
-        T.chunk4k.alloc(2 * (size_t)((n + 4095) / 4096));
-        T.chunk256k.alloc(2 * (size_t)((n + 262143) / 262144));
+        T.blk_box.alloc(2 * (size_t)grid_for(n, RB));
+        T.cross.alloc((size_t)n + 1);
         T.scene.alloc(2);
         T.partial.alloc(2 * 256);
     };
-    init_tree(ft, nf, leaf_stride<3>());
-    init_tree(et, ne, leaf_stride<2>());
+    init_tree(ft, nf);
+    init_tree(et, ne);
     c.cap = cap;
     c.type.alloc(cap);
     c.prim0.alloc(cap);
@@ -837,21 +1011,14 @@ Detector::Detector(int n_all_, int n_dyn_, int nv_, const int32_t* sv, int nf_, 
     c.bary.alloc(cap);
     c.nrm.alloc(cap);
     c.dist.alloc(cap);
-    counts.alloc((size_t)nv + ne + 8);
+    const size_t segs = ((size_t)nv + ne + 3) & ~(size_t)3;
+    counts.alloc(8 + 2 * segs);
     total = counts.p;
     ovf_count = counts.p + 3;
     qcount = counts.p + 8; // 16-byte aligned for the scan
+    qfill = qcount + segs;
     qoffset.alloc((size_t)nv + ne + 1);
     PA_HIP(hipHostMalloc((void**)&total_host, 3 * sizeof(uint32_t), hipHostMallocDefault));
-    stg.cap = cap;
-    stg.type.alloc(cap);
-    stg.prim0.alloc(cap);
-    stg.prim1.alloc(cap);
-    stg.v.alloc(cap);
-    stg.bary.alloc(cap);
-    stg.nrm.alloc(cap);
-    stg.dist.alloc(cap);
-    st_seg.alloc(cap);
     seg_key.alloc(cap);
     cand_pt.alloc((size_t)CAND * std::max(nv, 1));
     cand_ee.alloc((size_t)CAND * std::max(ne, 1));
@@ -879,18 +1046,24 @@ Detector::~Detector() {
 void Detector::build_tree(Tree& T, const double* x, bool faces, hipStream_t stream, PrimScratch& scratch, bool refit) {
     const int n = T.n;
     if (n == 0) return;
-    auto leaf_data = [&]() {
+    auto refit_boxes = [&]() {
         if (faces)
-            hipLaunchKernelGGL(k_leaf_data<3>, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, x, (const int32_t*)tris.p,
-                               (const uint32_t*)T.ids.p, n, T.leaf_box.p, T.leafd.p, (const int2*)T.lpos.p, T.rec.p);
+            hipLaunchKernelGGL(k_refit<3>, dim3(grid_for(n, RB)), dim3(RB), 0, stream, x, (const int4*)T.leafid.p, n,
+                               T.leaf_box.p, (const int2*)T.lpos.p, (const int2*)T.range.p, (const int32_t*)T.ipos.p, T.blk_box.p,
+                               T.rec.p);
         else
-            hipLaunchKernelGGL(k_leaf_data<2>, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, x, (const int32_t*)edges.p,
-                               (const uint32_t*)T.ids.p, n, T.leaf_box.p, T.leafd.p, (const int2*)T.lpos.p, T.rec.p);
+            hipLaunchKernelGGL(k_refit<2>, dim3(grid_for(n, RB)), dim3(RB), 0, stream, x, (const int4*)T.leafid.p, n,
+                               T.leaf_box.p, (const int2*)T.lpos.p, (const int2*)T.range.p, (const int32_t*)T.ipos.p, T.blk_box.p,
+                               T.rec.p);
+        PA_LAUNCH_CHECK();
+        if (n <= RB) return;
+        // the number of crossing nodes (a few per block) stays on the device: a grid-stride launch
+        hipLaunchKernelGGL(k_cross_boxes, dim3(std::min(1024, grid_for(n, 64))), dim3(BLK), 0, stream, (const int32_t*)T.cross.p,
+                           (const int2*)T.range.p, (const int32_t*)T.ipos.p, (const float4*)T.leaf_box.p, (const float4*)T.blk_box.p, T.rec.p);
         PA_LAUNCH_CHECK();
     };
     if (refit) { // same sorted order and Karras topology, new boxes and leaf data
-        leaf_data();
-        if (n > 1) node_boxes(T, stream);
+        refit_boxes();
         return;
     }
     hipLaunchKernelGGL(k_prim_boxes, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, x, faces ? tris.p : edges.p, faces ? 3 : 2, n,
@@ -903,25 +1076,31 @@ void Detector::build_tree(Tree& T, const double* x, bool faces, hipStream_t stre
     PA_LAUNCH_CHECK();
     if (nseg > 0) {
         hipLaunchKernelGGL(k_morton_seg, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, T.prim_box.p, faces ? tris.p : edges.p,
-                           faces ? 3 : 2, n, (const int32_t*)vseg.p, T.scene.p, T.keys.p, T.ids.p);
+                           faces ? 3 : 2, n, (const int32_t*)vseg.p, T.scene.p, T.keys.p, T.ids.p, T.cross.p);
         PA_LAUNCH_CHECK();
         radix_sort_pairs(T.keys.p, T.ids.p, n, 32, scratch, stream);
     } else {
-        hipLaunchKernelGGL(k_morton, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, T.prim_box.p, n, T.scene.p, T.keys.p, T.ids.p);
+        hipLaunchKernelGGL(k_morton, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, T.prim_box.p, n, T.scene.p, T.keys.p, T.ids.p,
+                           T.cross.p);
         PA_LAUNCH_CHECK();
         radix_sort_pairs(T.keys.p, T.ids.p, n, 30, scratch, stream);
     }
+    if (faces)
+        hipLaunchKernelGGL(k_leaf_ids<3>, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, (const int32_t*)tris.p, (const uint32_t*)T.ids.p, n,
+                           T.leafid.p);
+    else
+        hipLaunchKernelGGL(k_leaf_ids<2>, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, (const int32_t*)edges.p, (const uint32_t*)T.ids.p, n,
+                           T.leafid.p);
+    PA_LAUNCH_CHECK();
     if (n > 1) {
         hipLaunchKernelGGL(k_karras, dim3(grid_for(n - 1, BLK)), dim3(BLK), 0, stream, T.keys.p, T.ids.p, n, T.child.p, T.range.p);
         PA_LAUNCH_CHECK();
-        fill<int32_t>(T.ipos.p, -1, n - 1, stream);
-        fill<int32_t>(T.lpos.p, -1, 2 * (int64_t)n, stream);
-        hipLaunchKernelGGL(k_record_slots, dim3(grid_for(n - 1, BLK)), dim3(BLK), 0, stream, n, (const int32_t*)T.child.p, T.rec.p,
-                           T.ipos.p, T.lpos.p);
+        fill2<int32_t>(T.ipos.p, n - 1, T.lpos.p, 2 * (int64_t)n, -1, stream);
+        hipLaunchKernelGGL(k_record_slots, dim3(grid_for(n - 1, BLK)), dim3(BLK), 0, stream, n, (const int32_t*)T.child.p,
+                           (const int2*)T.range.p, T.rec.p, T.ipos.p, T.lpos.p, T.cross.p);
         PA_LAUNCH_CHECK();
     }
-    leaf_data();
-    if (n > 1) node_boxes(T, stream);
+    refit_boxes();
     if (nseg > 0) {
         fill<int32_t>(T.seg_first.p, -1, nseg, stream);
         fill<int32_t>(T.seg_last.p, -1, nseg, stream);
@@ -933,31 +1112,6 @@ void Detector::build_tree(Tree& T, const double* x, bool faces, hipStream_t stre
                            (const int32_t*)T.seg_first.p, (const int32_t*)T.seg_last.p, T.seg_root.p);
         PA_LAUNCH_CHECK();
     }
-}
-
-// Internal node boxes from the leaf boxes (chunk unions, range unions),
-// written into their record slots (the leaves' slots are written with the
-// leaf data).  The 262144-leaf level is built only where a range can hold
-// more than 64 of the 4096-leaf chunks.
-void Detector::node_boxes(Tree& T, hipStream_t stream) {
-    const int n = T.n;
-    const int n64 = (n + 63) / 64, n4k = (n + 4095) / 4096, n256k = (n + 262143) / 262144;
-    hipLaunchKernelGGL(k_chunk_union, dim3(grid_for((int64_t)n64 * 64, BLK)), dim3(BLK), 0, stream, (const float4*)T.leaf_box.p, n,
-                       T.chunk64.p, n64);
-    PA_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_chunk_union, dim3(grid_for((int64_t)n4k * 64, BLK)), dim3(BLK), 0, stream, (const float4*)T.chunk64.p, n64,
-                       T.chunk4k.p, n4k);
-    PA_LAUNCH_CHECK();
-    const bool top = n4k > 64;
-    if (top) {
-        hipLaunchKernelGGL(k_chunk_union, dim3(grid_for((int64_t)n256k * 64, BLK)), dim3(BLK), 0, stream, (const float4*)T.chunk4k.p,
-                           n4k, T.chunk256k.p, n256k);
-        PA_LAUNCH_CHECK();
-    }
-    hipLaunchKernelGGL(k_node_boxes, dim3(grid_for(n - 1, BLK)), dim3(BLK), 0, stream, n, (const int2*)T.range.p, (const int32_t*)T.ipos.p,
-                       (const float4*)T.leaf_box.p, (const float4*)T.chunk64.p, (const float4*)T.chunk4k.p,
-                       top ? (const float4*)T.chunk256k.p : nullptr, T.rec.p);
-    PA_LAUNCH_CHECK();
 }
 
 void Detector::set_segments(const int32_t* vs, int count) {
@@ -985,49 +1139,40 @@ void Detector::set_segments(const int32_t* vs, int count) {
 int Detector::detect(const double* x, bool refit, VertexCount vc) {
     refit = refit && built;
     // the edge tree (build, query) runs on the side stream beside the triangle tree
-    fill2<uint32_t>(counts.p, 8 + (int64_t)nv + ne, vc.cnt, vc.cnt ? vc.n : 0, 0u, stream);
+    fill2<uint32_t>(counts.p, (int64_t)counts.n, vc.cnt, vc.cnt ? vc.n : 0, 0u, stream);
     PA_HIP(hipEventRecord(ev_fork, stream));
     PA_HIP(hipStreamWaitEvent(side, ev_fork, 0));
     const float gap = (float)(dhat * 1.001);
     QueryOut o{c.type.p, c.prim0.p, c.prim1.p, c.v.p, c.bary.p, c.nrm.p, c.dist.p, c.cap};
-    QueryOut st{stg.type.p, stg.prim0.p, stg.prim1.p, stg.v.p, stg.bary.p, stg.nrm.p, stg.dist.p, stg.cap};
-    const int32_t* ee_roots = nseg > 0 ? (const int32_t*)et.seg_root.p : nullptr;
-    const int32_t* pt_roots = nseg > 0 ? (const int32_t*)ft.seg_root.p : nullptr;
-    // Per query a collect pass (traversal, leaf hits to the slab or the
-    // overflow list) and a test pass (FP64 predicate): pairs to the staging
-    // list (total[2] counts them, atomically from both streams), per-segment
-    // counts to qcount.  The edge tree and its queries, the longer chain, are
-    // enqueued first so the side stream starts while the host still enqueues
-    // the triangle tree.
-    auto ee_pass = [&](auto mode, auto sk, hipStream_t s, dim3 grid) {
-        hipLaunchKernelGGL((k_query_ee<decltype(mode)::value, decltype(sk)::value>), grid, dim3(QBLK), 0, s, ne, n_dyn,
-                           (const float4*)et.rec.p, (const double2*)et.leafd.p, dhat, gap, qcount + nv, nv, st, st_seg.p, total + 2,
-                           total, (const int32_t*)vseg.p, ee_roots, cand_ee.p, ccount_ee.p, ovf_ee.p, ovf_count + 1);
+    // Per query a collect pass and a test pass, which marks the accepted pairs
+    // and counts them per segment.  The edge tree and its queries, the longer
+    // chain, are enqueued first so the side stream starts while the host still
+    // enqueues the triangle tree.
+    const EEQuery EE{x, et.leafid.p, vseg.p, nseg > 0 ? (const int32_t*)et.seg_root.p : nullptr, ne, ne, n_dyn, nv};
+    const PTQuery PT{x, surf_verts.p, ft.leafid.p, vseg.p, nseg > 0 ? (const int32_t*)ft.seg_root.p : nullptr, nv, nf, n_dyn};
+    const ListOut el{cand_ee.p, ccount_ee.p, ovf_ee.p, ovf_count + 1, total}, pl{cand_pt.p, ccount_pt.p, ovf_pt.p, ovf_count, total};
+    auto two_pass = [&](auto K, const Tree& T, const ListOut& l, hipStream_t s) {
+        using QK = decltype(K);
+        const int qw = collect_qw(K.nq), per = qw * (CBLK / 64); // queries per wave and per block
+        hipLaunchKernelGGL((qw == 4 ? k_collect<QK, 4> : qw == 8 ? k_collect<QK, 8> : qw == 16 ? k_collect<QK, 16> : qw == 32 ? k_collect<QK, 32>
+                                                                                                          : k_collect<QK, 64>),
+                           dim3(query_grid(K.nq, per)), dim3(CBLK), 0, s, K, (const float4*)T.rec.p, gap, query_chunk(K.nq, per), l);
+        PA_LAUNCH_CHECK();
+        hipLaunchKernelGGL(k_test<QK>, dim3(grid_for(K.nq, TQ)), dim3(TBLK), 0, s, K, l, dhat, qcount);
         PA_LAUNCH_CHECK();
     };
-    auto pt_pass = [&](auto mode, auto sk, hipStream_t s, dim3 grid) {
-        hipLaunchKernelGGL((k_query_pt<decltype(mode)::value, decltype(sk)::value>), grid, dim3(QBLK), 0, s, x, surf_verts.p, nv,
-                           n_dyn, nf, (const float4*)ft.rec.p, (const double2*)ft.leafd.p, dhat, gap, qcount, st, st_seg.p,
-                           total + 2, total, (const int32_t*)vseg.p, pt_roots, cand_pt.p, ccount_pt.p, ovf_pt.p, ovf_count);
+    auto single_pass = [&](auto K, int mark, const Tree& T) {
+        using QK = decltype(K);
+        hipLaunchKernelGGL(k_single<QK>, dim3(grid_for(K.nq, QBLK)), dim3(QBLK), 0, stream, K, mark, (const float4*)T.rec.p, gap, dhat, qcount,
+                           single_pairs.p, c.cap, total + 2, total);
         PA_LAUNCH_CHECK();
     };
-    using M0 = std::integral_constant<int, 0>;
-    using M1 = std::integral_constant<int, 1>;
-    using M2 = std::integral_constant<int, 2>;
-    using SS = std::integral_constant<int, SHORT_STACK>;
-    using LS = std::integral_constant<int, STACK>;
-    const bool two = !force_single_pass;
+    const bool two = !force_single_pass && std::max(nf, ne) <= (int)COLLECT_MASK;
     build_tree(et, x, false, side, scratch_side, refit);
-    if (ne > 0 && two) {
-        ee_pass(M0{}, SS{}, side, dim3(query_grid(ne)));
-        ee_pass(M1{}, SS{}, side, dim3(grid_for(ne, QBLK), test_rows(ne)));
-    }
+    if (ne > 0 && two) two_pass(EE, et, el, side);
     build_tree(ft, x, true, stream, scratch, refit);
     built = true;
-    if (nv > 0 && two) {
-        pt_pass(M0{}, SS{}, stream, dim3(query_grid(nv)));
-        pt_pass(M1{}, SS{}, stream, dim3(grid_for(nv, QBLK), test_rows(nv)));
-    }
+    if (nv > 0 && two) two_pass(PT, ft, pl, stream);
     PA_HIP(hipEventRecord(ev_join, side));
     PA_HIP(hipStreamWaitEvent(stream, ev_join, 0));
     uint32_t h[3] = {0u, 0u, 0u};
@@ -1039,19 +1184,21 @@ int Detector::detect(const double* x, bool refit, VertexCount vc) {
     if (two) {
         count_found(h);
     }
-    if (!two || h[1] != 0) {
+    const bool single = !two || h[1] != 0;
+    if (single) {
         // the short stack or an overflow list was too small: the single pass
         // (traversal and test together, full stack) for both queries
-        fill<uint32_t>(counts.p, 0u, 8 + (int64_t)nv + ne, stream);
-        if (ne > 0) ee_pass(M2{}, LS{}, stream, dim3(query_grid(ne)));
-        if (nv > 0) pt_pass(M2{}, LS{}, stream, dim3(query_grid(nv)));
+        fill<uint32_t>(counts.p, 0u, (int64_t)counts.n, stream);
+        single_pairs.reserve(c.cap);
+        if (ne > 0) single_pass(EE, ACCEPTED, et);
+        if (nv > 0) single_pass(PT, 0, ft);
         count_found(h);
         if (two) single_pass_fallbacks++;
     }
     found_total = h[0];
     stack_overflow = h[1] != 0;
     PA_CHECK(!stack_overflow, PA_ERR_INVALID, "LBVH traversal stack overflow");
-    PA_CHECK(h[2] == h[0], PA_ERR_INVALID, "contact staging count differs from the segment counts");
+    PA_CHECK(!single || h[2] == h[0], PA_ERR_INVALID, "contact list length differs from the segment counts");
     if (found_total > c.cap) {
         n_contacts = 0;
         throw Error(PA_ERR_OVERFLOW, "contact capacity exceeded: found " + std::to_string(found_total) + " > " + std::to_string(c.cap));
@@ -1059,14 +1206,21 @@ int Detector::detect(const double* x, bool refit, VertexCount vc) {
     n_contacts = (int)found_total;
     peak = std::max(peak, n_contacts);
     if (n_contacts > 0) {
-        // canonical order: segments in query order (PT by vertex, EE by the
-        // smaller edge id), each sorted by partner id
-        hipLaunchKernelGGL(k_segment_keys, dim3(grid_for(n_contacts, BLK)), dim3(BLK), 0, stream, n_contacts, (const int2*)st_seg.p,
-                           (const int32_t*)stg.prim1.p, (const uint32_t*)qoffset.p, seg_key.p);
-        PA_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_place_contacts, dim3(grid_for(n_contacts, BLK)), dim3(BLK), 0, stream, n_contacts, (const int2*)st_seg.p, st,
-                           (const uint32_t*)qoffset.p, (const uint32_t*)qcount, (const int32_t*)seg_key.p, o, vc);
-        PA_LAUNCH_CHECK();
+        const PlaceArgs pa{qoffset.p, qcount, qfill, seg_key.p, dhat, o, vc};
+        if (single) {
+            const dim3 g(grid_for(n_contacts, TBLK));
+            hipLaunchKernelGGL(k_place_single<0>, g, dim3(TBLK), 0, stream, PT, EE, (const int2*)single_pairs.p, n_contacts, pa);
+            PA_LAUNCH_CHECK();
+            hipLaunchKernelGGL(k_place_single<1>, g, dim3(TBLK), 0, stream, PT, EE, (const int2*)single_pairs.p, n_contacts, pa);
+            PA_LAUNCH_CHECK();
+        } else {
+            const int pt_blocks = grid_for(nv, TQ);
+            const dim3 g(pt_blocks + grid_for(ne, TQ));
+            hipLaunchKernelGGL(k_place<0>, g, dim3(TBLK), 0, stream, PT, pl, pt_blocks, EE, el, pa);
+            PA_LAUNCH_CHECK();
+            hipLaunchKernelGGL(k_place<1>, g, dim3(TBLK), 0, stream, PT, pl, pt_blocks, EE, el, pa);
+            PA_LAUNCH_CHECK();
+        }
     }
     return n_contacts;
 }

@@ -95,6 +95,26 @@ def test_detector_orders_long_segments(pa, faces):
     _check_contacts_equal(gi, gr, oi, orr)
 
 
+@pytest.mark.parametrize("side", [2, 3, 9, 60, 110, 180])
+def test_query_passes_agree_over_sizes(pa, side):
+    """The two-pass queries against the single pass, bit for bit, on folded
+    cloths from one cell up to 97,000 edges: below and above a refit block, and
+    every number of queries per wave of the collect pass but the largest."""
+    from parallel_admm_amd.configs import config_for
+
+    cfg = config_for("cloth32")
+    x, sc = folded_cloth(side=side, spacing=0.01, gap=0.5 * cfg.thickness, jitter=0.1 * cfg.thickness, seed=side)
+    out = []
+    for single in (False, True):
+        det = pa.CollisionDetector.for_scene(sc, capacity=1 << 20, thickness=cfg.thickness)
+        det.set_single_pass(single)
+        det.detect(x)
+        out.append(det.contacts())
+    assert side < 3 or len(out[0][0]) > 0
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    np.testing.assert_array_equal(out[0][1], out[1][1])
+
+
 def test_single_pass_and_two_pass_queries_agree(pa):
     """The two query passes (collect leaf hits, then test them) and the single
     pass (traversal and FP64 test together) give the same list, bit for bit:
