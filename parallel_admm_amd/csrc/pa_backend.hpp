@@ -39,8 +39,6 @@ struct Backend {
     int device = 0;
     int verbose = 0;
     hipStream_t stream = nullptr;
-    hipStream_t side = nullptr;                       // the elastic local step beside the contact phase
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     std::string last_error;
 
     pa_admm_config cfg{};
@@ -256,7 +254,7 @@ struct Backend {
     void set_vertex_mu(const double* mu);
 
     // sub-phases (also used by step)
-    void local_step(hipStream_t s = nullptr);
+    void local_step();
     void contact_setup(float eps, float gamma, float hinv, bool counted = false);
     void contact_project(bool first_iter);
     void contact_sweep_once();
@@ -283,7 +281,7 @@ struct Backend {
     // level-0 pre-smoothing was already done by k_cg_update_pre.
     void precondition(const float* r, bool skip_pre0 = false);
     void dual_vertices(bool want_residual);
-    void elem_update(bool want_residual, bool last, bool next_check, hipStream_t s);
+    void elem_update(bool want_residual, bool last, bool next_check);
     void residual_read(double* rp, double* rd);
     void residual_enqueue(int it);
     int3 resid_blocks();

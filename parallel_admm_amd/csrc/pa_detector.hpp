@@ -79,8 +79,8 @@ struct Detector {
     int64_t single_pass_fallbacks = 0; // detections that reran as a single pass (short stack or overflow list too small)
     bool force_single_pass = false;    // every detection runs the single pass
     PrimScratch scratch;
-    // The edge tree is built and queried on a second stream, concurrently
-    // with the triangle tree (own sort scratch; joined before the scan).
+    // The edge tree is built on a second stream, concurrently with the
+    // triangle tree (own sort scratch; joined before the refit).
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     PrimScratch scratch_side;
@@ -112,7 +112,8 @@ struct Detector {
     void set_stream(hipStream_t s) { stream = s; }
 
   private:
-    void build_tree(Tree& T, const double* x, bool faces, hipStream_t s, PrimScratch& scr, bool refit);
+    void build_tree(Tree& T, const double* x, bool faces, hipStream_t s, PrimScratch& scr);
+    void refit_trees(const double* x);
     bool built = false; // trees built at least once (a refit needs their order and topology)
 };
 

@@ -266,13 +266,31 @@ __device__ inline void put_slot(float4* __restrict__ rec, int p, float4 lo, floa
 // from x), now 29 + 9; 350 + 60 + 222 us of a 160-scene batch's edges, now
 // 233 + 93.  Blocks of 128 and 64 leaves list two and four times the crossing
 // nodes and were slower in sum (19 + 12 and 17 + 21 us on the cloth's edges).
+//
+// Both trees share a launch here and in the kernels below: first the blocks of
+// the edge tree, the longer chain, then those of the triangle tree.  On two
+// streams their eight launches and four event calls left a small scene's host
+// behind its GPU, and a large scene's launches fill the chip by themselves.
 constexpr int RB = 256, RB_LEVELS = 9;
+struct TreeArgs {
+    int n; // leaves
+    const int4* leafid;
+    float4* leaf_box;
+    const int2* lpos;
+    const int2* range;
+    const int32_t* ipos;
+    float4* blk_box;
+    const int32_t* cross;
+    float4* rec;
+};
 template <int K>
-__global__ void __launch_bounds__(RB) k_refit(const double* __restrict__ x, const int4* __restrict__ leafid, int n,
-                                              float4* __restrict__ leaf_box, const int2* __restrict__ lpos, const int2* __restrict__ range, const int32_t* __restrict__ ipos, float4* __restrict__ blk_box,
-                                              float4* __restrict__ rec) {
-    __shared__ float win[RB_LEVELS][6][RB]; // win[l][.][a]: box of leaves [a, a + 2^l) of the block
-    const int t = threadIdx.x, b0 = blockIdx.x * RB, k = b0 + t;
+__device__ inline void refit_block(const TreeArgs& T, int block, const double* __restrict__ x, float (&win)[RB_LEVELS][6][RB]) {
+    const int n = T.n;
+    const int4* __restrict__ leafid = T.leafid;
+    const int2 *__restrict__ lpos = T.lpos, *__restrict__ range = T.range;
+    const int32_t* __restrict__ ipos = T.ipos;
+    float4 *__restrict__ leaf_box = T.leaf_box, *__restrict__ blk_box = T.blk_box, *__restrict__ rec = T.rec;
+    const int t = threadIdx.x, b0 = block * RB, k = b0 + t;
     const bool node = k < n - 1;
     const int p = node ? ipos[k] : -1; // the root and its children sit in no slot
     const int2 rg = node ? range[k] : make_int2(0, 0);
@@ -313,8 +331,8 @@ __global__ void __launch_bounds__(RB) k_refit(const double* __restrict__ x, cons
         put(l);
     }
     if (t == 0) {
-        blk_box[2 * blockIdx.x] = lo;
-        blk_box[2 * blockIdx.x + 1] = hi;
+        blk_box[2 * block] = lo;
+        blk_box[2 * block + 1] = hi;
     }
     __syncthreads();
     if (p < 0 || rg.x < b0 || rg.y >= b0 + RB) return; // the others: k_cross_boxes
@@ -322,15 +340,28 @@ __global__ void __launch_bounds__(RB) k_refit(const double* __restrict__ x, cons
     put_slot(rec, p, fmin4(get_lo(l, a), get_lo(l, b)), fmax4(get_hi(l, a), get_hi(l, b)), k, rg.y);
 }
 
+__global__ void __launch_bounds__(RB) k_refit(TreeArgs E, TreeArgs F, int e_blocks, const double* __restrict__ x) {
+    __shared__ float win[RB_LEVELS][6][RB]; // win[l][.][a]: box of leaves [a, a + 2^l) of the block
+    if ((int)blockIdx.x < e_blocks) refit_block<2>(E, blockIdx.x, x, win);
+    else refit_block<3>(F, (int)blockIdx.x - e_blocks, x, win);
+}
+
 // Boxes of the internal nodes whose range crosses a block boundary of k_refit
 // (cross[1 .. cross[0]], listed by the build), one wave each: the leaves of the
 // first and the last block that it covers in part, and the boxes of the blocks
 // between them, all loads independent.
-__global__ void __launch_bounds__(BLK) k_cross_boxes(const int32_t* __restrict__ cross, const int2* __restrict__ range,
-                                                     const int32_t* __restrict__ ipos, const float4* __restrict__ leaf_box,
-                                                     const float4* __restrict__ blk_box, float4* __restrict__ rec) {
+// The number of crossing nodes (a few per block) stays on the device, so the
+// launch strides over them.
+__global__ void __launch_bounds__(BLK) k_cross_boxes(TreeArgs E, TreeArgs F, int e_blocks) {
+    const bool edges = (int)blockIdx.x < e_blocks;
+    const TreeArgs& T = edges ? E : F;
+    const int32_t *__restrict__ cross = T.cross, *__restrict__ ipos = T.ipos;
+    const int2* __restrict__ range = T.range;
+    const float4 *__restrict__ leaf_box = T.leaf_box, *__restrict__ blk_box = T.blk_box;
+    float4* __restrict__ rec = T.rec;
+    const int block = edges ? (int)blockIdx.x : (int)blockIdx.x - e_blocks, blocks = edges ? e_blocks : (int)gridDim.x - e_blocks;
     const int lane = threadIdx.x & 63, count = cross[0];
-    for (int w = blockIdx.x * (BLK / 64) + (threadIdx.x >> 6); w < count; w += gridDim.x * (BLK / 64)) {
+    for (int w = block * (BLK / 64) + (threadIdx.x >> 6); w < count; w += blocks * (BLK / 64)) {
         const int i = cross[1 + w], p = ipos[i];
         if (p < 0) continue; // the root or a child of it
         const int2 rg = range[i];
@@ -679,19 +710,20 @@ struct EEQuery {
 // keeps a wave's LDS accesses in order).
 __device__ inline void wave_lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 
+template <int QW> struct CollectWave {
+    uint32_t stack[CSTACK];  // (query of the wave << COLLECT_BITS) | node
+    uint32_t hit[128];       // (query << COLLECT_BITS) | sorted leaf
+    float4 blo[QW], bhi[QW]; // query boxes grown by gap; w: the query's vertex ids
+    int cnt[QW];
+};
 template <class QK, int QW>
-__global__ void __launch_bounds__(CBLK) k_collect(QK K, const float4* __restrict__ rec, float gap, int chunk, ListOut out) {
-    constexpr int W = CBLK / 64;
-    __shared__ uint32_t stack_[W][CSTACK]; // (query of the wave << COLLECT_BITS) | node
-    __shared__ uint32_t hit_[W][128];      // (query << COLLECT_BITS) | sorted leaf
-    __shared__ float4 blo_[W][QW], bhi_[W][QW]; // query boxes grown by gap; w: the query's vertex ids
-    __shared__ int cnt_[W][QW];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint32_t* const stack = stack_[wave];
-    uint32_t* const hit = hit_[wave];
-    float4 *const blo = blo_[wave], *const bhi = bhi_[wave];
-    int* const cnt = cnt_[wave];
-    const int q0 = (xcd_block(blockIdx.x, chunk) * W + wave) * QW;
+__device__ inline void collect_wave(const QK& K, int block, const float4* __restrict__ rec, float gap, const ListOut& out, CollectWave<QW>& sh) {
+    const int lane = threadIdx.x & 63;
+    uint32_t* const stack = sh.stack;
+    uint32_t* const hit = sh.hit;
+    float4 *const blo = sh.blo, *const bhi = sh.bhi;
+    int* const cnt = sh.cnt;
+    const int q0 = (block * (CBLK / 64) + (int)(threadIdx.x >> 6)) * QW;
     const int leaf0 = K.nleaf - 1;
     auto rank = [&](unsigned long long m) { return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u)); };
     int sp = 0, nh = 0; // entries of stack and hit, the same in all lanes
@@ -791,6 +823,16 @@ __global__ void __launch_bounds__(CBLK) k_collect(QK K, const float4* __restrict
     if (lane < QW && q0 + lane < K.nq) out.ccount[q0 + lane] = (uint32_t)cnt[lane];
 }
 
+template <int QW>
+__global__ void __launch_bounds__(CBLK) k_collect(EEQuery EE, const float4* __restrict__ erec, ListOut el, int e_grid, int e_chunk, PTQuery PT,
+                                                  const float4* __restrict__ frec, ListOut pl, int p_chunk, float gap) {
+    __shared__ CollectWave<QW> sh[CBLK / 64];
+    if ((int)blockIdx.x < e_grid) // a multiple of 8 blocks: the XCD of a block of either part is its index mod 8
+        collect_wave<EEQuery, QW>(EE, xcd_block(blockIdx.x, e_chunk), erec, gap, el, sh[threadIdx.x >> 6]);
+    else
+        collect_wave<PTQuery, QW>(PT, xcd_block((int)blockIdx.x - e_grid, p_chunk), frec, gap, pl, sh[threadIdx.x >> 6]);
+}
+
 // Exclusive prefix sums of the slab entries of queries q0 .. q0 + TQ into pre
 // (TQ + 1 values); returns their number.
 __device__ inline int slab_prefix(const uint32_t* __restrict__ ccount, int q0, int nq, int* pre) {
@@ -826,9 +868,8 @@ __device__ inline int ovf_entries(const ListOut& l, int nq) { // none if the lis
 constexpr int ACCEPTED = (int)0x80000000;
 
 template <class QK>
-__global__ void __launch_bounds__(TBLK) k_test(QK K, ListOut l, double dhat, uint32_t* __restrict__ qcount) {
-    __shared__ int pre[TQ + 1];
-    const int q0 = blockIdx.x * TQ, total = slab_prefix(l.ccount, q0, K.nq, pre);
+__device__ inline void test_block(const QK& K, const ListOut& l, int block, double dhat, uint32_t* __restrict__ qcount, int* pre) {
+    const int q0 = block * TQ, total = slab_prefix(l.ccount, q0, K.nq, pre);
     auto test = [&](int q, int32_t* entry) {
         const auto Q = K.query(q);
         const int lf = *entry;
@@ -840,8 +881,15 @@ __global__ void __launch_bounds__(TBLK) k_test(QK K, ListOut l, double dhat, uin
         const int s = slab_query(pre, i);
         test(q0 + s, &l.cand[(size_t)(i - pre[s]) * K.nq + q0 + s]);
     }
-    const int i = blockIdx.x * TBLK + threadIdx.x; // the launch has at least nq lanes
+    const int i = block * TBLK + threadIdx.x; // the launch has at least nq lanes
     if (i < ovf_entries(l, K.nq)) test(l.ovf[i].x, &l.ovf[i].y);
+}
+
+__global__ void __launch_bounds__(TBLK) k_test(EEQuery EE, ListOut el, int e_blocks, PTQuery PT, ListOut pl, double dhat,
+                                               uint32_t* __restrict__ qcount) {
+    __shared__ int pre[TQ + 1];
+    if ((int)blockIdx.x < e_blocks) test_block(EE, el, blockIdx.x, dhat, qcount, pre);
+    else test_block(PT, pl, (int)blockIdx.x - e_blocks, dhat, qcount, pre);
 }
 
 // Canonical order of the accepted pairs: segment by segment (PT by vertex, EE
@@ -1043,29 +1091,11 @@ Detector::~Detector() {
     }
 }
 
-void Detector::build_tree(Tree& T, const double* x, bool faces, hipStream_t stream, PrimScratch& scratch, bool refit) {
+// Sorted order, topology, leaf ids and record slots of one tree; the boxes follow
+// in refit_trees.
+void Detector::build_tree(Tree& T, const double* x, bool faces, hipStream_t stream, PrimScratch& scratch) {
     const int n = T.n;
     if (n == 0) return;
-    auto refit_boxes = [&]() {
-        if (faces)
-            hipLaunchKernelGGL(k_refit<3>, dim3(grid_for(n, RB)), dim3(RB), 0, stream, x, (const int4*)T.leafid.p, n,
-                               T.leaf_box.p, (const int2*)T.lpos.p, (const int2*)T.range.p, (const int32_t*)T.ipos.p, T.blk_box.p,
-                               T.rec.p);
-        else
-            hipLaunchKernelGGL(k_refit<2>, dim3(grid_for(n, RB)), dim3(RB), 0, stream, x, (const int4*)T.leafid.p, n,
-                               T.leaf_box.p, (const int2*)T.lpos.p, (const int2*)T.range.p, (const int32_t*)T.ipos.p, T.blk_box.p,
-                               T.rec.p);
-        PA_LAUNCH_CHECK();
-        if (n <= RB) return;
-        // the number of crossing nodes (a few per block) stays on the device: a grid-stride launch
-        hipLaunchKernelGGL(k_cross_boxes, dim3(std::min(1024, grid_for(n, 64))), dim3(BLK), 0, stream, (const int32_t*)T.cross.p,
-                           (const int2*)T.range.p, (const int32_t*)T.ipos.p, (const float4*)T.leaf_box.p, (const float4*)T.blk_box.p, T.rec.p);
-        PA_LAUNCH_CHECK();
-    };
-    if (refit) { // same sorted order and Karras topology, new boxes and leaf data
-        refit_boxes();
-        return;
-    }
     hipLaunchKernelGGL(k_prim_boxes, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, x, faces ? tris.p : edges.p, faces ? 3 : 2, n,
                        T.prim_box.p);
     PA_LAUNCH_CHECK();
@@ -1100,7 +1130,6 @@ void Detector::build_tree(Tree& T, const double* x, bool faces, hipStream_t stre
                            (const int2*)T.range.p, T.rec.p, T.ipos.p, T.lpos.p, T.cross.p);
         PA_LAUNCH_CHECK();
     }
-    refit_boxes();
     if (nseg > 0) {
         fill<int32_t>(T.seg_first.p, -1, nseg, stream);
         fill<int32_t>(T.seg_last.p, -1, nseg, stream);
@@ -1112,6 +1141,22 @@ void Detector::build_tree(Tree& T, const double* x, bool faces, hipStream_t stre
                            (const int32_t*)T.seg_first.p, (const int32_t*)T.seg_last.p, T.seg_root.p);
         PA_LAUNCH_CHECK();
     }
+}
+
+// Boxes of both trees from x.
+void Detector::refit_trees(const double* x) {
+    auto args = [](const Tree& T) {
+        return TreeArgs{T.n, T.leafid.p, T.leaf_box.p, (const int2*)T.lpos.p, T.range.p, T.ipos.p, T.blk_box.p, T.cross.p, T.rec.p};
+    };
+    const TreeArgs E = args(et), F = args(ft);
+    const int eb = grid_for(et.n, RB), fb = grid_for(ft.n, RB);
+    if (eb + fb == 0) return;
+    hipLaunchKernelGGL(k_refit, dim3(eb + fb), dim3(RB), 0, stream, E, F, eb, x);
+    PA_LAUNCH_CHECK();
+    const int ec = et.n > RB ? std::min(1024, grid_for(et.n, 64)) : 0, fc = ft.n > RB ? std::min(1024, grid_for(ft.n, 64)) : 0;
+    if (ec + fc == 0) return;
+    hipLaunchKernelGGL(k_cross_boxes, dim3(ec + fc), dim3(BLK), 0, stream, E, F, ec);
+    PA_LAUNCH_CHECK();
 }
 
 void Detector::set_segments(const int32_t* vs, int count) {
@@ -1138,29 +1183,24 @@ void Detector::set_segments(const int32_t* vs, int count) {
 
 int Detector::detect(const double* x, bool refit, VertexCount vc) {
     refit = refit && built;
-    // the edge tree (build, query) runs on the side stream beside the triangle tree
     fill2<uint32_t>(counts.p, (int64_t)counts.n, vc.cnt, vc.cnt ? vc.n : 0, 0u, stream);
-    PA_HIP(hipEventRecord(ev_fork, stream));
-    PA_HIP(hipStreamWaitEvent(side, ev_fork, 0));
+    if (!refit) { // the edge tree is built on the side stream beside the triangle tree
+        PA_HIP(hipEventRecord(ev_fork, stream));
+        PA_HIP(hipStreamWaitEvent(side, ev_fork, 0));
+        build_tree(et, x, false, side, scratch_side);
+        build_tree(ft, x, true, stream, scratch);
+        PA_HIP(hipEventRecord(ev_join, side));
+        PA_HIP(hipStreamWaitEvent(stream, ev_join, 0));
+        built = true;
+    }
+    refit_trees(x); // a refit keeps the sorted order and the Karras topology
     const float gap = (float)(dhat * 1.001);
     QueryOut o{c.type.p, c.prim0.p, c.prim1.p, c.v.p, c.bary.p, c.nrm.p, c.dist.p, c.cap};
-    // Per query a collect pass and a test pass, which marks the accepted pairs
-    // and counts them per segment.  The edge tree and its queries, the longer
-    // chain, are enqueued first so the side stream starts while the host still
-    // enqueues the triangle tree.
+    // A collect pass and a test pass, which marks the accepted pairs and counts
+    // them per segment.
     const EEQuery EE{x, et.leafid.p, vseg.p, nseg > 0 ? (const int32_t*)et.seg_root.p : nullptr, ne, ne, n_dyn, nv};
     const PTQuery PT{x, surf_verts.p, ft.leafid.p, vseg.p, nseg > 0 ? (const int32_t*)ft.seg_root.p : nullptr, nv, nf, n_dyn};
     const ListOut el{cand_ee.p, ccount_ee.p, ovf_ee.p, ovf_count + 1, total}, pl{cand_pt.p, ccount_pt.p, ovf_pt.p, ovf_count, total};
-    auto two_pass = [&](auto K, const Tree& T, const ListOut& l, hipStream_t s) {
-        using QK = decltype(K);
-        const int qw = collect_qw(K.nq), per = qw * (CBLK / 64); // queries per wave and per block
-        hipLaunchKernelGGL((qw == 4 ? k_collect<QK, 4> : qw == 8 ? k_collect<QK, 8> : qw == 16 ? k_collect<QK, 16> : qw == 32 ? k_collect<QK, 32>
-                                                                                                          : k_collect<QK, 64>),
-                           dim3(query_grid(K.nq, per)), dim3(CBLK), 0, s, K, (const float4*)T.rec.p, gap, query_chunk(K.nq, per), l);
-        PA_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_test<QK>, dim3(grid_for(K.nq, TQ)), dim3(TBLK), 0, s, K, l, dhat, qcount);
-        PA_LAUNCH_CHECK();
-    };
     auto single_pass = [&](auto K, int mark, const Tree& T) {
         using QK = decltype(K);
         hipLaunchKernelGGL(k_single<QK>, dim3(grid_for(K.nq, QBLK)), dim3(QBLK), 0, stream, K, mark, (const float4*)T.rec.p, gap, dhat, qcount,
@@ -1168,13 +1208,17 @@ int Detector::detect(const double* x, bool refit, VertexCount vc) {
         PA_LAUNCH_CHECK();
     };
     const bool two = !force_single_pass && std::max(nf, ne) <= (int)COLLECT_MASK;
-    build_tree(et, x, false, side, scratch_side, refit);
-    if (ne > 0 && two) two_pass(EE, et, el, side);
-    build_tree(ft, x, true, stream, scratch, refit);
-    built = true;
-    if (nv > 0 && two) two_pass(PT, ft, pl, stream);
-    PA_HIP(hipEventRecord(ev_join, side));
-    PA_HIP(hipStreamWaitEvent(stream, ev_join, 0));
+    if (two && nv + ne > 0) {
+        const int qw = collect_qw(nv + ne), per = qw * (CBLK / 64); // queries per wave and per block
+        const int eg = ne > 0 ? query_grid(ne, per) : 0, pg = nv > 0 ? query_grid(nv, per) : 0;
+        hipLaunchKernelGGL((qw == 4 ? k_collect<4> : qw == 8 ? k_collect<8> : qw == 16 ? k_collect<16> : qw == 32 ? k_collect<32> : k_collect<64>),
+                           dim3(eg + pg), dim3(CBLK), 0, stream, EE, (const float4*)et.rec.p, el, eg, query_chunk(ne, per), PT,
+                           (const float4*)ft.rec.p, pl, query_chunk(nv, per), gap);
+        PA_LAUNCH_CHECK();
+        const int eb = grid_for(ne, TQ);
+        hipLaunchKernelGGL(k_test, dim3(eb + grid_for(nv, TQ)), dim3(TBLK), 0, stream, EE, el, eb, PT, pl, dhat, qcount);
+        PA_LAUNCH_CHECK();
+    }
     uint32_t h[3] = {0u, 0u, 0u};
     auto count_found = [&](uint32_t* o) { // segment offsets; the totals reach the host with the scan's last launch
         scan_exclusive(qcount, qoffset.p, (int64_t)nv + ne, total, scratch, stream, total_host);

@@ -2160,9 +2160,6 @@ Backend::Backend(const pa_device_opts* o) {
     PA_CHECK(device >= 0 && device < count, PA_ERR_INVALID, "device ordinal out of range");
     PA_HIP(hipSetDevice(device));
     PA_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-    PA_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking)); // default priority, as `stream`
-    PA_HIP(hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming));
-    PA_HIP(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming));
     for (auto& e : ev_chk) PA_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     PA_HIP(hipHostMalloc((void**)&chk_host, 16 * sizeof(double), hipHostMallocDefault));
     pa_admm_config_default(&cfg);
@@ -2177,12 +2174,6 @@ Backend::~Backend() {
     if (det && det != own_det.get()) det->stream = det->own_stream;
     own_det.reset();
     ws_mlp.reset(); // uses the stream
-    if (side) {
-        (void)hipStreamSynchronize(side);
-        (void)hipStreamDestroy(side);
-    }
-    if (ev_fork) (void)hipEventDestroy(ev_fork);
-    if (ev_join) (void)hipEventDestroy(ev_join);
     for (auto e : ev_chk)
         if (e) (void)hipEventDestroy(e);
     if (chk_host) (void)hipHostFree(chk_host);
@@ -2850,11 +2841,11 @@ static ElemArgs make_elem_args(const Backend& B) {
 static int elem_grid(const ElemArgs& a, int n_pin) { return a.blk_bend + grid_for(n_pin, BLK); }
 
 // z = prox(D x + Ue) at the step's first x.
-void Backend::local_step(hipStream_t s) {
+void Backend::local_step() {
     ElemArgs a = make_elem_args(*this);
     int g = elem_grid(a, hc.n_pin);
     if (g == 0) return;
-    hipLaunchKernelGGL(k_elem<ELEM_LOCAL>, dim3(g), dim3(BLK), 0, s ? s : stream, a, 0, x.p, Ue.p, z.p, (float*)nullptr, (double*)nullptr,
+    hipLaunchKernelGGL(k_elem<ELEM_LOCAL>, dim3(g), dim3(BLK), 0, stream, a, 0, x.p, Ue.p, z.p, (float*)nullptr, (double*)nullptr,
                        (const int32_t*)nullptr);
     PA_LAUNCH_CHECK();
 }
@@ -2871,11 +2862,11 @@ void Backend::dual_vertices(bool want_res) {
 
 // The elastic dual update of this iteration and, unless it is the last, the
 // local step of the next one (next_check: that one's residual needs zprev).
-void Backend::elem_update(bool want_res, bool last, bool next_check, hipStream_t s) {
+void Backend::elem_update(bool want_res, bool last, bool next_check) {
     ElemArgs a = make_elem_args(*this);
     const int g = elem_grid(a, hc.n_pin);
     if (g == 0) return;
-    hipLaunchKernelGGL((last ? k_elem<ELEM_DUAL> : k_elem<ELEM_DUAL | ELEM_LOCAL>), dim3(g), dim3(BLK), 0, s, a, want_res ? 1 : 0, x.p, Ue.p,
+    hipLaunchKernelGGL((last ? k_elem<ELEM_DUAL> : k_elem<ELEM_DUAL | ELEM_LOCAL>), dim3(g), dim3(BLK), 0, stream, a, want_res ? 1 : 0, x.p, Ue.p,
                        z.p, next_check ? zprev.p : (float*)nullptr, res_part.p, (const int32_t*)stop_guard);
     PA_LAUNCH_CHECK();
 }
@@ -3963,25 +3954,6 @@ int Backend::admm_loop(pa_step_stats& S, float eps, float gam_, float hinv) {
     res_log.clear(); // this attempt's checks
     double best = std::numeric_limits<double>::infinity();
     int it = 0;
-    // The elastic part (Ue and z from x) and the contact phase (detection,
-    // projection: p from x, x0, Uc) are independent until the right-hand
-    // side: the elastic pass runs on the side stream beside them.  Where an
-    // iteration is checked its elastic pass stays on the main stream, before
-    // the check (which must precede every later write).  Phase timing
-    // (profiling bit 1) keeps them in sequence.
-    const bool overlap = !(profiling & 2);
-    bool side_busy = false;
-    auto fork = [&]() {
-        PA_HIP(hipEventRecord(ev_fork, stream));
-        PA_HIP(hipStreamWaitEvent(side, ev_fork, 0));
-        side_busy = true;
-    };
-    auto join = [&]() {
-        if (!side_busy) return;
-        side_busy = false;
-        PA_HIP(hipEventRecord(ev_join, side));
-        PA_HIP(hipStreamWaitEvent(stream, ev_join, 0));
-    };
     auto checked = [&](int q) { return cfg.residual_tol > 0 && (q + 1) % cfg.residual_interval == 0; };
     // Stop test on the device (direct solve, no learned warm start): the
     // check of iteration q is read back once iteration q + 1 is enqueued, or
@@ -4016,9 +3988,10 @@ int Backend::admm_loop(pa_step_stats& S, float eps, float gam_, float hinv) {
                 break; // it == q + 1
             }
         }
-        if (it == 0 && overlap) {
-            fork();
-            local_step(side);
+        if (it == 0) {
+            mark_begin(1, &e);
+            local_step();
+            mark_end(1, e);
         }
         if (contact && it % cfg.dcd_interval == 0) {
             mark_begin(0, &e);
@@ -4027,30 +4000,19 @@ int Backend::admm_loop(pa_step_stats& S, float eps, float gam_, float hinv) {
                 mark_end(0, e);
                 break;
             }
-            try {
-                // rebuild at the step's first detection, refit later ones
-                det->detect(x.p, it > 0, VertexCount{vcnt.p, vloc.p, n_all});
-            } catch (...) {
-                join(); // the rollback writes x, which the side stream reads
-                throw;
-            }
+            // rebuild at the step's first detection, refit later ones
+            det->detect(x.p, it > 0, VertexCount{vcnt.p, vloc.p, n_all});
             contact_setup(eps, gam_, hinv, true);
             ws_window_begin();
             S.detections++;
             S.n_contacts_max = std::max(S.n_contacts_max, nc);
             mark_end(0, e);
         }
-        if (it == 0 && !overlap) {
-            mark_begin(1, &e);
-            local_step();
-            mark_end(1, e);
-        }
         if (contact) {
             mark_begin(2, &e);
             contact_project(it == 0);
             mark_end(2, e);
         }
-        join();
         const bool check = checked(it);
         mark_begin(3, &e);
         rhs(check, it == 0);
@@ -4062,13 +4024,7 @@ int Backend::admm_loop(pa_step_stats& S, float eps, float gam_, float hinv) {
         mark_end(4, e);
         mark_begin(1, &e);
         dual_vertices(check);
-        const bool last = it + 1 >= cfg.admm_max_iter;
-        if (overlap && !check && !last) {
-            fork();
-            elem_update(false, last, checked(it + 1), side);
-        } else {
-            elem_update(check, last, checked(it + 1), stream);
-        }
+        elem_update(check, it + 1 >= cfg.admm_max_iter, checked(it + 1));
         mark_end(1, e);
         if (lagged) {
             if (check) residual_enqueue(it);
@@ -4105,7 +4061,6 @@ int Backend::admm_loop(pa_step_stats& S, float eps, float gam_, float hinv) {
             }
         }
     }
-    join();
     if (lagged && pending >= 0 && take_check(pending)) S.converged = 1; // the last iteration's check
     if (ws_active && !ws_restart) ws_judge(); // the last window of the attempt
     return it;
