@@ -19,7 +19,6 @@ struct Tree {
     DBuf<int2> range;        // per internal node: first and last sorted leaf it covers
     DBuf<float4> rec;        // 8 per internal node: boxes, ids and last leaf of its up to four grandchildren
     DBuf<float4> blk_box;    // 2 per block of sorted leaves that the refit takes together
-    DBuf<int32_t> cross;     // [0] count, then the internal nodes whose range crosses such a block's boundary
     DBuf<int32_t> ipos;      // per internal node: float4 index of its record slot (-1: none)
     DBuf<int32_t> lpos;      // 2 per leaf: its slot in the parent's record, in the grandparent's (-1: none)
     DBuf<float4> scene;      // 2: scene box
@@ -79,8 +78,8 @@ struct Detector {
     int64_t single_pass_fallbacks = 0; // detections that reran as a single pass (short stack or overflow list too small)
     bool force_single_pass = false;    // every detection runs the single pass
     PrimScratch scratch;
-    // The edge tree is built on a second stream, concurrently with the
-    // triangle tree (own sort scratch; joined before the refit).
+    // A large edge tree is sorted on a second stream, concurrently with the
+    // triangle tree (own sort scratch; joined before the topology).
     hipStream_t side = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     PrimScratch scratch_side;
@@ -112,7 +111,9 @@ struct Detector {
     void set_stream(hipStream_t s) { stream = s; }
 
   private:
-    void build_tree(Tree& T, const double* x, bool faces, hipStream_t s, PrimScratch& scr);
+    void sort_leaves(Tree& T, const double* x, bool faces, hipStream_t s, PrimScratch& scr);
+    void build_topology();
+    void segment_roots(Tree& T);
     void refit_trees(const double* x);
     bool built = false; // trees built at least once (a refit needs their order and topology)
 };

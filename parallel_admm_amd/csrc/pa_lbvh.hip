@@ -125,24 +125,18 @@ __device__ inline uint32_t spread10(uint32_t v) {
     return v;
 }
 
-__device__ inline uint32_t quant10(float u) {
-    float q = fminf(fmaxf(u * 1024.0f, 0.0f), 1023.0f);
-    return (uint32_t)q;
+__device__ inline uint32_t morton_key(float4 lo, float4 hi, float4 slo, float4 shi, float cells, float last) {
+    const float ex = shi.x - slo.x, ey = shi.y - slo.y, ez = shi.z - slo.z;
+    const float cx = 0.5f * (lo.x + hi.x) - slo.x, cy = 0.5f * (lo.y + hi.y) - slo.y, cz = 0.5f * (lo.z + hi.z) - slo.z;
+    auto cell = [&](float u) { return (uint32_t)fminf(fmaxf(u * cells, 0.0f), last); };
+    return (spread10(cell(ex > 0.f ? cx / ex : 0.f)) << 2) | (spread10(cell(ey > 0.f ? cy / ey : 0.f)) << 1) | spread10(cell(ez > 0.f ? cz / ez : 0.f));
 }
 
 __global__ void k_morton(const float4* __restrict__ box, int n, const float4* __restrict__ scene, uint32_t* __restrict__ keys,
-                         uint32_t* __restrict__ ids, int32_t* __restrict__ cross) {
+                         uint32_t* __restrict__ ids) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0) cross[0] = 0; // for k_record_slots
     if (i >= n) return;
-    float4 slo = scene[0], shi = scene[1];
-    float4 lo = box[2 * i], hi = box[2 * i + 1];
-    float ex = shi.x - slo.x, ey = shi.y - slo.y, ez = shi.z - slo.z;
-    float cx = 0.5f * (lo.x + hi.x) - slo.x, cy = 0.5f * (lo.y + hi.y) - slo.y, cz = 0.5f * (lo.z + hi.z) - slo.z;
-    uint32_t qx = quant10(ex > 0.f ? cx / ex : 0.f);
-    uint32_t qy = quant10(ey > 0.f ? cy / ey : 0.f);
-    uint32_t qz = quant10(ez > 0.f ? cz / ez : 0.f);
-    keys[i] = (spread10(qx) << 2) | (spread10(qy) << 1) | spread10(qz);
+    keys[i] = morton_key(box[2 * i], box[2 * i + 1], scene[0], scene[1], 1024.0f, 1023.0f);
     ids[i] = (uint32_t)i;
 }
 
@@ -150,19 +144,130 @@ __global__ void k_morton(const float4* __restrict__ box, int n, const float4* __
 // (7 bits per axis) of the box centre in the box of all segments.
 __global__ void k_morton_seg(const float4* __restrict__ box, const int32_t* __restrict__ prims, int k, int n,
                              const int32_t* __restrict__ vseg, const float4* __restrict__ scene, uint32_t* __restrict__ keys,
-                             uint32_t* __restrict__ ids, int32_t* __restrict__ cross) {
+                             uint32_t* __restrict__ ids) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0) cross[0] = 0; // for k_record_slots
     if (i >= n) return;
-    float4 slo = scene[0], shi = scene[1];
-    float4 lo = box[2 * i], hi = box[2 * i + 1];
-    float ex = shi.x - slo.x, ey = shi.y - slo.y, ez = shi.z - slo.z;
-    float cx = 0.5f * (lo.x + hi.x) - slo.x, cy = 0.5f * (lo.y + hi.y) - slo.y, cz = 0.5f * (lo.z + hi.z) - slo.z;
-    auto q7 = [](float u) { return (uint32_t)fminf(fmaxf(u * 128.0f, 0.0f), 127.0f); };
-    const uint32_t qx = q7(ex > 0.f ? cx / ex : 0.f), qy = q7(ey > 0.f ? cy / ey : 0.f), qz = q7(ez > 0.f ? cz / ez : 0.f);
-    const uint32_t m = (spread10(qx) << 2) | (spread10(qy) << 1) | spread10(qz); // 21 bits
-    keys[i] = ((uint32_t)vseg[prims[k * i]] << 21) | m;
+    keys[i] = ((uint32_t)vseg[prims[k * i]] << 21) | morton_key(box[2 * i], box[2 * i + 1], scene[0], scene[1], 128.0f, 127.0f); // 21 bits
     ids[i] = (uint32_t)i;
+}
+
+// Sorted leaves of a tree of up to SMALL_BUILD primitives in one workgroup:
+// primitive boxes, scene box, keys, the radix sort (the elements of a pass in
+// registers, written back to LDS in their new order) and the leaf ids, with the
+// results of the kernels above and radix_sort_pairs.  Those take 17 launches
+// and about 110 us for a tree of 5000 primitives, little of it work; this takes
+// 34-47 us on one CU, and both trees run side by side (one detection of a
+// 33 x 33 cloth 399 -> 259 us).
+constexpr int SMALL_BUILD = 16384, SB_BLK = 1024, SB_ITEMS = SMALL_BUILD / SB_BLK, SB_WAVES = SB_BLK / 64;
+struct SmallTree {
+    const int32_t* prims;
+    int k, n; // vertices per primitive, primitives
+    uint32_t* keys;
+    uint32_t* ids;
+    int4* leafid;
+};
+__global__ void __launch_bounds__(SB_BLK) k_build_small(const double* __restrict__ x, const int32_t* __restrict__ vseg, SmallTree E, SmallTree F) {
+    __shared__ uint32_t lk[SMALL_BUILD], li[SMALL_BUILD / 2]; // keys; ids fit 14 bits, two to a word
+    __shared__ uint32_t cnt[SB_WAVES][256];
+    __shared__ float4 slo[SB_WAVES], shi[SB_WAVES];
+    const SmallTree& T = blockIdx.x == 0 ? E : F;
+    const int n = T.n;
+    if (n == 0) return;
+    uint16_t* const lid = reinterpret_cast<uint16_t*>(li);
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    // a wave owns consecutive elements, so that equal digits keep their order
+    const int items = (n + SB_BLK - 1) / SB_BLK, e0 = wave * 64 * items + lane;
+    float4 lo[SB_ITEMS], hi[SB_ITEMS], blo = make_float4(INFINITY, INFINITY, INFINITY, 0.f), bhi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
+    uint32_t key[SB_ITEMS], id[SB_ITEMS];
+#pragma unroll
+    for (int j = 0; j < SB_ITEMS; j++) {
+        const int e = e0 + 64 * j;
+        lo[j] = make_float4(INFINITY, INFINITY, INFINITY, 0.f);
+        hi[j] = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
+        if (j < items && e < n)
+            for (int q = 0; q < T.k; q++) {
+                const int v = T.prims[T.k * e + q];
+                lo[j] = fmin4(lo[j], pos_lo(x, v));
+                hi[j] = fmax4(hi[j], pos_hi(x, v));
+            }
+        blo = fmin4(blo, lo[j]);
+        bhi = fmax4(bhi, hi[j]);
+    }
+    blo = wave_min4(blo);
+    bhi = wave_max4(bhi);
+    if (lane == 0) {
+        slo[wave] = blo;
+        shi[wave] = bhi;
+    }
+    __syncthreads();
+    for (int w = 0; w < SB_WAVES; w++) {
+        blo = fmin4(blo, slo[w]);
+        bhi = fmax4(bhi, shi[w]);
+    }
+#pragma unroll
+    for (int j = 0; j < SB_ITEMS; j++) {
+        const int e = e0 + 64 * j;
+        key[j] = 0u;
+        id[j] = (uint32_t)e;
+        if (j < items && e < n)
+            key[j] = vseg ? (uint32_t)vseg[T.prims[T.k * e]] << 21 | morton_key(lo[j], hi[j], blo, bhi, 128.0f, 127.0f)
+                          : morton_key(lo[j], hi[j], blo, bhi, 1024.0f, 1023.0f);
+    }
+    for (int shift = 0; shift < 32; shift += 8) {
+        for (int c = t; c < SB_WAVES * 256; c += SB_BLK) cnt[c >> 8][c & 255] = 0;
+        __syncthreads();
+        uint32_t pos[SB_ITEMS];
+#pragma unroll
+        for (int j = 0; j < SB_ITEMS; j++)
+            pos[j] = j < items ? rs_rank((key[j] >> shift) & 255u, e0 + 64 * j < n, cnt[wave]) : 0u;
+        __syncthreads();
+        // digit d's start: the smaller digits' totals, then the waves before
+        uint32_t tot = 0;
+        if (t < 256)
+            for (int w = 0; w < SB_WAVES; w++) tot += cnt[w][t];
+        uint32_t inc = tot;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(inc, o, 64);
+            if (lane >= o) inc += y;
+        }
+        if (t < 256 && lane == 63) lk[wave] = inc; // lk is free here: the elements are in registers
+        __syncthreads();
+        if (t < 256) {
+            uint32_t run = inc - tot;
+            for (int w = 0; w < wave; w++) run += lk[w];
+            for (int w = 0; w < SB_WAVES; w++) {
+                const uint32_t c = cnt[w][t];
+                cnt[w][t] = run;
+                run += c;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < SB_ITEMS; j++)
+            if (j < items && e0 + 64 * j < n) {
+                const uint32_t p = cnt[wave][(key[j] >> shift) & 255u] + pos[j];
+                lk[p] = key[j];
+                lid[p] = (uint16_t)id[j];
+            }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < SB_ITEMS; j++)
+            if (j < items && e0 + 64 * j < n) {
+                key[j] = lk[e0 + 64 * j];
+                id[j] = lid[e0 + 64 * j];
+            }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int j = 0; j < SB_ITEMS; j++) {
+        const int e = e0 + 64 * j;
+        if (j < items && e < n) {
+            T.keys[e] = key[j];
+            T.ids[e] = id[j];
+            const int32_t* p = T.prims + T.k * (int)id[j];
+            T.leafid[e] = make_int4((int)id[j], p[0], p[1], T.k == 3 ? p[2] : -1);
+        }
+    }
 }
 
 // First and last sorted leaf of every segment (segments with no primitive keep -1).
@@ -198,11 +303,32 @@ __device__ inline int kdelta(const uint32_t* __restrict__ keys, const uint32_t* 
     return __clzll(a ^ b);
 }
 
-// Karras construction of internal node i over sorted unique 64-bit keys.
-__global__ void k_karras(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ ids, int n, int32_t* __restrict__ child,
-                         int2* __restrict__ range) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+// What the build of a tree's topology reads and writes.  Both trees share a
+// launch, as in a refit.
+struct TopoArgs {
+    int n;
+    const uint32_t* keys;
+    const uint32_t* ids;
+    int32_t* child;
+    int2* range;
+    int32_t* ipos;
+    int32_t* lpos;
+    float4* rec;
+};
+
+// Karras construction of internal node i over sorted unique 64-bit keys; also
+// clears the slot positions that k_record_slots then fills (-1: none).
+__global__ void k_karras(TopoArgs E, TopoArgs F, int e_blocks) {
+    const bool edges = (int)blockIdx.x < e_blocks;
+    const TopoArgs& T = edges ? E : F;
+    const uint32_t *__restrict__ keys = T.keys, *__restrict__ ids = T.ids;
+    int32_t* __restrict__ child = T.child;
+    int2* __restrict__ range = T.range;
+    const int n = T.n;
+    int i = (edges ? (int)blockIdx.x : (int)blockIdx.x - e_blocks) * (int)blockDim.x + (int)threadIdx.x;
+    if (i < n) reinterpret_cast<int2*>(T.lpos)[i] = make_int2(-1, -1);
     if (i >= n - 1) return;
+    T.ipos[i] = -1;
     const int d = (kdelta(keys, ids, n, i, i + 1) - kdelta(keys, ids, n, i, i - 1)) >= 0 ? 1 : -1;
     const int dmin = kdelta(keys, ids, n, i, i - d);
     int lmax = 2;
@@ -280,7 +406,6 @@ struct TreeArgs {
     const int2* range;
     const int32_t* ipos;
     float4* blk_box;
-    const int32_t* cross;
     float4* rec;
 };
 template <int K>
@@ -346,25 +471,28 @@ __global__ void __launch_bounds__(RB) k_refit(TreeArgs E, TreeArgs F, int e_bloc
     else refit_block<3>(F, (int)blockIdx.x - e_blocks, x, win);
 }
 
-// Boxes of the internal nodes whose range crosses a block boundary of k_refit
-// (cross[1 .. cross[0]], listed by the build), one wave each: the leaves of the
-// first and the last block that it covers in part, and the boxes of the blocks
-// between them, all loads independent.
-// The number of crossing nodes (a few per block) stays on the device, so the
-// launch strides over them.
-__global__ void __launch_bounds__(BLK) k_cross_boxes(TreeArgs E, TreeArgs F, int e_blocks) {
+// Boxes of the internal nodes whose range crosses a block boundary of k_refit:
+// the leaves of the first and the last block that a node covers in part, and the
+// boxes of the blocks between them, all loads independent.  A wave looks at
+// `per` nodes and works on its few crossing ones (most have none) with all
+// lanes, one after the other: 16 nodes up to CROSS_SMALL leaves, where the
+// longest wave is the launch (6.2 us against 8.3 with 64 on 3000 leaves), 64
+// above (14 us against 18 on 330,000, 110 against 148 on 2.5 million).  A list of the crossing nodes, made once per build, spread
+// them evenly but cost more than it gave: appending to it took 10-20 ns per
+// wave on one counter (37 us of the 256x256 cloth's build, 440 of a batch's).
+constexpr int CROSS_SMALL = 1 << 16;
+__global__ void __launch_bounds__(BLK) k_cross_boxes(TreeArgs E, TreeArgs F, int e_blocks, int per) {
     const bool edges = (int)blockIdx.x < e_blocks;
     const TreeArgs& T = edges ? E : F;
-    const int32_t *__restrict__ cross = T.cross, *__restrict__ ipos = T.ipos;
-    const int2* __restrict__ range = T.range;
     const float4 *__restrict__ leaf_box = T.leaf_box, *__restrict__ blk_box = T.blk_box;
-    float4* __restrict__ rec = T.rec;
-    const int block = edges ? (int)blockIdx.x : (int)blockIdx.x - e_blocks, blocks = edges ? e_blocks : (int)gridDim.x - e_blocks;
-    const int lane = threadIdx.x & 63, count = cross[0];
-    for (int w = block * (BLK / 64) + (threadIdx.x >> 6); w < count; w += blocks * (BLK / 64)) {
-        const int i = cross[1 + w], p = ipos[i];
-        if (p < 0) continue; // the root or a child of it
-        const int2 rg = range[i];
+    const int lane = threadIdx.x & 63;
+    const int i = (edges ? (int)blockIdx.x : (int)blockIdx.x - e_blocks) * (per * (BLK / 64)) + (int)(threadIdx.x >> 6) * per + lane;
+    const bool node = lane < per && i < T.n - 1;
+    const int2 r = node ? T.range[i] : make_int2(0, 0);
+    const int slot = node ? T.ipos[i] : -1; // none for the root and its children
+    for (unsigned long long todo = __ballot(slot >= 0 && r.x / RB != r.y / RB); todo; todo &= todo - 1) {
+        const int from = __ffsll(todo) - 1, p = __shfl(slot, from, 64), id = i - lane + from;
+        const int2 rg = make_int2(__shfl(r.x, from, 64), __shfl(r.y, from, 64));
         const int A = rg.x / RB, B = rg.y / RB;
         float4 lo = make_float4(INFINITY, INFINITY, INFINITY, 0.f), hi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.f);
         auto take = [&](const float4* arr, int u, int v) { // boxes [u, v): lane u + lane, .. + 64, ..., four in flight
@@ -388,7 +516,7 @@ __global__ void __launch_bounds__(BLK) k_cross_boxes(TreeArgs E, TreeArgs F, int
         take(blk_box, A + 1, B);
         lo = wave_min4(lo);
         hi = wave_max4(hi);
-        if (lane == 0) put_slot(rec, p, lo, hi, i, rg.y);
+        if (lane == 0) put_slot(T.rec, p, lo, hi, id, rg.y);
     }
 }
 
@@ -443,14 +571,15 @@ __global__ void k_leaf_ids(const int32_t* __restrict__ prims, const uint32_t* __
 // Record slots (build only): empty slots get their constant, and every node
 // that sits in a slot gets the slot's position (ipos for internal nodes;
 // lpos.x for a leaf kept by its parent, lpos.y in its grandparent's record),
-// each written by exactly one thread.  Nodes whose range crosses a block
-// boundary of k_refit are listed in cross (any order; cross[0] counts them).
-__global__ void k_record_slots(int n, const int32_t* __restrict__ child, const int2* __restrict__ range, float4* __restrict__ rec,
-                               int32_t* __restrict__ ipos, int32_t* __restrict__ lpos, int32_t* __restrict__ cross) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// each written by exactly one thread.
+__global__ void k_record_slots(TopoArgs E, TopoArgs F, int e_blocks) {
+    const bool edges = (int)blockIdx.x < e_blocks;
+    const TopoArgs& T = edges ? E : F;
+    const int n = T.n, i = (edges ? (int)blockIdx.x : (int)blockIdx.x - e_blocks) * (int)blockDim.x + (int)threadIdx.x;
     if (i >= n - 1) return;
-    const int2 rg = range[i];
-    if (rg.x / RB != rg.y / RB) cross[1 + stage_slot(reinterpret_cast<uint32_t*>(cross))] = i;
+    const int32_t* __restrict__ child = T.child;
+    float4* __restrict__ rec = T.rec;
+    int32_t *__restrict__ ipos = T.ipos, *__restrict__ lpos = T.lpos;
     const int l = child[2 * i], r = child[2 * i + 1];
     const bool li = l < n - 1, ri = r < n - 1;
     const int sl[4] = {li ? child[2 * l] : l, li ? child[2 * l + 1] : -1, ri ? child[2 * r] : r, ri ? child[2 * r + 1] : -1};
@@ -1045,7 +1174,6 @@ Detector::Detector(int n_all_, int n_dyn_, int nv_, const int32_t* sv, int nf_, 
         T.range.alloc(std::max(n - 1, 1));
         T.rec.alloc(8 * (size_t)std::max(n - 1, 1));
         T.blk_box.alloc(2 * (size_t)grid_for(n, RB));
-        T.cross.alloc((size_t)n + 1);
         T.scene.alloc(2);
         T.partial.alloc(2 * 256);
     };
@@ -1091,9 +1219,8 @@ Detector::~Detector() {
     }
 }
 
-// Sorted order, topology, leaf ids and record slots of one tree; the boxes follow
-// in refit_trees.
-void Detector::build_tree(Tree& T, const double* x, bool faces, hipStream_t stream, PrimScratch& scratch) {
+// Sorted leaves of one tree: keys, ids and leaf ids.
+void Detector::sort_leaves(Tree& T, const double* x, bool faces, hipStream_t stream, PrimScratch& scratch) {
     const int n = T.n;
     if (n == 0) return;
     hipLaunchKernelGGL(k_prim_boxes, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, x, faces ? tris.p : edges.p, faces ? 3 : 2, n,
@@ -1106,12 +1233,11 @@ void Detector::build_tree(Tree& T, const double* x, bool faces, hipStream_t stre
     PA_LAUNCH_CHECK();
     if (nseg > 0) {
         hipLaunchKernelGGL(k_morton_seg, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, T.prim_box.p, faces ? tris.p : edges.p,
-                           faces ? 3 : 2, n, (const int32_t*)vseg.p, T.scene.p, T.keys.p, T.ids.p, T.cross.p);
+                           faces ? 3 : 2, n, (const int32_t*)vseg.p, T.scene.p, T.keys.p, T.ids.p);
         PA_LAUNCH_CHECK();
         radix_sort_pairs(T.keys.p, T.ids.p, n, 32, scratch, stream);
     } else {
-        hipLaunchKernelGGL(k_morton, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, T.prim_box.p, n, T.scene.p, T.keys.p, T.ids.p,
-                           T.cross.p);
+        hipLaunchKernelGGL(k_morton, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, T.prim_box.p, n, T.scene.p, T.keys.p, T.ids.p);
         PA_LAUNCH_CHECK();
         radix_sort_pairs(T.keys.p, T.ids.p, n, 30, scratch, stream);
     }
@@ -1122,40 +1248,55 @@ void Detector::build_tree(Tree& T, const double* x, bool faces, hipStream_t stre
         hipLaunchKernelGGL(k_leaf_ids<2>, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, (const int32_t*)edges.p, (const uint32_t*)T.ids.p, n,
                            T.leafid.p);
     PA_LAUNCH_CHECK();
-    if (n > 1) {
-        hipLaunchKernelGGL(k_karras, dim3(grid_for(n - 1, BLK)), dim3(BLK), 0, stream, T.keys.p, T.ids.p, n, T.child.p, T.range.p);
+}
+
+// Topology, record slots and segment roots of both trees over their sorted
+// leaves; the boxes follow in refit_trees.
+void Detector::build_topology() {
+    auto args = [](const Tree& T) {
+        return TopoArgs{T.n, T.keys.p, T.ids.p, T.child.p, T.range.p, T.ipos.p, T.lpos.p, T.rec.p};
+    };
+    const TopoArgs E = args(et), F = args(ft);
+    const int eb = et.n > 1 ? grid_for(et.n, BLK) : 0, fb = ft.n > 1 ? grid_for(ft.n, BLK) : 0;
+    if (eb + fb > 0) {
+        hipLaunchKernelGGL(k_karras, dim3(eb + fb), dim3(BLK), 0, stream, E, F, eb);
         PA_LAUNCH_CHECK();
-        fill2<int32_t>(T.ipos.p, n - 1, T.lpos.p, 2 * (int64_t)n, -1, stream);
-        hipLaunchKernelGGL(k_record_slots, dim3(grid_for(n - 1, BLK)), dim3(BLK), 0, stream, n, (const int32_t*)T.child.p,
-                           (const int2*)T.range.p, T.rec.p, T.ipos.p, T.lpos.p, T.cross.p);
+        hipLaunchKernelGGL(k_record_slots, dim3(eb + fb), dim3(BLK), 0, stream, E, F, eb);
         PA_LAUNCH_CHECK();
     }
     if (nseg > 0) {
-        fill<int32_t>(T.seg_first.p, -1, nseg, stream);
-        fill<int32_t>(T.seg_last.p, -1, nseg, stream);
-        fill<int32_t>(T.seg_root.p, -1, nseg, stream);
-        hipLaunchKernelGGL(k_seg_bounds, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, (const uint32_t*)T.keys.p, n, T.seg_first.p,
-                           T.seg_last.p);
-        PA_LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_seg_roots, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, n, (const int2*)T.range.p, (const uint32_t*)T.keys.p,
-                           (const int32_t*)T.seg_first.p, (const int32_t*)T.seg_last.p, T.seg_root.p);
-        PA_LAUNCH_CHECK();
+        segment_roots(et);
+        segment_roots(ft);
     }
+}
+
+void Detector::segment_roots(Tree& T) {
+    const int n = T.n;
+    if (n == 0) return;
+    fill<int32_t>(T.seg_first.p, -1, nseg, stream);
+    fill<int32_t>(T.seg_last.p, -1, nseg, stream);
+    fill<int32_t>(T.seg_root.p, -1, nseg, stream);
+    hipLaunchKernelGGL(k_seg_bounds, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, (const uint32_t*)T.keys.p, n, T.seg_first.p, T.seg_last.p);
+    PA_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_seg_roots, dim3(grid_for(n, BLK)), dim3(BLK), 0, stream, n, (const int2*)T.range.p, (const uint32_t*)T.keys.p,
+                       (const int32_t*)T.seg_first.p, (const int32_t*)T.seg_last.p, T.seg_root.p);
+    PA_LAUNCH_CHECK();
 }
 
 // Boxes of both trees from x.
 void Detector::refit_trees(const double* x) {
     auto args = [](const Tree& T) {
-        return TreeArgs{T.n, T.leafid.p, T.leaf_box.p, (const int2*)T.lpos.p, T.range.p, T.ipos.p, T.blk_box.p, T.cross.p, T.rec.p};
+        return TreeArgs{T.n, T.leafid.p, T.leaf_box.p, (const int2*)T.lpos.p, T.range.p, T.ipos.p, T.blk_box.p, T.rec.p};
     };
     const TreeArgs E = args(et), F = args(ft);
     const int eb = grid_for(et.n, RB), fb = grid_for(ft.n, RB);
     if (eb + fb == 0) return;
     hipLaunchKernelGGL(k_refit, dim3(eb + fb), dim3(RB), 0, stream, E, F, eb, x);
     PA_LAUNCH_CHECK();
-    const int ec = et.n > RB ? std::min(1024, grid_for(et.n, 64)) : 0, fc = ft.n > RB ? std::min(1024, grid_for(ft.n, 64)) : 0;
+    const int per = et.n + ft.n <= CROSS_SMALL ? 16 : 64, block = per * (BLK / 64); // nodes per wave and per block
+    const int ec = et.n > RB ? grid_for(et.n, block) : 0, fc = ft.n > RB ? grid_for(ft.n, block) : 0;
     if (ec + fc == 0) return;
-    hipLaunchKernelGGL(k_cross_boxes, dim3(ec + fc), dim3(BLK), 0, stream, E, F, ec);
+    hipLaunchKernelGGL(k_cross_boxes, dim3(ec + fc), dim3(BLK), 0, stream, E, F, ec, per);
     PA_LAUNCH_CHECK();
 }
 
@@ -1184,13 +1325,21 @@ void Detector::set_segments(const int32_t* vs, int count) {
 int Detector::detect(const double* x, bool refit, VertexCount vc) {
     refit = refit && built;
     fill2<uint32_t>(counts.p, (int64_t)counts.n, vc.cnt, vc.cnt ? vc.n : 0, 0u, stream);
-    if (!refit) { // the edge tree is built on the side stream beside the triangle tree
-        PA_HIP(hipEventRecord(ev_fork, stream));
-        PA_HIP(hipStreamWaitEvent(side, ev_fork, 0));
-        build_tree(et, x, false, side, scratch_side);
-        build_tree(ft, x, true, stream, scratch);
-        PA_HIP(hipEventRecord(ev_join, side));
-        PA_HIP(hipStreamWaitEvent(stream, ev_join, 0));
+    if (!refit) {
+        if (std::max(et.n, ft.n) <= SMALL_BUILD) {
+            const SmallTree E{edges.p, 2, et.n, et.keys.p, et.ids.p, et.leafid.p};
+            const SmallTree F{tris.p, 3, ft.n, ft.keys.p, ft.ids.p, ft.leafid.p};
+            hipLaunchKernelGGL(k_build_small, dim3(2), dim3(SB_BLK), 0, stream, x, nseg > 0 ? (const int32_t*)vseg.p : nullptr, E, F);
+            PA_LAUNCH_CHECK();
+        } else { // the edge tree is sorted on the side stream beside the triangle tree
+            PA_HIP(hipEventRecord(ev_fork, stream));
+            PA_HIP(hipStreamWaitEvent(side, ev_fork, 0));
+            sort_leaves(et, x, false, side, scratch_side);
+            sort_leaves(ft, x, true, stream, scratch);
+            PA_HIP(hipEventRecord(ev_join, side));
+            PA_HIP(hipStreamWaitEvent(stream, ev_join, 0));
+        }
+        build_topology();
         built = true;
     }
     refit_trees(x); // a refit keeps the sorted order and the Karras topology

@@ -31,6 +31,25 @@ template <class T> inline void fill2(T* p, int64_t n, T* q, int64_t m, T v, hipS
     PA_LAUNCH_CHECK();
 }
 
+// Rank of this lane's 8-bit digit d among the wave's equal digits of this and
+// earlier calls (cnt: the wave's digit counts in LDS, updated); lanes with
+// valid = false take no part.
+__device__ inline uint32_t rs_rank(uint32_t d, bool valid, uint32_t* cnt) {
+    unsigned long long match = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < 8; b++) {
+        const bool bit = (d >> b) & 1u;
+        const unsigned long long m = __ballot(bit);
+        match &= bit ? m : ~m;
+    }
+    const uint32_t before = __builtin_amdgcn_mbcnt_hi((unsigned)(match >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)match, 0u));
+    const uint32_t start = valid ? cnt[d] : 0u;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // every lane reads before the first of its digit adds
+    if (valid && before == 0) cnt[d] = start + (uint32_t)__popcll(match);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    return start + before;
+}
+
 // Scratch for scan/sort; grown on demand.
 struct PrimScratch {
     DBuf<uint32_t> sums, hist, keys_alt, vals_alt;
