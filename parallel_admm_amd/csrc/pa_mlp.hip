@@ -1,15 +1,16 @@
 // MLP forward, backward and Adam on MFMA (gfx950, v_mfma_f32_16x16x32_bf16).
 //
-// Every product is one "NT" GEMM, C[M][N] = sum_k A[m][k] Bt[n][k], with both
-// operands BF16 and K contiguous, FP32 accumulation, one 16x16 output tile per
-// wave and a fused epilogue:
-//   forward hidden  a = C + b, H = SiLU(a) (also H^T and SiLU'(a) when training)
+// A pass is one launch (inference) or three (a training step): k_mlp takes 32
+// rows per workgroup through the whole network and back, k_weight_grads forms
+// every weight gradient, k_reduce sums its splits and takes the Adam step.
+// Every product is an "NT" one, C[M][N] = sum_k A[m][k] Bt[n][k], with both
+// operands BF16 and K contiguous, FP32 accumulation and 16x16 output tiles:
+//   forward hidden  a = C + b, H = SiLU(a) (H^T and SiLU'(a) when training)
 //   forward output  y = C + b, dY = (y - t) / n, loss partials
 //   backward        dA = C * SiLU'(a)  (and dA^T)
 //   weight grads    split-K partials of dA^T H (bias gradient via a ones row)
-// Activations are kept in both layouts so that each product reads K-contiguous
-// 16-byte fragments.  Partial weight gradients are summed in a fixed order, so
-// a training run is bit-reproducible.
+// Partial weight gradients are summed in a fixed order, so a training run is
+// bit-reproducible.
 #include "pa_mlp.hpp"
 
 #include <algorithm>
@@ -28,124 +29,226 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __device__ inline uint16_t to_bf16(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 
-enum { EPI_SILU = 0, EPI_OUT = 1, EPI_BWD = 2, EPI_PART = 3 };
+__device__ inline bf16x8 frag(const uint16_t* p) { return *reinterpret_cast<const bf16x8*>(p); }
+// Four BF16 values of consecutive rows of one column into a transposed array.
+__device__ inline void put4(uint16_t* p, const uint16_t (&v)[4]) {
+    *reinterpret_cast<uint2*>(p) = make_uint2((uint32_t)v[0] | (uint32_t)v[1] << 16, (uint32_t)v[2] | (uint32_t)v[3] << 16);
+}
 
-struct GemmArgs {
-    const uint16_t* A;
-    int lda;
-    const uint16_t* Bt;
-    int ldb;
-    int M, N, K, splits;
-    int train, n_real;
-    float inv_n;
-    const float* bias;
-    uint16_t* out;
-    int ldo;
-    uint16_t* outT;
-    int ldoT;
-    float* outS;
-    const float* inS;
-    int ldS;
-    float* outF;
-    const float* T;
+struct MlpArgs {
+    const float* src; // rows of `stride` floats: features, then 2 targets when training; via idx when given
+    int stride;
+    const int32_t* idx;
+    int n, cap; // real rows; leading dimension of the transposed arrays
+    const uint16_t *W1p, *W2, *W3, *W4p, *W2T, *W3T, *W4T;
+    const float* w; // FP32 parameters (biases)
+    float* Y;       // [rows][2]
+    // training only
+    uint16_t *XT, *H1T, *H2T, *H3T, *dYT, *dA1T, *dA2T, *dA3T;
     double* loss_part;
+    float inv_n;
 };
 
-// One 16x16 tile per wave; wave -> (split, tile m, tile n), n fastest.
+// 32 rows through the network, and with TRAIN back.  A layer over 8192 rows is
+// 0.27 GFLOP, under a microsecond of MFMA, so as launches of their own (12 of
+// 5-9 us in a training step) the layers cost only their latency; here
+// activations pass from layer to layer through LDS and SiLU' stays in
+// registers.  Wave w owns columns 32 w .. 32 w + 31 of every hidden layer in
+// both directions (2 x 2 tiles), so the SiLU' of its forward tiles is where its
+// backward tiles need it.  A layer's weight fragments come straight from L2,
+// one layer ahead of their use.
 // Fragment layout of the 16x16x32 product: lane l holds row (l % 16) of A and
 // column (l % 16) of B at k = 8 (l / 16) .. +7; the accumulator of lane l
 // holds column l % 16, rows 4 (l / 16) .. +3.
-template <int EPI> __global__ void __launch_bounds__(256) k_gemm_nt(GemmArgs g) {
-    const int lane = threadIdx.x & 63;
-    const int wave = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int tn_count = g.N >> 4, tiles = (g.M >> 4) * tn_count;
-    if (wave >= tiles * g.splits) return;
-    const int split = wave / tiles;
-    const int t = wave - split * tiles;
-    const int tm = t / tn_count, tn = t - tm * tn_count;
-    const int per = (g.K >> 5) / g.splits;
-    const int k0 = split * per * 32, k1 = k0 + per * 32;
-    const int r16 = lane & 15, kq = (lane >> 4) * 8;
-    const uint16_t* pa = g.A + (size_t)(tm * 16 + r16) * g.lda + kq;
-    const uint16_t* pb = g.Bt + (size_t)(tn * 16 + r16) * g.ldb + kq;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int k = k0; k < k1; k += 32) {
-        const bf16x8 a = *(const bf16x8*)(pa + k);
-        const bf16x8 b = *(const bf16x8*)(pb + k);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
+// Training step of 8192 rows: 15.4 us for this and 14.2 us for the weight
+// gradients, against 64 and 33 us as one launch per product.
+constexpr int FR = 32;         // rows per workgroup
+constexpr int AST = H + 8;     // LDS row strides (BF16): 16-byte aligned rows on rotating banks
+constexpr int XST = INP + 8;
+template <bool TRAIN> __global__ void __launch_bounds__(256) k_mlp(MlpArgs g) {
+    __shared__ __align__(16) uint16_t act[2][FR * AST];
+    __shared__ __align__(16) uint16_t xin[FR * XST]; // the input, then dY
+    __shared__ float tgt[FR][OUT];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, r16 = lane & 15, kq = (lane >> 4) * 8, rq = (lane >> 4) * 4;
+    const int tiles = gridDim.x, tile = tiles % 8 ? blockIdx.x : (blockIdx.x % 8) * (tiles / 8) + blockIdx.x / 8; // an XCD's tiles adjoin
+    const int row0 = tile * FR;
+    const int col[2] = {32 * wave + r16, 32 * wave + 16 + r16};
+    // the input rows (BF16, zero padded) and the targets
+    for (int e = t; e < FR * INP; e += 256) {
+        const int s = e / INP, k = e % INP, r = row0 + s;
+        float v = 0.f;
+        if (r < g.n && k < IN) v = g.src[(size_t)(g.idx ? g.idx[r] : r) * g.stride + k];
+        xin[s * XST + k] = to_bf16(v);
     }
-    const int col = tn * 16 + r16;
-    const int row0 = tm * 16 + (lane >> 4) * 4;
-    if (EPI == EPI_PART) {
-        float* o = g.outF + ((size_t)split * g.M + row0) * g.N + col;
+    if (TRAIN && t < FR * OUT) {
+        const int s = t / OUT, r = row0 + s;
+        tgt[s][t % OUT] = r < g.n ? g.src[(size_t)(g.idx ? g.idx[r] : r) * g.stride + IN + t % OUT] : 0.f;
+    }
+    bf16x8 w[2][4], wn[2][4];
+    auto load = [&](bf16x8(&o)[2][4], const uint16_t* W, int ld, int steps) {
 #pragma unroll
-        for (int r = 0; r < 4; r++) o[(size_t)r * g.N] = acc[r];
-    } else if (EPI == EPI_SILU) {
-        const float bc = g.bias[col];
+        for (int c = 0; c < 2; c++)
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int row = row0 + r;
-            const float a = acc[r] + bc;
-            const float sg = 1.f / (1.f + __expf(-a));
-            const uint16_t hb = to_bf16(a * sg);
-            g.out[(size_t)row * g.ldo + col] = hb;
-            if (g.train) {
-                g.outT[(size_t)col * g.ldoT + row] = hb;
-                g.outS[(size_t)row * g.ldS + col] = sg * (1.f + a * (1.f - sg));
+            for (int k = 0; k < 4; k++)
+                if (k < steps) o[c][k] = frag(W + (size_t)col[c] * ld + 32 * k + kq);
+    };
+    f32x4 acc[2][2]; // [row tile][column tile]
+    auto product = [&](const bf16x8(&b)[2][4], const uint16_t* A, int st, int steps) {
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int c = 0; c < 2; c++) acc[m][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (k < steps)
+#pragma unroll
+                for (int m = 0; m < 2; m++) {
+                    const bf16x8 a = frag(A + (16 * m + r16) * st + 32 * k + kq);
+#pragma unroll
+                    for (int c = 0; c < 2; c++) acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[c][k], acc[m][c], 0, 0, 0);
+                }
+    };
+    float S[3][2][2][4]; // SiLU' of the wave's tiles
+    auto silu = [&](int l, const float* bias, uint16_t* out, uint16_t* outT) {
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const float bc = bias[col[c]];
+#pragma unroll
+            for (int m = 0; m < 2; m++) {
+                uint16_t hb[4];
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const float a = acc[m][c][r] + bc;
+                    const float sg = 1.f / (1.f + __expf(-a));
+                    hb[r] = to_bf16(a * sg);
+                    out[(16 * m + rq + r) * AST + col[c]] = hb[r];
+                    if (TRAIN) S[l][m][c][r] = sg * (1.f + a * (1.f - sg));
+                }
+                if (TRAIN) put4(outT + (size_t)col[c] * g.cap + row0 + 16 * m + rq, hb);
             }
         }
-    } else if (EPI == EPI_BWD) {
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int row = row0 + r;
-            const uint16_t vb = to_bf16(acc[r] * g.inS[(size_t)row * g.ldS + col]);
-            g.out[(size_t)row * g.ldo + col] = vb;
-            g.outT[(size_t)col * g.ldoT + row] = vb;
+    };
+    load(w, g.W1p, INP, 1);
+    load(wn, g.W2, H, 4);
+    __syncthreads();
+    if (TRAIN)
+        for (int e = t; e < INA * FR; e += 256) { // X^T, row 10 = 1 on real rows
+            const int k = e / FR, s = e % FR;
+            g.XT[(size_t)k * g.cap + row0 + s] = k < IN ? xin[s * XST + k] : to_bf16(k == IN && row0 + s < g.n ? 1.f : 0.f);
         }
-    } else { // EPI_OUT
+    product(w, xin, XST, 1);
+    silu(0, g.w + OB1, act[0], g.H1T);
+    load(w, g.W3, H, 4);
+    __syncthreads();
+    product(wn, act[0], AST, 4);
+    silu(1, g.w + OB2, act[1], g.H2T);
+    if (TRAIN) load(wn, g.W4T, OUTK, 1);
+    bf16x8 w4[4]; // output layer: wave m < 2 takes row tile m
+#pragma unroll
+    for (int k = 0; k < 4; k++) w4[k] = frag(g.W4p + (size_t)r16 * H + 32 * k + kq);
+    __syncthreads();
+    product(w, act[1], AST, 4);
+    silu(2, g.w + OB3, act[0], g.H3T);
+    if (TRAIN) {
+        load(w, g.W3T, H, 4);
+        for (int e = t; e < FR * XST; e += 256) xin[e] = 0; // becomes dY: its last reader passed two barriers ago
+    }
+    __syncthreads();
+    if (wave < 2) {
+        f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < 4; k++) o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(act[0] + (16 * wave + r16) * AST + 32 * k + kq), w4[k], o, 0, 0, 0);
         double l = 0.0;
-        if (col < OUT) {
-            const float bc = g.bias[col];
+        if (r16 < OUT) {
+            const float bc = g.w[OB4 + r16];
+            uint16_t eb[4];
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int row = row0 + r;
-                const float y = acc[r] + bc;
-                g.outF[(size_t)row * OUT + col] = y;
-                if (g.train) {
-                    const float e = row < g.n_real ? y - g.T[(size_t)row * OUT + col] : 0.f;
+                const int s = 16 * wave + rq + r, row = row0 + s;
+                const float y = o[r] + bc;
+                g.Y[(size_t)row * OUT + r16] = y;
+                if (TRAIN) {
+                    const float e = row < g.n ? y - tgt[s][r16] : 0.f;
                     l += (double)e * (double)e;
-                    const uint16_t eb = to_bf16(e * g.inv_n);
-                    g.out[(size_t)row * g.ldo + col] = eb;
-                    g.outT[(size_t)col * g.ldoT + row] = eb;
+                    eb[r] = to_bf16(e * g.inv_n);
+                    xin[s * XST + r16] = eb[r];
                 }
             }
+            if (TRAIN) put4(g.dYT + (size_t)r16 * g.cap + row0 + 16 * wave + rq, eb);
         }
-        if (g.train) {
-            for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
-            if (lane == 0) g.loss_part[tm] = l;
+        if (TRAIN) {
+            for (int q = 32; q > 0; q >>= 1) l += __shfl_xor(l, q);
+            if (lane == 0) g.loss_part[2 * tile + wave] = l;
         }
+    }
+    if constexpr (TRAIN) {
+        auto back = [&](int l, uint16_t* out, uint16_t* outT) {
+#pragma unroll
+            for (int c = 0; c < 2; c++)
+#pragma unroll
+                for (int m = 0; m < 2; m++) {
+                    uint16_t vb[4];
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        vb[r] = to_bf16(acc[m][c][r] * S[l][m][c][r]);
+                        if (out) out[(16 * m + rq + r) * AST + col[c]] = vb[r];
+                    }
+                    put4(outT + (size_t)col[c] * g.cap + row0 + 16 * m + rq, vb);
+                }
+        };
+        __syncthreads();
+        product(wn, xin, XST, 1);
+        back(2, act[1], g.dA3T);
+        load(wn, g.W2T, H, 4);
+        __syncthreads();
+        product(w, act[1], AST, 4);
+        back(1, act[0], g.dA2T);
+        __syncthreads();
+        product(wn, act[0], AST, 4);
+        back(0, nullptr, g.dA1T);
     }
 }
 
-// Rows s < n of src (stride floats apart, via idx when given) into X
-// [rows][32] and X^T [16][cap] (row 10 = 1); padded rows are zero.
-__global__ void k_pack(const float* __restrict__ src, int stride, const int32_t* __restrict__ idx, int n, int rows, int cap, int targets,
-                       uint16_t* __restrict__ X, uint16_t* __restrict__ XT, float* __restrict__ T) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= rows) return;
-    const float* f = s < n ? src + (size_t)(idx ? idx[s] : s) * stride : nullptr;
+// Every weight gradient in one launch: split-K partials of dA^T H, one 16x16
+// tile and split per wave.  A layer's tiles start at first[l]; a wave's
+// fragments of eight K steps are in flight at once (as four launches of one
+// step at a time they took 33 us, now 14.2).  Workgroups of a split share an XCD, so
+// an L2 reads one eighth of the 7 MB that k_mlp left, mostly rows written there.
+struct GradArgs {
+    const uint16_t* A[4];
+    const uint16_t* Bt[4];
+    float* out[4];
+    int M[4], N[4], first[5];
+    int splits, per, cap; // K steps (32 rows) per split
+};
+__global__ void __launch_bounds__(256) k_weight_grads(GradArgs g) {
+    const int lane = threadIdx.x & 63;
+    const int s8 = min(g.splits, 8), ns = g.splits / s8; // splits are powers of two up to 16
+    const int split = (blockIdx.x % s8) * ns + (blockIdx.x / s8) % ns, t = (blockIdx.x / g.splits) * 4 + (threadIdx.x >> 6);
+    if (t >= g.first[4]) return;
+    int l = 0;
+    while (t >= g.first[l + 1]) l++;
+    const int tn_count = g.N[l] >> 4, q = t - g.first[l], tm = q / tn_count, tn = q - tm * tn_count;
+    const int r16 = lane & 15, kq = (lane >> 4) * 8;
+    const size_t k0 = (size_t)split * g.per * 32 + kq;
+    const uint16_t* pa = g.A[l] + (size_t)(tm * 16 + r16) * g.cap + k0;
+    const uint16_t* pb = g.Bt[l] + (size_t)(tn * 16 + r16) * g.cap + k0;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < g.per; s += 8) {
+        bf16x8 a[8], b[8];
 #pragma unroll
-    for (int k = 0; k < INP; k++) X[(size_t)s * INP + k] = (f && k < IN) ? to_bf16(f[k]) : (uint16_t)0;
+        for (int u = 0; u < 8; u++) {
+            const size_t k = 32 * (size_t)min(s + u, g.per - 1);
+            a[u] = frag(pa + k);
+            b[u] = frag(pb + k);
+        }
 #pragma unroll
-    for (int k = 0; k < INA; k++) {
-        float v = 0.f;
-        if (f) v = k < IN ? f[k] : (k == IN ? 1.f : 0.f);
-        XT[(size_t)k * cap + s] = to_bf16(v);
+        for (int u = 0; u < 8; u++)
+            if (s + u < g.per) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b[u], acc, 0, 0, 0);
     }
-    if (targets) {
-        T[2 * (size_t)s] = f ? f[IN] : 0.f;
-        T[2 * (size_t)s + 1] = f ? f[IN + 1] : 0.f;
-    }
+    float* o = g.out[l] + ((size_t)split * g.M[l] + tm * 16 + (lane >> 4) * 4) * g.N[l] + tn * 16 + r16;
+#pragma unroll
+    for (int r = 0; r < 4; r++) o[(size_t)r * g.N[l]] = acc[r];
 }
 
 struct Copies {
@@ -212,7 +315,14 @@ __global__ void k_reduce(int mode, int splits, const float* __restrict__ part, i
         else r = p - OB4, k = H;
     }
     float gsum = 0.f;
-    for (int s = 0; s < splits; s++) gsum += base[((size_t)s * rows + r) * cols + k];
+    for (int s = 0; s < splits; s += 8) { // at most 16 splits, eight loads in flight
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = base[((size_t)min(s + u, splits - 1) * rows + r) * cols + k];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (s + u < splits) gsum += v[u];
+    }
     if (mode == 0) {
         grad[p] = gsum;
         return;
@@ -237,39 +347,19 @@ __global__ void k_ones_rows(int cap, uint16_t* __restrict__ a, uint16_t* __restr
     c[(size_t)H * cap + s] = one;
 }
 
-template <int EPI> void launch(const GemmArgs& a, hipStream_t s) {
-    PA_CHECK(a.M % 16 == 0 && a.N % 16 == 0 && a.K % 32 == 0 && a.splits >= 1 && (a.K / 32) % a.splits == 0, PA_ERR_INVALID,
-             "mlp: product shape not tiled");
-    const int waves = (a.M / 16) * (a.N / 16) * a.splits;
-    hipLaunchKernelGGL(k_gemm_nt<EPI>, dim3((waves + 3) / 4), dim3(256), 0, s, a);
-    PA_LAUNCH_CHECK();
-}
-
 // ---------------------------------------------------------------------------
 // Scratch of the forward pass that allocates nothing (pa_mlp_forward_noalloc):
-// one file-scope device array per GPU, laid out for kNoAllocRows padded rows
-// (each region starts on a 256-byte boundary):
-//   staged input  float [rows][10]
-//   X             bf16  [rows][32]
-//   X^T           bf16  [16][rows]   (written by the packing kernel, unused by inference)
-//   H1, H2, H3    bf16  [rows][128]
-//   Y             float [rows][2]
-// Every byte a call reads is written earlier in the same call, so nothing is
-// cleared between calls.  Calls that overlap on one GPU share the array and
-// race; calls on different GPUs use each GPU's own copy.
+// one file-scope device array per GPU of the size that the C ABI states, holding
+// the staged input (float [rows][10]) and the output (float [rows][2]) of up to
+// kNoAllocRows padded rows; activations stay on chip.  Every byte a call reads
+// is written earlier in the same call, so nothing is cleared between calls.
+// Calls that overlap on one GPU share the array and race; calls on different
+// GPUs use each GPU's own copy.
 // ---------------------------------------------------------------------------
-constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
-constexpr size_t kSxIn = 0;
-constexpr size_t kSx = kSxIn + align256((size_t)kNoAllocRows * IN * sizeof(float));
-constexpr size_t kSxT = kSx + align256((size_t)kNoAllocRows * INP * sizeof(uint16_t));
-constexpr size_t kSh1 = kSxT + align256((size_t)INA * kNoAllocRows * sizeof(uint16_t));
-constexpr size_t kSh2 = kSh1 + align256((size_t)kNoAllocRows * H * sizeof(uint16_t));
-constexpr size_t kSh3 = kSh2 + align256((size_t)kNoAllocRows * H * sizeof(uint16_t));
-constexpr size_t kSy = kSh3 + align256((size_t)kNoAllocRows * H * sizeof(uint16_t));
-constexpr size_t kScratchBytes = kSy + align256((size_t)kNoAllocRows * OUT * sizeof(float));
-static_assert(kScratchBytes == kNoAllocScratchBytes, "scratch layout and its stated size differ");
+constexpr size_t kSy = (size_t)kNoAllocRows * IN * sizeof(float);
+static_assert(kSy % 256 == 0 && kSy + (size_t)kNoAllocRows * OUT * sizeof(float) <= kNoAllocScratchBytes, "scratch too small");
 
-__device__ __align__(256) unsigned char scratch[kScratchBytes];
+__device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 // Device address of `scratch` on each device, resolved once per device with
 // that device current (the array's name in host code is only a stand-in).
@@ -363,178 +453,68 @@ void Mlp::ensure(int rows) {
     if (rows <= cap) return;
     cap = rows;
     const size_t c = (size_t)cap;
-    X.alloc(c * INP);
     XT.alloc(c * INA);
-    for (DBuf<uint16_t>* b : {&H1, &H2, &H3, &dA1, &dA2, &dA3}) b->alloc(c * H);
     for (DBuf<uint16_t>* b : {&H1T, &H2T, &H3T}) b->alloc(c * HA);
     for (DBuf<uint16_t>* b : {&dA1T, &dA2T, &dA3T}) b->alloc(c * H);
-    dY.alloc(c * OUTK);
     dYT.alloc(c * OUTP);
-    for (DBuf<float>* b : {&S1, &S2, &S3}) b->alloc(c * H);
     Y.alloc(c * OUT);
-    T.alloc(c * OUT);
-    loss_part.alloc(c / 16);
     part.alloc((size_t)16 * (2 * H * HA + H * INA + OUTP * HA)); // up to 16 splits
-    for (DBuf<uint16_t>* b : {&H1T, &H2T, &H3T, &dY, &dYT}) b->zero(stream);
+    for (DBuf<uint16_t>* b : {&H1T, &H2T, &H3T, &dYT}) b->zero(stream);
     hipLaunchKernelGGL(k_ones_rows, dim3(grid_for(cap, 256)), dim3(256), 0, stream, cap, H1T.p, H2T.p, H3T.p);
     PA_LAUNCH_CHECK();
     PA_HIP(hipStreamSynchronize(stream));
 }
 
-void Mlp::pack(const float* src, int stride, const int32_t* idx, int n, int rows, bool targets) {
-    ensure(rows);
-    PA_CHECK(n >= 0 && n <= rows, PA_ERR_INVALID, "mlp: more samples than rows");
-    hipLaunchKernelGGL(k_pack, dim3(grid_for(rows, 256)), dim3(256), 0, stream, src, stride, idx, n, rows, cap, targets ? 1 : 0, X.p, XT.p,
-                       T.p);
+static MlpArgs mlp_args(const Mlp& m, const float* src, int stride, const int32_t* idx, int n, float* y) {
+    MlpArgs g{};
+    g.src = src;
+    g.stride = stride;
+    g.idx = idx;
+    g.n = n;
+    g.W1p = m.W1p.p;
+    g.W2 = m.W2.p;
+    g.W3 = m.W3.p;
+    g.W4p = m.W4p.p;
+    g.w = m.w.p;
+    g.Y = y;
+    return g;
+}
+
+void Mlp::infer(const float* src, int stride, int n, int rows, float* y) {
+    PA_CHECK(rows > 0 && rows % FR == 0 && n >= 0 && n <= rows, PA_ERR_INVALID, "mlp: bad forward shape");
+    hipLaunchKernelGGL(k_mlp<false>, dim3(rows / FR), dim3(256), 0, stream, mlp_args(*this, src, stride, nullptr, n, y));
     PA_LAUNCH_CHECK();
 }
 
-// Inference over `rows` padded rows from the packed input X ([rows][32]):
-// three SiLU layers into H1..H3 ([rows][128]) and the output layer into Y
-// ([rows][2]).  The buffers are the handle's or the allocation-free scratch.
-void Mlp::infer(int rows, const uint16_t* Xin, uint16_t* h1, uint16_t* h2, uint16_t* h3, float* y) {
-    PA_CHECK(rows > 0 && rows % 32 == 0, PA_ERR_INVALID, "mlp: bad forward shape");
-    GemmArgs a{};
-    a.M = rows;
-    a.splits = 1;
-    a.train = 0;
-    const uint16_t* in[3] = {Xin, h1, h2};
-    const uint16_t* wt[3] = {W1p.p, W2.p, W3.p};
-    uint16_t* out[3] = {h1, h2, h3};
-    const int bias[3] = {OB1, OB2, OB3};
-    for (int l = 0; l < 3; l++) {
-        a.A = in[l];
-        a.lda = l == 0 ? INP : H;
-        a.Bt = wt[l];
-        a.ldb = l == 0 ? INP : H;
-        a.N = H;
-        a.K = l == 0 ? INP : H;
-        a.bias = w.p + bias[l];
-        a.out = out[l];
-        a.ldo = H;
-        launch<EPI_SILU>(a, stream);
-    }
-    GemmArgs o{};
-    o.M = rows;
-    o.splits = 1;
-    o.train = 0;
-    o.A = h3;
-    o.lda = H;
-    o.Bt = W4p.p;
-    o.ldb = H;
-    o.N = OUTP;
-    o.K = H;
-    o.bias = w.p + OB4;
-    o.outF = y;
-    launch<EPI_OUT>(o, stream);
-}
-
-void Mlp::forward(int n, int rows, bool train) {
-    PA_CHECK(rows <= cap && rows % 32 == 0 && n <= rows, PA_ERR_INVALID, "mlp: bad forward shape");
-    if (!train) {
-        infer(rows, X.p, H1.p, H2.p, H3.p, Y.p);
-        return;
-    }
-    GemmArgs a{};
-    a.M = rows;
-    a.splits = 1;
-    a.train = train ? 1 : 0;
-    a.ldoT = cap;
-    a.ldS = H;
-    const uint16_t* in[3] = {X.p, H1.p, H2.p};
-    const uint16_t* wt[3] = {W1p.p, W2.p, W3.p};
-    uint16_t* out[3] = {H1.p, H2.p, H3.p};
-    uint16_t* outT[3] = {H1T.p, H2T.p, H3T.p};
-    float* outS[3] = {S1.p, S2.p, S3.p};
-    const int bias[3] = {OB1, OB2, OB3};
-    for (int l = 0; l < 3; l++) {
-        a.A = in[l];
-        a.lda = l == 0 ? INP : H;
-        a.Bt = wt[l];
-        a.ldb = l == 0 ? INP : H;
-        a.N = H;
-        a.K = l == 0 ? INP : H;
-        a.bias = w.p + bias[l];
-        a.out = out[l];
-        a.ldo = H;
-        a.outT = outT[l];
-        a.outS = outS[l];
-        launch<EPI_SILU>(a, stream);
-    }
-    a.A = H3.p;
-    a.lda = H;
-    a.Bt = W4p.p;
-    a.ldb = H;
-    a.N = OUTP;
-    a.K = H;
-    a.bias = w.p + OB4;
-    a.outF = Y.p;
-    a.T = T.p;
-    a.out = dY.p;
-    a.ldo = OUTK;
-    a.outT = dYT.p;
-    a.n_real = n;
+void Mlp::train_pass(const float* src, int stride, const int32_t* idx, int n, int rows, double* loss_out) {
+    PA_CHECK(rows > 0 && rows <= cap && rows % FR == 0 && n >= 0 && n <= rows, PA_ERR_INVALID, "mlp: bad training shape");
+    MlpArgs a = mlp_args(*this, src, stride, idx, n, Y.p);
+    a.cap = cap;
+    a.W2T = W2T.p;
+    a.W3T = W3T.p;
+    a.W4T = W4T.p;
+    a.XT = XT.p;
+    a.H1T = H1T.p;
+    a.H2T = H2T.p;
+    a.H3T = H3T.p;
+    a.dYT = dYT.p;
+    a.dA1T = dA1T.p;
+    a.dA2T = dA2T.p;
+    a.dA3T = dA3T.p;
+    a.loss_part = loss_out;
     a.inv_n = n > 0 ? 1.f / (float)n : 0.f;
-    a.loss_part = loss_part.p;
-    launch<EPI_OUT>(a, stream);
-}
-
-void Mlp::backward(int rows) {
-    GemmArgs a{};
-    a.M = rows;
-    a.splits = 1;
-    a.train = 1;
-    a.ldoT = cap;
-    a.ldS = H;
-    const uint16_t* in[3] = {dY.p, dA3.p, dA2.p};
-    const uint16_t* wt[3] = {W4T.p, W3T.p, W2T.p};
-    const float* inS[3] = {S3.p, S2.p, S1.p};
-    uint16_t* out[3] = {dA3.p, dA2.p, dA1.p};
-    uint16_t* outT[3] = {dA3T.p, dA2T.p, dA1T.p};
-    for (int l = 0; l < 3; l++) {
-        a.A = in[l];
-        a.lda = l == 0 ? OUTK : H;
-        a.Bt = wt[l];
-        a.ldb = l == 0 ? OUTK : H;
-        a.N = H;
-        a.K = l == 0 ? OUTK : H;
-        a.inS = inS[l];
-        a.out = out[l];
-        a.ldo = H;
-        a.outT = outT[l];
-        launch<EPI_BWD>(a, stream);
-    }
-    int slabs = rows / 32;
+    hipLaunchKernelGGL(k_mlp<true>, dim3(rows / FR), dim3(256), 0, stream, a);
+    PA_LAUNCH_CHECK();
+    const int slabs = rows / 32;
     splits = 16;
     while (slabs % splits) splits /= 2;
     const int64_t off2 = (int64_t)splits * H * INA, off3 = off2 + (int64_t)splits * H * HA, off4 = off3 + (int64_t)splits * H * HA;
-    GemmArgs g{};
-    g.K = rows;
-    g.splits = splits;
-    g.lda = cap;
-    g.ldb = cap;
-    // layer 4: dW4 = dY^T H3
-    g.A = dYT.p;
-    g.Bt = H3T.p;
-    g.M = OUTP;
-    g.N = HA;
-    g.outF = part.p + off4;
-    launch<EPI_PART>(g, stream);
-    g.A = dA3T.p;
-    g.Bt = H2T.p;
-    g.M = H;
-    g.N = HA;
-    g.outF = part.p + off3;
-    launch<EPI_PART>(g, stream);
-    g.A = dA2T.p;
-    g.Bt = H1T.p;
-    g.outF = part.p + off2;
-    launch<EPI_PART>(g, stream);
-    g.A = dA1T.p;
-    g.Bt = XT.p;
-    g.N = INA;
-    g.outF = part.p;
-    launch<EPI_PART>(g, stream);
+    // layers 4 to 1: dW4 = dY^T H3, dW3 = dA3^T H2, dW2 = dA2^T H1, dW1 = dA1^T X
+    GradArgs g{{dYT.p, dA3T.p, dA2T.p, dA1T.p}, {H3T.p, H2T.p, H1T.p, XT.p}, {part.p + off4, part.p + off3, part.p + off2, part.p},
+               {OUTP, H, H, H}, {HA, HA, HA, INA}, {0, 0, 0, 0, 0}, splits, slabs / splits, cap};
+    for (int l = 0; l < 4; l++) g.first[l + 1] = g.first[l] + (g.M[l] / 16) * (g.N[l] / 16);
+    hipLaunchKernelGGL(k_weight_grads, dim3((g.first[4] + 3) / 4 * splits), dim3(256), 0, stream, g);
+    PA_LAUNCH_CHECK();
 }
 
 void Mlp::reduce(int mode, float lr) {
@@ -551,6 +531,7 @@ void Mlp::reduce(int mode, float lr) {
     PA_LAUNCH_CHECK();
 }
 
+// Sum of the loss partials of `rows` rows, in row order.
 double Mlp::loss(int rows) {
     std::vector<double> h(rows / 16);
     loss_part.download(h.data(), h.size(), stream);
@@ -566,13 +547,12 @@ void Mlp::forward_host(const float* x, int n, float* y) {
     ensure(rows);
     samples.reserve((size_t)n * IN);
     samples.upload(x, (size_t)n * IN, stream);
-    pack(samples.p, IN, nullptr, n, rows, false);
-    forward(n, rows, false);
+    infer(samples.p, IN, n, rows, Y.p);
     Y.download(y, (size_t)n * OUT, stream);
     PA_HIP(hipStreamSynchronize(stream));
 }
 
-// The same forward as forward_host with every intermediate in the file-scope
+// The same forward as forward_host with input and output in the file-scope
 // scratch array: no device memory is allocated or freed.
 void Mlp::forward_noalloc(const float* x, int n, float* y) {
     PA_CHECK(n > 0, PA_ERR_INVALID, "mlp: no rows");
@@ -580,19 +560,10 @@ void Mlp::forward_noalloc(const float* x, int n, float* y) {
              "mlp: the allocation-free forward takes at most " + std::to_string(kNoAllocRows) + " rows per call");
     const int rows = pad_rows(n);
     unsigned char* base = static_cast<unsigned char*>(scratch_address());
-    float* xin = reinterpret_cast<float*>(base + kSxIn);
-    uint16_t* xp = reinterpret_cast<uint16_t*>(base + kSx);
-    uint16_t* xt = reinterpret_cast<uint16_t*>(base + kSxT);
-    uint16_t* h1 = reinterpret_cast<uint16_t*>(base + kSh1);
-    uint16_t* h2 = reinterpret_cast<uint16_t*>(base + kSh2);
-    uint16_t* h3 = reinterpret_cast<uint16_t*>(base + kSh3);
+    float* xin = reinterpret_cast<float*>(base);
     float* yo = reinterpret_cast<float*>(base + kSy);
     PA_HIP(hipMemcpyAsync(xin, x, sizeof(float) * (size_t)n * IN, hipMemcpyHostToDevice, stream));
-    // X^T's leading dimension is this call's padded row count (<= kNoAllocRows)
-    hipLaunchKernelGGL(k_pack, dim3(grid_for(rows, 256)), dim3(256), 0, stream, (const float*)xin, IN, (const int32_t*)nullptr, n, rows,
-                       rows, 0, xp, xt, (float*)nullptr);
-    PA_LAUNCH_CHECK();
-    infer(rows, xp, h1, h2, h3, yo);
+    infer(xin, IN, n, rows, yo);
     PA_HIP(hipMemcpyAsync(y, yo, sizeof(float) * (size_t)n * OUT, hipMemcpyDeviceToHost, stream));
     PA_HIP(hipStreamSynchronize(stream));
 }
@@ -613,9 +584,8 @@ double Mlp::gradients_host(const float* x, const float* t, int n, float* g) {
     const int rows = pad_rows(n);
     ensure(rows);
     stage_xt(samples, x, t, n, stream);
-    pack(samples.p, IN + OUT, nullptr, n, rows, true);
-    forward(n, rows, true);
-    backward(rows);
+    loss_part.reserve(rows / 16);
+    train_pass(samples.p, IN + OUT, nullptr, n, rows, loss_part.p);
     reduce(0, 0.f);
     grad.download(g, NPARAM, stream);
     return loss(rows) / (2.0 * n);
@@ -626,9 +596,8 @@ double Mlp::adam_host(const float* x, const float* t, int n, float lr) {
     const int rows = pad_rows(n);
     ensure(rows);
     stage_xt(samples, x, t, n, stream);
-    pack(samples.p, IN + OUT, nullptr, n, rows, true);
-    forward(n, rows, true);
-    backward(rows);
+    loss_part.reserve(rows / 16);
+    train_pass(samples.p, IN + OUT, nullptr, n, rows, loss_part.p);
     const double l = loss(rows) / (2.0 * n);
     reduce(1, lr);
     PA_HIP(hipStreamSynchronize(stream));
@@ -645,24 +614,32 @@ void Mlp::train_host(const float* samples_h, int64_t n, int epochs, int batch, f
     std::vector<int32_t> order((size_t)n);
     std::iota(order.begin(), order.end(), 0);
     std::mt19937_64 rng(seed);
+    std::shuffle(order.begin(), order.end(), rng);
+    // an epoch's loss partials stay on the device until its end: no wait per batch
+    const size_t per_batch = (size_t)batch / 16;
+    std::vector<double> h(((size_t)n + batch - 1) / batch * per_batch);
+    loss_part.reserve(h.size());
     for (int e = 0; e < epochs; e++) {
-        std::shuffle(order.begin(), order.end(), rng);
         perm.upload(order.data(), order.size(), stream);
-        double lsum = 0;
-        int64_t seen = 0;
-        for (int64_t b0 = 0; b0 < n; b0 += batch) {
+        size_t k = 0;
+        for (int64_t b0 = 0; b0 < n; b0 += batch, k++) {
             const int nb = (int)std::min<int64_t>(batch, n - b0);
-            const int rows = pad_rows(nb);
-            pack(samples.p, IN + OUT, perm.p + b0, nb, rows, true);
-            forward(nb, rows, true);
-            backward(rows);
+            train_pass(samples.p, IN + OUT, perm.p + b0, nb, pad_rows(nb), loss_part.p + k * per_batch);
             reduce(1, lr);
-            lsum += loss(rows) / 2.0;
-            seen += nb;
         }
-        if (epoch_loss) epoch_loss[e] = lsum / (double)seen;
+        if (e + 1 < epochs) std::shuffle(order.begin(), order.end(), rng); // the next epoch's order, beside this one's kernels
+        loss_part.download(h.data(), k * per_batch, stream);
+        PA_HIP(hipStreamSynchronize(stream));
+        double lsum = 0;
+        k = 0;
+        for (int64_t b0 = 0; b0 < n; b0 += batch, k++) {
+            const int parts = pad_rows((int)std::min<int64_t>(batch, n - b0)) / 16;
+            double l = 0;
+            for (int q = 0; q < parts; q++) l += h[k * per_batch + q];
+            lsum += l / 2.0;
+        }
+        if (epoch_loss) epoch_loss[e] = lsum / (double)n;
     }
-    PA_HIP(hipStreamSynchronize(stream));
 }
 
 double Mlp::time_ms(int which, int rows, int reps) {
@@ -672,16 +649,17 @@ double Mlp::time_ms(int which, int rows, int reps) {
     // a fixed synthetic batch: zero features and targets (timing only)
     samples.reserve((size_t)rows * (IN + OUT));
     PA_HIP(hipMemsetAsync(samples.p, 0, sizeof(float) * (size_t)rows * (IN + OUT), stream));
-    pack(samples.p, IN + OUT, nullptr, rows, rows, true);
+    loss_part.reserve(rows / 16);
     std::vector<float> keep(NPARAM);
     get_params(keep.data());
     hipEvent_t e0, e1;
     PA_HIP(hipEventCreate(&e0));
     PA_HIP(hipEventCreate(&e1));
     auto one = [&]() {
-        forward(rows, rows, which == 1);
-        if (which == 1) {
-            backward(rows);
+        if (which == 0) {
+            infer(samples.p, IN + OUT, rows, rows, Y.p);
+        } else {
+            train_pass(samples.p, IN + OUT, nullptr, rows, rows, loss_part.p);
             reduce(1, 0.f);
         }
     };

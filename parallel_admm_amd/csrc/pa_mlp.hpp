@@ -38,12 +38,12 @@ struct Mlp {
     DBuf<float> w, adam_m, adam_v;
     int adam_t = 0;
     DBuf<uint16_t> W1p, W2, W2T, W3, W3T, W4p, W4T;
-    // activations for up to `cap` rows (rows padded to a multiple of 32)
+    // what a pass over up to `cap` rows (padded to a multiple of 32) leaves in memory
     int cap = 0;
-    DBuf<uint16_t> X, XT, H1, H2, H3, H1T, H2T, H3T, dY, dYT, dA1, dA2, dA3, dA1T, dA2T, dA3T;
-    DBuf<float> S1, S2, S3, Y, T;
+    DBuf<uint16_t> XT, H1T, H2T, H3T, dYT, dA1T, dA2T, dA3T; // transposed, for the weight gradients
+    DBuf<float> Y;
     DBuf<float> part;        // split-K partial weight gradients
-    DBuf<double> loss_part;  // per output tile
+    DBuf<double> loss_part;  // per 16 rows (train_host: of an epoch)
     DBuf<float> grad;        // flat gradient (gradient-only mode)
     DBuf<float> samples;     // training set on the device, 12 floats per sample
     DBuf<int32_t> perm;      // sample order of the current epoch
@@ -61,14 +61,13 @@ struct Mlp {
     void get_params(float* host);
     void ensure(int rows);
 
-    // Packs rows of `src` (stride floats apart, features first, then 2
-    // targets when `targets`) into the input buffers; idx selects rows (or null).
-    void pack(const float* src, int stride, const int32_t* idx, int n, int rows, bool targets);
-    // Forward over `rows` padded rows (n real); with `train`, keeps what the
-    // backward pass needs and forms dY = (y - t) / n and the loss partials.
-    void forward(int n, int rows, bool train);
-    void infer(int rows, const uint16_t* Xin, uint16_t* h1, uint16_t* h2, uint16_t* h3, float* y);
-    void backward(int rows);
+    // Forward over `rows` padded rows, the first n from src (`stride` floats
+    // apart), into y [rows][2].
+    void infer(const float* src, int stride, int n, int rows, float* y);
+    // Forward and backward (features, then 2 targets per row; idx selects rows
+    // or null): loss partials to loss_out [rows / 16], split-K partial weight
+    // gradients to `part`.
+    void train_pass(const float* src, int stride, const int32_t* idx, int n, int rows, double* loss_out);
     // Sums the split-K partials; mode 0 writes the flat gradient, mode 1 takes an Adam step.
     void reduce(int mode, float lr);
     double loss(int rows);

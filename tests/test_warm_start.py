@@ -266,3 +266,26 @@ def test_trained_network_gain(pa):
         out[mode] = ws.summary(stats, wall)
         print(f"mode {mode}: {out[mode]}")
     assert out[1]["admm_iters_incl_wasted"] <= 1.1 * out[0]["admm_iters_mean"]
+
+
+@pytest.mark.parametrize("n", [1, 33, 511, 4640])
+def test_mlp_passes_at_row_tile_edges(pa, n):
+    """One row, one row past a tile of 32, a split of one tile each and a last
+    row short, and 145 row tiles (one split, not a multiple of the loads in
+    flight): gradients to the bars above; training at rate 0 over batches with
+    a ragged last one reports the loss of all rows (the same FP32 outputs
+    summed in FP64 in another order)."""
+    om = _oracle_mlp()
+    net = pa.MLP(seed=14)
+    w = net.params().astype(np.float64)
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((n, om.IN)).astype(np.float32)
+    t = rng.standard_normal((n, om.OUT)).astype(np.float32)
+    g, loss = net.gradients(x, t)
+    l16, g16 = om.loss_and_grad(w, x.astype(np.float64), t.astype(np.float64), emulate_bf16=True)
+    e16 = rel_err(g, g16)
+    losses = net.train(np.concatenate([x, t], axis=1), epochs=2, batch=96, lr=0.0, seed=3)
+    print(f"n={n}: rel err vs bf16 oracle {e16:.2e}, loss {loss:.9f} (oracle {l16:.9f}, trained {losses})")
+    assert abs(loss - l16) <= 1e-2 * l16 and e16 < 2e-2
+    np.testing.assert_allclose(losses, loss, rtol=1e-10)
+    np.testing.assert_array_equal(net.params().astype(np.float64), w)
