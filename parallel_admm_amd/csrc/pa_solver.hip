@@ -1410,9 +1410,10 @@ __global__ void __launch_bounds__(PBLK) k_cg_dir(int n, int slot, int nparts, do
 // ---------------------------------------------------------------------------
 // Next state slot (slot_old ^ 1) from |r|^2 at 3..5 and r.z at 6..8; every
 // thread gets beta, block 0 thread 0 writes the slot.
+template <int NT>
 __device__ inline void cg_advance(const double* __restrict__ part, int nparts, double* __restrict__ st, int slot_old, float (&be)[3]) {
     double s6[6];
-    block_reduce_parts<6, PBLK>(part, nparts, 9, 3, s6);
+    block_reduce_parts<6, NT>(part, nparts, 9, 3, s6);
     const double* so = st + slot_old * 8;
     double done[3];
     for (int k = 0; k < 3; k++) {
@@ -1432,7 +1433,7 @@ __device__ inline void cg_advance(const double* __restrict__ part, int nparts, d
 // one k_cg_dir_spmv does at the start of the next iteration.
 __global__ void __launch_bounds__(PBLK) k_cg_state(int slot_old, int nparts, double* __restrict__ st, const double* __restrict__ part) {
     float be[3];
-    cg_advance(part, nparts, st, slot_old, be);
+    cg_advance<PBLK>(part, nparts, st, slot_old, be);
 }
 
 // Up to RU entries of row i that lane `sub` of its row group owns (every
@@ -1474,19 +1475,31 @@ __device__ inline float3 ld3_or0(const float* __restrict__ a, int i, bool ok) { 
 // pass keeps the variant without the extra registers.
 inline bool multi_pass(int rows, int grid, int lpr) { return (int64_t)rows > 2 * (int64_t)grid * (PBLK / lpr); }
 
+// They run on workgroups of NT = 256 threads up to SMALL_LANES lanes (rows
+// times lanes per row) and of PBLK above.  4096 rows fill 16 workgroups of
+// PBLK, on 16 of the 256 CUs; a quarter of the size spreads the same waves over
+// 64 CUs.  At SMALL_LANES the grid leaves 256 partial sums, still one load per
+// thread and the cap of the grid; larger systems would need more passes.
+// AMG steps of a falling cloth (100 iterations), PBLK against SBLK: 4096 rows
+// 6.78 -> 5.56 ms (direction 12.1 -> 8.1 us, update 12.6 -> 7.8, post-smoothing
+// 8.9 -> 5.5), 16129 rows 8.47 -> 7.13 ms, 576 rows 3.08 -> 2.83 ms.
+constexpr int SBLK = 256;
+constexpr int64_t SMALL_LANES = 256 * 2 * SBLK;
+inline bool small_rows(int rows, int lpr) { return (int64_t)rows * lpr <= SMALL_LANES; }
+
 // The three SpMV-type kernels of the fused PCG iteration process two rows per
 // lane group (i and i + one grid's worth of rows) and issue every load that
 // does not depend on the reduced scalars (row pointers, entries, gathers, the
 // row's own values) before reducing the previous kernel's partial sums.
 
-template <int LPR, bool PF>
-__global__ void __launch_bounds__(PBLK) k_cg_dir_spmv(int n, int first, int slot_old, int nparts, double* __restrict__ st,
+template <int LPR, bool PF, int NT>
+__global__ void __launch_bounds__(NT) k_cg_dir_spmv(int n, int first, int slot_old, int nparts, double* __restrict__ st,
                                                      const int32_t* __restrict__ ptr, const int32_t* __restrict__ col,
                                                      const float* __restrict__ val, const float* __restrict__ diag,
                                                      const float* __restrict__ z, const float* __restrict__ p_old,
                                                      float* __restrict__ p_new, float* __restrict__ q, double* __restrict__ part) {
     const int sub = threadIdx.x % LPR;
-    const int rpb = PBLK / LPR, stride = gridDim.x * rpb;
+    const int rpb = NT / LPR, stride = gridDim.x * rpb;
     float be[3] = {0.f, 0.f, 0.f};
     bool need_be = !first;
     double acc[3] = {0, 0, 0};
@@ -1522,7 +1535,7 @@ __global__ void __launch_bounds__(PBLK) k_cg_dir_spmv(int n, int first, int slot
             pb[u] = first ? zb[u] : ld3(p_old, B.c[u]);
         }
         if (need_be) { // uniform per block (first row pass)
-            cg_advance(part, nparts, st, slot_old, be);
+            cg_advance<NT>(part, nparts, st, slot_old, be);
             need_be = false;
         }
         float3 sa = f3(0.f, 0.f, 0.f), sb = f3(0.f, 0.f, 0.f);
@@ -1562,12 +1575,12 @@ __global__ void __launch_bounds__(PBLK) k_cg_dir_spmv(int n, int first, int slot
             }
         }
     }
-    if (need_be) cg_advance(part, nparts, st, slot_old, be); // a block without rows still takes part
-    block_sum_write<3, PBLK>(acc, part, 9, 0);
+    if (need_be) cg_advance<NT>(part, nparts, st, slot_old, be); // a block without rows still takes part
+    block_sum_write<3, NT>(acc, part, 9, 0);
 }
 
-template <int LPR, bool PF>
-__global__ void __launch_bounds__(PBLK) k_cg_update_pre(int n, int slot, int nparts, double* __restrict__ st,
+template <int LPR, bool PF, int NT>
+__global__ void __launch_bounds__(NT) k_cg_update_pre(int n, int slot, int nparts, double* __restrict__ st,
                                                        const int32_t* __restrict__ ptr, const int32_t* __restrict__ col,
                                                        const float* __restrict__ val, const float* __restrict__ dinv, float w,
                                                        const float* __restrict__ pd, const float* __restrict__ q,
@@ -1575,12 +1588,12 @@ __global__ void __launch_bounds__(PBLK) k_cg_update_pre(int n, int slot, int npa
                                                        float* __restrict__ r_new, float* __restrict__ x0, float* __restrict__ res,
                                                        double* __restrict__ part) {
     const int sub = threadIdx.x % LPR;
-    const int rpb = PBLK / LPR, stride = gridDim.x * rpb;
+    const int rpb = NT / LPR, stride = gridDim.x * rpb;
     float al[3] = {0.f, 0.f, 0.f};
     bool need_al = true;
     auto take_alpha = [&] {
         double pq[3];
-        block_reduce_parts<3, PBLK>(part, nparts, 9, 0, pq);
+        block_reduce_parts<3, NT>(part, nparts, 9, 0, pq);
         const double* s = st + slot * 8;
         bool all_done = true;
         for (int k = 0; k < 3; k++) {
@@ -1666,7 +1679,7 @@ __global__ void __launch_bounds__(PBLK) k_cg_update_pre(int n, int slot, int npa
         }
     }
     if (need_al) take_alpha(); // a block without rows still takes part (block 0 counts the iteration)
-    block_sum_write<3, PBLK>(acc, part, 9, 3);
+    block_sum_write<3, NT>(acc, part, 9, 3);
 }
 
 // ---------------------------------------------------------------------------
@@ -1706,13 +1719,13 @@ __global__ void __launch_bounds__(BLK) k_amg_spmv(int rows, const int32_t* __res
 // Post-smoothing: xo = xi + w D^-1 (b - A xi); with part != null also b.xo at
 // 6..8 (on the finest level b is the PCG residual, so this is r.z).  Two rows
 // per lane group, as the fused PCG kernels.
-template <int LPR, bool PF>
-__global__ void __launch_bounds__(PBLK) k_amg_post(int n, const int32_t* __restrict__ ptr, const int32_t* __restrict__ col,
+template <int LPR, bool PF, int NT>
+__global__ void __launch_bounds__(NT) k_amg_post(int n, const int32_t* __restrict__ ptr, const int32_t* __restrict__ col,
                                                   const float* __restrict__ val, const float* __restrict__ dinv, float w,
                                                   const float* __restrict__ b, const float* __restrict__ xi, float* __restrict__ xo,
                                                   double* __restrict__ part) {
     const int sub = threadIdx.x % LPR;
-    const int rpb = PBLK / LPR, stride = gridDim.x * rpb;
+    const int rpb = NT / LPR, stride = gridDim.x * rpb;
     double acc[3] = {0, 0, 0};
     const int r_first = xcd_block() * rpb;
     int2 pra = make_int2(0, 0), prb = make_int2(0, 0);
@@ -1768,7 +1781,7 @@ __global__ void __launch_bounds__(PBLK) k_amg_post(int n, const int32_t* __restr
             }
         }
     }
-    if (part) block_sum_write<3, PBLK>(acc, part, 9, 6);
+    if (part) block_sum_write<3, NT>(acc, part, 9, 6);
 }
 
 // Partial r.z at 6..8.
@@ -2738,7 +2751,7 @@ void Backend::assemble_and_upload(const double* x0h) {
     cg_p2.alloc(3 * (size_t)n);
     a_lpr = lanes_per_row(nnz_a_off + n, n);
     // two rows per lane group in the fused PCG kernels
-    cg_blocks = std::max(1, std::min(grid_for((int64_t)n * a_lpr, 2 * PBLK), CG_MAX_BLOCKS));
+    cg_blocks = std::max(1, std::min(grid_for((int64_t)n * a_lpr, 2 * (small_rows(n, a_lpr) ? SBLK : PBLK)), CG_MAX_BLOCKS));
     cg_part.alloc(9 * (size_t)cg_blocks);
     cg_state.alloc(24);
     int elem_blocks = grid_for(hc.n_tri, BLK) + grid_for(hc.n_tet, BLK) + grid_for(hc.n_bend, BLK) + grid_for(hc.n_pin, BLK);
@@ -2958,8 +2971,10 @@ double Backend::spmv_time_ms(int reps) {
             with_lpr(a_lpr, [&](auto c) {
                 constexpr int P = decltype(c)::value;
                 if (fused)
-                    hipLaunchKernelGGL((multi_pass(n, nb, P) ? k_cg_dir_spmv<P, true> : k_cg_dir_spmv<P, false>), dim3(nb), dim3(PBLK), 0,
-                                       stream, n, 0, 0, nb, cg_state.p, a_ptr.p, a_col.p,
+                    hipLaunchKernelGGL((small_rows(n, a_lpr)     ? k_cg_dir_spmv<P, false, SBLK>
+                                        : multi_pass(n, nb, P) ? k_cg_dir_spmv<P, true, PBLK>
+                                                               : k_cg_dir_spmv<P, false, PBLK>),
+                                       dim3(nb), dim3(small_rows(n, a_lpr) ? SBLK : PBLK), 0, stream, n, 0, 0, nb, cg_state.p, a_ptr.p, a_col.p,
                                        a_val.p, a_diag.p, (const float*)cg_z.p, (const float*)cg_p.p, cg_p2.p, cg_q.p, cg_part.p);
                 else
                     hipLaunchKernelGGL(k_cg_spmv<P>, dim3(nb), dim3(PBLK), 0, stream, n, a_ptr.p, a_col.p, a_val.p, a_diag.p,
@@ -3045,8 +3060,12 @@ void Backend::precondition(const float* r, bool skip_pre0) {
         // level 0 emits r.z partials, so it runs on the partial-sum grid
         with_lpr(L.lpr_a, [&](auto c) {
             constexpr int P = decltype(c)::value;
-            const int grid = l == 0 ? nb : grid_for((int64_t)L.n * P, PBLK);
-            hipLaunchKernelGGL((multi_pass(L.n, grid, P) ? k_amg_post<P, true> : k_amg_post<P, false>), dim3(grid), dim3(PBLK), 0, stream,
+            const bool small = l == 0 ? small_rows(n, a_lpr) : small_rows(L.n, P);
+            const int grid = l == 0 ? nb : grid_for((int64_t)L.n * P, small ? SBLK : PBLK);
+            hipLaunchKernelGGL((small                     ? k_amg_post<P, false, SBLK>
+                                : multi_pass(L.n, grid, P) ? k_amg_post<P, true, PBLK>
+                                                           : k_amg_post<P, false, PBLK>),
+                               dim3(grid), dim3(small ? SBLK : PBLK), 0, stream,
                                L.n, L.aptr.p, L.acol.p, L.aval.p, L.dinv.p, L.omega,
                                bl, (const float*)L.x.p, out, l == 0 ? cg_part.p : (double*)nullptr);
         });
@@ -3080,7 +3099,10 @@ void Backend::pcg_iteration(int it, bool fused, int& pc, int& rc) {
     if (fused) {
         with_lpr(a_lpr, [&](auto c) {
             constexpr int P = decltype(c)::value;
-            hipLaunchKernelGGL((multi_pass(n, nb, P) ? k_cg_dir_spmv<P, true> : k_cg_dir_spmv<P, false>), dim3(nb), dim3(PBLK), 0, stream,
+            hipLaunchKernelGGL((small_rows(n, a_lpr)     ? k_cg_dir_spmv<P, false, SBLK>
+                                : multi_pass(n, nb, P) ? k_cg_dir_spmv<P, true, PBLK>
+                                                       : k_cg_dir_spmv<P, false, PBLK>),
+                               dim3(nb), dim3(small_rows(n, a_lpr) ? SBLK : PBLK), 0, stream,
                                n, it == 0 ? 1 : 0, slot ^ 1, nb, cg_state.p, a_ptr.p,
                                a_col.p, a_val.p, a_diag.p, (const float*)cg_z.p, (const float*)pbuf[pc], pbuf[pc ^ 1], cg_q.p,
                                cg_part.p);
@@ -3102,8 +3124,10 @@ void Backend::pcg_iteration(int it, bool fused, int& pc, int& rc) {
         DevLevel& L0 = *amg[0];
         with_lpr(L0.lpr_a, [&](auto c) {
             constexpr int P = decltype(c)::value;
-            hipLaunchKernelGGL((multi_pass(n, nb, P) ? k_cg_update_pre<P, true> : k_cg_update_pre<P, false>), dim3(nb), dim3(PBLK), 0,
-                               stream, n, slot, nb, cg_state.p, L0.aptr.p, L0.acol.p,
+            hipLaunchKernelGGL((small_rows(n, a_lpr)     ? k_cg_update_pre<P, false, SBLK>
+                                : multi_pass(n, nb, P) ? k_cg_update_pre<P, true, PBLK>
+                                                       : k_cg_update_pre<P, false, PBLK>),
+                               dim3(nb), dim3(small_rows(n, a_lpr) ? SBLK : PBLK), 0, stream, n, slot, nb, cg_state.p, L0.aptr.p, L0.acol.p,
                                L0.aval.p, L0.dinv.p, L0.omega, (const float*)pbuf[pc], (const float*)cg_q.p, cg_d.p,
                                (const float*)rbuf[rc], rbuf[rc ^ 1], L0.x.p, L0.r.p, cg_part.p);
         });

@@ -249,6 +249,32 @@ def test_global_solve_matches_llt(pa, precond):
             assert it <= 60
 
 
+@pytest.mark.parametrize("side", [2, 13, 128, 129])
+def test_amg_solve_at_workgroup_edges(pa, side):
+    """The AMG-preconditioned solve with one level, one part-filled workgroup,
+    and the last size on the small workgroups (16384 rows of 8 lanes) and the
+    first past it: the bar of test_global_solve_matches_llt."""
+    from parallel_admm_amd.configs import config_for
+
+    rng = np.random.default_rng(side)
+    cfg = config_for("cloth32")
+    cfg.global_tol = 1e-5
+    cfg.global_refine = 2
+    cfg.global_max_iter = 2000
+    cfg.precond = 1
+    sc = pa.Scene.generate(4, side=side, radius=0.1, drop=0.3)
+    m = sc.mesh()
+    b = pa.ADMMBackendHIP.from_scene(sc, cfg)
+    o = _oracle(m, cfg)
+    n = sc.info["n_dyn"]
+    xs = m["x"][:n] + 0.01 * rng.standard_normal((n, 3))
+    rhs = o.matrix(1) @ xs
+    xg, it = b.global_solve(rhs, m["x"][:n])
+    err = rel_err(xg, o.solve(rhs))
+    print(f"side {side}: PCG {it} iterations, rel err vs LLT {err:.2e}")
+    assert err < 1e-6 and it <= 60
+
+
 @pytest.mark.parametrize("passes", [1, 2])
 def test_direct_solve_matches_llt(pa, passes):
     """The direct global solve (precond 2: supernodal Cholesky factored on the
