@@ -42,9 +42,9 @@ def spmv_bytes(n: int, nnz_off: int) -> int:
 def top_bytes(top_cols: int, top_sq: int) -> int:
     """Algorithmic bytes of one launch of the direct solve's dense-top product
     (k_chol_top): S^-1 read once (4 sum m^2), and per top entry its assembled
-    right-hand side (12, written by k_chol_top_f), its unknown id and position
-    (8), the solution in elimination order and the correction (12 + 12)."""
-    return 4 * top_sq + 44 * top_cols
+    right-hand side (12, written by k_chol_top_f), its place (4) and the
+    correction (12)."""
+    return 4 * top_sq + 28 * top_cols
 
 
 def measured_traffic(workload: str, kernel: str) -> tuple[int | None, str | None]:

@@ -429,7 +429,7 @@ pa_status pa_mlp_forward(pa_mlp* m, const float* x, int32_t n, float* y);
 /* The same y[n][2] = MLP(x[n][10]) without allocating or freeing any device
  * memory.  No counterpart in the reference; it is for callers that cannot
  * allocate (code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc).  Every intermediate lives in one file-scope device array
+ * forbid hipMalloc).  Input and output are staged in one file-scope device array
  * per GPU of PA_MLP_NOALLOC_SCRATCH_BYTES (about 15 MB, held until the process
  * ends); n is at most PA_MLP_NOALLOC_MAX_ROWS per call (more is refused with
  * PA_ERR_INVALID).  Calls that overlap on one GPU share that array and race:
@@ -471,7 +471,7 @@ pa_status pa_scene_merge(const pa_scene* const* scenes, int32_t count, pa_scene*
 pa_status pa_detector_set_segments(pa_detector* d, const int32_t* seg, int32_t count);
 /* Query passes: 0 (default) a collect pass (traversal only, leaf hits to
  * per-query slabs and an overflow list) then a test pass (the FP64 predicate
- * on the hits), rerun as the single pass when the short traversal stack or the
+ * on the hits), rerun as the single pass when the shared traversal stack or the
  * overflow list was too small; 1 the single pass (traversal and predicate
  * together) always.  Both give the same list.  No counterpart in the
  * reference: a diagnostic for checking that they do. */

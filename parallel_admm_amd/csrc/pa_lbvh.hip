@@ -6,7 +6,7 @@
 // -> node boxes from leaf ranges -> 128-byte wide node records (the boxes,
 // ids and last sorted leaf of a node's up to four grandchildren, a leaf child
 // standing in for its own pair, so a traversal step descends two levels with
-// one dependent load) -> per query a traversal by 16 lanes that collects close
+// one dependent load) -> a traversal by waves that share a stack, collecting close
 // leaves, then the FP64 predicate on them, accepted pairs marked and counted
 // per segment.
 //

@@ -620,7 +620,7 @@ __global__ void k_contact_du(int nc, const int4* __restrict__ cv, const float4* 
 // entry of the sorted list: the lane of a vertex's first entry sums its run,
 // the others exit.  A run's entries are read eight at a time before they are
 // added (one at a time the longest run, 30 and more entries, set the kernel's
-// time: 9.9 us against 7.4 on a twice-folded 256x256 cloth, 9.6 against 6.0 on
+// time: 9.9 us, now 7.4, on a 256x256 cloth with a folded flap, 9.6, now 6.0, on
 // 160 merged cloths).  Lanes past the entry count read stale (allocated) run
 // markers beside the count and drop them.
 __global__ void k_vertex_gather(int ne_max, int n, float* __restrict__ p, const uint32_t* __restrict__ vptr,
