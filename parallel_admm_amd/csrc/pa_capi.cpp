@@ -686,10 +686,10 @@ pa_status pa_backend_set_contact_log(pa_backend* b, int64_t cap) {
     BK({
         PA_CHECK(cap >= 0 && cap <= ((int64_t)1 << 28), PA_ERR_INVALID, "log capacity out of range");
         pa::Backend& B = *b->b;
-        B.log_cap = cap;
+        B.log_cap = 0; // no log unless its buffer is there
         B.log_rows = 0;
-        if (cap) B.log_buf.alloc((size_t)cap * 12);
-        else B.log_buf.release();
+        B.log_buf.alloc((size_t)cap * 12);
+        B.log_cap = cap;
     });
 }
 

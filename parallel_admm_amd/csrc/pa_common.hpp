@@ -57,10 +57,15 @@ template <class T> struct DBuf {
         return *this;
     }
     ~DBuf() { release(); }
+    // A failed allocation leaves an empty buffer (n is set by a successful one
+    // only), so a later reserve() tries again.
     void alloc(size_t count) {
         release();
+        if (!count) return;
+        T* q = nullptr;
+        PA_HIP(hipMalloc(&q, sizeof(T) * count));
+        p = q;
         n = count;
-        if (count) PA_HIP(hipMalloc(&p, sizeof(T) * count));
     }
     // Grow-only reallocation (contents not preserved).
     void reserve(size_t count) {

@@ -1311,15 +1311,23 @@ void Detector::set_segments(const int32_t* vs, int count) {
     for (int f = 0; f < nf; f++)
         PA_CHECK(vs[t[3 * f]] == vs[t[3 * f + 1]] && vs[t[3 * f]] == vs[t[3 * f + 2]], PA_ERR_INVALID, "triangle spans two segments");
     for (int k = 0; k < ne; k++) PA_CHECK(vs[e[2 * k]] == vs[e[2 * k + 1]], PA_ERR_INVALID, "edge spans two segments");
-    vseg.alloc(n_all);
-    vseg.upload(vs, n_all, stream);
+    // all of it first: if an allocation fails, the detector stays as it was
+    DBuf<int32_t> seg(n_all), first[2], last[2], root[2];
+    seg.upload(vs, n_all, stream);
+    for (int k = 0; k < 2; k++) {
+        first[k].alloc(count);
+        last[k].alloc(count);
+        root[k].alloc(count);
+    }
+    vseg = std::move(seg);
+    Tree* const trees[2] = {&ft, &et};
+    for (int k = 0; k < 2; k++) {
+        trees[k]->seg_first = std::move(first[k]);
+        trees[k]->seg_last = std::move(last[k]);
+        trees[k]->seg_root = std::move(root[k]);
+    }
     nseg = count;
     built = false; // keys change: the next detection rebuilds
-    for (Tree* T : {&ft, &et}) {
-        T->seg_first.alloc(count);
-        T->seg_last.alloc(count);
-        T->seg_root.alloc(count);
-    }
 }
 
 int Detector::detect(const double* x, bool refit, VertexCount vc) {

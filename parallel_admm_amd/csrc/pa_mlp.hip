@@ -451,8 +451,8 @@ void Mlp::get_params(float* host) {
 void Mlp::ensure(int rows) {
     PA_CHECK(rows > 0 && rows % 32 == 0, PA_ERR_INVALID, "mlp: rows must be a positive multiple of 32");
     if (rows <= cap) return;
-    cap = rows;
-    const size_t c = (size_t)cap;
+    cap = 0; // until everything below is in place
+    const size_t c = (size_t)rows;
     XT.alloc(c * INA);
     for (DBuf<uint16_t>* b : {&H1T, &H2T, &H3T}) b->alloc(c * HA);
     for (DBuf<uint16_t>* b : {&dA1T, &dA2T, &dA3T}) b->alloc(c * H);
@@ -460,9 +460,10 @@ void Mlp::ensure(int rows) {
     Y.alloc(c * OUT);
     part.alloc((size_t)16 * (2 * H * HA + H * INA + OUTP * HA)); // up to 16 splits
     for (DBuf<uint16_t>* b : {&H1T, &H2T, &H3T, &dYT}) b->zero(stream);
-    hipLaunchKernelGGL(k_ones_rows, dim3(grid_for(cap, 256)), dim3(256), 0, stream, cap, H1T.p, H2T.p, H3T.p);
+    hipLaunchKernelGGL(k_ones_rows, dim3(grid_for(rows, 256)), dim3(256), 0, stream, rows, H1T.p, H2T.p, H3T.p);
     PA_LAUNCH_CHECK();
     PA_HIP(hipStreamSynchronize(stream));
+    cap = rows;
 }
 
 static MlpArgs mlp_args(const Mlp& m, const float* src, int stride, const int32_t* idx, int n, float* y) {

@@ -1,0 +1,125 @@
+"""Device allocations that fail: the call reports an error and the handle stays
+usable, so the same call repeated leaves the allocations of a handle that never
+failed (a size that is recorded before its allocation would be taken as
+allocated from then on, and kernels would run on null buffers).  The library's
+own host code runs on tests/fake_hip.cpp, a HIP runtime on host memory, in a
+process of its own per test.  CPU only."""
+import ctypes as C
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def fake_hip(tmp_path_factory):
+    out = tmp_path_factory.mktemp("fake_hip") / "libfake_hip.so"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-o", str(out), os.path.join(ROOT, "tests", "fake_hip.cpp")], check=True)
+    return str(out)
+
+
+def _fails_everywhere(pa, fake, make, call):
+    """`call` on fresh handles with each of its allocations failing in turn."""
+    h = make()
+    before, first = fake.fake_live(), fake.fake_allocs()
+    call(h)
+    want, count = fake.fake_live() - before, fake.fake_allocs() - first
+    assert count > 0
+    for k in range(1, count + 1):
+        h = make()
+        before = fake.fake_live()
+        fake.fake_fail_at(k)
+        try:
+            call(h)
+            raise AssertionError(f"allocation {k} of {count} failed unnoticed")
+        except pa.PAError as e:
+            assert e.code == pa.PA_ERR_HIP
+        fake.fake_fail_at(0)
+        call(h)
+        assert fake.fake_live() - before == want, f"allocation {k} of {count}"
+
+
+def _detector(pa, side):
+    sc = pa.Scene.generate(4, side=side, radius=0.1)
+    return pa.CollisionDetector.for_scene(sc, 1000, 1e-3), sc.mesh()["x"]
+
+
+def network(pa, fake):
+    x = np.zeros((100, pa.MLP_FEATURES), np.float32)
+    t = np.zeros((100, pa.MLP_OUTPUTS), np.float32)
+    rows = np.zeros((1000, 12), np.float32)
+    for call in (lambda m: m.forward(x), lambda m: m.gradients(x, t), lambda m: m.adam_step(x, t, 1e-3),
+                 lambda m: m.train(rows, 1, batch=96)):
+        _fails_everywhere(pa, fake, pa.MLP, call)
+
+
+def detection(pa, fake):
+    for side in (9, 90):  # leaves sorted in one workgroup, and by the radix sort with its scratch
+        x = _detector(pa, side)[1]
+        _fails_everywhere(pa, fake, lambda: _detector(pa, side)[0], lambda d: d.detect(x))
+
+
+def segments(pa, fake):
+    """A segmented detector keeps its segments when setting others fails."""
+    d, x = _detector(pa, 9)
+    d.set_segments(np.zeros(len(x), np.int32))
+    d.detect(x)
+    before, first = fake.fake_live(), fake.fake_allocs()
+    d.set_segments(np.zeros(len(x), np.int32))
+    for k in range(1, fake.fake_allocs() - first + 1):
+        fake.fake_fail_at(k)
+        try:
+            d.set_segments(np.ones(len(x), np.int32))
+            raise AssertionError("no error")
+        except pa.PAError as e:
+            assert e.code == pa.PA_ERR_HIP
+        fake.fake_fail_at(0)
+        assert fake.fake_live() == before
+        d.detect(x)
+
+
+def contact_log(pa, fake):
+    """No step logs into a buffer that was not allocated."""
+    from parallel_admm_amd.configs import config_for
+
+    sc = pa.Scene.generate(4, side=9, radius=0.1)
+    b = pa.ADMMBackendHIP.from_scene(sc, config_for("batch"))
+    fake.fake_last_pinned()[0] = 5  # the contacts that a detection finds
+    b.set_contact_log(1000)
+    b.step()
+    b.step()
+    logged = fake.fake_launches(b"k_ws_log")
+    assert logged > 0
+    b.set_contact_log(0)
+    fake.fake_fail_at(1)
+    try:
+        b.set_contact_log(2000)
+        raise AssertionError("no error")
+    except pa.PAError as e:
+        assert e.code == pa.PA_ERR_HIP
+    b.step()
+    b.step()
+    assert fake.fake_launches(b"k_ws_log") == logged
+
+
+@pytest.mark.parametrize("case", ["network", "detection", "segments", "contact_log"])
+def test_failed_allocation(fake_hip, case):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), fake_hip, case], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+if __name__ == "__main__":
+    _fake = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+    for _name in ("fake_live", "fake_var_bytes"):
+        getattr(_fake, _name).restype = C.c_size_t
+    for _name in ("fake_allocs", "fake_launches"):
+        getattr(_fake, _name).restype = C.c_long
+    _fake.fake_last_pinned.restype = C.POINTER(C.c_uint32)
+    sys.path.insert(0, ROOT)
+    import parallel_admm_amd as _pa
+
+    globals()[sys.argv[2]](_pa, _fake)
