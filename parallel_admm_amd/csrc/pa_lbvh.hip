@@ -1196,6 +1196,7 @@ Detector::Detector(int n_all_, int n_dyn_, int nv_, const int32_t* sv, int nf_, 
     qoffset.alloc((size_t)nv + ne + 1);
     PA_HIP(hipHostMalloc((void**)&total_host, 3 * sizeof(uint32_t), hipHostMallocDefault));
     seg_key.alloc(cap);
+    single_pairs.alloc(cap); // here, not on the first fallback: an allocation that fails inside a step would cost its rollback
     cand_pt.alloc((size_t)CAND * std::max(nv, 1));
     cand_ee.alloc((size_t)CAND * std::max(ne, 1));
     ccount_pt.alloc(std::max(nv, 1));
@@ -1390,7 +1391,6 @@ int Detector::detect(const double* x, bool refit, VertexCount vc) {
         // the short stack or an overflow list was too small: the single pass
         // (traversal and test together, full stack) for both queries
         fill<uint32_t>(counts.p, 0u, (int64_t)counts.n, stream);
-        single_pairs.reserve(c.cap);
         if (ne > 0) single_pass(EE, ACCEPTED, et);
         if (nv > 0) single_pass(PT, 0, ft);
         count_found(h);

@@ -63,6 +63,18 @@ def detection(pa, fake):
         _fails_everywhere(pa, fake, lambda: _detector(pa, side)[0], lambda d: d.detect(x))
 
 
+def single_pass(pa, fake):
+    """The single pass, which a step falls back to in the middle of its work,
+    allocates nothing of its own."""
+    for side in (9, 90):
+        d, x = _detector(pa, side)
+        d.detect(x)
+        before = fake.fake_allocs()
+        d.set_single_pass(True)
+        d.detect(x)
+        assert fake.fake_launches(b"k_single") > 0 and fake.fake_allocs() == before
+
+
 def segments(pa, fake):
     """A segmented detector keeps its segments when setting others fails."""
     d, x = _detector(pa, 9)
@@ -106,7 +118,7 @@ def contact_log(pa, fake):
     assert fake.fake_launches(b"k_ws_log") == logged
 
 
-@pytest.mark.parametrize("case", ["network", "detection", "segments", "contact_log"])
+@pytest.mark.parametrize("case", ["network", "detection", "single_pass", "segments", "contact_log"])
 def test_failed_allocation(fake_hip, case):
     r = subprocess.run([sys.executable, os.path.abspath(__file__), fake_hip, case], cwd=ROOT, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr
