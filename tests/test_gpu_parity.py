@@ -1040,3 +1040,140 @@ def test_step_with_point_track_matches_oracle(pa):
         print(f"point track frame {f}: contacts {st['n_contacts']}, step err {e:.2e}, |v_static| {np.abs(vg[n:]).max():.4f}")
     assert worst < 1e-5 and contacts > 0
     np.testing.assert_array_equal(b.track_frames(), [7])
+
+
+def _stacked_sheets(pa, layers, side, spacing, gap):
+    """Square sheets exactly one above the other, `gap` apart, as one mesh."""
+    k = np.arange(side * side)
+    sheet = spacing * np.stack([k // side, np.zeros(side * side), k % side], axis=1)
+    x = np.concatenate([sheet + [0, gap * q, 0] for q in range(layers)])
+    c = (side * np.arange(side - 1)[:, None] + np.arange(side - 1)).ravel()
+    cell = np.concatenate([np.stack([c, c + 1, c + side], axis=1), np.stack([c + 1, c + side + 1, c + side], axis=1)])
+    tris = np.concatenate([cell + q * side * side for q in range(layers)])
+    return x, pa.Scene.from_mesh(x, len(x), np.full(len(x), 1.0), tris=tris, tri_k=np.full(len(tris), 1e3))
+
+
+def test_overflowing_detection_falls_back_inside_a_step(pa):
+    """Eight sheets within the contact distance of each other: more close leaves
+    than the queries' slabs (16 each) and the overflow list (one entry per query)
+    hold, so a detection reruns as the single pass by itself.  Its list is the
+    oracle's, and steps with it are the forced single pass's, bit for bit."""
+    from parallel_admm_amd.configs import config_for
+
+    cfg = config_for("cloth32")
+    cfg.max_contacts = 1 << 18
+    cfg.admm_max_iter = 6  # two detections
+    d = cfg.thickness
+    x, sc = _stacked_sheets(pa, 8, 8, 0.01, 0.1 * d)
+    t = sc.topology()["surf_tris"].reshape(-1, 3)
+    lo, hi = x[t].min(axis=1), x[t].max(axis=1)
+    near = np.all((x[:, None] >= lo - d) & (x[:, None] <= hi + d), axis=2)
+    near[t, np.arange(len(t))[:, None]] = False
+    assert near.sum() > 17 * len(x)  # vertex queries alone overflow the list
+    o = _oracle(sc.mesh(), cfg)
+    o.detect(x, brute_force=True)
+    out = []
+    for single in (False, True):
+        det = _detector(pa, sc, cfg)
+        det.set_single_pass(single)
+        det.detect(x)
+        _check_contacts_equal(*det.contacts(), *o.contacts())
+        b = pa.ADMMBackendHIP.from_scene(sc, cfg)
+        b.attach_detector(det)
+        nc = [b.step()["n_contacts_max"] for _ in range(2)]
+        out.append((*b.get_state(), *b.get_duals()))
+    print(f"{near.sum()} close pairs of {len(x)} vertices, contacts per step {nc}")
+    assert min(nc) > 2048
+    for a, c in zip(*out):
+        np.testing.assert_array_equal(a, c)
+
+
+def test_single_pass_step_matches_two_pass_step(pa):
+    """A step whose detections run the single pass (which also counts and places
+    every vertex's contacts for the step) against one with the two passes, bit
+    for bit: a draped cloth (one contact per lane of the sweeps), a small folded
+    one (two per lane) and a larger one (a launch per sweep)."""
+    from parallel_admm_amd.configs import config_for
+
+    cfg = config_for("cloth32")
+    sc = pa.Scene.generate(1)
+    cases = [(sc, drape_on_obstacle(sc, cfg.thickness))]
+    for side in (11, 24):
+        xf, scf = folded_cloth(side=side, spacing=0.01, gap=0.5 * cfg.thickness, jitter=0.15 * cfg.thickness, seed=3)
+        cases.append((scf, xf))
+    peaks = []
+    for scene, x0 in cases:
+        out = []
+        for single in (False, True):
+            det = _detector(pa, scene, cfg)
+            det.set_single_pass(single)
+            b = pa.ADMMBackendHIP.from_scene(scene, cfg)
+            b.attach_detector(det)
+            b.set_state(x=x0)
+            nc = [b.step()["n_contacts_max"] for _ in range(2)]
+            out.append((*b.get_state(), *b.get_duals()))
+        peaks.append(max(nc))
+        for a, c in zip(*out):
+            np.testing.assert_array_equal(a, c)
+    print(f"contacts {peaks}")
+    assert 0 < peaks[0] <= 1024 < peaks[1] <= 2048 < peaks[2]
+
+
+@pytest.mark.parametrize("edges", [16383, 16384, 16385])
+def test_detector_at_the_small_build_limit(pa, edges):
+    """The last sizes whose leaves one workgroup sorts and the first beyond: the
+    list of a folded cloth cut to `edges` edges is that of the same edges with
+    others far away, 20,000 in all, which are sorted by the launches."""
+    from parallel_admm_amd.configs import config_for
+
+    cfg = config_for("cloth32")
+    x, sc = folded_cloth(side=76, spacing=0.01, gap=0.5 * cfg.thickness, jitter=0.15 * cfg.thickness, seed=7)
+    t = sc.topology()
+    e = t["surf_edges"].reshape(-1, 2)[:edges]
+    assert len(e) == edges
+    n = len(x)
+    lists = []
+    for far in (0, 20000 - edges):
+        k = np.arange(2 * far)
+        xx = np.concatenate([x, np.stack([9 + 0.1 * k, 9 + 0 * k, 9 + 0 * k], axis=1)])
+        ee = np.concatenate([e, n + k.reshape(-1, 2)])
+        det = pa.CollisionDetector(len(xx), n, t["surf_verts"], t["surf_tris"], ee, 1 << 18, cfg.thickness)
+        det.detect(xx)
+        lists.append(det.contacts())
+    print(f"{edges} edges: {len(lists[0][0])} contacts")
+    assert len(lists[0][0]) > 2000
+    np.testing.assert_array_equal(lists[0][0], lists[1][0])
+    np.testing.assert_array_equal(lists[0][1], lists[1][1])
+
+
+@pytest.mark.parametrize("side,refine,interval,precond", [(32, 2, 1, 2), (66, 2, 1, 2), (32, 1, 2, 2), (32, 1, 3, 2), (32, 1, 2, 1)])
+def test_refinement_and_check_interval_match_oracle(pa, side, refine, interval, precond):
+    """Two refinement passes per global solve (the second reads the stored
+    right-hand side), and a residual check every second or third iteration
+    (which reads the local step kept one iteration back), to the bars of
+    test_step_matches_fp64_oracle."""
+    from parallel_admm_amd.configs import config_for
+
+    cfg = config_for("cloth32")
+    cfg.residual_tol, cfg.global_refine, cfg.residual_interval, cfg.precond = 1e-4, refine, interval, precond
+    sc = pa.Scene.generate(4, side=side, radius=0.2, drop=0.002)
+    n = sc.info["n_dyn"]
+    b = pa.ADMMBackendHIP.from_scene(sc, cfg)
+    o = _oracle(sc.mesh(), cfg)
+    contacts = 0
+    for f in range(6):
+        x, v = b.get_state()
+        o.set_state(x, v)
+        o.set_duals(*b.get_duals())
+        n_log = len(o.residual_log())
+        st, so = b.step(), o.step()
+        contacts += st["n_contacts"]
+        e = step_err(b.get_state()[0], o.state()[0], x, n)
+        rg, ro = b.residual_log(), o.residual_log()[n_log:]
+        k = min(len(rg), len(ro))
+        dr = float(np.max(np.abs(rg[:k] - ro[:k]) / (np.abs(ro[:k]) + 1e-3)))
+        print(f"frame {f}: contacts {st['n_contacts']}, iterations {st['iterations']} oracle {so['iterations']}, checks {len(rg)}, "
+              f"step err {e:.2e}, residual rel diff {dr:.2e}")
+        assert k > 0 and abs(len(rg) - len(ro)) <= 1 and abs(st["iterations"] - so["iterations"]) <= interval
+        assert e < 1e-5 and dr < 1e-3
+    assert contacts > 0
