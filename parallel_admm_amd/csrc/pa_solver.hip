@@ -2283,6 +2283,10 @@ void Backend::init(const double* x0h, const double* massh, int n_all_, int n_dyn
     PA_CHECK(finalized, PA_ERR_INVALID, "init before finalize_constraints");
     PA_CHECK(!initialized, PA_ERR_INVALID, "init called twice");
     PA_CHECK(n_all_ > 0 && n_dyn > 0 && n_dyn <= n_all_, PA_ERR_INVALID, "bad vertex counts");
+    if (det) { // attached before these sizes were known: what attach_detector could not check
+        PA_CHECK(det->n_all <= n_all_, PA_ERR_INVALID, "attached detector has more vertices than the backend");
+        PA_CHECK(det->c.cap <= cfg.max_contacts, PA_ERR_INVALID, "detector capacity exceeds max_contacts");
+    }
     n_all = n_all_;
     n = n_dyn;
     auto chk_v = [&](int v) { PA_CHECK(v >= 0 && v < n, PA_ERR_INVALID, "constraint references a non-dynamic vertex"); };

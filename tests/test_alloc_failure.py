@@ -118,8 +118,41 @@ def contact_log(pa, fake):
     assert fake.fake_launches(b"k_ws_log") == logged
 
 
+def early_detector(pa, fake):
+    """A detector attached before apply_config and init, when the backend's sizes
+    are not known yet, is refused by init if it does not fit them: its contacts
+    index per-vertex counts and fill per-contact buffers of the backend."""
+    from parallel_admm_amd.configs import config_for
+
+    sc, big = pa.Scene.generate(4, side=9, radius=0.1), pa.Scene.generate(4, side=10, radius=0.1)
+    m = sc.mesh()
+    for scene, capacity, fits in ((sc, 1000, True), (big, 1000, False), (sc, 2000, False)):
+        cfg = config_for("batch")
+        cfg.max_contacts = 1000
+        b = pa.ADMMBackendHIP()
+        b.attach_detector(pa.CollisionDetector.for_scene(scene, capacity, 1e-3))
+        b.apply_config(cfg)
+        b.set_constraints(sc)
+        b.set_constraint_dim(sc.info["m_rows"])
+        b.finalize_constraints()
+        try:
+            b.init(m["x"], sc.mass(), sc.info["n_dyn"], sc.surface_flags(), m["pins"])
+            assert fits
+            b.step()
+        except pa.PAError as e:
+            assert not fits and e.code == pa.PA_ERR_INVALID
+
+
 @pytest.mark.parametrize("case", ["network", "detection", "single_pass", "segments", "contact_log"])
 def test_failed_allocation(fake_hip, case):
+    _run(fake_hip, case)
+
+
+def test_detector_attached_before_init(fake_hip):
+    _run(fake_hip, "early_detector")
+
+
+def _run(fake_hip, case):
     r = subprocess.run([sys.executable, os.path.abspath(__file__), fake_hip, case], cwd=ROOT, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stdout + r.stderr
 
