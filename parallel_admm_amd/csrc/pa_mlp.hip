@@ -448,8 +448,14 @@ void Mlp::get_params(float* host) {
     PA_HIP(hipStreamSynchronize(stream));
 }
 
-void Mlp::ensure(int rows) {
+float* Mlp::outputs(int rows) {
     PA_CHECK(rows > 0 && rows % 32 == 0, PA_ERR_INVALID, "mlp: rows must be a positive multiple of 32");
+    if ((size_t)rows * OUT > Y.n) Y.alloc(std::max((size_t)rows * OUT, Y.n + Y.n / 2));
+    return Y.p;
+}
+
+void Mlp::ensure(int rows) {
+    outputs(rows);
     if (rows <= cap) return;
     cap = 0; // until everything below is in place
     const size_t c = (size_t)rows;
@@ -457,7 +463,6 @@ void Mlp::ensure(int rows) {
     for (DBuf<uint16_t>* b : {&H1T, &H2T, &H3T}) b->alloc(c * HA);
     for (DBuf<uint16_t>* b : {&dA1T, &dA2T, &dA3T}) b->alloc(c * H);
     dYT.alloc(c * OUTP);
-    Y.alloc(c * OUT);
     part.alloc((size_t)16 * (2 * H * HA + H * INA + OUTP * HA)); // up to 16 splits
     for (DBuf<uint16_t>* b : {&H1T, &H2T, &H3T, &dYT}) b->zero(stream);
     hipLaunchKernelGGL(k_ones_rows, dim3(grid_for(rows, 256)), dim3(256), 0, stream, rows, H1T.p, H2T.p, H3T.p);
@@ -545,10 +550,9 @@ double Mlp::loss(int rows) {
 void Mlp::forward_host(const float* x, int n, float* y) {
     PA_CHECK(n > 0, PA_ERR_INVALID, "mlp: no rows");
     const int rows = pad_rows(n);
-    ensure(rows);
     samples.reserve((size_t)n * IN);
     samples.upload(x, (size_t)n * IN, stream);
-    infer(samples.p, IN, n, rows, Y.p);
+    infer(samples.p, IN, n, rows, outputs(rows));
     Y.download(y, (size_t)n * OUT, stream);
     PA_HIP(hipStreamSynchronize(stream));
 }
@@ -646,7 +650,8 @@ void Mlp::train_host(const float* samples_h, int64_t n, int epochs, int batch, f
 double Mlp::time_ms(int which, int rows, int reps) {
     PA_CHECK(reps > 0 && reps <= 100000 && (which == 0 || which == 1), PA_ERR_INVALID, "mlp: bad timing request");
     rows = pad_rows(rows);
-    ensure(rows);
+    if (which == 0) outputs(rows);
+    else ensure(rows);
     // a fixed synthetic batch: zero features and targets (timing only)
     samples.reserve((size_t)rows * (IN + OUT));
     PA_HIP(hipMemsetAsync(samples.p, 0, sizeof(float) * (size_t)rows * (IN + OUT), stream));

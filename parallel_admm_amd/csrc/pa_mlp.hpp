@@ -38,10 +38,10 @@ struct Mlp {
     DBuf<float> w, adam_m, adam_v;
     int adam_t = 0;
     DBuf<uint16_t> W1p, W2, W2T, W3, W3T, W4p, W4T;
-    // what a pass over up to `cap` rows (padded to a multiple of 32) leaves in memory
+    // what a training pass over up to `cap` rows (padded to a multiple of 32) leaves in memory
     int cap = 0;
     DBuf<uint16_t> XT, H1T, H2T, H3T, dYT, dA1T, dA2T, dA3T; // transposed, for the weight gradients
-    DBuf<float> Y;
+    DBuf<float> Y; // outputs of a pass, all that inference needs
     DBuf<float> part;        // split-K partial weight gradients
     DBuf<double> loss_part;  // per 16 rows (train_host: of an epoch)
     DBuf<float> grad;        // flat gradient (gradient-only mode)
@@ -59,7 +59,11 @@ struct Mlp {
     void init_params(uint64_t seed);
     void set_params(const float* host);
     void get_params(float* host);
+    // Buffers of a training pass over `rows` rows (outputs among them).
     void ensure(int rows);
+    // Y for at least `rows` rows, grown by half so that a step whose contacts
+    // grow slowly does not reallocate at every detection.
+    float* outputs(int rows);
 
     // Forward over `rows` padded rows, the first n from src (`stride` floats
     // apart), into y [rows][2].

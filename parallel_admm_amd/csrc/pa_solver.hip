@@ -3788,8 +3788,7 @@ void Backend::ws_window_begin() {
         if (ws_active) {
             if (use_mlp) {
                 const int rows = Mlp::pad_rows(nc);
-                ws_mlp->ensure(rows);
-                ws_mlp->infer(ws_norm.p, 10, nc, rows, ws_mlp->Y.p);
+                ws_mlp->infer(ws_norm.p, 10, nc, rows, ws_mlp->outputs(rows));
             }
             hipLaunchKernelGGL(k_ws_seed, dim3(grid_for(nc, BLK)), dim3(BLK), 0, stream, nc, ws.mode, (float)(cfg.thickness / cfg.dt),
                                (float)ws.clamp, use_mlp ? (const float*)ws_mlp->Y.p : nullptr, (const float*)ws_consts.p,

@@ -57,6 +57,16 @@ def network(pa, fake):
         _fails_everywhere(pa, fake, pa.MLP, call)
 
 
+def inference(pa, fake):
+    """Inference holds its input and output rows (48 bytes each), none of the
+    training buffers."""
+    m, before = pa.MLP(), fake.fake_live()
+    m.forward(np.zeros((4096, pa.MLP_FEATURES), np.float32))
+    assert fake.fake_live() - before <= 4096 * 48 and fake.fake_launches(b"k_ones_rows") == 0
+    m.forward(np.zeros((4097, pa.MLP_FEATURES), np.float32))
+    assert fake.fake_live() - before <= 4097 * 48 + 4096 * 4  # the output grows by half
+
+
 def detection(pa, fake):
     for side in (9, 90):  # leaves sorted in one workgroup, and by the radix sort with its scratch
         x = _detector(pa, side)[1]
@@ -146,6 +156,10 @@ def early_detector(pa, fake):
 @pytest.mark.parametrize("case", ["network", "detection", "single_pass", "segments", "contact_log"])
 def test_failed_allocation(fake_hip, case):
     _run(fake_hip, case)
+
+
+def test_inference_memory(fake_hip):
+    _run(fake_hip, "inference")
 
 
 def test_detector_attached_before_init(fake_hip):
