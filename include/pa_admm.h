@@ -430,12 +430,12 @@ pa_status pa_mlp_forward(pa_mlp* m, const float* x, int32_t n, float* y);
  * memory.  No counterpart in the reference; it is for callers that cannot
  * allocate (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  Input and output are staged in one file-scope device array
- * per GPU of PA_MLP_NOALLOC_SCRATCH_BYTES (about 15 MB, held until the process
+ * per GPU of PA_MLP_NOALLOC_SCRATCH_BYTES (0.8 MB, held until the process
  * ends); n is at most PA_MLP_NOALLOC_MAX_ROWS per call (more is refused with
  * PA_ERR_INVALID).  Calls that overlap on one GPU share that array and race:
  * serialise them. */
 #define PA_MLP_NOALLOC_MAX_ROWS 16384
-#define PA_MLP_NOALLOC_SCRATCH_BYTES 14942208
+#define PA_MLP_NOALLOC_SCRATCH_BYTES 786432
 pa_status pa_mlp_forward_noalloc(pa_mlp* m, const float* x, int32_t n, float* y);
 /* Gradient of L = 1/(2n) sum |MLP(x) - t|^2 (t[n][2]) in the flat layout; *loss = L. */
 pa_status pa_mlp_gradients(pa_mlp* m, const float* x, const float* t, int32_t n, float* grad, double* loss);

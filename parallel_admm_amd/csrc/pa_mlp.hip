@@ -357,7 +357,7 @@ __global__ void k_ones_rows(int cap, uint16_t* __restrict__ a, uint16_t* __restr
 // GPUs use each GPU's own copy.
 // ---------------------------------------------------------------------------
 constexpr size_t kSy = (size_t)kNoAllocRows * IN * sizeof(float);
-static_assert(kSy % 256 == 0 && kSy + (size_t)kNoAllocRows * OUT * sizeof(float) <= kNoAllocScratchBytes, "scratch too small");
+static_assert(kSy % 256 == 0 && kSy + (size_t)kNoAllocRows * OUT * sizeof(float) == kNoAllocScratchBytes, "scratch layout and size differ");
 
 __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 

@@ -25,9 +25,9 @@ constexpr int OUTK = 32;  // padded output-gradient width (MFMA K)
 constexpr int OW1 = 0, OB1 = OW1 + H * IN, OW2 = OB1 + H, OB2 = OW2 + H * H, OW3 = OB2 + H, OB3 = OW3 + H * H,
               OW4 = OB3 + H, OB4 = OW4 + OUT * H, NPARAM = OB4 + OUT;
 // Allocation-free forward: at most this many rows per call, with a device
-// scratch array of kNoAllocScratchBytes per GPU (14,942,208 bytes).
+// scratch array of kNoAllocScratchBytes per GPU (their inputs and outputs).
 constexpr int kNoAllocRows = 16384;
-constexpr size_t kNoAllocScratchBytes = 14942208;
+constexpr size_t kNoAllocScratchBytes = kNoAllocRows * (IN + OUT) * sizeof(float);
 } // namespace mlp
 
 struct Mlp {

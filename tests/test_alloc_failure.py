@@ -67,6 +67,12 @@ def inference(pa, fake):
     assert fake.fake_live() - before <= 4097 * 48 + 4096 * 4  # the output grows by half
 
 
+def noalloc_scratch(pa, fake):
+    """The allocation-free forward's device array holds its input and output rows
+    (48 bytes each) and nothing else."""
+    assert fake.fake_var_bytes(b"scratch") == pa.MLP_NOALLOC_MAX_ROWS * 48
+
+
 def detection(pa, fake):
     for side in (9, 90):  # leaves sorted in one workgroup, and by the radix sort with its scratch
         x = _detector(pa, side)[1]
@@ -158,8 +164,9 @@ def test_failed_allocation(fake_hip, case):
     _run(fake_hip, case)
 
 
-def test_inference_memory(fake_hip):
-    _run(fake_hip, "inference")
+@pytest.mark.parametrize("case", ["inference", "noalloc_scratch"])
+def test_inference_memory(fake_hip, case):
+    _run(fake_hip, case)
 
 
 def test_detector_attached_before_init(fake_hip):
@@ -181,4 +188,5 @@ if __name__ == "__main__":
     sys.path.insert(0, ROOT)
     import parallel_admm_amd as _pa
 
+    _pa.lib()
     globals()[sys.argv[2]](_pa, _fake)
