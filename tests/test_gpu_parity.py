@@ -1088,6 +1088,26 @@ def test_overflowing_detection_falls_back_inside_a_step(pa):
         np.testing.assert_array_equal(a, c)
 
 
+def test_overflowing_detection_of_many_waves(pa):
+    """Eight sheets of 3,600 vertices: some waves of the collect pass fill the
+    overflow list, the others stop where they meet it full.  The list is the
+    forced single pass's, and the detector's next detection, of the sheets moved
+    apart, is a fresh one's."""
+    d = 1e-3
+    x, sc = _stacked_sheets(pa, 8, 60, 0.01, 0.1 * d)
+    apart = x * [1, 20, 1]
+    apart[:3600, 1] = apart[3600, 1] + 0.5 * d  # two sheets stay close
+    dets = [pa.CollisionDetector.for_scene(sc, 1 << 21, d) for _ in range(2)]
+    dets[1].set_single_pass(True)
+    for pos in (x, apart, x):
+        n = [det.detect(pos) for det in dets]
+        lists = [det.contacts() for det in dets]
+        print(f"{n} contacts")
+        assert n[0] == n[1] > 0
+        np.testing.assert_array_equal(lists[0][0], lists[1][0])
+        np.testing.assert_array_equal(lists[0][1], lists[1][1])
+
+
 def test_single_pass_step_matches_two_pass_step(pa):
     """A step whose detections run the single pass (which also counts and places
     every vertex's contacts for the step) against one with the two passes, bit
