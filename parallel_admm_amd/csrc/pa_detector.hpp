@@ -75,7 +75,7 @@ struct Detector {
     DBuf<int32_t> cand_pt, cand_ee;
     DBuf<uint32_t> ccount_pt, ccount_ee;
     DBuf<int2> ovf_pt, ovf_ee;
-    int64_t single_pass_fallbacks = 0; // detections that reran as a single pass (short stack or overflow list too small)
+    int64_t single_pass_fallbacks = 0; // detections that reran as a single pass (shared stack or overflow list too small)
     bool force_single_pass = false;    // every detection runs the single pass
     PrimScratch scratch;
     // A large edge tree is sorted on a second stream, concurrently with the

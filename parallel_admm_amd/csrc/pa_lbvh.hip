@@ -156,8 +156,11 @@ __global__ void k_morton_seg(const float4* __restrict__ box, const int32_t* __re
 // registers, written back to LDS in their new order) and the leaf ids, with the
 // results of the kernels above and radix_sort_pairs.  Those take 17 launches
 // and about 110 us for a tree of 5000 primitives, little of it work; this takes
-// 34-47 us on one CU, and both trees run side by side (one detection of a
-// 33 x 33 cloth 399 -> 259 us).
+// 34-47 us on one CU, and both trees run side by side.  SMALL_BUILD is what LDS
+// holds, and it wins up to there: a detection of a cloth over its sphere takes
+// 0.12 ms with it against 0.20-0.23 with the launches at 2,625 edges, 0.16
+// against 0.21-0.24 at 6,800, 0.19 against 0.21-0.24 at 13,953 and 0.20-0.21
+// against 0.21-0.24 at 16,341 (ranges over two processes).
 constexpr int SMALL_BUILD = 16384, SB_BLK = 1024, SB_ITEMS = SMALL_BUILD / SB_BLK, SB_WAVES = SB_BLK / 64;
 struct SmallTree {
     const int32_t* prims;
@@ -386,17 +389,18 @@ __device__ inline void put_slot(float4* __restrict__ rec, int p, float4 lo, floa
 // of a power of two leaves (a union may count a leaf twice), read from a table
 // of all such windows that the block builds in LDS in log2(RB) steps: a node
 // costs two reads whatever its range.  Unions straight from the leaf boxes and
-// from 64- and 4096-leaf chunks in memory were a chain of up to 30 dependent
-// loads per node and three more launches: 33 + 4 + 4 us of the 256x256 cloth's
-// refit (28 us of FP64 leaf copies besides; the queries now take their vertices
-// from x), now 29 + 9; 350 + 60 + 222 us of a 160-scene batch's edges, now
-// 233 + 93.  Blocks of 128 and 64 leaves list two and four times the crossing
-// nodes and were slower in sum (19 + 12 and 17 + 21 us on the cloth's edges).
+// from chunks of them in memory are a chain of up to 30 dependent loads per node
+// (edges of a 160-scene batch: 632 us in three launches, against 233 for this
+// and 93 for k_cross_boxes).  Blocks of 128 and 64 leaves leave two and four
+// times the crossing nodes and were slower in sum (edges of the 256x256 cloth:
+// 19 + 12 and 17 + 21 us, 16 + 9 with 256).  Both trees of that cloth: 20 + 15
+// us; 512 scenes: 679 + 287 us, where the 55 KB of LDS that leave a CU two
+// blocks bound it.
 //
 // Both trees share a launch here and in the kernels below: first the blocks of
-// the edge tree, the longer chain, then those of the triangle tree.  On two
-// streams their eight launches and four event calls left a small scene's host
-// behind its GPU, and a large scene's launches fill the chip by themselves.
+// the edge tree, the longer chain, then those of the triangle tree.  Two
+// streams cost a small scene's host more than its GPU gains, and a large
+// scene's launches fill the chip by themselves.
 constexpr int RB = 256, RB_LEVELS = 9;
 struct TreeArgs {
     int n; // leaves
@@ -477,9 +481,10 @@ __global__ void __launch_bounds__(RB) k_refit(TreeArgs E, TreeArgs F, int e_bloc
 // `per` nodes and works on its few crossing ones (most have none) with all
 // lanes, one after the other: 16 nodes up to CROSS_SMALL leaves, where the
 // longest wave is the launch (6.2 us against 8.3 with 64 on 3000 leaves), 64
-// above (14 us against 18 on 330,000, 110 against 148 on 2.5 million).  A list of the crossing nodes, made once per build, spread
-// them evenly but cost more than it gave: appending to it took 10-20 ns per
-// wave on one counter (37 us of the 256x256 cloth's build, 440 of a batch's).
+// above (14 us against 18 on 330,000, 110 against 148 on 2.5 million).  A list of
+// the crossing nodes, made once per build, spreads them evenly but costs more
+// than it gives: appending to it takes 10-20 ns per wave on one counter (37 us
+// of the 256x256 cloth's build, 440 of a batch's).
 constexpr int CROSS_SMALL = 1 << 16;
 __global__ void __launch_bounds__(BLK) k_cross_boxes(TreeArgs E, TreeArgs F, int e_blocks, int per) {
     const bool edges = (int)blockIdx.x < e_blocks;
@@ -699,13 +704,13 @@ __device__ inline void traverse(const float4* __restrict__ rec, int start, int l
 // A step pops up to 16 pairs, four lanes each: every lane tests one child slot
 // of its node against its query's box; children that pass go back on the stack
 // and leaves to the wave's hit buffer, both packed by ballots.  With one lane
-// per query and a stack each, a launch took as long as its longest chain of
-// dependent loads (40 visits of 0.9 us on a 16 x 16 cloth, 130 at the fold of a
-// 256 x 256 one), the lanes that were done idled, and a visit read its 128-byte
-// record in eight 16-byte pieces per lane.  Here a wave's lanes are busy until
-// its last query is done, four of them read a record together, and a query's
-// nodes are visited many at a time.  Few queries give few waves, so QW falls
-// with their number (collect_qw) until a wave has four.
+// per query and a stack each (the single pass), a launch takes as long as its
+// longest chain of dependent loads (40 visits of 0.9 us on a 16 x 16 cloth, 130
+// at the fold of a 256 x 256 one), the lanes that are done idle, and a visit
+// reads its 128-byte record in eight 16-byte pieces per lane.  Here a wave's
+// lanes are busy until its last query is done, four of them read a record
+// together, and a query's nodes are visited many at a time.  Few queries give
+// few waves, so QW falls with their number (collect_qw) until a wave has four.
 // Hits are filtered 64 at a time by their vertex ids (pairs that share a vertex
 // or are both static, most of the hits in a cloth at rest) before they go to
 // the query's slab (the first CAND, strided by the query count:
@@ -723,10 +728,12 @@ __device__ inline void traverse(const float4* __restrict__ rec, int start, int l
 // (8 sheets of 120 x 120 vertices within the contact distance, 5 million
 // contacts: 19.1 ms a detection that way, 9.5 with the stop).
 //
-// 256 x 256 cloth: EE collect 82 -> 44 us, test 42 -> 12, PT collect 46 -> 24,
-// test 13 -> 5; 16 x 16 cloth: collects 38 -> 9.4 and 28 -> 9.0 us; 160-scene
-// batch (1.5 million edges): EE collect 505 -> 530, test 340 -> 68, PT collect
-// 230 -> 267, test 390 -> 73.
+// Both kinds in one launch, 256 x 256 cloth: collect 72 us, test 12; by a lane
+// per query the two collects took 82 and 46 us. 512 scenes: 1417 and 281 us. On
+// a 16 x 16 cloth the collects of the two kinds took 9.4 and 9.0 us in launches
+// of their own, by a lane per query 38 and 28.  A batch's collect gains nothing
+// (160 scenes 530 + 267 us, by a lane per query 505 + 230): its instructions and
+// loads bound it, not its chains.
 struct ListOut {
     int32_t* cand;
     uint32_t* ccount;
@@ -997,8 +1004,8 @@ __device__ inline int ovf_entries(const ListOut& l, int nq) { return (int)min(*l
 
 // Accepted entries keep a mark in the leaf index's sign bit, and their segment
 // counts them; nothing is appended to a common list: one counter that every
-// wave with a contact adds to took 10 to 20 ns a wave, 330 us of a 160-scene
-// batch's two test launches.
+// wave with a contact adds to costs 10 to 20 ns a wave (the two kinds of test of
+// a 160-scene batch 322 and 329 us with it, 68 and 73 without).
 constexpr int ACCEPTED = (int)0x80000000;
 
 template <class QK>
@@ -1033,9 +1040,10 @@ __global__ void __launch_bounds__(TBLK) k_test(EEQuery EE, ListOut el, int e_blo
 // the partner ids into their segments (any order inside one).  PASS 1: every
 // pair counts the smaller ids of its segment (a pair occurs once, so they are
 // distinct), evaluates its contact and writes it to its final place.  The
-// counts are independent loads over one lane per contact; an insertion sort by
-// one lane per segment moved each 68-byte record several times in a dependent
-// chain (13-30 us per detection for segments of 10 to 30).
+// counts are independent loads over one lane per contact, where an insertion
+// sort by one lane per segment moves each 68-byte record several times in a
+// dependent chain (13-30 us per detection for segments of 10 to 30, and 1.2 ms
+// for those of 8 sheets of 60 x 60 vertices, whose pairs this places in 0.25).
 struct PlaceArgs {
     const uint32_t* qoffset;
     const uint32_t* qcount;
@@ -1395,8 +1403,8 @@ int Detector::detect(const double* x, bool refit, VertexCount vc) {
     }
     const bool single = !two || h[1] != 0;
     if (single) {
-        // the short stack or an overflow list was too small: the single pass
-        // (traversal and test together, full stack) for both queries
+        // a wave's shared stack or an overflow list was too small: the single pass
+        // (traversal and test by one lane per query) for both queries
         fill<uint32_t>(counts.p, 0u, (int64_t)counts.n, stream);
         if (ne > 0) single_pass(EE, ACCEPTED, et);
         if (nv > 0) single_pass(PT, 0, ft);

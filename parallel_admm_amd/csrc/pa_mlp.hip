@@ -211,9 +211,9 @@ template <bool TRAIN> __global__ void __launch_bounds__(256) k_mlp(MlpArgs g) {
 
 // Every weight gradient in one launch: split-K partials of dA^T H, one 16x16
 // tile and split per wave.  A layer's tiles start at first[l]; a wave's
-// fragments of eight K steps are in flight at once (as four launches of one
-// step at a time they took 33 us, now 14.2).  Workgroups of a split share an XCD, so
-// an L2 reads one eighth of the 7 MB that k_mlp left, mostly rows written there.
+// fragments of eight K steps are in flight at once (14.2 us at 8192 rows; four
+// launches with one step at a time 33).  Workgroups of a split share an XCD, so an
+// L2 reads one eighth of the 7 MB that k_mlp left, mostly rows written there.
 struct GradArgs {
     const uint16_t* A[4];
     const uint16_t* Bt[4];

@@ -9,7 +9,7 @@ namespace {
 // tile adds up the sums before it (a few thousand values at most here, read by
 // 1024 lanes) and scans itself.  Launches bound these scans, not bytes: the
 // scans here are over 1e3 to 1e6 counts, and a launch costs 2-3 us and its
-// dependent dispatch as much again; the recursive tile scan took up to five.
+// dependent dispatch as much again; a recursive tile scan takes up to five.
 constexpr int SCAN_BLOCK = 1024;
 constexpr int SCAN_TILE = 4 * SCAN_BLOCK;
 constexpr int SCAN_ONE = 16 * SCAN_BLOCK;
@@ -124,8 +124,8 @@ __global__ void __launch_bounds__(RS_BLOCK) k_rs_hist(const uint32_t* __restrict
 // Stable scatter of one tile.  Wave w takes the tile's w-th quarter in rounds of
 // 64, so a wave ranks its elements by itself: 8 ballots find the lanes with the
 // same digit, and a digit count per wave in LDS carries over the rounds.  Only
-// then do the waves add up their counts: two barriers a tile (with all waves on
-// each round and a barrier between, 24, a tile took 8-15 us, now 5-6).
+// then do the waves add up their counts: two barriers and 5-6 us a tile (with
+// all waves on each round and a barrier between, 24 barriers and 8-15 us).
 __global__ void __launch_bounds__(RS_BLOCK) k_rs_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
                                                         uint32_t* __restrict__ kout, uint32_t* __restrict__ vout, int64_t n,
                                                         int shift, const uint32_t* __restrict__ offs, int ntiles) {

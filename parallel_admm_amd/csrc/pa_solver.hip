@@ -507,10 +507,10 @@ __global__ void k_contact_fill(int nc, int n, float eps, float gam, float hinv, 
 // number of smaller entries in its run.  vent gets the sorted entries, slot[c].k
 // the place of (contact c, vertex k), -1 for static vertices, and erun[e]
 // (vertex, end of its entries) on a vertex's first entry, (-1, 0) on the
-// others.  Counting reads a run eight entries at a time; the insertion sort by
-// one lane per vertex that stood here was a chain of dependent loads and
-// stores over runs of 10 to 40 entries, 32-85 us per detection on single
-// scenes.
+// others.  Counting reads a run eight entries at a time (3.9 us at 256x256
+// vertices); an insertion sort by one lane per vertex is a chain of dependent
+// loads and stores over runs of 10 to 40 entries, 32-85 us per detection on
+// single scenes.
 __global__ void k_contact_rank(int nc, int n, const int4* __restrict__ cv, const uint32_t* __restrict__ vptr,
                                const uint32_t* __restrict__ vraw, uint32_t* __restrict__ vent, int32_t* __restrict__ slot,
                                int2* __restrict__ erun) {
@@ -539,7 +539,7 @@ __global__ void k_contact_rank(int nc, int n, const int4* __restrict__ cv, const
 // p += Gamma r_c on the vertices with contacts (p holds (x - x0 + Uc) / h from
 // k_begin_step or k_dual_vert), one lane per entry of the sorted list: the lane
 // of a vertex's first entry sums its run in contact order, eight entries read
-// at a time (160 merged cloths: 38 -> 11.5 us against four).
+// at a time (160 merged cloths: 11.5 us, with four at a time 38).
 __global__ void k_vertex_p(int ne_max, int n, float* __restrict__ p, const uint32_t* __restrict__ vptr, const int2* __restrict__ erun,
                            const uint32_t* __restrict__ vent, const float4* __restrict__ G, const float4* __restrict__ rc) {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
@@ -619,9 +619,9 @@ __global__ void k_contact_du(int nc, const int4* __restrict__ cv, const float4* 
 // p_v += sum of the Gamma du entries of v (contact order), one lane per
 // entry of the sorted list: the lane of a vertex's first entry sums its run,
 // the others exit.  A run's entries are read eight at a time before they are
-// added (one at a time the longest run, 30 and more entries, set the kernel's
-// time: 9.9 us, now 7.4, on a 256x256 cloth with a folded flap, 9.6, now 6.0, on
-// 160 merged cloths).  Lanes past the entry count read stale (allocated) run
+// added; one at a time the longest run, 30 and more entries, sets the kernel's
+// time (9.9 us against 7.4 on a 256x256 cloth with a folded flap, 9.6 against
+// 6.0 on 160 merged cloths).  Lanes past the entry count read stale (allocated) run
 // markers beside the count and drop them.
 __global__ void k_vertex_gather(int ne_max, int n, float* __restrict__ p, const uint32_t* __restrict__ vptr,
                                 const int2* __restrict__ erun, const float4* __restrict__ gdu) {
@@ -662,10 +662,10 @@ __global__ void k_vertex_gather(int ne_max, int n, float* __restrict__ p, const 
 // - buf holds one float4 per entry (Gamma_k du), then the p of each run.  Runs
 //   that no longer fit behind the entries (only possible with over 1024
 //   contacts, most of whose vertices are distinct) keep p in global memory.
-// Ten sweeps (gs_max_iter 10), everything through L2 before: a side-16 cloth
-// draped over its sphere 36.6 -> 17.1 us, cloth256 landing (about 600
-// contacts) 38-48 -> 27.8 us, a side-95 cloth 47 -> 24 us (up to 1024
-// contacts) and 68 -> 36 us (above).
+// Ten sweeps (gs_max_iter 10), against everything through L2: a side-16 cloth
+// draped over its sphere 17.1 us (36.6), cloth256 landing (about 600
+// contacts) 27.8 (38-48), a side-95 cloth 24 (47) with up to 1024 contacts
+// and 36 (68) above, where two contacts per lane spill 18 registers.
 constexpr int CONTACT_WG_SLOTS = 10000;
 template <int NPT>
 __global__ void __launch_bounds__(1024) k_contact_sweeps_wg(int nc, int n, int sweeps, const int4* __restrict__ cv,
@@ -1888,8 +1888,9 @@ __global__ void __launch_bounds__(BLK) k_amg_coarse(int nc, int ncp, const float
 // in one descriptor, and where a row of F comes from is a table, so the chain
 // is descriptor -> (panel, table, r) -> children's u -> product.
 //
-// At 256x256 vertices (7 levels and the top): up 4 x 13.3 + 3 x 11.0 ->
-// 7 x 7.5 us, down 4 x (7.4 + 4.3) + 3 x 9.5 -> 6 x 5.0 + 7.4 us.
+// At 256x256 vertices (6 levels and the top): up 6 x 5.5-6.1 us, down 5 x
+// 4.5-4.8 and the leaves 10.1 us.  With L11^-1 and L21, over the 7 levels of
+// smaller leaves: up 4 x 13.3 + 3 x 11.0, down 4 x (7.4 + 4.3) + 3 x 9.5 us.
 // ---------------------------------------------------------------------------
 struct CholTile {
     int64_t panel;     // the supernode's [D; -W] in the panel array
@@ -1902,9 +1903,12 @@ struct CholTile {
 constexpr int CHOL_BLK = 256;
 // Dissection leaves hold up to 160 unknowns in systems of up to this many, 64
 // above.  Larger leaves save a level, two launches of about 6 us, and cost
-// host set-up (about 25,000 more flops per unknown): 256x256 cloth step
-// 12.5 -> 12.1 ms, tet box 4.31 -> 3.84, side-95 cloth 4.03 -> 3.67, but a
-// 160-scene batch of 500,000 unknowns, whose levels are wide, 36.9 -> 36.3.
+// host set-up (about 25,000 more flops per unknown).  Step with 160 against 64:
+// side-95 cloth 3.67 against 4.03 ms, tet box 3.84 / 4.31, 256x256 cloth 12.1 /
+// 12.5, 362x362 (131,044 unknowns) 7.1 / 7.2; above the line 420x420 9.4 / 9.4,
+// batches of 157,000 unknowns 6.6 / 7.1, of 304,000 11.2 / 11.7, of 500,000
+// 36.3 / 36.9.  Set-up is 2 to 5% longer throughout.  So the line gives up 0 to
+// 6% of a large system's step for 0.1 to 0.2 s of its set-up.
 constexpr int CHOL_BIG_LEAF_N = 1 << 17;
 constexpr int CHOL_INFLIGHT = 8; // float4 panel loads in flight per lane
 
@@ -2053,7 +2057,7 @@ __global__ void __launch_bounds__(CHOL_BLK) k_chol_down(const CholTile* __restri
 // padded to whole float4s), all in flight before f arrives in LDS; the lanes'
 // sums combine with shuffles.  NV follows the largest top, so a small one does
 // not step over the loads of a large one.  256x256 vertices (3036 columns,
-// 37 MB): 13.2 us against 15.5 with scalar loads and lane 0 adding 64 sums from
+// 37 MB): 11.9 us against 15.5 with scalar loads and lane 0 adding 64 sums from
 // LDS; a 256-column top 3.5 against 8.0.
 constexpr int CHOL_TOP_ROWS = 4;   // rows of S^-1 per workgroup (one per wave)
 constexpr int CHOL_TOP_BLK = 256;
