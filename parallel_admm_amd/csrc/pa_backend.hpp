@@ -233,6 +233,7 @@ struct Backend {
     int64_t spmv_launches = 0;
     std::vector<std::pair<hipEvent_t, hipEvent_t>> spmv_marks;
 
+    Backend() = default; // no device work; the constructor below delegates: one that fails half-way is destroyed
     explicit Backend(const pa_device_opts* o);
     ~Backend();
 

@@ -111,6 +111,7 @@ struct Detector {
     void set_stream(hipStream_t s) { stream = s; }
 
   private:
+    Detector() = default; // the public constructor delegates: one that fails half-way is destroyed
     void sort_leaves(Tree& T, const double* x, bool faces, hipStream_t s, PrimScratch& scr);
     void build_topology();
     void segment_roots(Tree& T);

@@ -1155,7 +1155,14 @@ __global__ void __launch_bounds__(TBLK) k_place_single(PTQuery PT, EEQuery EE, c
 
 Detector::Detector(int n_all_, int n_dyn_, int nv_, const int32_t* sv, int nf_, const int32_t* t, int ne_, const int32_t* e,
                    int cap, double dhat_, hipStream_t s)
-    : stream(s), n_all(n_all_), n_dyn(n_dyn_), nv(nv_), nf(nf_), ne(ne_), dhat(dhat_) {
+    : Detector() {
+    stream = s;
+    n_all = n_all_;
+    n_dyn = n_dyn_;
+    nv = nv_;
+    nf = nf_;
+    ne = ne_;
+    dhat = dhat_;
     PA_CHECK(cap > 0, PA_ERR_INVALID, "detector capacity must be positive");
     PA_CHECK(dhat > 0, PA_ERR_INVALID, "thickness must be positive");
     if (!stream) {

@@ -383,7 +383,7 @@ void* scratch_address() {
 
 } // namespace
 
-Mlp::Mlp(hipStream_t s) {
+Mlp::Mlp(hipStream_t s) : Mlp(Empty{}) {
     if (s) {
         stream = s;
     } else {

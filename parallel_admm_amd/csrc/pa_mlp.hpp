@@ -49,7 +49,8 @@ struct Mlp {
     DBuf<int32_t> perm;      // sample order of the current epoch
     int splits = 1;
 
-    explicit Mlp(hipStream_t s = nullptr);
+    Mlp() : Mlp(nullptr) {}
+    explicit Mlp(hipStream_t s);
     ~Mlp();
     Mlp(const Mlp&) = delete;
     Mlp& operator=(const Mlp&) = delete;
@@ -86,6 +87,10 @@ struct Mlp {
     // of one batch of `rows` rows, over `reps` back-to-back repetitions.  The
     // weights are kept; the Adam state is reset.
     double time_ms(int which, int rows, int reps);
+
+  private:
+    struct Empty {};
+    explicit Mlp(Empty) {} // the public constructors delegate: one that fails half-way is destroyed
 };
 
 } // namespace pa

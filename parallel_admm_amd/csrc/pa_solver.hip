@@ -2176,7 +2176,7 @@ __global__ void k_animate_points(int first, int count, const double* __restrict_
 // ===========================================================================
 // Host side
 // ===========================================================================
-Backend::Backend(const pa_device_opts* o) {
+Backend::Backend(const pa_device_opts* o) : Backend() {
     device = o ? o->device : 0;
     verbose = o ? o->verbose : 0;
     int count = 0;

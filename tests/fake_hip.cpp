@@ -19,6 +19,7 @@ std::map<std::string, size_t> var_bytes;
 std::map<const void*, void*> var_mem;
 long allocs = 0, fail_at = 0;
 size_t live = 0;
+long handles = 0; // streams, events and pinned allocations that are alive
 uint32_t* last_pinned = nullptr;
 char token; // handles: any address that is not null
 struct Dim3 {
@@ -33,6 +34,7 @@ void fake_fail_at(long nth) { // the nth allocation from now fails (0: none)
 }
 long fake_allocs() { return allocs; }
 size_t fake_live() { return live; }
+long fake_handles() { return handles; }
 long fake_launches(const char* part) { // of the kernels whose mangled name holds `part`
     long n = 0;
     for (auto& l : launches)
@@ -67,9 +69,11 @@ int hipFree(void* p) {
 int hipHostMalloc(void** p, size_t bytes, unsigned) {
     *p = std::calloc(bytes, 1);
     last_pinned = static_cast<uint32_t*>(*p);
+    handles++;
     return *p ? OK : OUT_OF_MEMORY;
 }
 int hipHostFree(void* p) {
+    handles--;
     std::free(p);
     return OK;
 }
@@ -133,9 +137,13 @@ int hipGetLastError() { return OK; }
 const char* hipGetErrorString(int) { return "fake HIP error"; }
 int hipStreamCreateWithFlags(void** s, unsigned) {
     *s = &token;
+    handles++;
     return OK;
 }
-int hipStreamDestroy(void*) { return OK; }
+int hipStreamDestroy(void*) {
+    handles--;
+    return OK;
+}
 int hipStreamSynchronize(void*) { return OK; }
 int hipStreamWaitEvent(void*, void*, unsigned) { return OK; }
 int hipStreamBeginCapture(void*, int) { return OK; }
@@ -145,10 +153,14 @@ int hipStreamEndCapture(void*, void** g) {
 }
 int hipEventCreate(void** e) {
     *e = &token;
+    handles++;
     return OK;
 }
 int hipEventCreateWithFlags(void** e, unsigned) { return hipEventCreate(e); }
-int hipEventDestroy(void*) { return OK; }
+int hipEventDestroy(void*) {
+    handles--;
+    return OK;
+}
 int hipEventRecord(void*, void*) { return OK; }
 int hipEventSynchronize(void*) { return OK; }
 int hipEventElapsedTime(float* ms, void*, void*) {

@@ -134,6 +134,29 @@ def contact_log(pa, fake):
     assert fake.fake_launches(b"k_ws_log") == logged
 
 
+def creation(pa, fake):
+    """A handle whose creation fails leaves nothing behind: no memory, stream,
+    event or pinned slot."""
+    from parallel_admm_amd.configs import config_for
+
+    sc = pa.Scene.generate(4, side=9, radius=0.1)
+    for make in (pa.MLP, lambda: _detector(pa, 9)[0], lambda: pa.ADMMBackendHIP.from_scene(sc, config_for("batch"))):
+        before = fake.fake_live(), fake.fake_handles()
+        first = fake.fake_allocs()
+        make()
+        count = fake.fake_allocs() - first
+        assert (fake.fake_live(), fake.fake_handles()) == before and count > 0
+        for k in range(1, count + 1):
+            fake.fake_fail_at(k)
+            try:
+                make()
+                raise AssertionError("no error")
+            except pa.PAError as e:
+                assert e.code == pa.PA_ERR_HIP
+            fake.fake_fail_at(0)
+            assert (fake.fake_live(), fake.fake_handles()) == before, f"allocation {k} of {count}"
+
+
 def early_detector(pa, fake):
     """A detector attached before apply_config and init, when the backend's sizes
     are not known yet, is refused by init if it does not fit them: its contacts
@@ -159,7 +182,7 @@ def early_detector(pa, fake):
             assert not fits and e.code == pa.PA_ERR_INVALID
 
 
-@pytest.mark.parametrize("case", ["network", "detection", "single_pass", "segments", "contact_log"])
+@pytest.mark.parametrize("case", ["network", "detection", "single_pass", "segments", "contact_log", "creation"])
 def test_failed_allocation(fake_hip, case):
     _run(fake_hip, case)
 
@@ -182,7 +205,7 @@ if __name__ == "__main__":
     _fake = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
     for _name in ("fake_live", "fake_var_bytes"):
         getattr(_fake, _name).restype = C.c_size_t
-    for _name in ("fake_allocs", "fake_launches"):
+    for _name in ("fake_allocs", "fake_launches", "fake_handles"):
         getattr(_fake, _name).restype = C.c_long
     _fake.fake_last_pinned.restype = C.POINTER(C.c_uint32)
     sys.path.insert(0, ROOT)
