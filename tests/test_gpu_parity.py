@@ -95,7 +95,7 @@ def test_detector_orders_long_segments(pa, faces):
     _check_contacts_equal(gi, gr, oi, orr)
 
 
-@pytest.mark.parametrize("side", [2, 3, 9, 60, 110, 180])
+@pytest.mark.parametrize("side", [2, 3, 9, 60, 110, 140, 180])
 def test_query_passes_agree_over_sizes(pa, side):
     """The two-pass queries against the single pass, bit for bit, on folded
     cloths from one cell up to 97,000 edges: below and above a refit block, and
